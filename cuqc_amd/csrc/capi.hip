@@ -230,7 +230,7 @@ int finish_result(EnumOut& eo, const Instance& I, qc_result* r, double t0, doubl
         r->st.t_nonmax_ms = eo.nonmax_ms;
     } else {
         const double tn = now_ms();
-        if ((rc = remove_nonmax_device(r->raw_off, r->raw_v, r->max_off, r->max_v, s))) return rc;
+        if ((rc = remove_nonmax_device(r->raw_off, r->raw_v, r->max_off, r->max_v, s, true))) return rc;
         r->st.t_nonmax_ms = now_ms() - tn;
     }
     r->st.max_cliques = r->max_off.size() - 1;

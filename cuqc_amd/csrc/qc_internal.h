@@ -237,8 +237,10 @@ int remove_nonmax_sets(const NmInput& in, int n_inst, std::vector<std::vector<ui
 // vertex-slot order, on the host
 int collect_raw(const CliqueRef* d_refs, const uint32_t* d_verts, uint64_t k, uint64_t nv, std::vector<uint64_t>& off,
                 std::vector<uint32_t>& v, hipStream_t s);
-// host raw sets (uploaded once)
+// host raw sets (uploaded once); distinct: no set names a vertex twice (a
+// search's own raw sets), so the cover filter may be used: its masks test
+// subsets of vertices, while a caller's sets are compared as multisets
 int remove_nonmax_device(const std::vector<uint64_t>& off, const std::vector<uint32_t>& v, std::vector<uint64_t>& mo,
-                         std::vector<uint32_t>& mv, hipStream_t s);
+                         std::vector<uint32_t>& mv, hipStream_t s, bool distinct = false);
 
 }  // namespace qc
