@@ -246,6 +246,7 @@ struct Ctx {
     int shard;                        // this wave's ring shard (blockIdx % q_shards)
     TaskRef* ptopref;                 // LDS: a copy of stack entry ptopi (the last pushed), ~0u: none
     uint32_t ptopi;
+    unsigned long long* clq;          // LDS, lane 0: the wave's refs and slots of the clique stream (clq_reserve)
     uint32_t* fl;                     // LDS: free block indices of the small classes, FL_LOCAL_MAX per class
     uint32_t* fln;                    // LDS: their counts
     TaskRef* pstack;
@@ -548,7 +549,9 @@ __device__ bool lu_bounds(Ctx& c, int m, int nc, int& ub, int& lb, int& med, int
             lb = nc + 1;
             invalid = true;
         }
-        int tq = min_tot < c.g.ubq_n ? c.g.p->ubq[min_tot] : c.g.p->ubq[c.g.ubq_n - 1];
+        // (a stale exdeg can make the sum negative: floor(d / gamma) is then
+        // below 0 and the bound too)
+        int tq = min_tot < 0 ? -1 : c.g.p->ubq[min(min_tot, c.g.ubq_n - 1)];
         ub = tq + 1 - m;
         if (ub > nc) ub = nc;
         if (lb < ub) {
@@ -930,35 +933,83 @@ __device__ __attribute__((always_inline)) int critical_prep(Ctx& c, int tc, int&
 // ---------------------------------------------------------------------------
 // emission
 // ---------------------------------------------------------------------------
-__device__ void emit_clique(Ctx& c, const int* ids, int len) {
+// A place for one raw set of `len` vertices in the clique stream: the ref's
+// index and the first vertex slot.  The persistent form takes CLQ_REFS refs
+// and CLQ_SLOTS slots at a time for the wave (lane 0 keeps what is left in
+// c.clq: next ref, end, next slot, end), since two device-scope atomics on one
+// pair of counters for each of a million raw sets cost as much as the search;
+// refs it does not use are marked empty when the wave ends (clq_close).  Sets of
+// more than CLQ_SLOTS / 4 vertices take their slots directly, so less than a
+// quarter of a wave's slots are lost at the ends.
+__device__ __attribute__((always_inline)) bool clq_reserve(Ctx& c, int len, unsigned long long& ri, unsigned long long& si) {
     const ExpandArgs& a = *c.a;
-    unsigned long long ri = 0, si = 0;
     if (c.lane == 0) {
-        ri = atomicAdd(&a.clq_ctr->items, 1ull);
-        si = atomicAdd(&a.clq_ctr->slots, (unsigned long long)len);
+        if (a.queue_mode) {
+            ri = c.clq[0];
+            if (ri == c.clq[1]) {
+                ri = atomicAdd(&a.clq_ctr->items, (unsigned long long)CLQ_REFS);
+                c.clq[1] = ri + CLQ_REFS;
+            }
+            c.clq[0] = ri + 1;
+            if (len > CLQ_SLOTS / 4) {
+                si = atomicAdd(&a.clq_ctr->slots, (unsigned long long)len);
+            } else {
+                si = c.clq[2];
+                if (si + len > c.clq[3]) {
+                    si = atomicAdd(&a.clq_ctr->slots, (unsigned long long)CLQ_SLOTS);
+                    c.clq[3] = si + CLQ_SLOTS;
+                }
+                c.clq[2] = si + len;
+            }
+        } else {
+            ri = atomicAdd(&a.clq_ctr->items, 1ull);
+            si = atomicAdd(&a.clq_ctr->slots, (unsigned long long)len);
+        }
     }
     ri = rdlane64(ri, 0);
     si = rdlane64(si, 0);
     if (ri >= a.clq_ref_cap || si + len > a.clq_vert_cap) {
         if (c.lane == 0) atomicOr(a.error, 1);
-        return;
+        return false;
     }
-    for (int k = c.lane; k < len; k += WAVE) a.clq_verts[si + k] = c.g.p->orig[ids[k]];
+    return true;
+}
+__device__ __forceinline__ void clq_ref(Ctx& c, unsigned long long ri, unsigned long long si, int len) {
     if (c.lane == 0) {
         CliqueRef r;
         r.off = si;
         r.len = (uint32_t)len;
         r.inst = c.inst;
-        a.clq_refs[ri] = r;
-    }
-    if (c.lane == 0) {
+        c.a->clq_refs[ri] = r;
         c.st->raw++;
         c.st->sum_clq += len;
     }
 }
+__device__ __attribute__((always_inline)) void emit_clique(Ctx& c, const int* ids, int len) {
+    const ExpandArgs& a = *c.a;
+    unsigned long long ri = 0, si = 0;
+    if (!clq_reserve(c, len, ri, si)) return;
+    for (int k = c.lane; k < len; k += WAVE) a.clq_verts[si + k] = c.g.p->orig[ids[k]];
+    clq_ref(c, ri, si, len);
+}
+// the vertices of the lanes in m
+__device__ __forceinline__ void emit_lanes(Ctx& c, uint64_t m, uint32_t orig) {
+    const int len = __popcll(m);
+    unsigned long long ri = 0, si = 0;
+    if (!clq_reserve(c, len, ri, si)) return;
+    if ((m >> c.lane) & 1ull) c.a->clq_verts[si + lanes_below(m)] = orig;
+    clq_ref(c, ri, si, len);
+}
+// the wave's unused refs, marked empty
+__device__ __forceinline__ void clq_close(Ctx& c) {
+    const ExpandArgs& a = *c.a;
+    wsync();
+    const unsigned long long end = min<unsigned long long>(c.clq[1], a.clq_ref_cap);
+    for (unsigned long long i = c.clq[0] + c.lane; i < end; i += WAVE) a.clq_refs[i] = CliqueRef{0, 0, CLQ_NONE};
+}
 
 // clique test, main.cu:1974-1995
-__device__ void check_for_clique(Ctx& c, int m) {
+__device__ __attribute__((always_inline)) void check_for_clique(Ctx& c, int m) {
     int req = md(c, m);
     bool bad = false;
     for (int k = c.lane; k < m; k += WAVE)
@@ -1438,6 +1489,570 @@ __device__ __attribute__((always_inline)) void write_child(Ctx& c, int tc, int m
     if (c.lane == 0) {
         c.st->children++;
         c.st->sum_tw += tc;
+    }
+}
+
+// ---------------------------------------------------------------------------
+// subtrees of at most 64 vertices, in registers
+// ---------------------------------------------------------------------------
+// A task of at most 64 vertices and its whole subtree need no memory: lane l
+// holds one vertex (ascending id order) with its 64-bit rows of the 1-hop and
+// 2-hop relations among the task's vertices, every set is a 64-bit mask in
+// scalar registers, a degree is the popcount of row & set, and a child of the
+// task is one 32-bit word per lane.  The rows are gathered once, when the
+// subtree's root is loaded; below it a vertex keeps its lane, children wait on
+// a stack in the LDS (which no other task uses meanwhile), and records are
+// written only for tasks handed to other waves.  The steps are those of
+// process_task; lists become masks, so only the order of the branches (the
+// key below) is kept of the records' order.
+//
+// Bound by the issue of dependent vector and scalar instructions (one or two
+// waves a SIMD).  Through records and lists in LDS a task of this size took
+// 40 us on a wave (load and matrix gathers 18%, flat LDS accesses and their
+// waits most of the rest), here about 12 us; whole kernels are compared at the
+// dispatch in expand_persistent.
+constexpr uint32_t TINY_MAX = WAVE;
+constexpr int TINY_EX_MAX = 8000;  // largest exdeg the word holds (stale exdegs can pass the task's size)
+constexpr int TINY_EX_MIN = -64;   // smallest at load: a subtree lowers an exdeg by at most 63 more
+constexpr int TINY_BIAS = 128;
+constexpr uint32_t TINY_ENTRY = WAVE * 4;  // bytes of a stack entry
+
+// State word of a vertex: [12:0] exdeg + 128, [18:13] indeg, [24:19] order
+// (lvl2adj, or 63 - position for a task loaded from a record), [25] member,
+// [26] present; 0: not in the task.
+constexpr uint32_t TW_MEMBER = 1u << 25, TW_PRESENT = 1u << 26;
+__device__ __forceinline__ uint32_t tiny_word(int in, int ex, int ord, bool member) {
+    return (uint32_t)(ex + TINY_BIAS) | ((uint32_t)in << 13) | ((uint32_t)ord << 19) | (member ? TW_MEMBER : 0u) |
+           TW_PRESENT;
+}
+__device__ __forceinline__ int tw_ex(uint32_t w) { return (int)(w & 0x1FFFu) - TINY_BIAS; }
+__device__ __forceinline__ int tw_in(uint32_t w) { return (int)((w >> 13) & 63u); }
+// Q order of candidates (main.cu:2059-2104): indeg, exdeg, lvl2adj, id, all
+// descending; the lane is the rank by id, so keys are unique and the last
+// branch vertex is the smallest key's lane
+__device__ __forceinline__ int tiny_key(uint32_t w, int lane) {
+    return (int)((((w >> 13) & 63u) << 25) | ((w & 0x1FFFu) << 12) | (((w >> 19) & 63u) << 6) | (uint32_t)lane);
+}
+
+struct Tiny {
+    uint64_t r1, r2;      // rows among the basis (bit = lane)
+    int id;               // root-local id (ascending over the lanes)
+    uint32_t orig;        // input id
+    int d1, d2;           // |N n root|, |N2 n root|
+    int mdt;              // mindeg[lane]
+    uint32_t s;           // word of the task to run next
+    uint32_t hot;         // the child pushed last, not yet in the LDS
+    int fr, ff;           // lane k: removed vertex and smallest failing member of the k-th failed removal
+    int nf;
+    uint32_t depth, hot_depth;
+    bool hot_on;
+    uint32_t n, bot;      // LDS stack: n entries from place bot (a ring)
+    uint32_t cap;
+    uint32_t tick;
+    uint32_t tasks, branches, children, beyond;  // counters since the last flush
+    unsigned long long sum_t, sum_tw;
+};
+
+// mindeg[i] for a uniform i >= 0
+__device__ __forceinline__ int tiny_md(const Ctx& c, const Tiny& y, int i) {
+    return i < WAVE ? rdlane(y.mdt, i) : uni(md(c, i));
+}
+
+// The basis from a record of t <= 64 vertices.  False (nothing changed but y)
+// when a degree does not fit the state word: the caller runs the general path.
+__device__ __attribute__((always_inline)) bool tiny_load(Ctx& c, const TaskRef& ref, Tiny& y) {
+    const int t = (int)ref.t;
+    const int lane = c.lane;
+    const bool on = lane < t;
+    Vrec v{0, 0, 0, 0};
+    if (on) v = c.a->in_verts[ref.off + lane];
+    if (ballot(on && (v.exdeg < TINY_EX_MIN || v.exdeg > TINY_EX_MAX || (uint32_t)v.indeg > 63u))) return false;
+    int rk = 0;
+    for (int i = 0; i < t; i++) rk += rdlane(v.id, i) < v.id ? 1 : 0;
+    const int to = (on ? rk : lane) << 2;
+    const uint32_t word = on ? tiny_word(v.indeg, v.exdeg, WAVE - 1 - lane, v.label == 1) : 0u;
+    y.id = __builtin_amdgcn_ds_permute(to, v.id);
+    y.s = (uint32_t)__builtin_amdgcn_ds_permute(to, (int)word);
+    const int rw = c.g.p->rw;
+    const uint64_t* __restrict__ A1 = c.g.p->A1;
+    const uint64_t* __restrict__ A2 = c.g.p->A2;
+    const int cw = y.id >> 6;
+    const uint64_t cm = 1ull << (y.id & 63);
+    y.d1 = on ? c.g.p->d1r[y.id] : 0;
+    y.d2 = on ? c.g.p->d2r[y.id] : 0;
+    y.orig = on ? c.g.p->orig[y.id] : 0u;
+    y.r1 = 0;
+    y.r2 = 0;
+    // (RU rows at a time: 2 RU gathers in flight per lane)
+    constexpr int RU = 8;
+    for (int i = 0; i < t; i += RU) {
+        uint64_t x[RU], z[RU];
+#pragma unroll
+        for (int q = 0; q < RU; q++) {
+            const int k = min(i + q, t - 1);
+            const size_t rb = (size_t)rdlane(y.id, k) * rw + cw;
+            x[q] = A1[rb];
+            z[q] = A2[rb];
+        }
+#pragma unroll
+        for (int q = 0; q < RU; q++) {
+            const uint64_t b = ballot(on && (x[q] & cm)), e = ballot(on && (z[q] & cm));
+            if (lane == min(i + q, t - 1)) {
+                y.r1 = b;
+                y.r2 = e;
+            }
+        }
+    }
+    y.mdt = md(c, lane);
+    y.depth = ref.depth;
+    y.hot_on = false;
+    y.hot = 0;
+    y.hot_depth = 0;
+    y.n = 0;
+    y.bot = 0;
+    y.nf = 0;
+    y.fr = 0;
+    y.ff = 0;
+    y.tick = 0;
+    y.tasks = y.branches = y.children = y.beyond = 0;
+    y.sum_t = y.sum_tw = 0;
+    return true;
+}
+
+// W_adj of the failed removals noted so far: the reference scans N(r) in
+// ascending id order and stops after the first failing member
+// (main.cu:1437-1450).  Noted per lane and counted here together: the row
+// loads of different removals do not wait for each other.
+__device__ __attribute__((always_inline)) void tiny_failed_scans(Ctx& c, Tiny& y) {
+    const int rw = c.g.p->rw;
+    const uint64_t* __restrict__ A1 = c.g.p->A1;
+    int rank = 0;
+    for (int k = 0; k < y.nf; k++) {
+        const int rid = rdlane(y.fr, k), fid = rdlane(y.ff, k);
+        const uint64_t* row = A1 + (size_t)rid * rw;
+        for (int wd = c.lane; wd <= (fid >> 6); wd += WAVE) {
+            uint64_t x = row[wd];
+            if (wd == (fid >> 6)) x &= (1ull << (fid & 63)) - 1ull;
+            rank += __popcll(x);
+        }
+    }
+    c.wadj_l += rank + (c.lane < y.nf ? 1 : 0);
+    y.nf = 0;
+}
+
+// counters into the wave's (LDS)
+__device__ __attribute__((always_inline)) void tiny_counters(Ctx& c, Tiny& y) {
+    if (c.lane == 0) {
+        c.st->tasks += y.tasks;
+        c.st->branches += y.branches;
+        c.st->children += y.children;
+        c.st->beyond += y.beyond;
+        c.st->sum_t += y.sum_t;
+        c.st->sum_tw += y.sum_tw;
+    }
+    y.tasks = y.branches = y.children = y.beyond = 0;
+    y.sum_t = y.sum_tw = 0;
+}
+
+// LU bounds (lu_bounds) and the member checks over lane masks: members M (m
+// of them), `cand` the lanes whose indegrees count (nc of them), in / ex per
+// lane.  True: the record fails.
+__device__ __forceinline__ bool tiny_bounds(Ctx& c, const Tiny& y, uint64_t M, int m, uint64_t cand, int nc, int in,
+                                            int ex, int mds, int& ub, int& lb, int& med) {
+    const bool mem = (M >> c.lane) & 1ull;
+    const int ms = c.g.min_size;
+    auto gm = [&](int s) { return s < ms ? mds : tiny_md(c, y, s); };  // get_mindeg
+    // the smallest (indeg, exdeg) pair, exdeg as an unsigned field
+    const int pair = wave_min(mem ? (in << 14) | (ex & 0x3FFF) : INT32_MAX);
+    const int min_in = pair >> 14;
+    bool invalid = false;
+    const int gmm = gm(m);
+    med = gm(m + 1);
+    if (min_in < tiny_md(c, y, m)) {
+        const int min_in_ex = (int)((uint32_t)pair << 18) >> 18;
+        int x = gmm - min_in;
+        for (;;) {
+            const int k = x + c.lane;
+            const uint64_t bm = ballot(k > min_in_ex || min_in + k >= md(c, m + k));
+            if (bm) {
+                x += __builtin_ctzll(bm);
+                break;
+            }
+            x += WAVE;
+        }
+        lb = x;
+        if (min_in + lb < tiny_md(c, y, m + lb)) {
+            lb = nc + 1;
+            invalid = true;
+        }
+        const int min_tot = wave_min(mem ? in + ex : INT32_MAX);
+        // (a stale exdeg can make the sum negative: floor(d / gamma) is then
+        // below 0 and the bound too)
+        const int tq = min_tot < 0 ? -1 : c.g.p->ubq[min(min_tot, c.g.ubq_n - 1)];
+        ub = tq + 1 - m;
+        if (ub > nc) ub = nc;
+        if (lb < ub) {
+            const int sum_in = wave_sum(mem ? in : 0);
+            // P(idx) = sum over v >= 1 of min(#{indeg >= v}, idx), idx = lane
+            const int xin = (cand >> c.lane) & 1ull ? in : 0;
+            int p = 0;
+            for (int v = 1;; v++) {
+                const int k = __popcll(ballot(xin >= v));
+                if (k == 0) break;
+                p += min(k, c.lane);
+            }
+            const uint64_t ok = ballot(c.lane <= ub && c.lane >= lb && sum_in + p >= m * md(c, m + c.lane));
+            if (ok == 0) {
+                lb = ub + 1;
+                invalid = true;
+            } else {
+                lb = __builtin_ctzll(ok);
+                ub = min(ub, 63 - __builtin_clzll(ok));
+                if (lb > 1) med = gm(m + lb);
+            }
+        }
+    } else {
+        ub = nc;
+        lb = m < ms ? ms - m : 0;
+    }
+    if (m + ub < ms || ub < 0 || ub < lb) invalid = true;
+    if (invalid) return true;
+    // vert_isextendable_LU (vert_ext): the checks that do not depend on the
+    // lane folded into two bounds; get_mindeg(m + ex) is mindeg[m + ex] under
+    // the first of them (mindeg is monotone)
+    const int tot = in + ex;
+    const int T = max(max(mds, med), gm(m + lb));
+    const bool f = mem && (tot < T || in + ub < tiny_md(c, y, m + ub) || tot < md(c, m + ex));
+    return ballot(f) != 0;
+}
+
+// degree_pruning over lane masks: `alive` are the candidates that may stay,
+// `dead` the others; on return `alive` holds those that stay.  True: fails.
+__device__ __attribute__((always_inline)) bool tiny_prune(Ctx& c, const Tiny& y, uint64_t M, int m, uint64_t& alive,
+                                                          uint64_t dead, int in, int& ex, bool map_empty, int mds, int& ub,
+                                                          int& lb, int& med) {
+    const int ms = c.g.min_size;
+    const uint64_t me = 1ull << c.lane;
+    int T = 0, U = 0;
+    auto bounds = [&]() {
+        const int g = m + lb < ms ? mds : tiny_md(c, y, m + lb);
+        T = max(max(mds, med), g);
+        U = tiny_md(c, y, m + lb) - ub + 1;
+    };
+    auto valid = [&]() { return in + ex >= T && in >= U && in + ex >= md(c, m + ex + 1); };  // cand_valid
+    uint64_t rem = alive, rmv = dead, cnt_set = alive;
+    bool first = true;
+    for (;;) {
+        if (tiny_bounds(c, y, M, m, cnt_set, __popcll(cnt_set), in, ex, mds, ub, lb, med)) return true;
+        bounds();
+        const uint64_t stay = ballot((rem & me) && valid());
+        rmv = first ? dead | (rem & ~stay) : rem & ~stay;
+        first = false;
+        rem = stay;
+        if (rem == 0 || rmv == 0) break;
+        // degree update, main.cu:1775-1807
+        const bool rc = __popcll(rem) < __popcll(rmv);
+        const uint64_t L = rc ? rem : rmv;
+        if (L & me) c.wadj_l += y.d1;
+        if ((M | rem) & me) {
+            if (map_empty) {
+                if (rc) ex = 0;
+            } else {
+                const int k = __popcll(y.r1 & L);
+                ex = rc ? k : ex - k;
+            }
+        }
+        // the indegrees that count: candidates valid under the old bounds
+        // with the new exdeg (main.cu:1811-1815)
+        cnt_set = ballot((rem & me) && valid());
+    }
+    alive = rem;
+    return false;
+}
+
+// One task (y.s): its branches, children pushed on the stack (the caller has
+// made room for them).
+__device__ __attribute__((always_inline)) void tiny_task(Ctx& c, Tiny& y, uint32_t* stk, uint16_t* sdep) {
+    const int lane = c.lane;
+    const uint64_t me = 1ull << lane;
+    const uint32_t w = y.s;
+    const uint64_t P = ballot(w & TW_PRESENT), M = ballot(w & TW_MEMBER);
+    const uint64_t C = P & ~M;
+    const int t0 = __popcll(P), nm = __popcll(M), nc = __popcll(C);
+    const int in = tw_in(w);
+    int ex = tw_ex(w);
+    const int ms = c.g.min_size;
+    const int mds = tiny_md(c, y, ms);
+    y.tasks++;
+    y.sum_t += t0;
+    // ---- lookahead ----
+    const int req = tiny_md(c, y, t0);
+    int l2 = 0;
+    if (ballot((M & me) && in + ex < req) == 0) {
+        if (C & me) {
+            c.wadj_l += y.d2;
+            l2 = __popcll(y.r2 & C);
+        }
+        if (ballot((C & me) && (l2 < nc - 1 || in + ex < req)) == 0) {
+            emit_lanes(c, P, y.orig);
+            return;
+        }
+    }
+    // ---- branches ----
+    const int mdg = nm < ms ? mds : tiny_md(c, y, nm);  // get_mindeg(nm)
+    const bool keys = !(c.g.max_depth >= 0 && (int)y.depth + 1 > c.g.max_depth);
+    uint64_t Cr = C;
+    const int key = tiny_key(w, lane);
+    int v = 0;
+    for (int b = 0; b < nc; b++) {
+        if (b > 0) {
+            // remove_one_vertex: the last branch's vertex
+            const uint64_t vb = 1ull << v;
+            Cr &= ~vb;
+            const bool adj = (y.r1 & vb) != 0;
+            if (adj) ex--;
+            const uint64_t fail = ballot(adj && (M & me) && in + ex < mdg);
+            if (fail) {
+                // (lanes are in id order: the lowest failing lane is scanned first)
+                const int rid = rdlane(y.id, v), fid = rdlane(y.id, __builtin_ctzll(fail));
+                if (lane == y.nf) {
+                    y.fr = rid;
+                    y.ff = fid;
+                }
+                if (++y.nf == WAVE) tiny_failed_scans(c, y);
+                break;
+            }
+            if (lane == v) c.wadj_l += y.d1;
+        }
+        v = wave_min((Cr & me) ? key : INT32_MAX) & (WAVE - 1);
+        y.branches++;
+        if (lane == v) c.wadj_l += y.d1 + y.d2;
+        // the child: members and v, candidates inside N2(v)
+        uint64_t Mc = M | (1ull << v);
+        int m = nm + 1;
+        const uint64_t rest = Cr & ~(1ull << v);
+        uint64_t alive = rest & rdlane64(y.r2, v), dead = rest & ~alive;
+        const int a1 = (int)((y.r1 >> v) & 1ull);
+        int ci = in + a1, ce = ex - a1;
+        int ub = 0, lb = 0, med = 0;
+        bool map_empty = false, first = true, fails;
+        for (;;) {
+            fails = tiny_prune(c, y, Mc, m, alive, dead, ci, ce, map_empty, mds, ub, lb, med);
+            if (!first || fails) break;
+            first = false;
+            // critical_prep
+            const int thr = tiny_md(c, y, m + lb);
+            const uint64_t cm = ballot((Mc & me) && ci + ce == thr && ce > 0);
+            if (cm & me) c.wadj_l += y.d1;
+            const uint64_t F = cm ? ballot((alive & me) && (y.r1 & cm)) : 0ull;
+            dead = 0;
+            if (F == 0) {
+                map_empty = true;
+                continue;
+            }
+            const int ncrit = __popcll(F);
+            if (F & me) c.wadj_l += y.d1 + y.d2;
+            const int x1 = __popcll(y.r1 & F), x2 = __popcll(y.r2 & F);
+            ci += x1;
+            ce -= x1;
+            if (ballot(((Mc & me) && x2 != ncrit) || ((F & me) && x2 < ncrit - 1))) {
+                m = -1;  // the reference's 2: neither a clique test nor a child
+                break;
+            }
+            Mc |= F;
+            m += ncrit;
+            const uint64_t left = alive & ~F;
+            alive = left & ballot(x2 == ncrit);
+            dead = left & ~alive;
+        }
+        if (m < 0) continue;
+        if (m >= ms && ballot((Mc & me) && ci < tiny_md(c, y, m)) == 0) emit_lanes(c, Mc, y.orig);
+        if (fails || alive == 0) continue;
+        y.children++;
+        y.sum_tw += m + __popcll(alive);
+        if (!keys) {
+            y.beyond++;
+            continue;
+        }
+        if (y.hot_on) {
+            uint32_t at = y.bot + y.n;
+            if (at >= y.cap) at -= y.cap;
+            stk[at * WAVE + lane] = y.hot;
+            if (lane == 0) sdep[at] = (uint16_t)y.hot_depth;
+            y.n++;
+        }
+        y.hot_on = true;
+        y.hot_depth = y.depth + 1;
+        y.hot = ((Mc | alive) & me) ? tiny_word(ci, ce, l2, (Mc & me) != 0) : 0u;
+    }
+}
+
+// the task after this one (the child pushed last, else the top of the stack)
+__device__ __forceinline__ bool tiny_next(Ctx& c, Tiny& y, const uint32_t* stk, const uint16_t* sdep) {
+    if (y.hot_on) {
+        y.s = y.hot;
+        y.depth = y.hot_depth;
+        y.hot_on = false;
+        return true;
+    }
+    if (y.n == 0) return false;
+    y.n--;
+    uint32_t at = y.bot + y.n;
+    if (at >= y.cap) at -= y.cap;
+    wsync();
+    y.s = stk[at * WAVE + c.lane];
+    y.depth = (uint32_t)uni((int)sdep[at]);
+    return true;
+}
+
+// place of every lane's vertex in the record of task word w: members first
+// (ascending id), then the candidates in Q order
+__device__ __forceinline__ int tiny_place(Ctx& c, uint32_t w, uint64_t M, uint64_t C) {
+    const int key = tiny_key(w, c.lane);
+    int rank = __popcll(M);
+    for (uint64_t s = C; s; s &= s - 1) rank += rdlane(key, __builtin_ctzll(s)) > key ? 1 : 0;
+    return (M >> c.lane) & 1ull ? lanes_below(M) : rank;
+}
+
+// The k oldest tasks of the stack become records on the wave's own task stack
+// (for the rings, or because the LDS stack needs room).
+__device__ __attribute__((always_inline)) void tiny_spill(Ctx& c, Tiny& y, const uint32_t* stk, const uint16_t* sdep,
+                                                          uint32_t k) {
+    const ExpandArgs& a = *c.a;
+    wsync();
+    for (; k > 0; k--) {
+        const uint32_t w = stk[y.bot * WAVE + c.lane];
+        const uint32_t depth = (uint32_t)uni((int)sdep[y.bot]);
+        if (++y.bot == y.cap) y.bot = 0;
+        y.n--;
+        const uint64_t P = ballot(w & TW_PRESENT), M = ballot(w & TW_MEMBER);
+        const int t = __popcll(P);
+        unsigned long long si = 0;
+        if (c.lane == 0) si = pool_alloc(c, (uint32_t)t);
+        si = rdlane64(si, 0);
+        if (si == ~0ull) {
+            if (c.lane == 0) atomicOr(a.error, 1);
+            continue;
+        }
+        const int at = tiny_place(c, w, M, P & ~M);
+        if (w & TW_PRESENT) a.pool[si + at] = Vrec{y.id, (w & TW_MEMBER) ? 1 : 0, tw_in(w), tw_ex(w)};
+        TaskRef r;
+        r.off = si;
+        r.t = (uint32_t)t;
+        r.depth = (uint16_t)depth;
+        r.inst = (uint16_t)c.inst;
+        r.bound = 0;
+        r.b0 = 0;
+        r.b1 = 0;
+        push_ref(c, r, 0, !a.use_priv, nullptr);
+    }
+}
+
+// moves the child pushed last to the stack
+__device__ __forceinline__ void tiny_unhot(Ctx& c, Tiny& y, uint32_t* stk, uint16_t* sdep) {
+    if (!y.hot_on) return;
+    uint32_t at = y.bot + y.n;
+    if (at >= y.cap) at -= y.cap;
+    stk[at * WAVE + c.lane] = y.hot;
+    if (c.lane == 0) sdep[at] = (uint16_t)y.hot_depth;
+    y.n++;
+    y.hot_on = false;
+}
+
+// Runs the subtree; returns true when it stopped to hand tasks over (their
+// records are on the wave's own stack) and has to be resumed, false when it
+// is done.  One task only, its children all made records, in the static order
+// (whose tasks are dealt to the waves in turn).
+__device__ __attribute__((always_inline)) bool tiny_run(Ctx& c, Tiny& y, uint32_t* stk, uint16_t* sdep, bool go_on) {
+    const ExpandArgs& a = *c.a;
+    bool more = go_on ? tiny_next(c, y, stk, sdep) : true;
+    while (more) {
+        const uint32_t nc = (uint32_t)__popcll(ballot((y.s & (TW_PRESENT | TW_MEMBER)) == TW_PRESENT));
+        uint32_t out = y.n + nc > y.cap ? y.n + nc - y.cap : 0u;
+        bool give = false;
+        if (!a.static_sched && (++y.tick & 3u) == 0) {
+            // more waves wait for work than the rings hold (as between
+            // tasks of the general loop, with the word read at one check and
+            // used at the next): up to 16 of the oldest tasks go out
+            const unsigned long long ph = rdlane64(c.share_v, 0);
+            if (c.lane == 0) c.share_v = __hip_atomic_load(a.pending, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            const long long hg = (long long)(ph >> 32), pd = (long long)(ph & 0xFFFFFFFFull);
+            const long long waiting = pd - ((long long)gridDim.x - hg);
+            const long long need = hg - (waiting > 0 ? waiting : 0);
+            // every busy wave reads the same need: each answers with the
+            // chance that twice the need is met between them (a record made
+            // and not taken costs its basis again)
+            const long long busy = (long long)gridDim.x - hg;
+            const uint32_t dice = (blockIdx.x * 0x9E3779B9u + y.tick * 0x85EBCA6Bu) >> 8;
+            if (need > 0 && y.n > 0 && (2 * need >= busy || (long long)(((unsigned long long)dice * busy) >> 24) < 2 * need)) {
+                give = true;
+                const long long share = need / max(1ll, busy) + 1;
+                out = max(out, (uint32_t)min<long long>(min<long long>(share, 16ll), (long long)y.n));
+            }
+        }
+        if (out) tiny_spill(c, y, stk, sdep, out);
+        if (give) {
+            // the task to run next waits in front of the stack
+            y.hot = y.s;
+            y.hot_depth = y.depth;
+            y.hot_on = true;
+            return true;
+        }
+        tiny_task(c, y, stk, sdep);
+        if (a.static_sched) {
+            tiny_unhot(c, y, stk, sdep);
+            tiny_spill(c, y, stk, sdep, y.n);
+        }
+        more = tiny_next(c, y, stk, sdep);
+    }
+    tiny_failed_scans(c, y);
+    tiny_counters(c, y);
+    return false;
+}
+
+// Level-synchronous form: one task, its children written to the output
+// stream with one claim for all of them.
+__device__ __attribute__((always_inline)) void tiny_level(Ctx& c, Tiny& y, uint32_t* stk, uint16_t* sdep) {
+    const ExpandArgs& a = *c.a;
+    tiny_task(c, y, stk, sdep);
+    tiny_unhot(c, y, stk, sdep);
+    const uint32_t n = y.n;
+    const unsigned long long slots = y.beyond ? 0ull : y.sum_tw;
+    tiny_failed_scans(c, y);
+    tiny_counters(c, y);
+    if (n == 0) return;
+    unsigned long long ri = 0, si = 0;
+    if (c.lane == 0) {
+        ri = atomicAdd(&a.out_ctr[0].items, (unsigned long long)n);
+        si = atomicAdd(&a.out_ctr[0].slots, slots);
+    }
+    ri = rdlane64(ri, 0);
+    si = rdlane64(si, 0);
+    if (ri + n > a.out_ref_cap[0] || si + slots > a.out_vert_cap[0]) {
+        if (c.lane == 0) atomicOr(a.error, 1);
+        return;
+    }
+    wsync();
+    for (uint32_t k = 0; k < n; k++) {
+        const uint32_t w = stk[k * WAVE + c.lane];
+        const uint64_t P = ballot(w & TW_PRESENT), M = ballot(w & TW_MEMBER), C = P & ~M;
+        const int t = __popcll(P), nm = __popcll(M);
+        const int at = tiny_place(c, w, M, C);
+        if (w & TW_PRESENT) a.out_verts[0][si + at] = Vrec{y.id, (w & TW_MEMBER) ? 1 : 0, tw_in(w), tw_ex(w)};
+        // slot bound of this child's own children (see TaskRef)
+        const int bnd = wave_sum((C >> c.lane) & 1ull ? min(y.d2 + nm + 1, t) : 0);
+        if (c.lane == 0) {
+            TaskRef r;
+            r.off = si;
+            r.t = (uint32_t)t;
+            r.depth = (uint16_t)(c.depth + 1);
+            r.inst = (uint16_t)c.inst;
+            r.bound = (uint64_t)bnd;
+            r.b0 = 0;
+            r.b1 = 0;
+            a.out_refs[0][ri + k] = r;
+        }
+        si += t;
     }
 }
 
@@ -1994,7 +2609,7 @@ __device__ __forceinline__ void flush_stats(Ctx& c, DevStats* d) {
 __device__ __forceinline__ void flush_stats(Ctx& c) { flush_stats(c, c.a->stats); }
 
 template <bool LOCAL>
-__device__ __forceinline__ void task_loop(Ctx& c) {
+__device__ __forceinline__ void task_loop(Ctx& c, char* lds, uint16_t* sdep) {
     const ExpandArgs& a = *c.a;
     const uint32_t nw = gridDim.x;
     uint32_t i;
@@ -2007,7 +2622,18 @@ __device__ __forceinline__ void task_loop(Ctx& c) {
     }
     while (i < a.n_in) {
         TaskRef ref = a.in_refs[i];
-        if (ref.t <= c.cap)
+        bool done = false;
+        if (LOCAL && ref.t <= TINY_MAX && ref.depth > 0) {
+            Tiny y;
+            done = tiny_load(c, ref, y);
+            if (done) {
+                c.depth = ref.depth;
+                y.cap = TINY_MAX;
+                tiny_level(c, y, (uint32_t*)lds, sdep);
+            }
+        }
+        if (done) {
+        } else if (ref.t <= c.cap)
             process_task<LOCAL>(c, ref);
         else if (c.lane == 0)
             atomicOr(a.error, 2);
@@ -2026,8 +2652,11 @@ __device__ __forceinline__ void task_loop(Ctx& c) {
 template <int TL>
 __global__ __launch_bounds__(64) void expand_local(const ExpandArgs* __restrict__ ap) {
     const ExpandArgs& a = *ap;
-    constexpr size_t BYTES = ws_bytes(TL, true, (TL + 63) / 64);
+    // the LDS workspace, or the children of a task of at most 64 vertices
+    constexpr size_t WS_BYTES = ws_bytes(TL, true, (TL + 63) / 64);
+    constexpr size_t BYTES = WS_BYTES > TINY_MAX * TINY_ENTRY ? WS_BYTES : TINY_MAX * TINY_ENTRY;
     __shared__ __attribute__((aligned(16))) char lds[BYTES];
+    __shared__ uint16_t s_dep[TINY_MAX];
     Ctx c;
     c.wadj_l = 0;
     c.a = ap;
@@ -2044,7 +2673,7 @@ __global__ __launch_bounds__(64) void expand_local(const ExpandArgs* __restrict_
     c.ph = s_ph;
     if (c.lane == 0) s_st = LStats{0, 0, 0, 0, 0, 0, 0, 0, 0};
     ph_start(c);
-    task_loop<true>(c);
+    task_loop<true>(c, lds, s_dep);
 }
 
 __global__ __launch_bounds__(64) void expand_hbm(const ExpandArgs* __restrict__ ap) {
@@ -2066,7 +2695,17 @@ __global__ __launch_bounds__(64) void expand_hbm(const ExpandArgs* __restrict__ 
     c.ph = s_ph;
     if (c.lane == 0) s_st = LStats{0, 0, 0, 0, 0, 0, 0, 0, 0};
     ph_start(c);
-    task_loop<false>(c);
+    task_loop<false>(c, nullptr, nullptr);
+}
+
+// diagnostics: one task's row of the timeline
+__device__ __forceinline__ void timeline_row(Ctx& c, const TaskRef& ref, long long gslot, long long start) {
+    if (c.lane != 0) return;
+    unsigned long long* r = c.a->timeline + 4 * (unsigned long long)gslot;
+    r[0] = (unsigned long long)start;
+    r[1] = (unsigned long long)wall_clock64();
+    r[2] = ((unsigned long long)blockIdx.x << 32) | ref.t;
+    r[3] = (unsigned long long)ref.depth | ((unsigned long long)ref.b0 << 16) | ((unsigned long long)ref.b1 << 40);
 }
 
 // ---------------------------------------------------------------------------
@@ -2125,6 +2764,15 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void ex
     // (registers are the scarce resource of this kernel)
     __shared__ TaskRef s_claim[4];
     __shared__ TaskRef s_top;
+    // the wave's part of the clique stream (none yet)
+    __shared__ unsigned long long s_clq[4];
+    c.clq = s_clq;
+    if (c.lane < 4) s_clq[c.lane] = 0;
+    // the subtree of at most 64 vertices in hand (tiny_run), its children's
+    // depths; the children themselves use the dynamic LDS
+    __shared__ uint16_t s_dep[TINY_STACK_MAX];
+    Tiny y{};
+    bool tiny = false;  // to be resumed after a hand-over
     c.ptopref = &s_top;
     c.ptopi = ~0u;
     c.share_v = 0;  // reads as nobody waiting
@@ -2141,18 +2789,20 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void ex
     for (;;) {
         TaskRef ref;
         long long gslot;
-        if (qi < nq) {
+        if (!tiny && qi < nq) {
             ref = s_claim[qi];
             if (c.phase_on && c.lane == 0) c.ph[PH_N_RING]++;
             gslot = (long long)(qbase + (qh + (unsigned long long)qi) % a.q_cap);
             qi++;
         } else if (a.static_sched && c.ptop != c.pbot && static_flush(c)) {
             continue;
-        } else if (c.ptop != c.pbot) {
+        } else if (tiny || c.ptop != c.pbot) {
             // this wave's own stack (depth first)
             idle = 0;
             ph_mark(c, PH_POP);
-            if (!a.static_sched && c.ptop - c.pbot > 1) {
+            // (a wave with a subtree in hand can give every record away)
+            const uint32_t own = tiny ? 0u : 1u;
+            if (!a.static_sched && c.ptop - c.pbot > own) {
                 // more waves wait for work than the rings hold: hand over
                 // the oldest (shallowest, so largest) records, up to 16 at
                 // once, into the bucket of the oldest one.  The rings hold
@@ -2166,7 +2816,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void ex
                 const long long waiting = pd - ((long long)G - hg);
                 const long long need = hg - (waiting > 0 ? waiting : 0);
                 if (need > 0) {
-                    const int want = (int)min<long long>(min<long long>((long long)(c.ptop - c.pbot - 1), 16ll), need);
+                    const int want = (int)min<long long>(min<long long>((long long)(c.ptop - c.pbot - own), 16ll), need);
                     if (a.n_buckets > 1) {
                         // cost order: the 16 oldest records are ordered by
                         // predicted bucket, largest first (stable), so the
@@ -2174,7 +2824,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void ex
                         // Lane j holds record j; its rank is the number of
                         // records before it in that order.
                         wsync();  // lane 0's stack stores, visible to every lane
-                        const int span = (int)min<uint32_t>(c.ptop - c.pbot - 1, 16u);
+                        const int span = (int)min<uint32_t>(c.ptop - c.pbot - own, 16u);
                         const uint32_t at = (c.pbot + (uint32_t)c.lane) % a.priv_cap;
                         const int bj = c.lane < span ? (int)c.pbkt[at] : -1;
                         int rank = 0;
@@ -2220,6 +2870,11 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void ex
                 }
             }
             ph_mark(c, PH_GIVE);
+            if (tiny) {
+                tiny = tiny_run(c, y, (uint32_t*)lds, s_dep, true);
+                ph_mark(c, PH_TINY);
+                continue;
+            }
             c.ptop--;
             TaskRef r;
             // the newest entry is usually still in LDS (pushed last)
@@ -2383,6 +3038,26 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void ex
         c.share_ok = ref.t >= SHARE_MIN_T;
         // workspace: LDS with local matrices, LDS arrays with root
         // matrices, slab with local matrices, or slab in root space
+        // A task that fits one vertex a lane runs with its whole subtree in
+        // registers.  64 is the width of a wave and of a mask in scalar
+        // registers; split items (prepared records) and the root (labels
+        // other than member and candidate) take the general path.  Against
+        // that path for every size (kernel, medians): a full search of 1.86
+        // million tasks of 23 vertices 59 -> 22 ms, a power-law window of
+        // 252,000 tasks of 29 34 -> 16 ms, 3,051 tasks of 17 16.3 -> 9.0 ms;
+        // a window whose tasks are all larger is unchanged.
+        if (ref.t <= TINY_MAX && ref.depth > 0 && ref.b1 == 0 && a.tiny_cap && tiny_load(c, ref, y)) {
+            y.cap = a.tiny_cap;
+            // (the record is in registers: its block can go back at once)
+            wsync();
+            if (c.lane == 0) pool_free(c, ref.off, ref.t);
+            ph_mark(c, PH_LOAD);
+            tiny = tiny_run(c, y, (uint32_t*)lds, s_dep, false);
+            ph_mark(c, PH_TINY);
+            if (a.timeline && gslot >= 0) timeline_row(c, ref, gslot, tl_start);
+            continue;
+        }
+        y = Tiny{};  // nothing of it lives across the general path
         const bool fits = ref.t <= a.slab_tcap;
         const bool local = ref.t <= (uint32_t)TL || (ref.t > wide && ref.t <= mid);
         // (built per task: only one workspace descriptor is live)
@@ -2457,14 +3132,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void ex
             process_task<false>(c, ref);
         }
         wsync();
-        if (a.timeline && gslot >= 0 && c.lane == 0) {
-            unsigned long long* r = a.timeline + 4 * (unsigned long long)gslot;
-            r[0] = (unsigned long long)tl_start;
-            r[1] = (unsigned long long)wall_clock64();
-            r[2] = ((unsigned long long)blockIdx.x << 32) | ref.t;
-            r[3] = (unsigned long long)ref.depth | ((unsigned long long)ref.b0 << 16) |
-                   ((unsigned long long)ref.b1 << 40);
-        }
+        if (a.timeline && gslot >= 0) timeline_row(c, ref, gslot, tl_start);
         ph_mark(c, PH_CHILD);
         if (c.lane == 0) {
             // the record's block: a split item's prepared record is freed by
@@ -2482,6 +3150,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void ex
     }
     ph_mark(c, PH_IDLE);
     ph_flush(c);
+    clq_close(c);
     if (sinst >= 0)
         flush_stats(c, &a.inst_stats[sinst]);
     else

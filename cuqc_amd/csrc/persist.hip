@@ -211,6 +211,11 @@ int enumerate_persistent(const Instance* const* insts, const qc_params* params, 
     const size_t mask_b = (size_t)2 * std::max<size_t>((size_t)maxrw, midw) * 8;
     const bool mask_lds = mask_b <= MASK_LDS_MAX;
     size_t lds_b = std::max(ws_bytes(TL, true, (TL + 63) / 64), arr_b + (mask_lds ? mask_b : 0));
+    // (traces number every task by its ring position: no subtree runs unseen)
+    const bool tiny = p.trace == 0;
+    // room for the children of any task of 64 vertices; the registers allow
+    // 8 waves per CU, and 8 x 16 KB fit its LDS
+    if (tiny) lds_b = std::max<size_t>(lds_b, (size_t)64 * 256);
     QC_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, 64, lds_b));
     {
         // A workgroup's LDS (static + dynamic) is allocated in granules of
@@ -284,6 +289,14 @@ int enumerate_persistent(const Instance* const* insts, const qc_params* params, 
     uint64_t clq_slots = fixed_clq ? p.clique_capacity
                                    : std::max<uint64_t>(ws.clq_slots, std::min<uint64_t>(max_clq, 1ull << 24));
     uint64_t clq_refs = std::max<uint64_t>(ws.clq_refs_cap, clq_slots / 8 + 1024);
+    // a caller's clique capacity bounds the raw sets' vertices (and their
+    // number); the waves take refs and slots several at a time, so the stream
+    // itself is larger by what they can leave unused
+    const uint64_t fixed_slots = clq_slots, fixed_refs = clq_slots / 8 + 1024;
+    if (fixed_clq) {
+        clq_slots = clq_slots + clq_slots / 3 + (uint64_t)grid * CLQ_SLOTS;
+        clq_refs = std::max<uint64_t>(clq_refs, fixed_refs + (uint64_t)grid * CLQ_REFS);
+    }
     // private stacks: a power of two of refs per wave (the stack is a ring
     // indexed by 32-bit counters)
     const uint64_t max_priv = 1ull << 20;
@@ -342,6 +355,8 @@ int enumerate_persistent(const Instance* const* insts, const qc_params* params, 
     RunState first{};
     std::vector<DevStats> first_stats;
     float first_ms = 0;
+    uint64_t last_items = 0;
+    uint64_t raw_k = 0, raw_nv = 0;  // raw sets and their vertices, over all instances
     for (int attempt = 0;; attempt++) {
         if ((rc = ensure(ws.pool, pool_cap * sizeof(Vrec))) || (rc = ensure(ws.q, nr * q_cap * sizeof(TaskRef))) ||
             (rc = ensure(ws.seq, nr * q_cap * 8)) || (rc = ensure(ws.clq_refs, clq_refs * sizeof(CliqueRef))) ||
@@ -406,6 +421,7 @@ int enumerate_persistent(const Instance* const* insts, const qc_params* params, 
         A.pool_top = ctr + 2 * nr * QSTRIDE;
         A.pending = ctr + (2 * nr + 1) * QSTRIDE;
         A.overflow = ctr + (2 * nr + 2) * QSTRIDE;
+        A.tiny_cap = tiny ? (uint32_t)std::min<size_t>(TINY_STACK_MAX, lds_b / 256) : 0u;
         A.n_buckets = nb;
         A.q_shards = ns;
         A.n_roots = (int32_t)roots.size();
@@ -481,6 +497,7 @@ int enumerate_persistent(const Instance* const* insts, const qc_params* params, 
             QC_HIP(hipMemcpy(&rs.clq, ws.clq_ctr.p, sizeof(rs.clq), hipMemcpyDeviceToHost));
             QC_HIP(hipMemcpy(&rs.err, ws.err.p, sizeof(int), hipMemcpyDeviceToHost));
             QC_HIP(hipMemcpy(ist.data(), d_istats.p, (size_t)count * sizeof(DevStats), hipMemcpyDeviceToHost));
+            last_items = rs.clq.items;  // refs taken (of the launch whose buffers are read below: the last)
             if (rs.err) {
                 if (rs.err == 1 && rep == 0) {
                     // grow what ran out (its counter kept counting) and rerun
@@ -523,8 +540,17 @@ int enumerate_persistent(const Instance* const* insts, const qc_params* params, 
                 first = rs;
                 first_stats = ist;
                 first_ms = ms;
-            } else if (first.clq.items != rs.clq.items || first.clq.slots != rs.clq.slots ||
-                       memcmp(first_stats.data(), ist.data(), (size_t)count * sizeof(DevStats)) != 0) {
+                raw_k = raw_nv = 0;
+                for (const DevStats& d : ist) {
+                    raw_k += d.raw_cliques;
+                    raw_nv += d.sum_clique_len;
+                }
+                if (fixed_clq && (raw_k > fixed_refs || raw_nv > fixed_slots)) {
+                    set_error("persistent expansion: %llu raw sets of %llu vertices exceed the clique capacity",
+                              (unsigned long long)raw_k, (unsigned long long)raw_nv);
+                    status = QC_EOVERFLOW;
+                }
+            } else if (memcmp(first_stats.data(), ist.data(), (size_t)count * sizeof(DevStats)) != 0) {
                 set_error("graph replay %d differs from the first launch", rep);
                 status = QC_EDEVICE;
             }
@@ -566,7 +592,7 @@ int enumerate_persistent(const Instance* const* insts, const qc_params* params, 
         unsigned long long ph[PH_COUNT];
         QC_HIP(hipMemcpy(ph, d_phase.p, sizeof(ph), hipMemcpyDeviceToHost));
         static const char* names[] = {"load", "lookahead", "remove", "add", "prune", "child", "prepare", "idle",
-                                      "lu", "degupd", "classify", "critical", "compact", "hist", "pool", "pop", "give", "sync"};
+                                      "lu", "degupd", "classify", "critical", "compact", "hist", "pool", "pop", "give", "sync", "tiny"};
         double tot = 0;
         for (int k = 0; k < PH_CYCLES; k++) tot += (double)ph[k];
         fprintf(stderr, "[qcmine] phases (grid %u waves, %.3g wave-cycles):", grid, tot);
@@ -578,12 +604,16 @@ int enumerate_persistent(const Instance* const* insts, const qc_params* params, 
 
     // per-instance outputs (the last replay's buffers; replays are identical
     // in every counter, the raw sets only in their order)
-    StreamCtr cc = first.clq;
+    // (the stream's counters run ahead of the raw sets: refs and slots are
+    // taken several at a time)
+    StreamCtr cc{raw_k, raw_nv};
+    DBuf d_sets;  // the raw sets' refs, instances in order
     {
         std::vector<uint64_t> go;
         std::vector<uint32_t> gv;
-        if ((rc = collect_raw(ws.clq_refs.as<CliqueRef>(), ws.clq_verts.as<uint32_t>(), cc.items, cc.slots, go, gv,
-                              s)))
+        const uint64_t taken = std::min<uint64_t>(last_items, clq_refs);
+        if ((rc = collect_raw(ws.clq_refs.as<CliqueRef>(), taken, ws.clq_verts.as<uint32_t>(), cc.items, cc.slots, go, gv,
+                              d_sets, s)))
             return rc;
         if (count == 1) {
             outs[0].raw_off = std::move(go);
@@ -632,7 +662,7 @@ int enumerate_persistent(const Instance* const* insts, const qc_params* params, 
                t.sum_t_written, (unsigned long long)first.ctr[2 * nr], t.raw_cliques, t.sum_clique_len);
         printf("\nTASKS SIZE: %llu\nBUFFER SIZE: %llu\nCLIQUES SIZE: %llu\nCLIQUES OFFSET SIZE: %llu\n\n",
                (unsigned long long)pool_cap, (unsigned long long)first.ctr[2 * nr],
-               (unsigned long long)first.clq.slots, (unsigned long long)first.clq.items);
+               (unsigned long long)raw_nv, (unsigned long long)raw_k);
         fflush(stdout);
     }
     // RemoveNonMax runs on the raw sets where the kernel left them, all
@@ -657,7 +687,7 @@ int enumerate_persistent(const Instance* const* insts, const qc_params* params, 
         NmInput in;
         in.k = cc.items;
         in.nv = cc.slots;
-        in.refs = ws.clq_refs.as<CliqueRef>();
+        in.refs = d_sets.as<CliqueRef>();
         in.verts = ws.clq_verts.as<uint32_t>();
         in.base = d_base.as<uint32_t>();
         in.limit = d_limit.as<uint32_t>();

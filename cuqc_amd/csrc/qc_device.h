@@ -49,7 +49,7 @@ __host__ __device__ constexpr uint32_t pow2_at_least(uint32_t x) {
 // per-vertex int arrays of pow2(tcap) entries, then (`mat`) the task-local
 // 1-hop / 2-hop matrices (tcap rows of ceil(tcap/64) words), then two masks of
 // `mwords` words (ceil(tcap/64) with local matrices, rw in root space).
-__host__ __device__ constexpr size_t ws_bytes(uint32_t tcap, bool mat, uint32_t mwords) {
+__host__ __device__ __attribute__((always_inline)) constexpr size_t ws_bytes(uint32_t tcap, bool mat, uint32_t mwords) {
     uint32_t T2 = pow2_at_least(tcap < 64 ? 64 : tcap);
     uint32_t W = (tcap + 63) / 64;
     size_t b = 0;
@@ -87,6 +87,14 @@ struct CliqueRef {
     uint32_t len;
     uint32_t inst;
 };
+
+// clique stream of the persistent form: refs and vertex slots a wave takes at
+// a time, and the instance of a ref that holds no set
+constexpr int CLQ_REFS = 32;
+constexpr int CLQ_SLOTS = 2048;
+constexpr uint32_t CLQ_NONE = 0xFFFFFFFFu;
+// most tasks of at most 64 vertices a wave keeps in its dynamic LDS
+constexpr uint32_t TINY_STACK_MAX = 256;
 
 // Counters of one output stream (children or cliques).
 struct StreamCtr {
@@ -220,6 +228,8 @@ struct ExpandArgs {
     long long* trace_parent;
     unsigned int* trace_beyond;  // per slot: children past the depth window
 
+    uint32_t tiny_cap;               // persistent mode: tasks of 64 vertices that the dynamic LDS holds
+                                     // (tiny_run; 0: tasks of that size take the general path)
     int32_t n_buckets;               // 1 = FIFO
     int32_t n_roots;                 // root tasks of the launch (root split width)
     int32_t q_shards;                // rings per bucket (ring b q_shards + s; wave w uses shard w mod q_shards)
@@ -256,6 +266,7 @@ enum PhaseId {
     PH_POP,           // persistent form: taking the next task (own stack, rings)
     PH_GIVE,          // persistent form: deciding on and making hand-overs from the own stack
     PH_SYNC,          // persistent form: a ring claim's acquire and the cells' return
+    PH_TINY,          // subtrees of at most 64 vertices, in registers
     PH_CYCLES,        // (the entries above count cycles, the ones below events)
     PH_N_OWN = PH_CYCLES,  // tasks taken from the wave's own stack
     PH_N_RING,        // tasks taken from the rings

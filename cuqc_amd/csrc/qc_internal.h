@@ -232,11 +232,11 @@ int nonmax_run(const NmInput& in, char* scratch, size_t scratch_bytes, const NmO
 // nonmax_run in allocated scratch, results copied to the host per instance
 int remove_nonmax_sets(const NmInput& in, int n_inst, std::vector<std::vector<uint64_t>*> mo,
                        std::vector<std::vector<uint32_t>*> mv, hipStream_t s);
-// the raw sets of a persistent launch's clique stream (k refs, nv vertex
-// slots) as one array, instances in order and each instance's sets in
-// vertex-slot order, on the host
-int collect_raw(const CliqueRef* d_refs, const uint32_t* d_verts, uint64_t k, uint64_t nv, std::vector<uint64_t>& off,
-                std::vector<uint32_t>& v, hipStream_t s);
+// the raw sets of a persistent launch's clique stream (k sets of nv vertices
+// among `taken` refs) as one array, instances in order and each instance's sets
+// in vertex-slot order, on the host; their refs in that order stay in `sets`
+int collect_raw(const CliqueRef* d_refs, uint64_t taken, const uint32_t* d_verts, uint64_t k, uint64_t nv,
+                std::vector<uint64_t>& off, std::vector<uint32_t>& v, DBuf& sets, hipStream_t s);
 // host raw sets (uploaded once); distinct: no set names a vertex twice (a
 // search's own raw sets), so the cover filter may be used: its masks test
 // subsets of vertices, while a caller's sets are compared as multisets
