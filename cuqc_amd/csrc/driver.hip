@@ -2,8 +2,9 @@
 // the reference's search() loop (main.cu:606-678) on the device.
 //
 // Tasks wait on two LIFO stacks (vertex pool in HBM, task refs mirrored on
-// the host): tasks of at most `TL` vertices are expanded from LDS by
-// expand_local<TL>, larger ones from per-wave HBM slabs by expand_hbm.  Each
+// the host): tasks of at most `TL` vertices, launched with many waves per CU,
+// and larger ones, launched with a quarter of a CU's LDS and an HBM slab per
+// wave.  Each
 // host iteration pops a batch from the top of one stack (large first), runs
 // one launch, and pushes the children it wrote back on top, so the search
 // proceeds depth-first in batches, like the reference's width-bounded levels
@@ -20,9 +21,7 @@
 #include "qc_internal.h"
 
 namespace qcdev {
-template <int TL>
-__global__ void expand_local(const ExpandArgs*);
-__global__ void expand_hbm(const ExpandArgs*);
+__global__ void expand_level(const ExpandArgs*);
 }  // namespace qcdev
 
 namespace qc {
@@ -35,15 +34,6 @@ struct Stack {
     uint64_t top = 0;              // slots in use
     std::vector<TaskRef> refs;     // host mirror, increasing off
 };
-
-size_t slab_bytes_for(uint32_t tcap, uint32_t rw) {
-    uint32_t T2 = 64;
-    while (T2 < tcap) T2 <<= 1;
-    size_t b = (size_t)15 * T2 * 4;
-    b = (b + 15) & ~(size_t)15;
-    b += (size_t)2 * rw * 8;
-    return (b + 255) & ~(size_t)255;
-}
 
 }  // namespace
 
@@ -113,20 +103,23 @@ int enumerate_plain(const Instance& I, const qc_params& p, EnumOut& out, hipStre
     QC_HIP(hipMemsetAsync(d_stats.p, 0, sizeof(DevStats), s));
     QC_HIP(hipMemsetAsync(d_err.p, 0, sizeof(int), s));
 
-    // HBM slabs for tasks above the LDS tile (root-space addressing)
-    const uint32_t slab_tcap = (uint32_t)I.R;
-    const size_t slab_b = slab_bytes_for(slab_tcap, (uint32_t)I.rw);
-    uint32_t n_slabs = 256;
-    while (n_slabs > 1 && (size_t)n_slabs * slab_b > budget / 8) n_slabs >>= 1;
-    DBuf d_slab;
-    if ((rc = d_slab.alloc((size_t)n_slabs * slab_b))) return rc;
-
     int dev = 0;
     QC_HIP(hipGetDevice(&dev));
     int n_cu = 0;
     QC_HIP(hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, dev));
+    // HBM slabs, one per wave of a large-task launch: 4 waves per CU, as many as
+    // LARGE_LDS allows.  Small tasks fit SMALL_LDS (a task of 64 vertices' children;
+    // the arrays of up to 256 vertices with any rows that are staged).
+    constexpr size_t LARGE_LDS = 79 * 512, SMALL_LDS = 64 * 256;
+    const size_t slab_b = wide_slab_bytes((uint32_t)I.R);
+    uint32_t n_slabs = (uint32_t)std::max(1, n_cu) * 4;
+    while (n_slabs > 1 && (size_t)n_slabs * slab_b > budget / 8) n_slabs >>= 1;
     const uint32_t small_grid_max =
         p.workgroups > 0 ? (uint32_t)p.workgroups : (uint32_t)std::max(1, n_cu) * 16;
+    // (a small task only needs its slab for degrees beyond the LDS form's fields)
+    const size_t small_slab_b = wide_slab_bytes(std::min<uint32_t>(TL, (uint32_t)I.R));
+    DBuf d_slab;
+    if ((rc = d_slab.alloc(std::max((size_t)n_slabs * slab_b, (size_t)small_grid_max * small_slab_b)))) return rc;
 
     // ---- root ----
     // (a window's leading removals applied at once when they are many)
@@ -162,8 +155,7 @@ int enumerate_plain(const Instance& I, const qc_params& p, EnumOut& out, hipStre
     A.clq_vert_cap = clq_slots;
     A.slab = d_slab.as<char>();
     A.slab_bytes = slab_b;
-    A.slab_tcap = slab_tcap;
-    A.slab_mwords = (uint32_t)I.rw;
+    A.slab_tcap = (uint32_t)I.R;
     A.stats = d_stats.as<DevStats>();
     A.error = d_err.as<int>();
     A.g.root_b0 = cut.b0;
@@ -243,22 +235,15 @@ int enumerate_plain(const Instance& I, const qc_params& p, EnumOut& out, hipStre
         A.in_refs = d_in_refs.as<TaskRef>();
         A.in_verts = S.verts.as<Vrec>();
         A.n_in = (uint32_t)take;
+        A.lds_bytes = (uint32_t)(k == 1 ? LARGE_LDS : SMALL_LDS);
+        A.slab_bytes = k == 1 ? slab_b : small_slab_b;
         QC_HIP(hipMemcpyAsync(d_args.p, &A, sizeof(A), hipMemcpyHostToDevice, s));
         QC_HIP(hipMemsetAsync(d_ctr.p, 0, 2 * sizeof(StreamCtr), s));
         QC_HIP(hipMemsetAsync(d_task_ctr.p, 0, sizeof(unsigned int), s));
         QC_HIP(hipEventRecord(e0, s));
-        if (k == 1) {
-            uint32_t grid = std::min<uint32_t>((uint32_t)take, n_slabs);
-            hipLaunchKernelGGL(qcdev::expand_hbm, dim3(grid), dim3(64), 0, s, d_args.as<ExpandArgs>());
-        } else {
-            uint32_t grid = std::min<uint32_t>((uint32_t)take, small_grid_max);
-            if (TL == 64)
-                hipLaunchKernelGGL(qcdev::expand_local<64>, dim3(grid), dim3(64), 0, s, d_args.as<ExpandArgs>());
-            else if (TL == 128)
-                hipLaunchKernelGGL(qcdev::expand_local<128>, dim3(grid), dim3(64), 0, s, d_args.as<ExpandArgs>());
-            else
-                hipLaunchKernelGGL(qcdev::expand_local<256>, dim3(grid), dim3(64), 0, s, d_args.as<ExpandArgs>());
-        }
+        const uint32_t grid = std::min<uint32_t>((uint32_t)take, k == 1 ? n_slabs : small_grid_max);
+        hipLaunchKernelGGL(qcdev::expand_level, dim3(grid), dim3(64), k == 1 ? LARGE_LDS : SMALL_LDS, s,
+                           d_args.as<ExpandArgs>());
         QC_HIP(hipGetLastError());
         QC_HIP(hipEventRecord(e1, s));
         StreamCtr oc[2];

@@ -6,14 +6,15 @@
 // remove-one-vertex, add-one-vertex with diameter and degree pruning,
 // critical-vertex pruning, the clique test and the Q-ordered child write.
 //
+// Three forms of the same steps, by the task's size: up to 64 vertices in
+// registers, with the whole subtree below (tiny_*); up to what the wave's LDS
+// holds (WideLds); larger ones from the wave's HBM slab (WideSlab).
+//
 // Adjacency.  Every task is a subset of the root task, so vertex ids are
 // root-local (0..R-1) and the 1-hop / 2-hop relations are kept as R x R bit
-// matrices in HBM (A1, A2).  A task of t <= TL vertices is staged in LDS
-// together with its own t x t sub-matrices (row = position in the task
-// record as loaded), so each pruning step is a row AND mask popcount; larger
-// tasks run from a per-wave HBM slab and address A1/A2 directly.  Where the
-// reference scans adjacency lists through its id->position map
-// (vertex_order_map), this code tests bits: the two are the same relation.
+// matrices in HBM (A1, A2).  Where the reference scans adjacency lists through
+// its id->position map (vertex_order_map), this code tests bits: the two are
+// the same relation.
 //
 // Semantics follow the host column of the reference (main.cu:1349-2198),
 // including the two degree-update branches of a degree-pruning round
@@ -110,82 +111,7 @@ __device__ __forceinline__ uint64_t wave_min_u64(uint64_t v) {
 __device__ __forceinline__ int wave_max(int v) {
     return wave_reduce32(v, INT32_MIN, [](int x, int y) { return max(x, y); });
 }
-// inclusive prefix sum across the wave
-__device__ __forceinline__ long long wave_incl_scan64(long long v) {
-    int l = lane_id();
-#pragma unroll
-    for (int o = 1; o < WAVE; o <<= 1) {
-        long long u = __shfl_up(v, o, WAVE);
-        if (l >= o) v += u;
-    }
-    return v;
-}
-
 __device__ __forceinline__ void wsync() { __syncthreads(); }
-
-__device__ __forceinline__ bool gbit(const uint64_t* M, int W, int row, int col) {
-    return (M[(size_t)row * W + (col >> 6)] >> (col & 63)) & 1ull;
-}
-
-// ---------------------------------------------------------------------------
-// workspace
-// ---------------------------------------------------------------------------
-struct WS {
-    int *pid, *plab, *pin, *pex, *pl2;           // parent record
-    int *cid, *cpp, *clab, *cin, *cex, *cl2;     // child under construction
-    int *rem, *rmv, *cind, *adjc;                // lists (4 x T2 ints)
-    uint64_t *khi, *klo;                         // sort keys, alias the lists
-    uint64_t *M1, *M2;                           // local matrices (LDS mode)
-    uint64_t *mk0, *mk1;                         // masks (W words each)
-    int T2;                                      // capacity rounded to 2^k
-};
-
-
-__device__ inline WS make_ws(char* base, uint32_t tcap, bool mat, uint32_t mwords) {
-    WS w;
-    uint32_t T2 = pow2_at_least(tcap < 64 ? 64 : tcap);
-    uint32_t W = (tcap + 63) / 64;
-    int* ip = (int*)base;
-    w.pid = ip; ip += T2;
-    w.plab = ip; ip += T2;
-    w.pin = ip; ip += T2;
-    w.pex = ip; ip += T2;
-    w.pl2 = ip; ip += T2;
-    w.cid = ip; ip += T2;
-    w.cpp = ip; ip += T2;
-    w.clab = ip; ip += T2;
-    w.cin = ip; ip += T2;
-    w.cex = ip; ip += T2;
-    w.cl2 = ip; ip += T2;
-    w.rem = ip; ip += T2;
-    w.rmv = ip; ip += T2;
-    w.cind = ip; ip += T2;
-    w.adjc = ip; ip += T2;
-    w.khi = (uint64_t*)w.rem;
-    w.klo = (uint64_t*)w.cind;
-    size_t b = (size_t)15 * T2 * 4;
-    b = (b + 15) & ~(size_t)15;
-    uint64_t* up = (uint64_t*)(base + b);
-    if (mat) {
-        w.M1 = up; up += (size_t)tcap * W;
-        w.M2 = up; up += (size_t)tcap * W;
-    } else {
-        w.M1 = w.M2 = nullptr;
-    }
-    w.mk0 = up; up += mwords;
-    w.mk1 = up; up += mwords;
-    w.T2 = (int)T2;
-    return w;
-}
-
-// per-vertex arrays at `arrays` (LDS), masks of `mwords` words at `masks`
-// (root space, in the wave's HBM slab); no local matrices
-__device__ inline WS make_ws_split(char* arrays, uint32_t tcap, uint64_t* masks, uint32_t mwords) {
-    WS w = make_ws(arrays, tcap, false, 0);
-    w.mk0 = masks;
-    w.mk1 = masks + mwords;
-    return w;
-}
 
 // ---------------------------------------------------------------------------
 // per-task state
@@ -225,14 +151,9 @@ __device__ __forceinline__ GConst load_graph(const DevGraph* p) {
 struct Ctx {
     const ExpandArgs* a;
     GConst g;             // tables of the instance being expanded
-    WS w;
-    const uint64_t* M1;   // matrix used for tests (local or root space)
-    const uint64_t* M2;
-    int W;                // words per row of M1/M2 = words per mask
     int lane;
     LStats* st;           // counters of this wave (LDS; lane 0 updates them)
     uint32_t depth;
-    uint32_t cap;         // largest task the workspace holds
     uint32_t inst;        // instance of the task being expanded
     long long slot;       // queue slot of the task being expanded (trace)
     unsigned long long* ph;           // phase cycles (LDS, diagnostics)
@@ -288,49 +209,6 @@ __device__ __forceinline__ int get_mindeg(const Ctx& c, int s) {
     return s < ms ? md(c, ms) : md(c, s);
 }
 
-// main.cu:2153-2173
-__device__ __forceinline__ bool cand_valid(const Ctx& c, int in, int ex, int m, int ub, int lb, int med) {
-    int tot = in + ex;
-    if (tot < md(c, c.g.min_size)) return false;
-    if (tot < get_mindeg(c, m + ex + 1)) return false;
-    if (tot < med) return false;
-    if (in + ub - 1 < md(c, m + lb)) return false;
-    if (tot < get_mindeg(c, m + lb)) return false;
-    return true;
-}
-// main.cu:2175-2198
-__device__ __forceinline__ bool vert_ext(const Ctx& c, int in, int ex, int m, int ub, int lb, int med) {
-    int tot = in + ex;
-    if (tot < md(c, c.g.min_size)) return false;
-    if (tot < get_mindeg(c, m + ex)) return false;
-    if (tot < med) return false;
-    if (ex == 0 && in < get_mindeg(c, m + ex)) return false;
-    if (in + ub < md(c, m + ub)) return false;
-    if (tot < get_mindeg(c, m + lb)) return false;
-    return true;
-}
-
-__device__ __forceinline__ int rowpop(const Ctx& c, const uint64_t* M, int row, const uint64_t* mask) {
-    const uint64_t* r = M + (size_t)row * c.W;
-    int s = 0;
-    for (int w = 0; w < c.W; w++) s += __popcll(r[w] & mask[w]);
-    return s;
-}
-// rowpop with four independent loads per step (the gather latency
-// overlapped), for the loops that run it over whole records
-__device__ __forceinline__ int rowpop4(const Ctx& c, const uint64_t* M, int row, const uint64_t* mask) {
-    const uint64_t* r = M + (size_t)row * c.W;
-    const int W = c.W;
-    int s0 = 0, s1 = 0, w = 0;
-    for (; w + 4 <= W; w += 4) {
-        const uint64_t x0 = r[w], x1 = r[w + 1], x2 = r[w + 2], x3 = r[w + 3];
-        s0 += __popcll(x0 & mask[w]) + __popcll(x2 & mask[w + 2]);
-        s1 += __popcll(x1 & mask[w + 1]) + __popcll(x3 & mask[w + 3]);
-    }
-    for (; w < W; w++) s0 += __popcll(r[w] & mask[w]);
-    return s0 + s1;
-}
-
 // W_adj bookkeeping: adjacency entries the reference's list scans visit
 // (restricted to root vertices), summed over ids.  Each lane keeps its own
 // partial sum; the wave sums them when the counters are flushed.
@@ -341,593 +219,8 @@ __device__ __forceinline__ void wadj_lanes(Ctx& c, long long x) {  // x per lane
     c.wadj_l += x;
 }
 
-__device__ inline void clear_mask(Ctx& c, uint64_t* mk) {
-    for (int w = c.lane; w < c.W; w += WAVE) mk[w] = 0;
-    wsync();
-}
-
 __device__ inline void set_mask_bit(uint64_t* mk, int b) {
     atomicOr((unsigned long long*)&mk[b >> 6], 1ull << (b & 63));
-}
-
-// descending sort of ints a[0..n) (bitonic, padded with INT_MIN)
-__device__ void sort_desc_int(Ctx& c, int* a, int n) {
-    if (n <= 1) return;
-    int n2 = 1;
-    while (n2 < n) n2 <<= 1;
-    for (int i = n + c.lane; i < n2; i += WAVE) a[i] = INT32_MIN;
-    wsync();
-    for (int k = 2; k <= n2; k <<= 1) {
-        for (int j = k >> 1; j > 0; j >>= 1) {
-            for (int i = c.lane; i < n2; i += WAVE) {
-                int ixj = i ^ j;
-                if (ixj > i) {
-                    int x = a[i], y = a[ixj];
-                    bool desc = (i & k) == 0;
-                    if (desc ? (x < y) : (x > y)) {
-                        a[i] = y;
-                        a[ixj] = x;
-                    }
-                }
-            }
-            wsync();
-        }
-    }
-}
-
-// ascending sort of 128-bit keys (hi, lo) over [0, n)
-__device__ void sort_keys(Ctx& c, uint64_t* hi, uint64_t* lo, int n) {
-    if (n <= 1) return;
-    int n2 = 1;
-    while (n2 < n) n2 <<= 1;
-    for (int i = n + c.lane; i < n2; i += WAVE) {
-        hi[i] = ~0ull;
-        lo[i] = ~0ull;
-    }
-    wsync();
-    for (int k = 2; k <= n2; k <<= 1) {
-        for (int j = k >> 1; j > 0; j >>= 1) {
-            for (int i = c.lane; i < n2; i += WAVE) {
-                int ixj = i ^ j;
-                if (ixj > i) {
-                    uint64_t xh = hi[i], xl = lo[i], yh = hi[ixj], yl = lo[ixj];
-                    bool gt = xh > yh || (xh == yh && xl > yl);
-                    bool asc = (i & k) == 0;
-                    if (asc == gt) {
-                        hi[i] = yh;
-                        lo[i] = yl;
-                        hi[ixj] = xh;
-                        lo[ixj] = xl;
-                    }
-                }
-            }
-            wsync();
-        }
-    }
-}
-
-// ---------------------------------------------------------------------------
-// Candidate indegrees for the LU bounds.  The bounds only need P(k), the sum
-// of the k largest indegrees (main.cu:1919-1940 walks them sorted), and
-// indegrees lie in [0, m].  With the suffix counts C[v] = #{x >= v},
-// P(k) = sum over v >= 1 of min(C[v], k): each of the k largest values x
-// adds 1 for every v in [1, x].
-//   m < 64: lane v holds C[v] in a register (creg, one ballot per value and
-//           chunk); reg = true.
-//   else:   tables C[v] (in adjc) and suffix sums S[v] = sum{x : x >= v}
-//           (in cind), v in [0, V + 1]; P(k) = S[v + 1] + (k - C[v + 1]) v
-//           with v the largest value whose C[v] >= k.
-// Returns V = the largest value, or -1 when the tables do not fit (the
-// caller sorts).
-// ---------------------------------------------------------------------------
-// One chunk of candidate indegrees (x < 0: no value in this lane) into the
-// register table of the m < 64 case: lane v counts the values >= v, V is the
-// largest value.  Loops that produce the indegrees call it on the values in
-// their registers, so the table costs no pass of its own.
-__device__ __forceinline__ void hist_chunk(const Ctx& c, int x, int& creg, int& V) {
-    const int top = uni(wave_max(x));
-    V = max(V, top);
-    for (int v = 1; v <= top; v++) {
-        const int k = __popcll(ballot(x >= v));
-        if (c.lane == v) creg += k;
-    }
-}
-
-__device__ int indeg_dist(Ctx& c, int n, int m, int& creg, bool& reg) {
-    WS& w = c.w;
-    if (m < WAVE) {
-        int cnt = 0, V = 0;
-        for (int base = 0; base < n; base += WAVE) {
-            const int i = base + c.lane;
-            hist_chunk(c, i < n ? w.cind[i] : -1, cnt, V);
-        }
-        creg = cnt;
-        reg = true;
-        return V;
-    }
-    reg = false;
-    int mx = 0;
-    for (int i = c.lane; i < n; i += WAVE) mx = max(mx, w.cind[i]);
-    const int V = uni(wave_max(mx));
-    if (V + 2 > w.T2) return -1;
-    int* C = w.adjc;
-    int* S = w.cind;
-    for (int v = c.lane; v <= V + 1; v += WAVE) C[v] = 0;
-    wsync();
-    for (int i = c.lane; i < n; i += WAVE) atomicAdd(&C[w.cind[i]], 1);
-    wsync();
-    // suffix scans from the top bin down: C <- counts >= v, S <- sums >= v
-    long long cc = 0, cs = 0;
-    for (int top = V; top >= 0; top -= WAVE) {
-        const int v = top - c.lane;  // lane 0 holds the highest bin of the chunk
-        const long long h = v >= 0 ? C[v] : 0;
-        const long long ic = wave_incl_scan64(h) + cc;
-        const long long is = wave_incl_scan64(h * (v >= 0 ? v : 0)) + cs;
-        cc = (long long)rdlane64((unsigned long long)ic, WAVE - 1);
-        cs = (long long)rdlane64((unsigned long long)is, WAVE - 1);
-        wsync();
-        if (v >= 0) {
-            C[v] = (int)ic;
-            S[v] = (int)is;
-        }
-        wsync();
-    }
-    if (c.lane == 0) {
-        C[V + 1] = 0;
-        S[V + 1] = 0;
-    }
-    wsync();
-    return V;
-}
-
-// P(k) = sum_{v=1..V} min(C[v], k) with lane v's register holding C[v]
-__device__ __forceinline__ int top_sum_reg(int creg, int V, int k) {
-    int p = 0;
-    for (int v = 1; v <= V; v++) p += min(__builtin_amdgcn_readlane(creg, v), k);
-    return p;
-}
-
-// P(k) from the distribution tables (k <= n)
-__device__ __forceinline__ long long top_sum(const WS& w, int V, int k) {
-    if (k <= 0) return 0;
-    const int* C = w.adjc;
-    const int* S = w.cind;
-    int lo = 0, hi = V;  // C[0] = n >= k
-    while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (C[mid] >= k)
-            lo = mid;
-        else
-            hi = mid - 1;
-    }
-    return (long long)S[lo + 1] + (long long)(k - C[lo + 1]) * lo;
-}
-
-// ---------------------------------------------------------------------------
-// LU bounds, main.cu:1857-1972.  Members are child positions [0, m).  With
-// V >= 0 the candidate indegrees are given by indeg_dist (creg / reg), with
-// V < 0 cind[0..nc) holds them sorted descending.
-// ---------------------------------------------------------------------------
-__device__ bool lu_bounds(Ctx& c, int m, int nc, int& ub, int& lb, int& med, int V, int creg, bool reg) {
-    WS& w = c.w;
-    const ExpandArgs& a = *c.a;
-    // one pass: the smallest (indeg, exdeg) pair in lexicographic order
-    // gives min_in and the smallest exdeg among the members at min_in
-    uint64_t min_pair = ((uint64_t)INT32_MAX << 32) | (uint64_t)INT32_MAX;
-    int min_tot = INT32_MAX;
-    long long sum_in = 0;
-    for (int i = c.lane; i < m; i += WAVE) {
-        int in = w.cin[i], ex = w.cex[i];
-        min_pair = min(min_pair, ((uint64_t)(uint32_t)in << 32) | (uint32_t)ex);
-        min_tot = min(min_tot, in + ex);
-        sum_in += in;
-    }
-    min_pair = wave_min_u64(min_pair);
-    const int min_in = uni((int)(min_pair >> 32));
-    const int min_in_ex = uni((int)(uint32_t)min_pair);
-    min_tot = uni(wave_min(min_tot));
-    sum_in = wave_sum64(sum_in);
-
-    bool invalid = false;
-    med = get_mindeg(c, m + 1);
-    if (min_in < md(c, m)) {
-        int lb0 = get_mindeg(c, m) - min_in;
-        // first x >= lb0 with x > min_in_ex || min_in + x >= mindeg[m + x]
-        int x = lb0;
-        for (;;) {
-            int y = x + c.lane;
-            bool stop = (y > min_in_ex) || (min_in + y >= md(c, m + y));
-            uint64_t bm = ballot(stop);
-            if (bm) {
-                x += __builtin_ctzll(bm);
-                break;
-            }
-            x += WAVE;
-        }
-        lb = x;
-        if (min_in + lb < md(c, m + lb)) {
-            lb = nc + 1;
-            invalid = true;
-        }
-        // (a stale exdeg can make the sum negative: floor(d / gamma) is then
-        // below 0 and the bound too)
-        int tq = min_tot < 0 ? -1 : c.g.p->ubq[min(min_tot, c.g.ubq_n - 1)];
-        ub = tq + 1 - m;
-        if (ub > nc) ub = nc;
-        if (lb < ub) {
-            // P(idx) = sum of the idx largest candidate indegrees;
-            // cond(idx) = sum_in + P(idx) >= m * mindeg[m + idx]
-            // i0 = first idx in [lb, ub) with cond, else ub
-            long long carry = 0;
-            int first = -1, last = -1;
-            for (int base = 0; base <= ub; base += WAVE) {
-                int idx = base + c.lane;  // P(idx) = prefix over [0, idx)
-                long long inc;
-                if (V >= 0 && reg) {
-                    inc = top_sum_reg(creg, V, idx);
-                } else if (V >= 0) {
-                    inc = idx <= ub ? top_sum(w, V, idx) : 0;
-                } else {
-                    long long v = (idx - 1 >= 0 && idx - 1 < nc && idx <= ub) ? (long long)w.cind[idx - 1] : 0;
-                    inc = wave_incl_scan64(v) + carry;  // = P(idx)
-                    carry = (long long)rdlane64((unsigned long long)inc, WAVE - 1);
-                }
-                bool inr = idx <= ub;
-                bool cnd = inr && (sum_in + inc >= (long long)m * md(c, m + idx));
-                uint64_t bfirst = ballot(cnd && idx >= lb);
-                if (first < 0 && bfirst) first = base + __builtin_ctzll(bfirst);
-                uint64_t blast = ballot(cnd && idx >= lb);
-                if (blast) last = base + 63 - __builtin_clzll(blast);
-            }
-            first = uni(first);
-            last = uni(last);
-            if (first < 0) {
-                lb = ub + 1;
-                invalid = true;
-            } else {
-                // the reference's first loop stops at idx == ub even when
-                // cond(ub) is false; first > ub is impossible here
-                lb = first;
-                int tub = last > first ? last : first;
-                if (ub > tub) ub = tub;
-                if (lb > 1) med = get_mindeg(c, m + lb);
-            }
-        }
-    } else {
-        ub = nc;
-        int ms = c.g.min_size;
-        lb = m < ms ? ms - m : 0;
-    }
-    if (m + ub < c.g.min_size) invalid = true;
-    if (ub < 0 || ub < lb) invalid = true;
-    return invalid;
-}
-
-__device__ inline bool members_fail(Ctx& c, int m, int ub, int lb, int med) {
-    bool f = false;
-    for (int k = c.lane; k < m; k += WAVE)
-        if (!vert_ext(c, c.w.cin[k], c.w.cex[k], m, ub, lb, med)) f = true;
-    return ballot(f) != 0;
-}
-
-// ---------------------------------------------------------------------------
-// degree pruning, main.cu:1735-1855.  cind[0..nind) = candidate indegrees.
-// ---------------------------------------------------------------------------
-// map_empty: the reference's id->position map holds no entry during this call
-// (critical-vertex pruning without critical-adjacent candidates).  pre_V >= 0:
-// the caller built the register table of cind[0..nind) (pre_V, pre_creg).
-__device__ __attribute__((always_inline)) bool degree_pruning(Ctx& c, int& tc, int& nc, int m, int& ub, int& lb,
-                                                              int& med, int nind, bool map_empty, int pre_V,
-                                                              int pre_creg) {
-    WS& w = c.w;
-    ph_mark(c, PH_PRUNE);
-    int creg = pre_creg;
-    bool reg = pre_V >= 0;
-    int V = pre_V;
-    if (!reg) {
-        V = indeg_dist(c, nind, m, creg, reg);
-        if (V < 0) sort_desc_int(c, w.cind, nind);
-    }
-    ph_mark(c, PH_HIST);
-    if (lu_bounds(c, m, nind, ub, lb, med, V, creg, reg) || members_fail(c, m, ub, lb, med)) {
-        ph_mark(c, PH_LU);
-        return true;
-    }
-    ph_mark(c, PH_LU);
-    // classify candidates, stable; first_out = the smallest position ever
-    // removed (positions below it stay in place in the compaction)
-    int nrem = 0, nrmv = 0, first_out = tc;
-    for (int base = m; base < tc; base += WAVE) {
-        int i = base + c.lane;
-        bool in = i < tc;
-        bool ok = in && w.clab[i] == 0 && cand_valid(c, w.cin[i], w.cex[i], m, ub, lb, med);
-        uint64_t bo = ballot(ok), bx = ballot(in && !ok);
-        if (ok) w.rem[nrem + lanes_below(bo)] = i;
-        if (in && !ok) w.rmv[nrmv + lanes_below(bx)] = i;
-        if (first_out == tc && bx) first_out = base + __builtin_ctzll(bx);
-        nrem += __popcll(bo);
-        nrmv += __popcll(bx);
-    }
-    wsync();
-    ph_mark(c, PH_COMPACT);
-    while (nrem > 0 && nrmv > 0) {
-        // degree update, main.cu:1775-1807
-        {
-            const bool rc = nrem < nrmv;
-            const int nl = rc ? nrem : nrmv;
-            const int* L = rc ? w.rem : w.rmv;
-            long long sw = 0;
-            for (int k = c.lane; k < nl; k += WAVE) sw += c.g.p->d1r[w.cid[L[k]]];
-            wadj_lanes(c, sw);
-        }
-        // only members and remaining candidates are updated: the removed
-        // ones never return, so their exdeg is never read again.  The same
-        // pass gathers the indegrees of the remaining candidates that are
-        // valid under the previous bounds with the new exdeg
-        // (main.cu:1811-1815).
-        const int nupd = m + nrem;
-        const bool rc = nrem < nrmv;
-        const int nl = rc ? nrem : nrmv;
-        const int* L = rc ? w.rem : w.rmv;
-        // 0: exdeg unchanged, 1: all zero (empty map, recompute),
-        // 2: bit tests against few vertices, 3: row popcounts against a mask
-        const int mode = map_empty ? (rc ? 1 : 0) : (nl < c.W ? 2 : 3);
-        if (mode == 2) {
-            for (int k = c.lane; k < nl; k += WAVE) w.adjc[k] = w.cpp[L[k]];
-            wsync();
-        } else if (mode == 3) {
-            clear_mask(c, w.mk0);
-            for (int k = c.lane; k < nl; k += WAVE) set_mask_bit(w.mk0, w.cpp[L[k]]);
-            wsync();
-        }
-        int nv = 0, hV = 0, hc = 0;
-        for (int base = 0; base < nupd; base += WAVE) {
-            const int j = base + c.lane;
-            bool ok = false;
-            int in = 0;
-            if (j < nupd) {
-                const int i = j < m ? j : w.rem[j - m];
-                int ex = w.cex[i];
-                if (mode == 1) {
-                    ex = 0;
-                } else if (mode >= 2) {
-                    int cnt = 0;
-                    if (mode == 2) {
-                        const int row = w.cpp[i];
-                        for (int k = 0; k < nl; k++) cnt += (int)gbit(c.M1, c.W, row, w.adjc[k]);
-                    } else {
-                        cnt = rowpop(c, c.M1, w.cpp[i], w.mk0);
-                    }
-                    ex = rc ? cnt : ex - cnt;
-                }
-                if (mode != 0) w.cex[i] = ex;
-                if (j >= m) {
-                    in = w.cin[i];
-                    ok = cand_valid(c, in, ex, m, ub, lb, med);
-                }
-            }
-            const uint64_t bo = ballot(ok);
-            // (with m < 64 the register table replaces the list)
-            if (ok && m >= WAVE) w.cind[nv + lanes_below(bo)] = in;
-            nv += __popcll(bo);
-            if (m < WAVE) hist_chunk(c, ok ? in : -1, hc, hV);
-        }
-        wsync();
-        ph_mark(c, PH_DEGUPD);
-        ph_mark(c, PH_COMPACT);
-        if (m < WAVE) {
-            V = hV;
-            creg = hc;
-            reg = true;
-        } else {
-            V = indeg_dist(c, nv, m, creg, reg);
-            if (V < 0) sort_desc_int(c, w.cind, nv);
-        }
-        ph_mark(c, PH_HIST);
-        if (lu_bounds(c, m, nv, ub, lb, med, V, creg, reg) || members_fail(c, m, ub, lb, med)) {
-            ph_mark(c, PH_LU);
-            return true;
-        }
-        ph_mark(c, PH_LU);
-        // re-classify the remaining set under the new bounds (in place)
-        int kept = 0;
-        nrmv = 0;
-        for (int base = 0; base < nrem; base += WAVE) {
-            int k = base + c.lane;
-            bool in = k < nrem;
-            int i = in ? w.rem[k] : 0;
-            bool ok = in && cand_valid(c, w.cin[i], w.cex[i], m, ub, lb, med);
-            uint64_t bo = ballot(ok), bx = ballot(in && !ok);
-            if (bx) first_out = min(first_out, rdlane(i, __builtin_ctzll(bx)));
-            wsync();
-            if (ok) w.rem[kept + lanes_below(bo)] = i;
-            if (in && !ok) w.rmv[nrmv + lanes_below(bx)] = i;
-            kept += __popcll(bo);
-            nrmv += __popcll(bx);
-            wsync();
-        }
-        nrem = kept;
-    }
-    // compaction: child[m + k] = child[rem[k]] (rem ascending, m + k <= rem[k]);
-    // rem[k] = m + k below first_out - m
-    ph_mark(c, PH_COMPACT);
-    for (int base = first_out - m; base < nrem; base += WAVE) {
-        int k = base + c.lane;
-        int i = 0, id = 0, pp = 0, lab = 0, in = 0, ex = 0, l2 = 0;
-        if (k < nrem) {
-            i = w.rem[k];
-            id = w.cid[i];
-            pp = w.cpp[i];
-            lab = w.clab[i];
-            in = w.cin[i];
-            ex = w.cex[i];
-            if (c.keys) l2 = w.cl2[i];
-        }
-        wsync();
-        if (k < nrem) {
-            int d = m + k;
-            w.cid[d] = id;
-            w.cpp[d] = pp;
-            w.clab[d] = lab;
-            w.cin[d] = in;
-            w.cex[d] = ex;
-            if (c.keys) w.cl2[d] = l2;
-        }
-        wsync();
-    }
-    tc = tc - nc + nrem;
-    nc = nrem;
-    ph_mark(c, PH_MOVE);
-    return false;
-}
-
-// ---------------------------------------------------------------------------
-// critical vertex pruning, main.cu:1526-1707, up to its closing degree
-// pruning: returns 2 when the task fails (the reference's 2), else 0 with the
-// arguments of the degree-pruning call that ends the step (candidate
-// indegrees in cind[0..nind), map_empty).  The caller runs that call; its
-// result gives the reference's 0 / 1.
-// ---------------------------------------------------------------------------
-__device__ __attribute__((always_inline)) int critical_prep(Ctx& c, int tc, int& nc, int& m, int lb, int& nind_out,
-                                                            bool& map_empty) {
-    WS& w = c.w;
-    int thr = md(c, m + lb);
-    // mask of critical members
-    // critical members: matrix indices listed in rmv[0..ncm)
-    int ncm = 0;
-    long long sw = 0;
-    for (int base = 0; base < m; base += WAVE) {
-        const int k = base + c.lane;
-        const bool cr = k < m && w.cin[k] + w.cex[k] == thr && w.cex[k] > 0;
-        const uint64_t bc = ballot(cr);
-        if (cr) {
-            w.rmv[ncm + lanes_below(bc)] = w.cpp[k];
-            sw += c.g.p->d1r[w.cid[k]];
-        }
-        ncm += __popcll(bc);
-    }
-    wadj_lanes(c, sw);
-    wsync();
-    // critical-adjacent candidates
-    int ncrit = 0;
-    if (ncm > 0) {
-        const bool sparse = ncm < c.W;
-        if (!sparse) {
-            clear_mask(c, w.mk0);
-            for (int k = c.lane; k < ncm; k += WAVE) set_mask_bit(w.mk0, w.rmv[k]);
-            wsync();
-        }
-        for (int base = m; base < tc; base += WAVE) {
-            int i = base + c.lane;
-            bool f = false;
-            if (i < tc) {
-                const int row = w.cpp[i];
-                if (sparse) {
-                    for (int k = 0; k < ncm && !f; k++) f = gbit(c.M1, c.W, row, w.rmv[k]);
-                } else {
-                    f = rowpop(c, c.M1, row, w.mk0) > 0;
-                }
-            }
-            ncrit += __popcll(ballot(f));
-            if (f) w.clab[i] = 4;
-        }
-        wsync();
-    }
-    if (ncrit == 0) {
-        // every candidate passes the 2-hop filter; the map stays empty
-        int nind = 0;
-        for (int base = m; base < tc; base += WAVE) {
-            int i = base + c.lane;
-            bool in = i < tc;
-            uint64_t bo = ballot(in);
-            if (in) w.cind[nind + lanes_below(bo)] = w.cin[i];
-            nind += __popcll(bo);
-        }
-        wsync();
-        nind_out = nind;
-        map_empty = true;
-        return 0;
-    }
-    // stable partition of [m, tc): label 4 first (perm in rmv, temp in cind)
-    {
-        int nf = 0, nn = 0;
-        for (int base = m; base < tc; base += WAVE) {
-            int i = base + c.lane;
-            bool in = i < tc;
-            bool f = in && w.clab[i] == 4;
-            uint64_t bf = ballot(f), bn = ballot(in && !f);
-            if (f) w.rmv[nf + lanes_below(bf)] = i;
-            if (in && !f) w.rmv[ncrit + nn + lanes_below(bn)] = i;
-            nf += __popcll(bf);
-            nn += __popcll(bn);
-        }
-        wsync();
-        int cnt = tc - m;
-        auto permute = [&](int* F) {
-            for (int k = c.lane; k < cnt; k += WAVE) w.cind[k] = F[w.rmv[k]];
-            wsync();
-            for (int k = c.lane; k < cnt; k += WAVE) F[m + k] = w.cind[k];
-            wsync();
-        };
-        permute(w.cid);
-        permute(w.cpp);
-        permute(w.clab);
-        permute(w.cin);
-        permute(w.cex);
-        if (c.keys) permute(w.cl2);
-    }
-    // add the critical-adjacent vertices: degree updates and 2-hop counts
-    const bool sparse = ncrit < c.W;
-    if (!sparse) clear_mask(c, w.mk1);
-    sw = 0;
-    for (int k = c.lane; k < ncrit; k += WAVE) {
-        if (!sparse) set_mask_bit(w.mk1, w.cpp[m + k]);
-        sw += c.g.p->d1r[w.cid[m + k]] + c.g.p->d2r[w.cid[m + k]];
-    }
-    wadj_lanes(c, sw);
-    wsync();
-    for (int i = c.lane; i < tc; i += WAVE) {
-        int pp = w.cpp[i];
-        int d1 = 0, d2 = 0;
-        if (sparse) {
-            for (int k = 0; k < ncrit; k++) {
-                const int col = w.cpp[m + k];
-                d1 += (int)gbit(c.M1, c.W, pp, col);
-                d2 += (int)gbit(c.M2, c.W, pp, col);
-            }
-        } else {
-            d1 = rowpop(c, c.M1, pp, w.mk1);
-            d2 = rowpop(c, c.M2, pp, w.mk1);
-        }
-        w.cin[i] += d1;
-        w.cex[i] -= d1;
-        w.adjc[i] = d2;
-    }
-    wsync();
-    bool fail = false;
-    for (int k = c.lane; k < m; k += WAVE)
-        if (w.adjc[k] != ncrit) fail = true;
-    for (int k = m + c.lane; k < m + ncrit; k += WAVE)
-        if (w.adjc[k] < ncrit - 1) fail = true;
-    if (ballot(fail)) return 2;
-    for (int k = m + c.lane; k < m + ncrit; k += WAVE) w.clab[k] = 1;
-    m += ncrit;
-    nc -= ncrit;
-    // diameter step around the added vertices
-    int nind = 0;
-    for (int base = m; base < tc; base += WAVE) {
-        int i = base + c.lane;
-        bool in = i < tc;
-        bool ok = in && w.adjc[i] == ncrit;
-        uint64_t bo = ballot(ok);
-        if (ok) w.cind[nind + lanes_below(bo)] = w.cin[i];
-        if (in && !ok) w.clab[i] = -1;
-        nind += __popcll(bo);
-    }
-    wsync();
-    nind_out = nind;
-    map_empty = false;
-    return 0;
 }
 
 // ---------------------------------------------------------------------------
@@ -985,13 +278,6 @@ __device__ __forceinline__ void clq_ref(Ctx& c, unsigned long long ri, unsigned 
         c.st->sum_clq += len;
     }
 }
-__device__ __attribute__((always_inline)) void emit_clique(Ctx& c, const int* ids, int len) {
-    const ExpandArgs& a = *c.a;
-    unsigned long long ri = 0, si = 0;
-    if (!clq_reserve(c, len, ri, si)) return;
-    for (int k = c.lane; k < len; k += WAVE) a.clq_verts[si + k] = c.g.p->orig[ids[k]];
-    clq_ref(c, ri, si, len);
-}
 // the vertices of the lanes in m
 __device__ __forceinline__ void emit_lanes(Ctx& c, uint64_t m, uint32_t orig) {
     const int len = __popcll(m);
@@ -1008,44 +294,12 @@ __device__ __forceinline__ void clq_close(Ctx& c) {
     for (unsigned long long i = c.clq[0] + c.lane; i < end; i += WAVE) a.clq_refs[i] = CliqueRef{0, 0, CLQ_NONE};
 }
 
-// clique test, main.cu:1974-1995
-__device__ __attribute__((always_inline)) void check_for_clique(Ctx& c, int m) {
-    int req = md(c, m);
-    bool bad = false;
-    for (int k = c.lane; k < m; k += WAVE)
-        if (c.w.cin[k] < req) bad = true;
-    if (ballot(bad)) return;
-    emit_clique(c, c.w.cid, m);
-}
-
-static __device__ __forceinline__ uint32_t label_rank(int l) {
-    return l == 1 ? 0u : l == 2 ? 1u : l == 0 ? 2u : l == 3 ? 3u : 4u;
-}
-
-// Q order (main.cu:2059-2104) as an ascending 128-bit key
-__device__ __forceinline__ void q_key(int lab, int in, int ex, int l2, int id, uint64_t& hi, uint64_t& lo) {
-    hi = ((uint64_t)label_rank(lab) << 61) | ((uint64_t)(0x3FFFFFFF - in) << 30) | (uint64_t)(0x3FFFFFFF - ex);
-    lo = ((uint64_t)(0x7FFFFFFFu - (uint32_t)l2) << 32) | (uint64_t)(0xFFFFFFFFu - (uint32_t)id);
-}
-
-// Cost-model features of a record held in child positions [0, tc) (members
-// first): members, candidates, min/max/mean indeg, min/max/mean exdeg, depth,
+// Cost-model features of a record from per-lane partial values (lane 0 holds
+// the row): members, candidates, min/max/mean indeg, min/max/mean exdeg, depth,
 // ub - lb, mean |N2 n root| over candidates, size.  Means are
 // float(sum) / float(count), as in the oracle.
-__device__ void task_features(Ctx& c, int tc, int mem, int depth, int gap, float* f /* lane 0 */) {
-    WS& w = c.w;
-    int mi = INT32_MAX, ma = INT32_MIN, me = INT32_MAX, mx = INT32_MIN;
-    long long si = 0, se = 0, s2 = 0;
-    for (int i = c.lane; i < tc; i += WAVE) {
-        int in = w.cin[i], ex = w.cex[i];
-        mi = min(mi, in);
-        ma = max(ma, in);
-        me = min(me, ex);
-        mx = max(mx, ex);
-        si += in;
-        se += ex;
-        if (i >= mem) s2 += c.g.p->d2r[w.cid[i]];
-    }
+__device__ __forceinline__ void feature_row(int tc, int mem, int depth, int gap, int mi, int ma, int me, int mx,
+                                            long long si, long long se, long long s2, float* f) {
     mi = wave_min(mi);
     ma = wave_max(ma);
     me = wave_min(me);
@@ -1053,7 +307,7 @@ __device__ void task_features(Ctx& c, int tc, int mem, int depth, int gap, float
     si = wave_sum64(si);
     se = wave_sum64(se);
     s2 = wave_sum64(s2);
-    if (c.lane == 0) {
+    if (lane_id() == 0) {
         const int cnd = tc - mem;
         f[0] = (float)mem;
         f[1] = (float)cnd;
@@ -1276,6 +530,30 @@ __device__ __attribute__((always_inline)) int ring_claim(Ctx& c, int b, int n, u
     return 0;
 }
 
+// The ring a producer's next task goes to: this wave's own shard when waves wait
+// there (head ahead of tail) or nowhere, else the shard where most wait.
+__device__ __attribute__((always_inline)) int ring_for(Ctx& c, int* waiting = nullptr) {
+    const ExpandArgs& a = *c.a;
+    if (a.q_shards == 1) return 0;
+    int w = 0;
+    if (c.lane < a.q_shards) {
+        const unsigned long long h = __hip_atomic_load(&a.q_head[c.lane * QSTRIDE], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const unsigned long long t = __hip_atomic_load(&a.q_tail[c.lane * QSTRIDE], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        w = h > t ? (int)(h - t) : 0;
+    }
+    int r = c.shard, n = rdlane(w, c.shard);
+    if (n == 0) {
+        // (the lane in the low bits: the maximum names its shard)
+        const int best = wave_max(w << 6 | c.lane);
+        if (best >> 6) {
+            r = best & 63;
+            n = best >> 6;
+        }
+    }
+    if (waiting) *waiting = n;
+    return r;
+}
+
 // Publishes positions [pos, pos + k) of bucket b (their refs are written):
 // one release fence for the wave's record and ref stores, then the
 // sequence words (lanes < k).
@@ -1329,10 +607,10 @@ __device__ __forceinline__ bool share_child(Ctx& c) {
 // then reports a capacity overflow).
 __device__ __attribute__((always_inline)) bool push_ref(Ctx& c, const TaskRef& r, int bkt, bool shared, const float* feat) {
     const ExpandArgs& a = *c.a;
-    const int rg = bkt * a.q_shards + c.shard;
     for (int pass = 0; pass < 2; pass++) {
         const bool ring = (pass == 0) == (shared || !a.use_priv);
         if (ring) {
+            const int rg = ring_for(c);
             unsigned long long pos = 0;
             if (ring_claim(c, rg, 1, &pos) == 1) {
                 const unsigned long long gi = (unsigned long long)rg * a.q_cap + pos % a.q_cap;
@@ -1399,97 +677,6 @@ __device__ __forceinline__ TaskRef bcast_ref(const TaskRef& mine, int l) {
     TaskRef r;
     __builtin_memcpy(&r, w, sizeof(r));
     return r;
-}
-
-__device__ __attribute__((always_inline)) void write_child(Ctx& c, int tc, int mem, int gap) {
-    const ExpandArgs& a = *c.a;
-    WS& w = c.w;
-    if (c.g.max_depth >= 0 && (int)c.depth + 1 > c.g.max_depth) {
-        // outside the depth window: counted, never expanded
-        if (c.lane == 0) {
-            c.st->children++;
-            c.st->sum_tw += tc;
-            c.st->beyond++;
-            if (a.trace_beyond && c.slot >= 0) atomicAdd(&a.trace_beyond[c.slot], 1u);
-        }
-        return;
-    }
-    for (int i = c.lane; i < tc; i += WAVE) q_key(w.clab[i], w.cin[i], w.cex[i], w.cl2[i], w.cid[i], w.khi[i], w.klo[i]);
-    wsync();
-    sort_keys(c, w.khi, w.klo, tc);
-    const bool q = a.queue_mode != 0;
-    int s = (uint32_t)tc <= a.small_max ? 0 : 1;
-    int bucket = 0;
-    float feat[12];
-    // cost order: children that fit the LDS tile take the lowest bucket
-    // without the model (their subtrees are small, and on trees of tiny
-    // tasks the features and the forward pass would cost as much as the task)
-    const bool predict = q && a.n_buckets > 1 && (uint32_t)tc > a.cost_min_t;
-    if (q && (a.trace_feat || predict)) task_features(c, tc, mem, (int)c.depth + 1, gap, feat);
-    if (predict) bucket = cost_bucket(c, feat);
-    unsigned long long ri = 0, si = 0;
-    if (q) ph_mark(c, PH_CHILD);
-    if (c.lane == 0) {
-        if (q) {
-            si = pool_alloc(c, (uint32_t)tc);
-        } else {
-            ri = atomicAdd(&a.out_ctr[s].items, 1ull);
-            si = atomicAdd(&a.out_ctr[s].slots, (unsigned long long)tc);
-        }
-    }
-    ri = rdlane64(ri, 0);
-    si = rdlane64(si, 0);
-    if (q ? si == ~0ull : (ri >= a.out_ref_cap[s] || si + tc > a.out_vert_cap[s])) {
-        if (c.lane == 0) atomicOr(a.error, 1);
-        return;
-    }
-    Vrec* dst = (q ? a.pool : a.out_verts[s]) + si;
-    for (int i = c.lane; i < tc; i += WAVE) {
-        uint64_t hi = w.khi[i], lo = w.klo[i];
-        uint32_t rank = (uint32_t)(hi >> 61);
-        Vrec v;
-        v.id = (int32_t)(0xFFFFFFFFu - (uint32_t)lo);
-        v.label = rank == 0 ? 1 : rank == 1 ? 2 : rank == 2 ? 0 : rank == 3 ? 3 : -1;
-        v.indeg = 0x3FFFFFFF - (int32_t)((hi >> 30) & 0x3FFFFFFFull);
-        v.exdeg = 0x3FFFFFFF - (int32_t)(hi & 0x3FFFFFFFull);
-        dst[i] = v;
-    }
-    TaskRef r;
-    r.off = si;
-    r.t = (uint32_t)tc;
-    r.depth = (uint16_t)(c.depth + 1);
-    r.inst = (uint16_t)c.inst;
-    r.bound = 0;
-    r.b0 = 0;
-    r.b1 = 0;
-    if (q) {
-        // dynamic order: children stay on this wave's stack (depth first),
-        // with their predicted bucket when a cost model orders the work;
-        // static order: the stack only stages them, and the wave moves them
-        // to the ring (whose positions are dealt to the waves in turn) in
-        // one claim when the task ends
-        const bool shared = !a.use_priv || (!a.static_sched && share_child(c));
-        const bool pushed = push_ref(c, r, bucket, shared, feat);
-        ph_mark(c, PH_POOL);
-        if (!pushed) return;
-    } else {
-        // slot bound of this child's own children (see TaskRef)
-        unsigned long long bnd = 0;
-        for (int i = mem + c.lane; i < tc; i += WAVE) {
-            unsigned long long x =
-                (unsigned long long)c.g.p->d2r[(int32_t)(0xFFFFFFFFu - (uint32_t)w.klo[i])] + mem + 1;
-            bnd += x < (unsigned long long)tc ? x : (unsigned long long)tc;
-        }
-        bnd = (unsigned long long)wave_sum64((long long)bnd);
-        if (c.lane == 0) {
-            r.bound = bnd;
-            a.out_refs[s][ri] = r;
-        }
-    }
-    if (c.lane == 0) {
-        c.st->children++;
-        c.st->sum_tw += tc;
-    }
 }
 
 // ---------------------------------------------------------------------------
@@ -2056,533 +1243,1350 @@ __device__ __attribute__((always_inline)) void tiny_level(Ctx& c, Tiny& y, uint3
     }
 }
 
-// first index in [from, t) where pred holds, else t
-template <class P>
-__device__ __forceinline__ int first_where(Ctx& c, int from, int t, P pred) {
-    for (int base = from; base < t; base += WAVE) {
-        int i = base + c.lane;
-        uint64_t b = ballot(i < t && pred(i));
-        if (b) return base + __builtin_ctzll(b);
-    }
-    return t;
+// ---------------------------------------------------------------------------
+// tasks of more than 64 vertices
+// ---------------------------------------------------------------------------
+// The steps of h_expand_level's body (main.cu:1060-1181) on a compact layout: a
+// vertex's indeg and exdeg are one 32-bit word, a child vertex is that word
+// and its position in the parent, 20 bytes a vertex for parent and child
+// together.  With WideLds all of it is in LDS (about 1,700 vertices at 4 waves
+// per CU); with WideSlab the arrays are in the wave's HBM slab, read and
+// written in order, and only bit masks, rows and short sorts use the LDS.
+//   * A branch reads two matrix rows (N and N2 of its vertex), loaded while
+//     the branch before it runs and kept in LDS; the bits of N are kept per
+//     position for the removal that follows (main.cu:1437-1450).
+//   * Every access is a ds_ or global_ instruction on an array known to be
+//     there; several chunks of 64 are loaded before the first is used.
+//   * Removed candidates leave the arrays at once (one list of positions,
+//     only written when there are any): nothing scans what was removed.
+//   * The indegree counts of the LU bounds are made only when the bounds
+//     get that far, and their index search stops at the first hit from
+//     either end.
+//   * Counts against a set of vertices walk the set's rows (one scalar row
+//     address for 64 lanes, neighbouring words) while the set is small.
+// The order of members and of candidates inside a child is free: the record
+// written is sorted by a key that is unique.
+constexpr uint32_t WIDE_LDS_MAX = 4095;   // WideLds: positions, indegrees and the sort key's fields
+constexpr int WIDE_LDS_R_MAX = 1 << 20;   // WideLds: ids in a sort key
+constexpr int WIDE_ROW_WORDS = 256;       // rows up to this size (R <= 16,384) are staged in LDS
+
+// orders this wave's LDS and memory accesses among its lanes (they execute
+// in order: only the compiler is held, no outstanding load is waited for)
+__device__ __forceinline__ void lsync() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); }
+
+template <class T>
+using gptr = __attribute__((address_space(1))) T*;
+template <class T>
+__device__ __forceinline__ gptr<const T> glob(const T* p) {
+    return (gptr<const T>)p;
+}
+template <class T>
+__device__ __forceinline__ gptr<T> globw(T* p) {
+    return (gptr<T>)p;
 }
 
-// ---------------------------------------------------------------------------
-// one task record, main.cu:1060-1181
-// ---------------------------------------------------------------------------
-template <bool LOCAL>
-__device__ __attribute__((always_inline)) void process_task(Ctx& c, const TaskRef ref) {
-    const ExpandArgs& a = *c.a;
-    WS& w = c.w;
-    const int t0 = (int)ref.t;
-    c.depth = ref.depth;
-    c.keys = !(c.g.max_depth >= 0 && (int)c.depth + 1 > c.g.max_depth);
-    const bool item = ref.b1 > 0;
-    if (!item) {  // a split item's task is counted by its prepare step
-        if (c.lane == 0) {
-            c.st->tasks++;
-            c.st->sum_t += t0;
-            if ((uint32_t)t0 > c.a->small_max) c.st->large++;
+// Vertex word: indeg above EXB bits of exdeg + BIAS; exdeg is accepted at load
+// within LIMIT of 0 (a task lowers it by less than its size after that).
+template <class W, int EXB_, int BIAS_, int LIMIT_>
+struct WideWord {
+    using word = W;
+    static constexpr int EXB = EXB_, BIAS = BIAS_, LIMIT = LIMIT_;
+    static constexpr W MASK = ((W)1 << EXB) - 1;
+    static constexpr W ADJ1 = ((W)1 << EXB) - 1;  // indeg + 1, exdeg - 1
+    static __device__ __forceinline__ int in(W w) { return (int)(w >> EXB); }
+    static __device__ __forceinline__ int ex(W w) { return (int)(w & MASK) - BIAS; }
+    static __device__ __forceinline__ W make(int in, int ex) { return ((W)(uint32_t)in << EXB) | (W)(uint32_t)(ex + BIAS); }
+    static __device__ __forceinline__ W set_ex(W w, int ex) { return (w & ~MASK) | (W)(uint32_t)(ex + BIAS); }
+};
+struct WideLds : WideWord<uint32_t, 20, 1 << 17, 1 << 16> {
+    static constexpr bool slab = false;
+    static constexpr int U = 2;  // chunks of 64 in flight
+    using u32p = uint32_t*;
+    using wordp = uint32_t*;
+    using posp = uint16_t*;
+    using pos_t = uint16_t;
+    using keyp = uint64_t*;
+};
+struct WideSlab : WideWord<uint64_t, 32, 1 << 30, 1 << 29> {
+    static constexpr bool slab = true;
+    static constexpr int U = 4;
+    using u32p = gptr<uint32_t>;
+    using wordp = gptr<uint64_t>;
+    using posp = gptr<uint32_t>;
+    using pos_t = uint32_t;
+    using keyp = gptr<uint64_t>;
+};
+
+__device__ __forceinline__ bool wide_rows_staged(uint32_t rw, uint32_t lds_bytes) {
+    return rw <= (uint32_t)WIDE_ROW_WORDS && 24u * rw <= lds_bytes;
+}
+
+template <class P>
+struct Wide {
+    uint64_t* row1;         // LDS: rows of the branch vertex (rl)
+    uint64_t* row2;
+    uint64_t* lmask;        // LDS: a set of vertices in root space (rl)
+    uint64_t* nbits;        // N of the branch vertex by parent position (LDS; in the slab when too large)
+    uint64_t* flag;         // a bit per candidate (as nbits)
+    typename P::u32p pid;   // parent: root-local id
+    typename P::wordp pw;   //         indeg / exdeg word
+    typename P::posp pl2;   //         lvl2adj
+    typename P::posp cpos;  // child: position in the parent
+    typename P::wordp cw;   //        word
+    typename P::posp list;  // positions (parent) of removed candidates, and other short lists (T entries)
+    typename P::posp tab;   // counts per indegree (T entries)
+    typename P::keyp keys;  // sort keys (WideLds: in the place of cw, list and tab; WideSlab: 2 T entries)
+    char* spare;            // LDS behind the masks and rows (WideSlab: short sorts)
+    uint32_t spare_bytes;
+    gptr<const uint64_t> A1, A2;
+    gptr<const int32_t> d1r, d2r;
+    int T;             // capacity of the arrays
+    int rw;            // words per row
+    int idb;           // WideLds: bits of the id in a sort key
+    int mdt;           // mindeg[lane]
+    int mds;           // mindeg[min_size]
+    bool rl;           // rows are staged in LDS
+    int tb, ub1;       // cand_valid's lane-independent bounds, from the last wide_bounds
+};
+
+template <class P>
+__device__ __forceinline__ int wide_md(const Ctx& c, const Wide<P>& z, int i) {
+    return i < WAVE ? rdlane(z.mdt, i) : uni(md(c, i));
+}
+
+// cand_valid (main.cu:2153-2173) with the lane-independent checks in tb, ub1
+template <class P>
+__device__ __forceinline__ bool wide_valid(const Ctx& c, int tb, int ub1, int m, typename P::word w) {
+    const int in = P::in(w), ex = P::ex(w), tot = in + ex;
+    return tot >= tb && in >= ub1 && tot >= md(c, m + ex + 1);
+}
+
+// LU bounds (main.cu:1857-1972) and the member checks of a child with members
+// [0, m): nc candidates count, all of [m, m + n) or, with `sub`, those valid
+// under the bounds (tb0, ub0).  True: the record fails.
+template <class P>
+__device__ __attribute__((always_inline)) bool wide_bounds(Ctx& c, Wide<P>& z, int m, int n, int nc, bool sub, int tb0,
+                                                           int ub0, int& ub, int& lb, int& med) {
+    const int ms = c.g.min_size;
+    auto gm = [&](int s) { return s < ms ? z.mds : wide_md(c, z, s); };
+    // smallest (indeg, exdeg) pair, exdeg compared as an unsigned value
+    int min_in, min_in_ex, min_tot = INT32_MAX, sum_in = 0;
+    if constexpr (!P::slab) {
+        // (in one word, compared as signed with the top bit flipped)
+        int pair = INT32_MAX;
+        for (int i = c.lane; i < m; i += WAVE) {
+            const uint32_t w = z.cw[i];
+            const int in = P::in(w), ex = P::ex(w);
+            pair = min(pair, (int)((((uint32_t)in << P::EXB) | ((uint32_t)ex & P::MASK)) ^ 0x80000000u));
+            min_tot = min(min_tot, in + ex);
+            sum_in += in;
         }
+        const uint32_t mp = (uint32_t)wave_min(pair) ^ 0x80000000u;
+        min_in = (int)(mp >> P::EXB);
+        min_in_ex = (int)(mp << (32 - P::EXB)) >> (32 - P::EXB);
+    } else {
+        uint64_t pair = ~0ull;
+        for (int i = c.lane; i < m; i += WAVE) {
+            const uint64_t w = z.cw[i];
+            const int in = P::in(w), ex = P::ex(w);
+            pair = min(pair, ((uint64_t)(uint32_t)in << 32) | (uint32_t)ex);
+            min_tot = min(min_tot, in + ex);
+            sum_in += in;
+        }
+        pair = wave_min_u64(pair);
+        min_in = (int)(pair >> 32);
+        min_in_ex = (int)(uint32_t)pair;
     }
-
-    for (int i = c.lane; i < t0; i += WAVE) {
-        Vrec v = a.in_verts[ref.off + i];
-        w.pid[i] = v.id;
-        w.plab[i] = item ? (v.label & 15) : v.label;
-        w.pin[i] = v.indeg;
-        w.pex[i] = v.exdeg;
-        w.pl2[i] = item ? (v.label >> 4) : 0;
-    }
-    wsync();
-    const int nm = uni(first_where(c, 0, t0, [&](int i) { return w.plab[i] != 1; }));
-    const int cov = uni(first_where(c, nm, t0, [&](int i) { return w.plab[i] != 2; })) - nm;
-
-    // position -> matrix index: local position (LOCAL) or root id
-    int* P2M = LOCAL ? nullptr : w.pid;
-    if (LOCAL) {
-        // t0 x t0 sub-matrices of A1 / A2, rows in position order
-        const int W = (t0 + 63) / 64;
-        c.W = W;
-        c.M1 = w.M1;
-        c.M2 = w.M2;
-        const int rw = c.g.p->rw;
-        const uint64_t* __restrict__ A1 = c.g.p->A1;
-        const uint64_t* __restrict__ A2 = c.g.p->A2;
-        // lane = column; the rows' words holding the columns' bits are
-        // gathered RU rows at a time (2 RU loads in flight per lane: tasks
-        // here are small, and the build is a few rounds of memory latency);
-        // the last group masks the rows past t0
-        constexpr int RU = 8;
-        for (int wd = 0; wd < W; wd++) {
-            int col = wd * 64 + c.lane;
-            bool cv = col < t0;
-            int cb = cv ? w.pid[col] : 0;
-            int cw = cb >> 6;
-            uint64_t cm = 1ull << (cb & 63);
-            for (int i = 0; i < t0; i += RU) {
-                uint64_t x[RU], y[RU];
+    bool invalid = false;
+    med = gm(m + 1);
+    if (min_in < wide_md(c, z, m)) {
+        int x = gm(m) - min_in;
+        for (;;) {
+            const int k = x + c.lane;
+            const uint64_t bm = ballot(k > min_in_ex || min_in + k >= md(c, m + k));
+            if (bm) {
+                x += __builtin_ctzll(bm);
+                break;
+            }
+            x += WAVE;
+        }
+        lb = uni(x);
+        if (min_in + lb < wide_md(c, z, m + lb)) {
+            lb = nc + 1;
+            invalid = true;
+        }
+        min_tot = wave_min(min_tot);
+        // (a stale exdeg can make the sum negative: floor(d / gamma) is then
+        // below 0 and the bound too)
+        const int tq = min_tot < 0 ? -1 : glob(c.g.p->ubq)[min(min_tot, c.g.ubq_n - 1)];
+        ub = tq + 1 - m;
+        if (ub > nc) ub = nc;
+        ub = uni(ub);
+        if (lb < ub) {
+            const long long sum_all = wave_sum64((long long)sum_in);
+            // C[v] = #{indeg >= v}: lane v holds it while every value is
+            // below 64, else a table
+            int V = 0, creg = 0;
+            const bool reg = m < WAVE;
+            auto indeg = [&](int i) {  // of candidate i, 0 when it does not count
+                if (i >= m + n) return 0;
+                const typename P::word w = z.cw[i];
+                return !sub || wide_valid<P>(c, tb0, ub0, m, w) ? P::in(w) : 0;
+            };
+            if (m < 16 && n > 2 * WAVE) {
+                // values below 16: every lane counts its own in 8-bit fields
+                // (of at most 255 chunks at a time), then sums of 16- and
+                // 32-bit fields over the lanes
+                int cnt[16];
 #pragma unroll
-                for (int q = 0; q < RU; q++) {
-                    x[q] = 0;
-                    y[q] = 0;
-                    if (i + q < t0) {
-                        const size_t rb = (size_t)w.pid[i + q] * rw + cw;
-                        x[q] = A1[rb];
-                        y[q] = A2[rb];
+                for (int v = 0; v < 16; v++) cnt[v] = 0;
+                for (int b0 = m; b0 < m + n; b0 += 255 * WAVE) {
+                    unsigned long long lo = 0, hi = 0;
+                    const int b1 = min(m + n, b0 + 255 * WAVE);
+#pragma unroll 4
+                    for (int base = b0; base < b1; base += WAVE) {
+                        const int x = indeg(base + c.lane);
+                        const unsigned long long one = 1ull << ((x & 7) * 8);
+                        lo += x < 8 ? one : 0ull;
+                        hi += x < 8 ? 0ull : one;
+                    }
+                    constexpr unsigned long long EV = 0x00FF00FF00FF00FFull;
+                    auto sum = [](unsigned long long x, unsigned long long y) { return x + y; };
+                    // (64 lanes x 255 fit 16 bits)
+                    const unsigned long long f0 = wave_reduce64(lo & EV, 0ull, sum);
+                    const unsigned long long f1 = wave_reduce64((lo >> 8) & EV, 0ull, sum);
+                    unsigned long long f2 = 0, f3 = 0;
+                    if (m >= 8) {
+                        f2 = wave_reduce64(hi & EV, 0ull, sum);
+                        f3 = wave_reduce64((hi >> 8) & EV, 0ull, sum);
+                    }
+#pragma unroll
+                    for (int v = 1; v < 16; v++) {
+                        const unsigned long long f = v & 8 ? (v & 1 ? f3 : f2) : (v & 1 ? f1 : f0);
+                        cnt[v] += (int)((f >> (((v & 7) >> 1) * 16)) & 0xFFFFull);
                     }
                 }
+                int run = 0;
 #pragma unroll
-                for (int q = 0; q < RU; q++) {
-                    const uint64_t b = ballot(cv && (x[q] & cm)), e = ballot(cv && (y[q] & cm));
-                    if (c.lane == 0 && i + q < t0) {
-                        w.M1[(size_t)(i + q) * W + wd] = b;
-                        w.M2[(size_t)(i + q) * W + wd] = e;
+                for (int v = 15; v >= 1; v--) {
+                    run += cnt[v];
+                    if (run && V == 0) V = v;
+                    if (c.lane == v) creg = run;
+                }
+            } else if (reg) {
+                for (int base = m; base < m + n; base += WAVE) {
+                    const int xin = indeg(base + c.lane);
+                    int v = 1;
+                    for (;; v++) {
+                        const int k = __popcll(ballot(xin >= v));
+                        if (k == 0) break;
+                        if (c.lane == v) creg += k;
+                    }
+                    V = max(V, v - 1);
+                }
+            } else {
+                for (int v = 1;; v++) {
+                    int k = 0;
+                    for (int base = m; base < m + n; base += WAVE) k += __popcll(ballot(indeg(base + c.lane) >= v));
+                    if (k == 0) break;
+                    if (c.lane == 0) z.tab[v] = (typename P::pos_t)k;
+                    V = v;
+                }
+                lsync();
+            }
+            // the condition for 64 values of idx, P(idx) = sum of
+            // min(C[v], idx) over v >= 1; the first value that holds is looked
+            // for from lb up, the last from ub down (nearly always in the
+            // first 64 on either side)
+            auto holds = [&](int base) -> uint64_t {
+                const int idx = base + c.lane;
+                long long p = 0;
+                if (reg) {
+                    int q = 0;
+                    for (int v = 1; v <= V; v++) q += min(rdlane(creg, v), idx);
+                    p = q;
+                } else {
+                    for (int v = 1; v <= V; v++) p += min((int)z.tab[v], idx);
+                }
+                return ballot(idx <= ub && idx >= lb && sum_all + p >= (long long)m * md(c, m + idx));
+            };
+            int first = -1, last = -1, base = lb & ~(WAVE - 1);
+            uint64_t ok = 0;
+            for (; base <= ub; base += WAVE) {
+                ok = holds(base);
+                if (ok) break;
+            }
+            if (ok) {
+                first = base + __builtin_ctzll(ok);
+                int top = ub & ~(WAVE - 1);
+                for (; top > base; top -= WAVE) {
+                    const uint64_t up = holds(top);
+                    if (up) {
+                        ok = up;
+                        break;
                     }
                 }
+                last = top + 63 - __builtin_clzll(ok);
+            }
+            if (first < 0) {
+                lb = ub + 1;
+                invalid = true;
+            } else {
+                lb = first;
+                ub = min(ub, last);
+                if (lb > 1) med = gm(m + lb);
             }
         }
-        wsync();
     } else {
-        c.W = c.g.p->rw;
-        c.M1 = c.g.p->A1;
-        c.M2 = c.g.p->A2;
+        ub = nc;
+        lb = m < ms ? ms - m : 0;
     }
-#define PM(i) (LOCAL ? (i) : P2M[(i)])
+    if (m + ub < ms || ub < 0 || ub < lb) invalid = true;
+    if (invalid) return true;
+    // vert_isextendable_LU (vert_ext) for the members: the checks that do not
+    // depend on the vertex folded into two bounds; get_mindeg(m + ex) is
+    // mindeg[m + ex] under the first of them (mindeg is monotone)
+    const int g = gm(m + lb);
+    const int tb = max(max(z.mds, med), g);
+    const int um = wide_md(c, z, m + ub) - ub;
+    bool f = false;
+    for (int i = c.lane; i < m; i += WAVE) {
+        const typename P::word w = z.cw[i];
+        const int in = P::in(w), ex = P::ex(w), tot = in + ex;
+        if (tot < tb || in < um || tot < md(c, m + ex)) f = true;
+    }
+    if (ballot(f)) return true;
+    z.tb = tb;
+    z.ub1 = wide_md(c, z, m + lb) - ub + 1;
+    return false;
+}
+
+// |row(id) n L| for this lane's id against the vertices of L: lane k of
+// `ids` holds L's k-th vertex of the group, nl <= 64 of them (X: A1 or A2)
+__device__ __forceinline__ int wide_count(gptr<const uint64_t> X, int rw, int ids, int nl, int id) {
+    const int wd = id >> 6, sh = id & 63;
+    int n = 0, k = 0;
+    for (; k + 4 <= nl; k += 4) {
+        uint64_t x[4];
+#pragma unroll
+        for (int q = 0; q < 4; q++) x[q] = X[(size_t)rdlane(ids, k + q) * rw + wd];
+#pragma unroll
+        for (int q = 0; q < 4; q++) n += (int)((x[q] >> sh) & 1ull);
+    }
+    for (; k < nl; k++) n += (int)((X[(size_t)rdlane(ids, k) * rw + wd] >> sh) & 1ull);
+    return n;
+}
+// the same against a mask in LDS
+__device__ __forceinline__ int wide_rowpop(gptr<const uint64_t> X, int rw, const uint64_t* mask, int id) {
+    gptr<const uint64_t> r = X + (size_t)id * rw;
+    int s = 0, w = 0;
+    for (; w + 8 <= rw; w += 8) {
+        uint64_t x[8];
+#pragma unroll
+        for (int q = 0; q < 8; q++) x[q] = r[w + q];
+#pragma unroll
+        for (int q = 0; q < 8; q++) s += __popcll(x[q] & mask[w + q]);
+    }
+    for (; w < rw; w++) s += __popcll(r[w] & mask[w]);
+    return s;
+}
+
+// A set of nl vertices, vertex k = at(k): counts by its rows, or by a mask of
+// it when it has more than two vertices per row word (a lane then reads its own
+// row, 64 rows at once, instead of the same words of one row).
+template <class P, class At>
+__device__ __attribute__((always_inline)) bool wide_set(Ctx& c, Wide<P>& z, int nl, At at) {
+    const bool mask = z.rl && nl > 2 * z.rw;
+    if (mask) {
+        for (int w = c.lane; w < z.rw; w += WAVE) z.lmask[w] = 0;
+        lsync();
+        for (int k = c.lane; k < nl; k += WAVE) set_mask_bit(z.lmask, (int)at(k));
+        lsync();
+    }
+    return mask;
+}
+template <class P, class At>
+__device__ __attribute__((always_inline)) int wide_in_set(Ctx& c, Wide<P>& z, gptr<const uint64_t> X, bool mask, int nl,
+                                                          At at, int id) {
+    if (mask) return wide_rowpop(X, z.rw, z.lmask, id);
+    int n = 0;
+    for (int g = 0; g < nl; g += WAVE) {
+        const int ids = g + c.lane < nl ? (int)at(g + c.lane) : 0;
+        n += wide_count(X, z.rw, ids, min(nl - g, WAVE), id);
+    }
+    return n;
+}
+
+// Keeps the candidates [m, m + n) valid under (z.tb, z.ub1), in place; the
+// others go on the list (their positions) from nl on.  Returns how many stay.
+template <class P>
+__device__ __attribute__((always_inline)) int wide_keep(Ctx& c, Wide<P>& z, int m, int n, int& nl) {
+    // (most children keep every candidate: the words are only read up to the
+    // first that goes)
+    int from = 0;
+    for (; from < n; from += P::U * WAVE) {
+        bool go = false;
+#pragma unroll
+        for (int u = 0; u < P::U; u++) {
+            const int i = from + u * WAVE + c.lane;
+            if (i < n) go |= !wide_valid<P>(c, z.tb, z.ub1, m, z.cw[m + i]);
+        }
+        if (ballot(go)) break;
+    }
+    if (from >= n) return n;
+    int kept = from;
+    for (int base = from; base < n; base += P::U * WAVE) {
+        typename P::word w[P::U];
+        uint32_t p[P::U];
+#pragma unroll
+        for (int u = 0; u < P::U; u++) {
+            const int i = base + u * WAVE + c.lane;
+            w[u] = i < n ? z.cw[m + i] : (typename P::word)0;
+            p[u] = i < n ? (uint32_t)z.cpos[m + i] : 0u;
+        }
+        lsync();
+#pragma unroll
+        for (int u = 0; u < P::U; u++) {
+            const int i = base + u * WAVE + c.lane;
+            const bool in = i < n;
+            const bool ok = in && wide_valid<P>(c, z.tb, z.ub1, m, w[u]);
+            const uint64_t bo = ballot(ok), bx = ballot(in && !ok);
+            if (ok) {
+                const int d = m + kept + lanes_below(bo);
+                z.cw[d] = w[u];
+                z.cpos[d] = (typename P::pos_t)p[u];
+            } else if (in) {
+                z.list[nl + lanes_below(bx)] = (typename P::pos_t)p[u];
+            }
+            kept += __popcll(bo);
+            nl += __popcll(bx);
+        }
+        lsync();
+    }
+    return kept;
+}
+
+// degree_pruning (main.cu:1735-1855): members [0, m), candidates [m, m + n),
+// nl removed ones on the list.  True: the record fails (n is then meaningless).
+// map_empty: the reference's id->position map holds no entry during this call
+// (critical-vertex pruning without critical-adjacent candidates).
+template <class P>
+__device__ __attribute__((always_inline)) bool wide_prune(Ctx& c, Wide<P>& z, int m, int& n, int nl, bool map_empty, int& ub,
+                                                          int& lb, int& med) {
+    int nc = n;
+    bool sub = false;
+    int tb0 = 0, ub0 = 0;
+    for (;;) {
+        ph_mark(c, PH_PRUNE);
+        const bool fail = wide_bounds(c, z, m, n, nc, sub, tb0, ub0, ub, lb, med);
+        ph_mark(c, PH_LU);
+        if (fail) return true;
+        if (sub) nl = 0;
+        n = wide_keep(c, z, m, n, nl);
+        lsync();
+        ph_mark(c, PH_COMPACT);
+        if (n == 0 || nl == 0) return false;
+        // degree update, main.cu:1775-1807: recomputed from the remaining
+        // candidates when they are fewer than the removed ones, else lowered
+        const bool rc = n < nl;
+        const int k = rc ? n : nl;
+        auto at = [&](int q) { return z.pid[rc ? z.cpos[m + q] : z.list[q]]; };
+        long long sw = 0;
+        for (int q = c.lane; q < k; q += WAVE) sw += z.d1r[at(q)];
+        wadj_lanes(c, sw);
+        const bool mask = map_empty ? false : wide_set(c, z, k, at);
+        tb0 = z.tb;
+        ub0 = z.ub1;
+        sub = true;
+        nc = 0;
+        for (int base = 0; base < m + n; base += WAVE) {
+            const int i = base + c.lane;
+            bool ok = false;
+            typename P::word w = 0;
+            int id = 0;
+            if (i < m + n) {
+                w = z.cw[i];
+                id = (int)z.pid[z.cpos[i]];
+            }
+            if (!map_empty) {
+                const int cnt = wide_in_set(c, z, z.A1, mask, k, at, id);
+                w = P::set_ex(w, rc ? cnt : P::ex(w) - cnt);
+            } else if (rc) {
+                w = P::set_ex(w, 0);
+            }
+            if (i < m + n) {
+                z.cw[i] = w;
+                // indegrees of the candidates valid under the old bounds
+                // with the new exdeg (main.cu:1811-1815)
+                ok = i >= m && wide_valid<P>(c, tb0, ub0, m, w);
+            }
+            nc += __popcll(ballot(ok));
+        }
+        lsync();
+        ph_mark(c, PH_DEGUPD);
+    }
+}
+
+// critical vertex pruning (main.cu:1526-1707) up to its closing degree pruning:
+// 2 when the record fails, else 0 with the candidates, the list and map_empty
+// as that pruning takes them.
+template <class P>
+__device__ __attribute__((always_inline)) int wide_critical(Ctx& c, Wide<P>& z, int& m, int& n, int& nl, int lb,
+                                                            bool& map_empty) {
+    using pos_t = typename P::pos_t;
+    const int thr = wide_md(c, z, m + lb);
+    int ncm = 0;
+    long long sw = 0;
+    for (int base = 0; base < m; base += WAVE) {
+        const int i = base + c.lane;
+        typename P::word w = 0;
+        if (i < m) w = z.cw[i];
+        const bool cr = i < m && P::in(w) + P::ex(w) == thr && P::ex(w) > 0;
+        const uint64_t bc = ballot(cr);
+        if (cr) {
+            const pos_t p = z.cpos[i];
+            z.list[ncm + lanes_below(bc)] = p;
+            sw += z.d1r[z.pid[p]];
+        }
+        ncm += __popcll(bc);
+    }
+    nl = 0;
+    map_empty = true;
+    if (ncm == 0) return 0;
+    wadj_lanes(c, sw);
+    lsync();
+    // critical-adjacent candidates, moved to the front of the candidates: the
+    // ones beyond the first ncrit places change places with the others there
+    auto crit = [&](int q) { return z.pid[z.list[q]]; };
+    int ncrit = 0;
+    const bool cmask = wide_set(c, z, ncm, crit);
+    for (int base = 0; base < n; base += WAVE) {
+        const int i = base + c.lane;
+        const int id = i < n ? (int)z.pid[z.cpos[m + i]] : 0;
+        const int k = wide_in_set(c, z, z.A1, cmask, ncm, crit, id);
+        const uint64_t bf = ballot(i < n && k > 0);
+        if (c.lane == 0) z.flag[base / WAVE] = bf;
+        ncrit += __popcll(bf);
+    }
+    if (ncrit == 0) return 0;
+    map_empty = false;
+    lsync();
+    int na = 0, nb = 0;
+    const int half = z.T / 2;  // adjacent at ncrit or beyond: list[0 ..); not adjacent before it: list[half ..)
+    for (int base = 0; base < n; base += WAVE) {
+        const int i = base + c.lane;
+        const bool f = (z.flag[base / WAVE] >> c.lane) & 1ull;
+        const bool xa = f && i >= ncrit, xb = i < n && !f && i < ncrit;
+        const uint64_t ba = ballot(xa), bb = ballot(xb);
+        if (xa) z.list[na + lanes_below(ba)] = (pos_t)(m + i);
+        if (xb) z.list[half + nb + lanes_below(bb)] = (pos_t)(m + i);
+        na += __popcll(ba);
+        nb += __popcll(bb);
+    }
+    lsync();
+    for (int k = c.lane; k < na; k += WAVE) {  // (na == nb)
+        const int i = z.list[k], j = z.list[half + k];
+        const typename P::word wi = z.cw[i], wj = z.cw[j];
+        const pos_t pi = z.cpos[i], pj = z.cpos[j];
+        z.cw[i] = wj;
+        z.cpos[i] = pj;
+        z.cw[j] = wi;
+        z.cpos[j] = pi;
+    }
+    lsync();
+    auto at = [&](int q) { return z.pid[z.cpos[m + q]]; };
+    sw = 0;
+    for (int q = c.lane; q < ncrit; q += WAVE) {
+        const uint32_t id = at(q);
+        sw += z.d1r[id] + z.d2r[id];
+    }
+    wadj_lanes(c, sw);
+    const bool mask = wide_set(c, z, ncrit, at);
+    // degrees and 2-hop counts against the added vertices; candidates not
+    // within 2 hops of all of them leave.  (The entries of the set itself,
+    // [m, m + ncrit), stay where they are: later chunks read them.)
+    bool bad = false;
+    const int all = m + n, fixed = m + ncrit;
+    int kept = 0;
+    for (int base = 0; base < all; base += WAVE) {
+        const int i = base + c.lane;
+        const bool in = i < all;
+        typename P::word w = 0;
+        uint32_t p = 0;
+        int id = 0;
+        if (in) {
+            w = z.cw[i];
+            p = z.cpos[i];
+            id = (int)z.pid[p];
+        }
+        const int x1 = wide_in_set(c, z, z.A1, mask, ncrit, at, id);
+        const int x2 = wide_in_set(c, z, z.A2, mask, ncrit, at, id);
+        w += (typename P::word)x1 * P::ADJ1;
+        if (in && ((i < m && x2 != ncrit) || (i >= m && i < fixed && x2 < ncrit - 1))) bad = true;
+        const bool cand = in && i >= fixed;
+        const bool ok = cand && x2 == ncrit;
+        const uint64_t bo = ballot(ok), bx = ballot(cand && !ok);
+        lsync();
+        if (in && i < fixed) z.cw[i] = w;
+        if (ok) {
+            const int d = fixed + kept + lanes_below(bo);
+            z.cw[d] = w;
+            z.cpos[d] = (pos_t)p;
+        } else if (cand) {
+            z.list[nl + lanes_below(bx)] = (pos_t)p;
+        }
+        kept += __popcll(bo);
+        nl += __popcll(bx);
+        lsync();
+    }
+    if (ballot(bad)) return 2;
+    m = fixed;
+    n = kept;
+    return 0;
+}
+
+// a raw set of `len` vertices, id_at(i) the i-th one's root-local id
+template <class At>
+__device__ __attribute__((always_inline)) void wide_emit(Ctx& c, int len, At id_at) {
+    unsigned long long ri = 0, si = 0;
+    if (!clq_reserve(c, len, ri, si)) return;
+    for (int k = c.lane; k < len; k += WAVE) c.a->clq_verts[si + k] = glob(c.g.p->orig)[id_at(k)];
+    clq_ref(c, ri, si, len);
+}
+
+// Descending bitonic sort of n keys, any n: every comparator has the larger key
+// to the lower index, so places from n on (the smallest possible key) would
+// never move.  swap_if(lo, hi) exchanges the two places when out of order.
+template <class F>
+__device__ __forceinline__ void wide_sort(Ctx& c, int n, F swap_if) {
+    int n2 = 1;
+    while (n2 < n) n2 <<= 1;
+    for (int k = 2; k <= n2; k <<= 1) {
+        for (int j = k >> 1; j > 0; j >>= 1) {
+            for (int x = c.lane; x < n2 / 2; x += WAVE) {
+                const int lo = ((x & ~(j - 1)) << 1) | (x & (j - 1));
+                const int hi = j == k >> 1 ? (lo ^ (k - 1)) : lo + j;
+                if (hi < n) swap_if(lo, hi);
+            }
+            lsync();
+        }
+    }
+}
+
+// The child's record: members, then the candidates in Q order
+// (main.cu:2059-2104: indeg, exdeg, lvl2adj, id, all descending).
+template <class P>
+__device__ __attribute__((always_inline)) void wide_child(Ctx& c, Wide<P>& z, int m, int n, int gap) {
+    const ExpandArgs& a = *c.a;
+    const int tc = m + n;
+    if (!c.keys) {
+        // outside the depth window: counted, never expanded
+        if (c.lane == 0) {
+            c.st->children++;
+            c.st->sum_tw += tc;
+            c.st->beyond++;
+            if (a.trace_beyond && c.slot >= 0) atomicAdd(&a.trace_beyond[c.slot], 1u);
+        }
+        return;
+    }
+    const bool q = a.queue_mode != 0;
+    const int s = (uint32_t)tc <= a.small_max ? 0 : 1;
+    int bucket = 0;
+    float feat[12];
+    // cost order: children that fit the LDS tile take the lowest bucket
+    // without the model (their subtrees are small, and on trees of tiny
+    // tasks the features and the forward pass would cost as much as the task)
+    const bool predict = q && a.n_buckets > 1 && (uint32_t)tc > a.cost_min_t;
+    if (q && (a.trace_feat || predict)) {
+        int mi = INT32_MAX, ma = INT32_MIN, me = INT32_MAX, mx = INT32_MIN;
+        long long si = 0, se = 0, s2 = 0;
+        for (int i = c.lane; i < tc; i += WAVE) {
+            const typename P::word w = z.cw[i];
+            const int in = P::in(w), ex = P::ex(w);
+            mi = min(mi, in);
+            ma = max(ma, in);
+            me = min(me, ex);
+            mx = max(mx, ex);
+            si += in;
+            se += ex;
+            if (i >= m) s2 += z.d2r[z.pid[z.cpos[i]]];
+        }
+        feature_row(tc, m, (int)c.depth + 1, gap, mi, ma, me, mx, si, se, s2, feat);
+    }
+    if (predict) bucket = cost_bucket(c, feat);
+    unsigned long long ri = 0, si = 0;
+    ph_mark(c, PH_CHILD);
+    if (c.lane == 0) {
+        if (q) {
+            si = pool_alloc(c, (uint32_t)tc);
+        } else {
+            ri = atomicAdd(&a.out_ctr[s].items, 1ull);
+            si = atomicAdd(&a.out_ctr[s].slots, (unsigned long long)tc);
+        }
+    }
+    ri = rdlane64(ri, 0);
+    si = rdlane64(si, 0);
+    if (q ? si == ~0ull : (ri >= a.out_ref_cap[s] || si + tc > a.out_vert_cap[s])) {
+        if (c.lane == 0) atomicOr(a.error, 1);
+        return;
+    }
+    gptr<Vrec> dst = globw((q ? a.pool : a.out_verts[s]) + si);
+    auto put = [&](int i, uint32_t id, int label, typename P::word w) {
+        typedef int v4 __attribute__((ext_vector_type(4)));
+        *(gptr<v4>)(dst + i) = v4{(int)id, label, P::in(w), P::ex(w)};
+    };
+    for (int i = c.lane; i < m; i += WAVE) put(i, z.pid[z.cpos[i]], 1, z.cw[i]);
+    unsigned long long bnd = 0;
+    auto bound_of = [&](uint32_t id) {  // slot bound of the child's own children (see TaskRef)
+        const unsigned long long x = (unsigned long long)z.d2r[id] + m + 1;
+        return x < (unsigned long long)tc ? x : (unsigned long long)tc;
+    };
+    lsync();
+    if constexpr (!P::slab) {
+        // keys in the words' place: from the top down a chunk's keys only cover
+        // words that have been read, when the candidates start at word 0
+        if (m > WAVE) {
+            for (int base = 0; base < n; base += WAVE) {
+                const int i = base + c.lane;
+                uint32_t w = 0;
+                if (i < n) w = z.cw[m + i];
+                lsync();
+                if (i < n) z.cw[i] = w;
+                lsync();
+            }
+        }
+        const int w0 = m > WAVE ? 0 : m;
+        for (int base = (n - 1) & ~(WAVE - 1); base >= 0; base -= WAVE) {
+            const int i = base + c.lane;
+            uint64_t key = 0;
+            if (i < n) {
+                const uint32_t w = z.cw[w0 + i], p = z.cpos[m + i];
+                const uint32_t id = z.pid[p];
+                key = ((uint64_t)w << 32) | ((uint32_t)z.pl2[p] << z.idb) | id;
+                if (!q) bnd += bound_of(id);
+            }
+            lsync();
+            if (i < n) z.keys[i] = key;
+            lsync();
+        }
+        wide_sort(c, n, [&](int lo, int hi) {
+            const uint64_t u = z.keys[lo], v = z.keys[hi];
+            if (u < v) {
+                z.keys[lo] = v;
+                z.keys[hi] = u;
+            }
+        });
+        for (int i = c.lane; i < n; i += WAVE) {
+            const uint64_t key = z.keys[i];
+            put(m + i, (uint32_t)key & ((1u << z.idb) - 1u), 0, (uint32_t)(key >> 32));
+        }
+    } else {
+        // 128-bit keys (word, lvl2adj and id), in LDS when they fit there
+        auto run = [&](auto khi, auto klo) {
+            for (int i = c.lane; i < n; i += WAVE) {
+                const uint32_t p = z.cpos[m + i], id = z.pid[p];
+                khi[i] = z.cw[m + i];
+                klo[i] = ((uint64_t)z.pl2[p] << 32) | id;
+                if (!q) bnd += bound_of(id);
+            }
+            lsync();
+            wide_sort(c, n, [&](int lo, int hi) {
+                const uint64_t uh = khi[lo], vh = khi[hi], ul = klo[lo], vl = klo[hi];
+                if (uh < vh || (uh == vh && ul < vl)) {
+                    khi[lo] = vh;
+                    khi[hi] = uh;
+                    klo[lo] = vl;
+                    klo[hi] = ul;
+                }
+            });
+            for (int i = c.lane; i < n; i += WAVE) put(m + i, (uint32_t)klo[i], 0, khi[i]);
+        };
+        if (16u * (uint32_t)n <= z.spare_bytes)
+            run((uint64_t*)z.spare, (uint64_t*)z.spare + n);
+        else
+            run(z.keys, z.keys + (size_t)z.T);
+    }
+    TaskRef r;
+    r.off = si;
+    r.t = (uint32_t)tc;
+    r.depth = (uint16_t)(c.depth + 1);
+    r.inst = (uint16_t)c.inst;
+    r.bound = 0;
+    r.b0 = 0;
+    r.b1 = 0;
+    if (q) {
+        // dynamic order: children stay on this wave's stack (depth first),
+        // with their predicted bucket when a cost model orders the work;
+        // static order: the stack only stages them, and the wave moves them
+        // to the ring (whose positions are dealt to the waves in turn) in
+        // one claim when the task ends
+        const bool shared = !a.use_priv || (!a.static_sched && share_child(c));
+        const bool pushed = push_ref(c, r, bucket, shared, feat);
+        ph_mark(c, PH_POOL);
+        if (!pushed) return;
+    } else {
+        bnd = (unsigned long long)wave_sum64((long long)bnd);
+        if (c.lane == 0) {
+            r.bound = bnd;
+            a.out_refs[s][ri] = r;
+        }
+    }
+    if (c.lane == 0) {
+        c.st->children++;
+        c.st->sum_tw += tc;
+    }
+}
+
+// exdeg of positions [0, keep) minus their neighbours among positions
+// [keep, keep + nr): several removals at once
+template <class P>
+__device__ __attribute__((always_inline)) void wide_bulk_remove(Ctx& c, Wide<P>& z, int keep, int nr) {
+    if (nr <= 0) return;
+    auto gone = [&](int q) { return z.pid[keep + q]; };
+    const bool mask = wide_set(c, z, nr, gone);
+    for (int base = 0; base < keep; base += WAVE) {
+        const int i = base + c.lane;
+        const int id = i < keep ? (int)z.pid[i] : 0;
+        const int k = wide_in_set(c, z, z.A1, mask, nr, gone, id);
+        if (i < keep) z.pw[i] -= (typename P::word)k;
+    }
+    lsync();
+}
+
+// W_adj of a removal that fails: the reference scans N(r) in ascending id
+// order and stops after the first failing member (main.cu:1437-1450)
+template <class P>
+__device__ __attribute__((always_inline)) void wide_failed_scan(Ctx& c, Wide<P>& z, int rid, int fid) {
+    const size_t r0 = (size_t)rid * z.rw;
+    int rank = 0;
+    for (int wd = c.lane; wd <= (fid >> 6); wd += WAVE) {
+        uint64_t x = z.A1[r0 + wd];
+        if (wd == (fid >> 6)) x &= (1ull << (fid & 63)) - 1ull;
+        rank += __popcll(x);
+    }
+    wadj_lanes(c, rank + (c.lane == 0));
+}
+
+// Split step of a task whose branches [bbeg, bend) go to several waves: finds
+// the first failing removal, counts the removals' scans, stores the record as
+// it stands before the first branch of the window (with lvl2adj) and pushes
+// the items, ch branches each on average.
+template <class P>
+__device__ __attribute__((always_inline)) void wide_split(Ctx& c, Wide<P>& z, const TaskRef& ref, int nm, int bbeg, int bend,
+                                                          int ch) {
+    const ExpandArgs& a = *c.a;
+    const int t0 = (int)ref.t;
+    // Removal k (branch b = k) takes position t0 - k.  Member i fails at
+    // the removal of its need_i-th neighbour counted from the end, with
+    // need_i = max(pin + pex - mindeg(nm) + 1, 1); kb = the first such
+    // removal over all members (bend: none before the window's end).
+    const int mdg = get_mindeg(c, nm);
+    int kb = bend;
+    for (int i = 0; i < nm; i++) {
+        const typename P::word w = z.pw[i];
+        const int need = max(P::in(w) + P::ex(w) - mdg + 1, 1);
+        const size_t r0 = (size_t)z.pid[i] * z.rw;
+        // removals up to kb inclusive: a member failing at the same
+        // removal as an earlier one must be seen (smallest failing id)
+        const int lim = min(kb, bend - 1);
+        int cnt = 0, ki = INT32_MAX;
+        for (int k0 = 1; k0 <= lim && ki == INT32_MAX; k0 += WAVE) {
+            const int k = k0 + c.lane;
+            bool adj = false;
+            if (k <= lim) {
+                const uint32_t id = z.pid[t0 - k];
+                adj = (z.A1[r0 + (id >> 6)] >> (id & 63)) & 1ull;
+            }
+            const uint64_t bm = ballot(adj);
+            const int pc = __popcll(bm);
+            if (cnt + pc >= need) {
+                const uint64_t hit = ballot(adj && cnt + lanes_below(bm) + 1 == need);
+                ki = k0 + __builtin_ctzll(hit);
+            }
+            cnt += pc;
+        }
+        if (c.lane == 0) z.list[i] = (typename P::pos_t)min(ki, bend);  // (bend: none)
+        kb = min(kb, ki);
+    }
+    lsync();
+    // W_adj of the removals: full scans of N(r) for removals 1..kb-1,
+    // the partial scan up to the smallest failing member for removal kb
+    long long sw = 0;
+    for (int k = 1 + c.lane; k < kb; k += WAVE) sw += z.d1r[z.pid[t0 - k]];
+    wadj_lanes(c, sw);
+    if (kb < bend) {
+        int fid = INT32_MAX;
+        for (int i = c.lane; i < nm; i += WAVE)
+            if ((int)z.list[i] == kb) fid = min(fid, (int)z.pid[i]);
+        wide_failed_scan(c, z, (int)z.pid[t0 - kb], wave_min(fid));
+    }
+    const int hi = min(kb, bend);
+    if (hi <= bbeg) return;
+    // removals 1..bbeg happen before the window: apply them once here
+    const int pre = bbeg;
+    const int ts = t0 - pre;
+    wide_bulk_remove(c, z, ts, pre);
+    // the record plus one Vrec after it whose id counts the items still
+    // to run (the last one frees the block)
+    unsigned long long slot = 0;
+    if (c.lane == 0) slot = pool_alloc(c, (uint32_t)ts + 1u);
+    slot = rdlane64(slot, 0);
+    if (slot == ~0ull) {
+        if (c.lane == 0) atomicOr(a.error, 1);
+        return;
+    }
+    for (int i = c.lane; i < ts; i += WAVE) {
+        const typename P::word w = z.pw[i];
+        a.pool[slot + i] = Vrec{(int32_t)z.pid[i], (i < nm ? 1 : 0) | ((int32_t)z.pl2[i] << 4), P::in(w), P::ex(w)};
+    }
+    const int n_items = (hi - bbeg + ch - 1) / ch;
+    if (c.lane == 0) a.pool[slot + ts] = Vrec{n_items, 0, 0, 0};
+    // item boundaries balance the work rather than the branch count:
+    // branch b builds a child from about t0 - b vertices, so with
+    // S(b) = sum of (t0 - x) over x in [bbeg, b), boundary j is the first
+    // b with S(b) >= j S(hi) / n_items (kept strictly increasing)
+    const long long t0l = t0;
+    auto S = [&](long long b) { return (b - bbeg) * t0l - (b * (b - 1) - (long long)bbeg * (bbeg - 1)) / 2; };
+    const long long s_tot = S(hi);
+    auto boundary = [&](int j) -> int {
+        if (j <= 0) return bbeg;
+        if (j >= n_items) return hi;
+        const long long target = s_tot * j / n_items;
+        int lo = bbeg, up = hi;
+        while (lo < up) {
+            const int mid = (lo + up) >> 1;
+            if (S(mid) >= target)
+                up = mid;
+            else
+                lo = mid + 1;
+        }
+        return min(max(lo, bbeg + j), hi - (n_items - j));
+    };
+    auto item_ref = [&](int j) {
+        TaskRef r;
+        r.off = slot;
+        r.t = (uint32_t)ts;
+        r.depth = ref.depth;
+        r.inst = ref.inst;
+        r.bound = (uint64_t)c.slot;  // the task the item belongs to (trace)
+        r.b0 = (uint32_t)(boundary(j) - pre);
+        r.b1 = (uint32_t)(boundary(j + 1) - pre);
+        return r;
+    };
+    // the items go to the rings in chunks of up to 64 claimed at once
+    // (lanes write the refs, one release fence per chunk), as many as wait at a
+    // ring, the rest to this wave's own; what the rings cannot take stays on
+    // this wave's stack
+    int done = 0;
+    while (done < n_items) {
+        unsigned long long pos = 0;
+        int waiting = 0;
+        const int rg = ring_for(c, &waiting);
+        const int k = ring_claim(c, rg, min(n_items - done, waiting > 0 ? min(waiting, WAVE) : WAVE), &pos);
+        if (k == 0) break;
+        if (c.lane == 0)
+            __hip_atomic_fetch_add(a.pending, (unsigned long long)k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (c.lane < k) {
+            const unsigned long long gi = (unsigned long long)rg * a.q_cap + (pos + c.lane) % a.q_cap;
+            if (a.trace_parent) a.trace_parent[gi] = -2;
+            a.q_refs[gi] = item_ref(done + c.lane);
+        }
+        ring_publish(c, rg, pos, k);
+        done += k;
+    }
+    for (; done < n_items; done++)
+        if (!push_ref(c, item_ref(done), a.n_buckets - 1, false, nullptr)) break;
+}
+
+// One task or split item.  False, with nothing done, when a degree or lvl2adj
+// does not fit WideLds' fields (WideSlab then runs it; its own are never
+// exceeded).  The caller has checked wide_fits (WideLds) or the slab's size.
+template <class P>
+__device__ __attribute__((always_inline)) bool process_wide(Ctx& c, const TaskRef ref, char* lds, uint32_t lds_bytes,
+                                                            char* slab) {
+    const ExpandArgs& a = *c.a;
+    const int t0 = (int)ref.t;
+    const bool item = ref.b1 > 0;
+    const bool root = ref.depth == 0;
+    Wide<P> z;
+    z.rw = c.g.p->rw;
+    const uint32_t T = wide_T((uint32_t)t0);
+    z.T = (int)T;
+    z.rl = wide_rows_staged((uint32_t)z.rw, lds_bytes);
+    z.idb = c.g.p->R <= 65536 ? 16 : 20;
+    {
+        char* at = lds;
+        z.row1 = (uint64_t*)at;
+        z.row2 = z.row1 + z.rw;
+        z.lmask = z.row2 + z.rw;
+        if (z.rl) at += 24 * z.rw;
+        if constexpr (!P::slab) {
+            z.keys = (uint64_t*)at;
+            z.cw = (uint32_t*)at;
+            z.list = (uint16_t*)(at + 4 * T);
+            z.tab = (uint16_t*)(at + 6 * T);
+            at += 8 * T;
+            z.pid = (uint32_t*)at;
+            at += 4 * T;
+            z.pw = (uint32_t*)at;
+            at += 4 * T;
+            z.pl2 = (uint16_t*)at;
+            at += 2 * T;
+            z.cpos = (uint16_t*)at;
+            at += 2 * T;
+            z.nbits = (uint64_t*)at;
+            z.flag = z.nbits + T / 64;
+        } else {
+            // WIDE_SLAB bytes a vertex
+            gptr<char> g = globw(slab);
+            z.keys = (gptr<uint64_t>)g;
+            z.pw = z.keys + (size_t)2 * T;
+            z.cw = z.keys + (size_t)3 * T;
+            gptr<uint32_t> u = (gptr<uint32_t>)(z.keys + (size_t)4 * T);
+            z.pid = u;
+            z.pl2 = u + (size_t)T;
+            z.cpos = u + (size_t)2 * T;
+            z.list = u + (size_t)3 * T;
+            z.tab = u + (size_t)4 * T;
+            if ((uint32_t)(at - lds) + T / 4 <= lds_bytes) {
+                z.nbits = (uint64_t*)at;
+                at += T / 4;
+            } else {
+                z.nbits = (uint64_t*)(slab + (size_t)52 * T);
+            }
+            z.flag = z.nbits + T / 64;
+        }
+        z.spare = at;
+        z.spare_bytes = lds_bytes - (uint32_t)(at - lds);
+    }
+    // ---- record ----
+    bool bad = false;
+    int nm = 0, cov = 0;
+    gptr<const Vrec> src = glob(a.in_verts + ref.off);
+    // lvl2adj has to fit its field (an item of the root takes it from the whole root)
+    const uint32_t l2_max = P::slab ? 0xFFFFFFFFu : z.idb == 16 ? 0xFFFFu : 0xFFFu;
+    for (int base = 0; base < t0; base += P::U * WAVE) {
+        typedef int v4 __attribute__((ext_vector_type(4)));
+        v4 v[P::U];
+#pragma unroll
+        for (int u = 0; u < P::U; u++) {
+            const int i = base + u * WAVE + c.lane;
+            v[u] = v4{0, 0, 0, 0};
+            if (i < t0) v[u] = *(gptr<const v4>)(src + i);
+        }
+#pragma unroll
+        for (int u = 0; u < P::U; u++) {
+            const int i = base + u * WAVE + c.lane;
+            const bool in = i < t0;
+            const int lab = item ? v[u].y & 15 : v[u].y;
+            const uint32_t l2 = item ? (uint32_t)v[u].y >> 4 : 0u;
+            if (v[u].w < -P::LIMIT || v[u].w > P::LIMIT || l2 > l2_max) bad = true;
+            nm += __popcll(ballot(in && lab == 1));
+            cov += __popcll(ballot(in && lab == 2));
+            if (in) {
+                z.pid[i] = (uint32_t)v[u].x;
+                z.pw[i] = P::make(v[u].z, v[u].w);
+                z.pl2[i] = (typename P::pos_t)l2;
+            }
+        }
+    }
+    if (ballot(bad)) return false;
+    int nc = t0 - nm;
+    const int nb = nc - cov;
+    int bend = nb;
+    if (root && c.g.p->root_b1 >= 0 && c.g.p->root_b1 < bend) bend = (int)c.g.p->root_b1;
+    // a negative window start counts from the end of the root's branches
+    const long long rb0 = c.g.p->root_b0 >= 0 ? c.g.p->root_b0 : max(0ll, (long long)nb + c.g.p->root_b0);
+    const int bbeg = root ? (int)min<long long>(rb0, (long long)nb) : 0;
+    c.depth = ref.depth;
+    c.keys = !(c.g.max_depth >= 0 && (int)c.depth + 1 > c.g.max_depth);
+    if (!item && c.lane == 0) {  // (a split item's task is counted by its prepare step)
+        c.st->tasks++;
+        c.st->sum_t += t0;
+        if ((uint32_t)t0 > a.small_max) c.st->large++;
+    }
+    z.A1 = glob(c.g.p->A1);
+    z.A2 = glob(c.g.p->A2);
+    z.d1r = glob(c.g.p->d1r);
+    z.d2r = glob(c.g.p->d2r);
+    z.mdt = md(c, c.lane);
+    z.mds = uni(md(c, c.g.min_size));
+    lsync();
     ph_mark(c, PH_LOAD);
 
     // ---- lookahead, main.cu:1349-1405 ----
-    int nc = t0 - nm;
     if (!item) {
-        int req = md(c, t0);
+        const int req = wide_md(c, z, t0);
         bool f = false;
-        for (int i = c.lane; i < nm; i += WAVE)
-            if (w.pin[i] + w.pex[i] < req) f = true;
+        for (int i = c.lane; i < nm; i += WAVE) {
+            const typename P::word w = z.pw[i];
+            if (P::in(w) + P::ex(w) < req) f = true;
+        }
         if (ballot(f) == 0) {
             // a record holding every root vertex and no member is the whole
             // root: |N2(v) n candidates| is then |N2(v) n root| = d2r[v],
-            // with no row scans (O(R^2 / 64) words at the root otherwise).
-            // A root shortened by a window's leading removals (root_cut) takes
-            // the whole root's values too: its lookahead ran on the whole
-            // root, where it failed (the host checked), so nothing is emitted
-            const bool cut_root = nm == 0 && ref.depth == 0 && c.g.p->root_cut > 0;
+            // with no row scans.  A root shortened by a window's leading
+            // removals (root_cut) takes the whole root's values too: its
+            // lookahead ran on the whole root, where it failed (the host
+            // checked), so nothing is emitted
+            const bool cut_root = nm == 0 && root && c.g.p->root_cut > 0;
             const bool whole_root = nm == 0 && (t0 == c.g.p->R || cut_root);
-            if (!whole_root) clear_mask(c, w.mk0);
+            auto cand = [&](int q) { return z.pid[nm + q]; };
+            const bool mask = whole_root ? false : wide_set(c, z, nc, cand);
             long long sw = 0;
-            for (int i = nm + c.lane; i < t0; i += WAVE) {
-                if (!whole_root) set_mask_bit(w.mk0, PM(i));
-                sw += c.g.p->d2r[w.pid[i]];
+            bool low = false, known = false;
+            // (from the end of the record, where the degrees are lowest: when
+            // the children are not kept, lvl2adj only serves this test)
+            for (int base = nm + ((nc - 1) & ~(WAVE - 1)); base >= nm; base -= WAVE) {
+                const int i = base + c.lane;
+                const int id = i < t0 ? (int)z.pid[i] : 0;
+                const int d2 = i < t0 ? z.d2r[id] : 0;
+                sw += d2;
+                if (known) continue;
+                const int l2 = whole_root ? d2 : wide_in_set(c, z, z.A2, mask, nc, cand, id);
+                if (i < t0) {
+                    const typename P::word w = z.pw[i];
+                    z.pl2[i] = (typename P::pos_t)l2;
+                    if (l2 < nc - 1 || P::in(w) + P::ex(w) < req) low = true;
+                }
+                known = !c.keys && ballot(low) != 0;
             }
             wadj_lanes(c, sw);
-            wsync();
-            bool bad = false;
-            for (int i = nm + c.lane; i < t0; i += WAVE) {
-                int l2 = whole_root ? c.g.p->d2r[w.pid[i]] : rowpop(c, c.M2, PM(i), w.mk0);
-                w.pl2[i] = l2;
-                if (l2 < nc - 1 || w.pin[i] + w.pex[i] < req) bad = true;
-            }
-            wsync();
-            if (ballot(bad) == 0 && !cut_root) {
-                emit_clique(c, w.pid, t0);
+            lsync();
+            if (ballot(low) == 0 && !cut_root) {
+                wide_emit(c, t0, [&](int i) { return z.pid[i]; });
                 ph_mark(c, PH_LOOKAHEAD);
-                return;
+                return true;
             }
         }
     }
     ph_mark(c, PH_LOOKAHEAD);
 
     // ---- branch loop, main.cu:1094-1180 ----
-    // Branch ordinal b = j - covered.  Branch b >= 1 first removes the last
-    // parent vertex (remove_one_vertex); a failing member ends the loop.
+    // Branch ordinal b takes position t0 - 1 - b.  Branch b >= 1 first removes
+    // the vertex of the branch before; a failing member ends the loop.
     int tp = t0;
-    const int expansions = nc;
-    const bool root = ref.depth == 0;
-    const int nb = expansions - cov;
-    int bend = nb;
-    if (root && c.g.p->root_b1 >= 0 && c.g.p->root_b1 < bend) bend = (int)c.g.p->root_b1;
-    // a negative window start counts from the end of the root's branches
-    const long long rb0 = c.g.p->root_b0 >= 0 ? c.g.p->root_b0 : max(0ll, (long long)nb + c.g.p->root_b0);
-    const int bbeg = root ? (int)min<long long>(rb0, (long long)nb) : 0;
-
-    // remove one vertex, main.cu:1408-1462; returns true on a member failure
-    // With members_only, candidates keep their exdeg and `pend` names the
-    // removed vertex: the child build applies it to them in its own pass.
-    int pend = -1;
-    auto remove_step = [&](bool count, bool members_only) -> bool {
-        int mdg = get_mindeg(c, nm);
-        nc--;
-        tp--;
-        int rr = PM(tp);
-        pend = members_only ? rr : -1;
-        bool fail = false;
-        int fid = INT32_MAX;  // smallest failing member id
-        const int upto = members_only ? nm : tp;
-        for (int i = c.lane; i < upto; i += WAVE) {
-            if (gbit(c.M1, c.W, rr, PM(i))) {
-                int ex = w.pex[i] - 1;
-                w.pex[i] = ex;
-                if (i < nm && w.pin[i] + ex < mdg) {
-                    fail = true;
-                    fid = min(fid, w.pid[i]);
-                }
-            }
+    int b_lo = 0, b_hi = bend;
+    if (item) {
+        // removals 1..b0 at once (the prepare step found no failure before
+        // the item's range); b0 and b1 count from the record it stored
+        b_lo = (int)ref.b0;
+        b_hi = (int)ref.b1;
+        tp = t0 - b_lo;
+        nc -= b_lo;
+        wide_bulk_remove(c, z, tp, b_lo);
+        ph_mark(c, PH_REMOVE);
+    } else {
+        // a root's branches are split finer, to about one item per resident
+        // wave over all roots: until the roots' items produce children nothing
+        // else can run
+        int ch = a.queue_mode ? a.split_chunk : 0;
+        if (root && ch > 0 && a.n_roots > 0) {
+            const long long want = ((long long)(bend - bbeg) * a.n_roots + gridDim.x - 1) / gridDim.x;
+            ch = (int)max(1ll, min((long long)ch, want));
         }
-        wsync();
-        if (ballot(fail)) {
-            if (count) {
-                // the reference scans N(r) in ascending id order and stops
-                // after the first failing member
-                fid = uni(wave_min(fid));
-                const int rid = w.pid[tp];
-                const uint64_t* row = c.g.p->A1 + (size_t)rid * c.g.p->rw;
-                int rank = 0;
-                for (int wd = c.lane; wd <= (fid >> 6); wd += WAVE) {
-                    uint64_t x = row[wd];
-                    if (wd == (fid >> 6)) x &= (1ull << (fid & 63)) - 1ull;
-                    rank += __popcll(x);
-                }
-                wadj_lanes(c, rank + (c.lane == 0));
-            }
+        if (ch > 0 && (uint32_t)t0 > a.split_min_t && bend - bbeg > ch) {
+            wide_split(c, z, ref, nm, bbeg, bend, ch);
+            ph_mark(c, PH_PREPARE);
             return true;
         }
-        if (count) wadj_add(c, c.g.p->d1r[w.pid[tp]]);
-        return false;
-    };
-
-    // exdeg of positions [0, keep) minus their neighbours among positions
-    // [keep, keep + nr): several removals at once
-    auto bulk_remove = [&](int keep, int nr) {
-        if (nr <= 0) return;
-        if (nr < c.W) {
-            for (int k = c.lane; k < nr; k += WAVE) w.adjc[k] = PM(keep + k);
-            wsync();
-            for (int i = c.lane; i < keep; i += WAVE) {
-                const int row = PM(i);
-                int cnt = 0;
-                for (int k = 0; k < nr; k++) cnt += (int)gbit(c.M1, c.W, row, w.adjc[k]);
-                w.pex[i] -= cnt;
-            }
-        } else {
-            clear_mask(c, w.mk0);
-            for (int q = keep + c.lane; q < keep + nr; q += WAVE) set_mask_bit(w.mk0, PM(q));
-            wsync();
-            for (int i = c.lane; i < keep; i += WAVE) w.pex[i] -= rowpop4(c, c.M1, PM(i), w.mk0);
-        }
-        wsync();
-    };
-
-    int b_lo = 0, b_hi = nb;
-    bool count_removes = true;
-    // a root's branches are split finer, to about one item per resident wave
-    // over all roots: until the roots' items produce children nothing else
-    // can run
-    int ch = a.split_chunk;
-    if (ref.depth == 0 && ch > 0 && a.n_roots > 0) {
-        const long long want = ((long long)(bend - bbeg) * a.n_roots + gridDim.x - 1) / gridDim.x;
-        ch = (int)max(1ll, min((long long)ch, want));
-    }
-    if (item) {
-        // split item: apply removals 1..b0 at once (the prepare step found no
-        // failure before its range), then run branches [b0, b1); b0 and b1
-        // count from the record the prepare step stored
-        const int b0 = (int)ref.b0;
-        if (b0 > 0) {
-            bulk_remove(t0 - b0, b0);
-            tp = t0 - b0;
-            nc -= b0;
-        }
-        ph_mark(c, PH_REMOVE);
-        b_lo = b0;
-        b_hi = (int)ref.b1;
-        count_removes = false;
-    } else if (a.queue_mode && ch > 0 && (uint32_t)t0 > a.split_min_t && bend - bbeg > ch) {
-        // prepare step: find the first failing removal, count the
-        // removals' scans, store the record as it stands before the first
-        // branch of the window (with lvl2adj) and push the items
-        // Removal k (branch b = k) takes position t0 - k.  Member i fails at
-        // the removal of its need_i-th neighbour counted from the end, with
-        // need_i = max(pin + pex - mindeg(nm) + 1, 1); kb = the first such
-        // removal over all members (bend: none before the window's end).
-        const int mdg = get_mindeg(c, nm);
-        int kb = bend;
-        for (int i = 0; i < nm; i++) {
-            const int need = max(w.pin[i] + w.pex[i] - mdg + 1, 1);
-            const int row = PM(i);
-            // removals up to kb inclusive: a member failing at the same
-            // removal as an earlier one must be seen (smallest failing id)
-            const int lim = min(kb, bend - 1);
-            int cnt = 0, ki = INT32_MAX;
-            for (int k0 = 1; k0 <= lim && ki == INT32_MAX; k0 += WAVE) {
-                const int k = k0 + c.lane;
-                const bool nb_ = k <= lim && gbit(c.M1, c.W, row, PM(t0 - k));
-                const uint64_t bm = ballot(nb_);
-                const int pc = __popcll(bm);
-                if (cnt + pc >= need) {
-                    const uint64_t hit = ballot(nb_ && cnt + lanes_below(bm) + 1 == need);
-                    ki = k0 + __builtin_ctzll(hit);
-                }
-                cnt += pc;
-            }
-            w.rem[i] = ki;
-            kb = min(kb, ki);
-        }
-        wsync();
-        // W_adj of the removals: full scans of N(r) for removals 1..kb-1,
-        // the partial scan up to the smallest failing member for removal kb
-        long long sw = 0;
-        for (int k = 1 + c.lane; k < kb; k += WAVE) sw += c.g.p->d1r[w.pid[t0 - k]];
-        wadj_lanes(c, sw);
-        if (kb < bend) {
-            int fid = INT32_MAX;
-            for (int i = c.lane; i < nm; i += WAVE)
-                if (w.rem[i] == kb) fid = min(fid, w.pid[i]);
-            fid = uni(wave_min(fid));
-            const uint64_t* rrow = c.g.p->A1 + (size_t)w.pid[t0 - kb] * c.g.p->rw;
-            int rank = 0;
-            for (int wd = c.lane; wd <= (fid >> 6); wd += WAVE) {
-                uint64_t x = rrow[wd];
-                if (wd == (fid >> 6)) x &= (1ull << (fid & 63)) - 1ull;
-                rank += __popcll(x);
-            }
-            wadj_lanes(c, rank + (c.lane == 0));
-        }
-        const int hi = min(kb, bend);
-        if (hi <= bbeg) {
-            ph_mark(c, PH_PREPARE);
-            return;
-        }
-        // removals 1..bbeg happen before the window: apply them once here
-        const int pre = bbeg;
-        const int ts = t0 - pre;
-        bulk_remove(ts, pre);
-        // the record plus one Vrec after it whose id counts the items still
-        // to run (the last one frees the block)
-        unsigned long long slot = 0;
-        if (c.lane == 0) slot = pool_alloc(c, (uint32_t)ts + 1u);
-        slot = rdlane64(slot, 0);
-        if (slot == ~0ull) {
-            if (c.lane == 0) atomicOr(a.error, 1);
-            return;
-        }
-        for (int i = c.lane; i < ts; i += WAVE) {
-            Vrec v;
-            v.id = w.pid[i];
-            v.label = w.plab[i] | (w.pl2[i] << 4);
-            v.indeg = w.pin[i];
-            v.exdeg = w.pex[i];
-            a.pool[slot + i] = v;
-        }
-        const int n_items = (hi - bbeg + ch - 1) / ch;
-        if (c.lane == 0) a.pool[slot + ts] = Vrec{n_items, 0, 0, 0};
-        // item boundaries balance the work rather than the branch count:
-        // branch b builds a child from about t0 - b vertices, so with
-        // S(b) = sum of (t0 - x) over x in [bbeg, b), boundary j is the first
-        // b with S(b) >= j S(hi) / n_items (kept strictly increasing)
-        const long long t0l = t0;
-        auto S = [&](long long b) {
-            return (b - bbeg) * t0l - (b * (b - 1) - (long long)bbeg * (bbeg - 1)) / 2;
-        };
-        const long long s_tot = S(hi);
-        auto boundary = [&](int j) -> int {
-            if (j <= 0) return bbeg;
-            if (j >= n_items) return hi;
-            const long long target = s_tot * j / n_items;
-            int lo = bbeg, up = hi;
-            while (lo < up) {
-                const int mid = (lo + up) >> 1;
-                if (S(mid) >= target)
-                    up = mid;
-                else
-                    lo = mid + 1;
-            }
-            return min(max(lo, bbeg + j), hi - (n_items - j));
-        };
-        auto item_ref = [&](int j) {
-            TaskRef r;
-            r.off = slot;
-            r.t = (uint32_t)ts;
-            r.depth = ref.depth;
-            r.inst = ref.inst;
-            r.bound = (uint64_t)c.slot;  // the task the item belongs to (trace)
-            r.b0 = (uint32_t)(boundary(j) - pre);
-            r.b1 = (uint32_t)(boundary(j + 1) - pre);
-            return r;
-        };
-        // the items go to the top ring in chunks of up to 64 claimed at once
-        // (lanes write the refs, one release fence per chunk); what the ring
-        // cannot take stays on this wave's stack
-        const int top = a.n_buckets - 1;
-        const int rg = top * a.q_shards + c.shard;
-        int done = 0;
-        while (done < n_items) {
-            unsigned long long pos = 0;
-            const int k = ring_claim(c, rg, min(n_items - done, WAVE), &pos);
-            if (k == 0) break;
-            if (c.lane == 0)
-                __hip_atomic_fetch_add(a.pending, (unsigned long long)k, __ATOMIC_RELAXED,
-                                       __HIP_MEMORY_SCOPE_AGENT);
-            if (c.lane < k) {
-                const unsigned long long gi = (unsigned long long)rg * a.q_cap + (pos + c.lane) % a.q_cap;
-                if (a.trace_parent) a.trace_parent[gi] = -2;
-                a.q_refs[gi] = item_ref(done + c.lane);
-            }
-            ring_publish(c, rg, pos, k);
-            done += k;
-        }
-        for (; done < n_items; done++)
-            if (!push_ref(c, item_ref(done), top, false, nullptr)) break;
-        ph_mark(c, PH_PREPARE);
-        return;
-    }
-
-    // A window that starts at branch bbeg > 0 first needs removals
-    // 1..bbeg.  Without members none of them can fail, so they are applied at
-    // once (their adjacency scans counted as the sequential removals count
-    // them) and the loop starts at bbeg.
-    if (!item && bbeg > 0 && nm == 0 && bbeg < bend) {
-        long long sw = 0;
-        for (int k = 1 + c.lane; k <= bbeg; k += WAVE) sw += c.g.p->d1r[w.pid[t0 - k]];
-        if (count_removes) wadj_lanes(c, sw);
-        bulk_remove(t0 - bbeg, bbeg);
-        tp = t0 - bbeg;
-        nc -= bbeg;
-        b_lo = bbeg;
-        ph_mark(c, PH_REMOVE);
-    }
-
-    for (int b = b_lo; b < b_hi; b++) {
-        if (!item && b >= bend) break;
-        pend = -1;
-        if (b > b_lo || (!item && b > 0 && b_lo == 0)) {
-            // before the window (no child built) the removal is applied
-            // whole; otherwise the child build applies it to the candidates
-            const bool stop = remove_step(count_removes, item || b >= bbeg);
+        if (bbeg > 0 && bbeg < bend) {
+            // a window that starts at branch bbeg: removals 1..bbeg at once
+            // (the root has no members: none of them can fail)
+            long long sw = 0;
+            for (int k = 1 + c.lane; k <= bbeg; k += WAVE) sw += z.d1r[z.pid[t0 - k]];
+            wadj_lanes(c, sw);
+            b_lo = bbeg;
+            tp = t0 - bbeg;
+            nc -= bbeg;
+            wide_bulk_remove(c, z, tp, bbeg);
             ph_mark(c, PH_REMOVE);
-            if (stop) break;
+        } else if (bbeg > 0) {
+            // an empty window: the removals before it are counted as the
+            // reference makes them, up to the window's end
+            long long sw = 0;
+            for (int k = 1 + c.lane; k < bend; k += WAVE) sw += z.d1r[z.pid[t0 - k]];
+            wadj_lanes(c, sw);
+            return true;
         }
-        if (!item && b < bbeg) continue;
-        // child record (main.cu:1094-1180 with add_one_vertex, main.cu:1465-1523,
-        // and diameter pruning, main.cu:1709-1732, applied while it is built):
-        // members, then the branch vertex (parent position tp - 1) as a
-        // member, then the candidates inside N2(v) in parent order with their
-        // degrees updated for v; candidates outside N2(v) follow with id and
-        // matrix index only (label -1: degree pruning counts them as removed)
-        if (c.lane == 0) c.st->branches++;
+    }
+    const int ms = c.g.min_size;
+    const int mdg = nm < ms ? z.mds : wide_md(c, z, nm);  // get_mindeg(nm)
+    // rows of the next branch vertex, in registers until its branch starts
+    constexpr int NJ = WIDE_ROW_WORDS / WAVE;
+    uint64_t n1[NJ], n2[NJ];
+    int nd1 = 0, nd2 = 0;  // its |N n root|, |N2 n root|
+    auto fetch = [&](int p) {
+        const int id = uni((int)z.pid[p]);
+        nd1 = z.d1r[id];
+        nd2 = z.d2r[id];
+        if (!z.rl) return;
+        const size_t r0 = (size_t)id * z.rw;
+#pragma unroll
+        for (int j = 0; j < NJ; j++) {
+            const int wd = j * WAVE + c.lane;
+            n1[j] = 0;
+            n2[j] = 0;
+            if (wd < z.rw) {
+                n1[j] = z.A1[r0 + wd];
+                n2[j] = z.A2[r0 + wd];
+            }
+        }
+    };
+    if (b_lo < b_hi) fetch(tp - 1);
+    int d1v = 0;
+    for (int b = b_lo; b < b_hi; b++) {
+        const bool pend = b > b_lo;
+        if (pend) {
+            // remove_one_vertex (main.cu:1408-1462) for the last branch's
+            // vertex: the members here, the candidates with the child's build
+            nc--;
+            tp--;
+            bool fail = false;
+            int fid = INT32_MAX;
+            for (int i = c.lane; i < nm; i += WAVE) {
+                if ((z.nbits[i >> 6] >> (i & 63)) & 1ull) {
+                    const typename P::word w = z.pw[i] - 1u;
+                    z.pw[i] = w;
+                    if (P::in(w) + P::ex(w) < mdg) {
+                        fail = true;
+                        fid = min(fid, (int)z.pid[i]);
+                    }
+                }
+            }
+            if (ballot(fail)) {
+                if (!item) wide_failed_scan(c, z, uni((int)z.pid[tp]), wave_min(fid));
+                break;
+            }
+            if (!item) wadj_add(c, d1v);
+            ph_mark(c, PH_REMOVE);
+        }
         const int vsrc = tp - 1;
-        const int vpp = PM(vsrc);
-        wadj_add(c, (long long)c.g.p->d1r[w.pid[vsrc]] + c.g.p->d2r[w.pid[vsrc]]);
-        for (int i = c.lane; i < nm; i += WAVE) {
-            const int pp = PM(i);
-            const int a1 = (int)gbit(c.M1, c.W, vpp, pp);
-            w.cid[i] = w.pid[i];
-            w.cpp[i] = pp;
-            w.clab[i] = w.plab[i];
-            w.cin[i] = w.pin[i] + a1;
-            w.cex[i] = w.pex[i] - a1;
-            if (c.keys) w.cl2[i] = w.pl2[i];
+        const int vid = uni((int)z.pid[vsrc]);
+        d1v = nd1;
+        wadj_add(c, (long long)nd1 + nd2);
+        if (z.rl) {
+#pragma unroll
+            for (int j = 0; j < NJ; j++) {
+                const int wd = j * WAVE + c.lane;
+                if (wd < z.rw) {
+                    z.row1[wd] = n1[j];
+                    z.row2[wd] = n2[j];
+                }
+            }
         }
+        lsync();
+        if (b + 1 < b_hi) fetch(vsrc - 1);
+        if (c.lane == 0) c.st->branches++;
+        // the child: members, the branch vertex, then the candidates inside
+        // N2(v) with their degrees updated (add_one_vertex, main.cu:1465-1523,
+        // diameter pruning, main.cu:1709-1732); the others go on the list
+        int m = nm + 1, n = 0, nl = 0;
         if (c.lane == 0) {
-            int pv = w.pex[vsrc];
-            if (pend >= 0 && gbit(c.M1, c.W, pend, vpp)) w.pex[vsrc] = --pv;
-            w.cid[nm] = w.pid[vsrc];
-            w.cpp[nm] = vpp;
-            w.clab[nm] = 1;
-            w.cin[nm] = w.pin[vsrc];
-            w.cex[nm] = pv;
-            if (c.keys) w.cl2[nm] = w.pl2[vsrc];
+            typename P::word w = z.pw[vsrc];
+            if (pend) w -= (uint32_t)(z.nbits[vsrc >> 6] >> (vsrc & 63)) & 1u;
+            z.cw[nm] = w;
+            z.cpos[nm] = (typename P::pos_t)vsrc;
         }
-        int m = nm + 1, cc = nc - 1;
-        // one pass over the candidates: the survivors of the 2-hop test go
-        // to [m, m + ns) in parent order with their degrees updated for v;
-        // the others (id and matrix index only) are staged in rem / rmv and
-        // appended after the survivors
-        int nsd = 0, ndd = 0, hV = 0, hc = 0;
-        for (int base = nm; base < vsrc; base += WAVE) {
-            const int q = base + c.lane;
-            const bool in = q < vsrc;
-            const int pp = in ? PM(q) : 0;
-            const bool ok = in && gbit(c.M2, c.W, vpp, pp);
-            const uint64_t bo = ballot(ok), bx = ballot(in && !ok);
-            int pexq = 0;
-            if (in) {
-                // the removal of this branch (main.cu:1437-1450) for the
-                // parent's candidate q
-                pexq = w.pex[q];
-                if (pend >= 0 && gbit(c.M1, c.W, pend, pp)) w.pex[q] = --pexq;
+        const size_t r0 = (size_t)vid * z.rw;
+        lsync();
+        for (int base = 0; base < vsrc; base += P::U * WAVE) {
+            uint32_t id[P::U];
+            typename P::word w[P::U];
+            uint64_t x1[P::U], x2[P::U], ob[P::U];
+#pragma unroll
+            for (int u = 0; u < P::U; u++) {
+                const int i = base + u * WAVE + c.lane;
+                id[u] = i < vsrc ? z.pid[i] : 0u;
+                w[u] = i < vsrc ? z.pw[i] : (typename P::word)0;
+                ob[u] = pend && base + u * WAVE < vsrc ? z.nbits[base / WAVE + u] : 0ull;
             }
-            int xin = -1;
-            if (ok) {
-                const int r = lanes_below(bo);
-                const int d = m + nsd + r;
-                const int a1 = (int)gbit(c.M1, c.W, vpp, pp);
-                const int cin_ = w.pin[q] + a1;
-                xin = cin_;
-                w.cid[d] = w.pid[q];
-                w.cpp[d] = pp;
-                w.clab[d] = 0;
-                w.cin[d] = cin_;
-                w.cex[d] = pexq - a1;
-                if (c.keys) w.cl2[d] = w.pl2[q];
-                if (m >= WAVE) w.cind[nsd + r] = cin_;  // else the register table
-            } else if (in) {
-                const int d = ndd + lanes_below(bx);
-                w.rem[d] = w.pid[q];
-                w.rmv[d] = pp;
+#pragma unroll
+            for (int u = 0; u < P::U; u++) {
+                if (z.rl) {
+                    x1[u] = z.row1[id[u] >> 6];
+                    x2[u] = z.row2[id[u] >> 6];
+                } else {
+                    x1[u] = z.A1[r0 + (id[u] >> 6)];
+                    x2[u] = z.A2[r0 + (id[u] >> 6)];
+                }
             }
-            nsd += __popcll(bo);
-            ndd += __popcll(bx);
-            if (m < WAVE) hist_chunk(c, xin, hc, hV);
+            lsync();
+#pragma unroll
+            for (int u = 0; u < P::U; u++) {
+                const int i = base + u * WAVE + c.lane;
+                if (base + u * WAVE >= vsrc) break;
+                const bool in = i < vsrc, cand = in && i >= nm;
+                const uint32_t a1 = (uint32_t)(x1[u] >> (id[u] & 63)) & 1u;
+                const uint32_t a2 = (uint32_t)(x2[u] >> (id[u] & 63)) & 1u;
+                const uint32_t o = (uint32_t)(ob[u] >> c.lane) & 1u;
+                if (cand && o) {
+                    w[u] -= 1u;
+                    z.pw[i] = w[u];
+                }
+                const uint64_t bm = ballot(in && a1);
+                if (c.lane == 0) z.nbits[base / WAVE + u] = bm;
+                const typename P::word wc = w[u] + (a1 ? P::ADJ1 : (typename P::word)0);
+                const bool ok = cand && a2;
+                const uint64_t bo = ballot(ok), bx = ballot(cand && !a2);
+                if (ok || (in && i < nm)) {
+                    const int d = ok ? m + n + lanes_below(bo) : i;
+                    z.cw[d] = wc;
+                    z.cpos[d] = (typename P::pos_t)i;
+                }
+                if (bx) {
+                    if (cand && !a2) z.list[nl + lanes_below(bx)] = (typename P::pos_t)i;
+                    nl += __popcll(bx);
+                }
+                n += __popcll(bo);
+            }
+            lsync();
         }
-        const int ns = nsd;
-        wsync();
-        for (int k = c.lane; k < ndd; k += WAVE) {
-            const int d = m + ns + k;
-            w.cid[d] = w.rem[k];
-            w.cpp[d] = w.rmv[k];
-            w.clab[d] = -1;
-        }
-        int tc = m + ns + ndd;
-        int nind = ns;
-        wsync();
         ph_mark(c, PH_ADD);
         int ub = 0, lb = 0, med = 0;
         // degree pruning, then critical-vertex pruning, which ends in a
-        // second degree pruning (one call site: the call is inlined)
-        bool first = true, map_empty = false, skip = false;
-        int r = 0;
-        int preV = m < WAVE ? hV : -1;  // the build's table of the survivors' indegrees
+        // second degree pruning
+        bool first = true, map_empty = false, fails;
         for (;;) {
-            const bool fail = degree_pruning(c, tc, cc, m, ub, lb, med, nind, map_empty, preV, hc);
-            preV = -1;
-            if (!first) {
-                r = fail ? 1 : 0;
-                break;
-            }
-            if (fail) {
-                if (m >= c.g.min_size) check_for_clique(c, m);
-                skip = true;
-                break;
-            }
-            const int crit = critical_prep(c, tc, cc, m, lb, nind, map_empty);
-            ph_mark(c, PH_CRIT);
-            if (crit == 2) {
-                skip = true;
-                break;
-            }
+            fails = wide_prune(c, z, m, n, nl, map_empty, ub, lb, med);
+            if (!first || fails) break;
             first = false;
+            if (wide_critical(c, z, m, n, nl, lb, map_empty) == 2) {
+                m = -1;  // neither a clique test nor a child
+                break;
+            }
+            ph_mark(c, PH_CRIT);
         }
-        if (skip) {
-            ph_mark(c, PH_PRUNE);
+        if (m < 0) {
+            ph_mark(c, PH_CRIT);
             continue;
         }
-        if (m >= c.g.min_size) check_for_clique(c, m);
+        if (m >= ms) {
+            // clique test, main.cu:1974-1995
+            const int req = wide_md(c, z, m);
+            bool low = false;
+            for (int i = c.lane; i < m; i += WAVE) low |= P::in(z.cw[i]) < req;
+            if (ballot(low) == 0) wide_emit(c, m, [&](int i) { return z.pid[z.cpos[i]]; });
+        }
         ph_mark(c, PH_PRUNE);
-        if (r == 1) continue;
-        if (cc > 0) write_child(c, tc, m, ub - lb);
-        wsync();
+        if (!fails && n > 0) wide_child(c, z, m, n, ub - lb);
+        lsync();
         ph_mark(c, PH_CHILD);
     }
-#undef PM
+    return true;
+}
+
+// whether a task of t vertices runs from LDS
+__device__ __forceinline__ bool wide_fits(const Ctx& c, uint32_t t, uint32_t lds_bytes) {
+    return t <= WIDE_LDS_MAX && c.g.p->R <= WIDE_LDS_R_MAX &&
+           wide_lds_bytes(t, (uint32_t)c.g.p->rw) <= lds_bytes;
+}
+
+// a task of any size and kind
+__device__ __attribute__((always_inline)) void process_task(Ctx& c, const TaskRef& ref, char* lds, uint32_t lds_bytes,
+                                                            char* slab) {
+    if (wide_fits(c, ref.t, lds_bytes) && process_wide<WideLds>(c, ref, lds, lds_bytes, slab)) return;
+    process_wide<WideSlab>(c, ref, lds, lds_bytes, slab);
 }
 
 // ---------------------------------------------------------------------------
@@ -2608,9 +2612,29 @@ __device__ __forceinline__ void flush_stats(Ctx& c, DevStats* d) {
 }
 __device__ __forceinline__ void flush_stats(Ctx& c) { flush_stats(c, c.a->stats); }
 
-template <bool LOCAL>
-__device__ __forceinline__ void task_loop(Ctx& c, char* lds, uint16_t* sdep) {
-    const ExpandArgs& a = *c.a;
+// Level-synchronous form (expand_level): one wave per task of the batch.  Small
+// tasks are launched with little LDS and many waves per CU, large ones with a
+// quarter of a CU's LDS and a slab each.
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void expand_level(
+    const ExpandArgs* __restrict__ ap) {
+    const ExpandArgs& a = *ap;
+    extern __shared__ __attribute__((aligned(16))) char lds[];
+    __shared__ uint16_t s_dep[TINY_MAX];
+    __shared__ LStats s_st;
+    __shared__ unsigned long long s_ph[PH_COUNT];
+    Ctx c;
+    c.wadj_l = 0;
+    c.a = ap;
+    c.g = load_graph(&ap->g);
+    c.phase_on = ap->phase != nullptr;
+    c.inst = 0;
+    c.slot = -1;
+    c.lane = lane_id();
+    c.st = &s_st;
+    c.ph = s_ph;
+    if (c.lane == 0) s_st = LStats{0, 0, 0, 0, 0, 0, 0, 0, 0};
+    ph_start(c);
+    char* const slab = a.slab + (size_t)blockIdx.x * a.slab_bytes;
     const uint32_t nw = gridDim.x;
     uint32_t i;
     if (a.static_sched) {
@@ -2621,22 +2645,15 @@ __device__ __forceinline__ void task_loop(Ctx& c, char* lds, uint16_t* sdep) {
         i = (uint32_t)rdlane((int)x, 0);
     }
     while (i < a.n_in) {
-        TaskRef ref = a.in_refs[i];
-        bool done = false;
-        if (LOCAL && ref.t <= TINY_MAX && ref.depth > 0) {
-            Tiny y;
-            done = tiny_load(c, ref, y);
-            if (done) {
-                c.depth = ref.depth;
-                y.cap = TINY_MAX;
-                tiny_level(c, y, (uint32_t*)lds, sdep);
-            }
+        const TaskRef ref = a.in_refs[i];
+        Tiny y;
+        if (ref.t <= TINY_MAX && ref.depth > 0 && ref.b1 == 0 && tiny_load(c, ref, y)) {
+            c.depth = ref.depth;
+            y.cap = TINY_MAX;
+            tiny_level(c, y, (uint32_t*)lds, s_dep);
+        } else {
+            process_task(c, ref, lds, a.lds_bytes, slab);
         }
-        if (done) {
-        } else if (ref.t <= c.cap)
-            process_task<LOCAL>(c, ref);
-        else if (c.lane == 0)
-            atomicOr(a.error, 2);
         wsync();
         if (a.static_sched) {
             i += nw;
@@ -2649,55 +2666,6 @@ __device__ __forceinline__ void task_loop(Ctx& c, char* lds, uint16_t* sdep) {
     flush_stats(c);
 }
 
-template <int TL>
-__global__ __launch_bounds__(64) void expand_local(const ExpandArgs* __restrict__ ap) {
-    const ExpandArgs& a = *ap;
-    // the LDS workspace, or the children of a task of at most 64 vertices
-    constexpr size_t WS_BYTES = ws_bytes(TL, true, (TL + 63) / 64);
-    constexpr size_t BYTES = WS_BYTES > TINY_MAX * TINY_ENTRY ? WS_BYTES : TINY_MAX * TINY_ENTRY;
-    __shared__ __attribute__((aligned(16))) char lds[BYTES];
-    __shared__ uint16_t s_dep[TINY_MAX];
-    Ctx c;
-    c.wadj_l = 0;
-    c.a = ap;
-    c.g = load_graph(&ap->g);
-    c.phase_on = ap->phase != nullptr;
-    c.inst = 0;
-    c.slot = -1;
-    c.lane = lane_id();
-    c.w = make_ws(lds, TL, true, (TL + 63) / 64);
-    c.cap = TL;
-    __shared__ LStats s_st;
-    __shared__ unsigned long long s_ph[PH_COUNT];
-    c.st = &s_st;
-    c.ph = s_ph;
-    if (c.lane == 0) s_st = LStats{0, 0, 0, 0, 0, 0, 0, 0, 0};
-    ph_start(c);
-    task_loop<true>(c, lds, s_dep);
-}
-
-__global__ __launch_bounds__(64) void expand_hbm(const ExpandArgs* __restrict__ ap) {
-    const ExpandArgs& a = *ap;
-    Ctx c;
-    c.wadj_l = 0;
-    c.a = ap;
-    c.g = load_graph(&ap->g);
-    c.phase_on = ap->phase != nullptr;
-    c.inst = 0;
-    c.slot = -1;
-    c.lane = lane_id();
-    char* base = a.slab + (size_t)blockIdx.x * a.slab_bytes;
-    c.w = make_ws(base, a.slab_tcap, false, a.slab_mwords);
-    c.cap = a.slab_tcap;
-    __shared__ LStats s_st;
-    __shared__ unsigned long long s_ph[PH_COUNT];
-    c.st = &s_st;
-    c.ph = s_ph;
-    if (c.lane == 0) s_st = LStats{0, 0, 0, 0, 0, 0, 0, 0, 0};
-    ph_start(c);
-    task_loop<false>(c, nullptr, nullptr);
-}
-
 // diagnostics: one task's row of the timeline
 __device__ __forceinline__ void timeline_row(Ctx& c, const TaskRef& ref, long long gslot, long long start) {
     if (c.lane != 0) return;
@@ -2708,17 +2676,29 @@ __device__ __forceinline__ void timeline_row(Ctx& c, const TaskRef& ref, long lo
     r[3] = (unsigned long long)ref.depth | ((unsigned long long)ref.b0 << 16) | ((unsigned long long)ref.b1 << 40);
 }
 
+// The block of a task that ran: a split item's prepared record is freed by the
+// last of its items (count in the Vrec after the record); roots live outside
+// the pool's blocks.
+__device__ __attribute__((always_inline)) void release_record(Ctx& c, const TaskRef& ref) {
+    if (c.lane != 0) return;
+    if (ref.b1 > 0) {
+        const int left = __hip_atomic_fetch_add(&c.a->pool[ref.off + ref.t].id, -1, __ATOMIC_ACQ_REL,
+                                                __HIP_MEMORY_SCOPE_AGENT);
+        if (left == 1) pool_free(c, ref.off, ref.t + 1u);
+    } else if (ref.depth > 0) {
+        pool_free(c, ref.off, ref.t);
+    }
+}
+
 // ---------------------------------------------------------------------------
-// persistent kernel: every wave pops task refs from the FIFO queue until the
-// pending counter reaches zero; tasks of at most TL vertices run from LDS,
-// larger ones from the wave's HBM slab.
+// persistent kernel: every wave takes tasks from its own stack and the shared
+// rings until the pending counter reaches zero
 // ---------------------------------------------------------------------------
 // (two resident waves per SIMD: the register allocation is held to 256)
-template <int TL>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void expand_persistent(
     const ExpandArgs* __restrict__ ap) {
     const ExpandArgs& a = *ap;
-    // dynamic LDS: max(TL workspace with local matrices, arrays of wide tasks)
+    // a task's arrays, or the stack of a subtree of at most 64 vertices
     extern __shared__ __attribute__((aligned(16))) char lds[];
     Ctx c;
     c.wadj_l = 0;
@@ -2741,8 +2721,6 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void ex
     if (c.lane < FL_SMALL) s_fln[c.lane] = 0;
     wsync();
     char* const slab = a.slab + (size_t)blockIdx.x * a.slab_bytes;
-    const uint32_t mid = a.mid_tcap;
-    const uint32_t wide = a.lds_wide;
     __shared__ LStats s_st;
     __shared__ unsigned long long s_ph[PH_COUNT];
     c.st = &s_st;
@@ -2751,7 +2729,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void ex
     ph_start(c);
     // consecutive idle polls before the launch is declared stuck (about a
     // minute of back-off): every wave then leaves with error bit 4
-    constexpr int IDLE_LIMIT = 1 << 22;
+    constexpr int IDLE_LIMIT = 1 << 24;
     const unsigned long long G = gridDim.x;
     int idle = 0;       // consecutive empty polls (back-off)
     int idle_total = 0;
@@ -2760,9 +2738,6 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void ex
     // the single ring
     unsigned long long spos = blockIdx.x;
 
-    // positions claimed from a ring and not yet run: their refs wait in LDS
-    // (registers are the scarce resource of this kernel)
-    __shared__ TaskRef s_claim[4];
     __shared__ TaskRef s_top;
     // the wave's part of the clique stream (none yet)
     __shared__ unsigned long long s_clq[4];
@@ -2779,22 +2754,18 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void ex
     c.share_n = 0;
     c.share_left = 0;
     c.share_ok = false;
-    int nq = 0, qi = 0;
-    unsigned long long qbase = 0, qh = 0;
+    // the position this wave has taken in a ring and not yet run
+    bool ticket = false;
+    unsigned long long tpos = 0, tbase = 0;
     // `pending` counts the tasks waiting in the rings plus the waves that hold
-    // work (claimed positions or a non-empty stack); `hungry` counts the
+    // work (a published position or a non-empty stack); `hungry` counts the
     // waves that hold none.  A wave changes them only when it takes work
     // from the rings, hands work to them or runs out, not per task.
     bool busy = false;
     for (;;) {
         TaskRef ref;
         long long gslot;
-        if (!tiny && qi < nq) {
-            ref = s_claim[qi];
-            if (c.phase_on && c.lane == 0) c.ph[PH_N_RING]++;
-            gslot = (long long)(qbase + (qh + (unsigned long long)qi) % a.q_cap);
-            qi++;
-        } else if (a.static_sched && c.ptop != c.pbot && static_flush(c)) {
+        if (a.static_sched && c.ptop != c.pbot && static_flush(c)) {
             continue;
         } else if (tiny || c.ptop != c.pbot) {
             // this wave's own stack (depth first)
@@ -2844,9 +2815,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void ex
                             wsync();
                         }
                     }
-                    int bk = 0;
-                    if (c.lane == 0) bk = c.pbkt[c.pbot % a.priv_cap];
-                    const int rg = rdlane(bk, 0) * a.q_shards + c.shard;
+                    const int rg = ring_for(c);
                     // a hand-over is optional: one attempt, and when another
                     // producer moved the tail first the wave keeps its records
                     // (retrying under contention cost more than the records
@@ -2885,144 +2854,105 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void ex
             if (c.phase_on && c.lane == 0) c.ph[PH_N_OWN]++;
         } else {
             // ---- the shared rings ----
-            int state = 0;  // 0 nothing published, 1 got positions, 2 done, 3 retry now
-            unsigned long long h = 0;
-            int nk = 1;     // consecutive positions claimed
-            int bsel = 0;   // their ring
-            if (a.static_sched) {
-                if (c.lane == 0) {
-                    const unsigned long long sq =
-                        __hip_atomic_load(&a.q_seq[spos % a.q_cap], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    if (sq == spos + 1ull) {
-                        state = 1;
-                        h = spos;
-                        spos += G;
+            // A wave without work takes a ticket, the next position of a ring
+            // (one add on its head), and waits for that position's own
+            // sequence word: no two waves want the same task, so a published
+            // task wakes one wave and nobody retries.  (Waves that all read
+            // every ring's counters and raced for each task by compare and
+            // swap slowed the working ones down: with 2,048 waves a power-law
+            // window took 29 ms against 13 with 1,024.)  Heads may run ahead
+            // of tails by the waves that wait; hand-overs go to such rings
+            // (ring_for).  Tasks pushed where nobody waits are found by the
+            // pushing wave itself at the latest: it looks at every ring
+            // before it waits.
+            if (!ticket) {
+                if (a.static_sched) {
+                    tpos = spos;
+                    tbase = 0;
+                    spos += G;
+                } else {
+                    const int NS = a.q_shards;
+                    unsigned long long hl = 0, tl = 0;
+                    if (c.lane < NS) {
+                        hl = __hip_atomic_load(&a.q_head[c.lane * QSTRIDE], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                        tl = __hip_atomic_load(&a.q_tail[c.lane * QSTRIDE], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                     }
-                }
-            } else {
-                // every ring at once: lane l reads the head and tail of ring l
-                // (bucket l / q_shards, shard l % q_shards)
-                const int NS = a.q_shards;
-                const int NR = a.n_buckets * NS;
-                unsigned long long hl = 0, tl = 0;
-                if (c.lane < NR) {
-                    hl = __hip_atomic_load(&a.q_head[c.lane * QSTRIDE], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    tl = __hip_atomic_load(&a.q_tail[c.lane * QSTRIDE], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                }
-                const uint64_t m = ballot(c.lane < NR && tl > hl);
-                if (m) {
                     // this wave's own shard first (its XCD's L2 holds the
-                    // records its neighbours wrote), the highest bucket with
-                    // work there; else the highest bucket with work anywhere,
-                    // from the next shard after this one
-                    uint64_t own = 0;
-                    for (int q = 0; q < a.n_buckets; q++) own |= 1ull << (q * NS + c.shard);
-                    const uint64_t mo = m & own;
-                    const int b = (63 - __builtin_clzll(mo ? mo : m)) / NS;
-                    const uint64_t full = NS == 64 ? ~0ull : (1ull << NS) - 1;
-                    const uint64_t sm = (m >> (b * NS)) & full;
-                    const uint64_t rot = ((sm >> c.shard) | (sm << ((NS - c.shard) & 63))) & full;
-                    const int rsel = b * NS + (c.shard + __builtin_ctzll(rot)) % NS;
-                    const unsigned long long hb = rdlane64(hl, rsel), tb = rdlane64(tl, rsel);
-                    if (c.lane == 0) {
-                        // a very deep ring hands out several consecutive
-                        // positions per claim: one head update per claim limits
-                        // how fast tiny tasks can be taken.  Only very deep: the
-                        // positions of one claim run one after another, which
-                        // lengthens the critical path when they are heavy.  Only
-                        // published positions are claimed.
-                        const unsigned long long avail = tb - hb;
-                        const unsigned long long per = G / (unsigned long long)NS + 1;
-                        const int k = avail >= 32 * per ? 4 : avail >= 16 * per ? 2 : 1;
-                        const unsigned long long* seq = a.q_seq + (size_t)rsel * a.q_cap;
-                        int pub = 0;
-                        while (pub < k && __hip_atomic_load(&seq[(hb + pub) % a.q_cap], __ATOMIC_RELAXED,
-                                                            __HIP_MEMORY_SCOPE_AGENT) == hb + pub + 1ull)
-                            pub++;
-                        if (pub == 0) {
-                            state = 3;  // claimed by a producer, about to be published
-                        } else {
-                            unsigned long long e = hb;
-                            if (__hip_atomic_compare_exchange_strong(&a.q_head[rsel * QSTRIDE], &e,
-                                                                     hb + (unsigned long long)pub, __ATOMIC_RELAXED,
-                                                                     __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
-                                state = 1;
-                                h = hb;
-                                nk = pub;
-                                bsel = rsel;
-                            } else {
-                                state = 3;
-                            }
-                        }
+                    // records its neighbours wrote), else the next one with
+                    // tasks, else wait at its own
+                    const uint64_t m = ballot(c.lane < NS && tl > hl);
+                    int r = c.shard;
+                    if (m && !((m >> r) & 1ull)) {
+                        const uint64_t up = m & ~((2ull << r) - 1ull);
+                        r = __builtin_ctzll(up ? up : m);
                     }
+                    if (c.lane == 0)
+                        tpos = __hip_atomic_fetch_add(&a.q_head[r * QSTRIDE], 1ull, __ATOMIC_RELAXED,
+                                                      __HIP_MEMORY_SCOPE_AGENT);
+                    tpos = rdlane64(tpos, 0);
+                    tbase = (unsigned long long)r * a.q_cap;
                 }
+                ticket = true;
             }
-            // every ring looked empty: finished once nothing is pending (no
-            // ring task and no busy wave: a wave counts itself out only when
-            // its stack is empty, after pushing what it made).  Polls are
-            // relaxed: an acquire invalidates the CU's vector L1 under the
-            // waves still working.
-            if (c.lane == 0 && state == 0 &&
-                (__hip_atomic_load(a.pending, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & 0xFFFFFFFFull) == 0)
-                state = 2;
-            state = rdlane(state, 0);
-            if (state == 2) break;
-            if (state == 3) continue;
-            if (state == 0) {
+            unsigned long long* const cell = &a.q_seq[tbase + tpos % a.q_cap];
+            unsigned long long sq = 0;
+            if (c.lane == 0) sq = __hip_atomic_load(cell, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (rdlane64(sq, 0) != tpos + 1ull) {
                 if (busy) {
                     // out of work: no longer counted in pending, now hungry
                     busy = false;
-                    if (c.lane == 0) {
-                        __hip_atomic_fetch_add(a.pending, PH_HUNGRY - 1ull, __ATOMIC_RELAXED,
-                                               __HIP_MEMORY_SCOPE_AGENT);
-                    }
+                    if (c.lane == 0)
+                        __hip_atomic_fetch_add(a.pending, PH_HUNGRY - 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                     continue;  // look once more before sleeping
                 }
-                // a lost task or another wave's fault: leave (error bit 4)
-                if (rdlane(c.lane == 0 ? __hip_atomic_load(a.error, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0,
-                           0) & 4)
-                    break;
-                idle = idle < 16 ? idle + 1 : 16;
+                // Finished once nothing is pending (no ring task and no busy
+                // wave: a wave counts itself out only when its stack is
+                // empty, after pushing what it made): looked up on every
+                // fourth poll, as is a lost task or another wave's fault
+                // (error bit 4).  Polls are relaxed: an acquire invalidates the
+                // CU's vector L1 under the waves still working.
+                if ((idle_total & 3) == 0) {
+                    int leave = 0;
+                    if (c.lane == 0) {
+                        const unsigned long long pd = __hip_atomic_load(a.pending, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                        const int er = __hip_atomic_load(a.error, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                        leave = (pd & 0xFFFFFFFFull) == 0 || (er & 4) != 0;
+                    }
+                    if (rdlane(leave, 0)) break;
+                }
                 if (++idle_total >= IDLE_LIMIT) {
                     if (c.lane == 0) atomicOr(a.error, 4);
                     break;
                 }
-                for (int k = 0; k < idle; k++) __builtin_amdgcn_s_sleep(32);
+                idle = idle < 8 ? idle + 1 : 8;
+                for (int k = 0; k < idle; k++) __builtin_amdgcn_s_sleep(16);
                 ph_mark(c, PH_IDLE);
                 continue;
             }
             idle = 0;
             idle_total = 0;
-            h = rdlane64(h, 0);
-            nk = rdlane(nk, 0);
-            bsel = rdlane(bsel, 0);
-            // the claimed tasks leave the rings; an idle wave becomes busy
+            ticket = false;
+            // the task leaves the ring; an idle wave becomes busy
             if (c.lane == 0) {
-                const unsigned long long d =
-                    (unsigned long long)((busy ? 0 : 1) - (long long)nk) - (busy ? 0ull : PH_HUNGRY);
-                if (d) __hip_atomic_fetch_add(a.pending, d, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                const unsigned long long d = busy ? 0ull - 1ull : 0ull - PH_HUNGRY;
+                __hip_atomic_fetch_add(a.pending, d, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
             busy = true;
-            // one acquire per claim (pairs with the producers' release before
-            // the sequence words), then lane q reads the ref of position h + q
-            // and gives the cell back for the next lap
+            // the acquire pairs with the producer's release before the
+            // sequence word; the ref is read before the cell goes back for the
+            // next lap, with a plain relaxed store: no release, whose
+            // agent-scope form writes back this XCD's L2
             ph_mark(c, PH_POP);
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-            const unsigned long long base = (unsigned long long)bsel * a.q_cap;
-            if (c.lane < nk) s_claim[c.lane] = a.q_refs[base + (h + c.lane) % a.q_cap];
+            gslot = (long long)(tbase + tpos % a.q_cap);
+            TaskRef r;
+            if (c.lane == 0) r = a.q_refs[gslot];
+            ref = bcast_ref(r, 0);
             wsync();
-            // the refs are in LDS (the barrier waited for their loads), so
-            // the cells go back with plain relaxed stores: no release, whose
-            // agent-scope form writes back this XCD's L2
-            if (c.lane < nk)
-                __hip_atomic_store(&a.q_seq[base + (h + c.lane) % a.q_cap], h + (unsigned long long)c.lane + a.q_cap,
-                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (c.lane == 0)
+                __hip_atomic_store(cell, tpos + a.q_cap, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (c.phase_on && c.lane == 0) c.ph[PH_N_RING]++;
             ph_mark(c, PH_SYNC);
-            nq = nk;
-            qi = 0;
-            qbase = base;
-            qh = h;
-            continue;
         }
         ph_mark(c, PH_POP);
         const long long tl_start = a.timeline ? wall_clock64() : 0;
@@ -3058,94 +2988,15 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void ex
             continue;
         }
         y = Tiny{};  // nothing of it lives across the general path
-        const bool fits = ref.t <= a.slab_tcap;
-        const bool local = ref.t <= (uint32_t)TL || (ref.t > wide && ref.t <= mid);
-        // (built per task: only one workspace descriptor is live)
-        if (ref.t <= (uint32_t)TL) {
-            c.w = make_ws(lds, TL, true, (TL + 63) / 64);
-            c.cap = TL;
-        } else if (ref.t <= wide) {
-            c.w = make_ws_split(lds, wide,
-                                a.lds_masks >= 0 ? (uint64_t*)(lds + a.lds_masks)
-                                                 : (uint64_t*)(slab + ws_bytes(a.slab_tcap, false, 0)),
-                                a.slab_mwords);
-            c.cap = wide;
-        } else if (ref.t <= mid) {
-            c.w = make_ws(slab, mid, true, (mid + 63) / 64);
-            if (a.lds_masks >= 0) {
-                c.w.mk0 = (uint64_t*)(lds + a.lds_masks);
-                c.w.mk1 = c.w.mk0 + (mid + 63) / 64;
-            }
-            c.cap = mid;
-        } else {
-            c.w = make_ws(slab, a.slab_tcap, false, a.slab_mwords);
-            if (a.lds_masks >= 0) {
-                c.w.mk0 = (uint64_t*)(lds + a.lds_masks);
-                c.w.mk1 = c.w.mk0 + a.slab_mwords;
-                // the LDS below the masks (the wide tier's arrays) is free
-                // during a slab task: as many of the task's arrays as fit go
-                // there, in slots of S = t rounded up to 64 entries plus 64
-                // (every array and list of a task holds at most t + 2
-                // entries: positions below t, and the LU tables over
-                // indegrees 0..V+1 with V <= members), in this order: the
-                // child's arrays every pruning pass reads (indegree,
-                // exdegree, label, id, matrix index, lvl2adj), the pruning
-                // lists (rem, rmv, cind, adjc), then the parent's arrays
-                // (indegree, exdegree, label, id, lvl2adj).  When the
-                // children lie past the depth window their lvl2adj is never
-                // kept, and the parent's exdegree, updated by every branch,
-                // takes its slot.  The sort keys keep their slab addresses
-                // (the bitonic sort pads them to a power of two).
-                const uint32_t S = ((ref.t + 63u) & ~63u) + 64u;
-                const uint32_t k = (uint32_t)a.lds_masks / (S * 4);
-                const bool keys = !(c.g.max_depth >= 0 && (int)ref.depth + 1 > c.g.max_depth);
-                int* lp = (int*)lds;
-                uint32_t n = 0;
-                auto put = [&](int*& p) {
-                    if (n < k) p = lp + n * S;
-                    n++;
-                };
-                put(c.w.cin);
-                put(c.w.cex);
-                put(c.w.clab);
-                put(c.w.cid);
-                put(c.w.cpp);
-                put(keys ? c.w.cl2 : c.w.pex);
-                put(c.w.rem);
-                put(c.w.rmv);
-                put(c.w.cind);
-                put(c.w.adjc);
-                if (k > 8) c.w.T2 = (int)S;  // the LU tables' capacity (cind, adjc)
-                put(c.w.pin);
-                if (keys) put(c.w.pex);
-                put(c.w.plab);
-                put(c.w.pid);
-                if (keys) put(c.w.pl2);
-            }
-            c.cap = a.slab_tcap;
-        }
-        if (!fits) {
+        if (ref.t > a.slab_tcap) {
             if (c.lane == 0) atomicOr(a.error, 2);
-        } else if (local) {
-            process_task<true>(c, ref);
         } else {
-            process_task<false>(c, ref);
+            process_task(c, ref, lds, a.lds_bytes, slab);
         }
         wsync();
         if (a.timeline && gslot >= 0) timeline_row(c, ref, gslot, tl_start);
         ph_mark(c, PH_CHILD);
-        if (c.lane == 0) {
-            // the record's block: a split item's prepared record is freed by
-            // the last of its items (count in the Vrec after the record);
-            // roots live outside the pool's blocks
-            if (ref.b1 > 0) {
-                const int left = __hip_atomic_fetch_add(&a.pool[ref.off + ref.t].id, -1, __ATOMIC_ACQ_REL,
-                                                        __HIP_MEMORY_SCOPE_AGENT);
-                if (left == 1) pool_free(c, ref.off, ref.t + 1u);
-            } else if (ref.depth > 0) {
-                pool_free(c, ref.off, ref.t);
-            }
-        }
+        release_record(c, ref);
         ph_mark(c, PH_POOL);
     }
     ph_mark(c, PH_IDLE);
@@ -3158,12 +3009,3 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void ex
 }
 
 }  // namespace qcdev
-
-template __global__ void qcdev::expand_persistent<64>(const ExpandArgs*);
-template __global__ void qcdev::expand_persistent<128>(const ExpandArgs*);
-template __global__ void qcdev::expand_persistent<256>(const ExpandArgs*);
-
-// explicit instantiations exported for the host driver
-template __global__ void qcdev::expand_local<64>(const ExpandArgs*);
-template __global__ void qcdev::expand_local<128>(const ExpandArgs*);
-template __global__ void qcdev::expand_local<256>(const ExpandArgs*);

@@ -21,31 +21,27 @@
 #include "qc_internal.h"
 
 namespace qcdev {
-template <int TL>
 __global__ void expand_persistent(const ExpandArgs*);
 
-// Queue state for a fresh run: the roots dealt over the top bucket's ns
-// rings (root i at position i / ns of shard i mod ns, published), every
-// other cell free for its first lap, the free lists empty, counters reset.
-// ctr = heads[nr], tails[nr], pool top, hungry|pending, overflow (nr =
-// nb ns rings), QSTRIDE words apart.  Root records sit at the start of the
+// Queue state for a fresh run: the roots dealt over the nr rings (root i
+// at position i / nr of ring i mod nr, published), every other cell free for
+// its first lap, the free lists empty, counters reset.  ctr = heads[nr],
+// tails[nr], pool top, hungry|pending, overflow, QSTRIDE words apart.  Root records sit at the start of the
 // pool; allocated blocks start at the next unit boundary.
 __global__ void persist_reset(const TaskRef* __restrict__ roots, uint32_t nroots, const Vrec* __restrict__ root_verts,
-                              uint64_t root_slots, TaskRef* q_refs, unsigned long long* q_seq, uint64_t q_cap, int nb,
-                              int ns, Vrec* pool, unsigned long long* ctr, unsigned long long* fl_head,
+                              uint64_t root_slots, TaskRef* q_refs, unsigned long long* q_seq, uint64_t q_cap,
+                              uint32_t nr, Vrec* pool, unsigned long long* ctr, unsigned long long* fl_head,
                               uint32_t n_waves, StreamCtr* clq_ctr,
                               DevStats* stats, DevStats* inst_stats, uint32_t n_inst, int* error,
                               const float* __restrict__ root_feat, float* trace_feat, long long* trace_parent,
                               unsigned int* trace_beyond) {
     const uint64_t tid = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x;
     const uint64_t nt = (uint64_t)gridDim.x * blockDim.x;
-    const uint64_t nr = (uint64_t)nb * ns;
-    const uint64_t top = (uint64_t)(nb - 1) * ns;  // first ring of the top bucket
     for (uint64_t i = tid; i < nr * q_cap; i += nt) {
         const uint64_t r = i / q_cap, pos = i % q_cap;
-        q_seq[i] = (r >= top && pos * ns + (r - top) < nroots) ? pos + 1 : pos;
+        q_seq[i] = pos * nr + r < nroots ? pos + 1 : pos;
     }
-    for (uint64_t i = tid; i < nroots; i += nt) q_refs[(top + i % ns) * q_cap + i / ns] = roots[i];
+    for (uint64_t i = tid; i < nroots; i += nt) q_refs[(i % nr) * q_cap + i / nr] = roots[i];
     if (trace_feat) {
         // (one ring: root i at position i)
         for (uint64_t i = tid; i < (uint64_t)nroots * 12; i += nt) trace_feat[i] = root_feat[i];
@@ -59,11 +55,11 @@ __global__ void persist_reset(const TaskRef* __restrict__ roots, uint32_t nroots
         for (uint64_t r = 0; r < nr; r++) {
             ctr[r * QSTRIDE] = 0;  // head
             // tail: the roots dealt to this ring
-            ctr[(nr + r) * QSTRIDE] = r >= top && r - top < nroots ? (nroots - (r - top) + ns - 1) / ns : 0;
+            ctr[(nr + r) * QSTRIDE] = r < nroots ? (nroots - r + nr - 1) / nr : 0;
         }
-        ctr[2 * nr * QSTRIDE] = (root_slots + POOL_UNIT - 1) / POOL_UNIT * POOL_UNIT;  // pool top
-        ctr[(2 * nr + 1) * QSTRIDE] = (uint64_t)n_waves << 32 | nroots;  // hungry: every wave, pending: the roots
-        ctr[(2 * nr + 2) * QSTRIDE] = 0;                      // overflow
+        ctr[2ull * nr * QSTRIDE] = (root_slots + POOL_UNIT - 1) / POOL_UNIT * POOL_UNIT;  // pool top
+        ctr[(2ull * nr + 1) * QSTRIDE] = (uint64_t)n_waves << 32 | nroots;  // hungry: every wave, pending: the roots
+        ctr[(2ull * nr + 2) * QSTRIDE] = 0;                      // overflow
         clq_ctr->items = 0;
         clq_ctr->slots = 0;
         *stats = DevStats{0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
@@ -76,16 +72,8 @@ namespace qc {
 
 namespace {
 
-// Per-wave HBM slab: the root-space workspace for tasks above the mid size
-// and, in the same bytes, the local-matrix workspace for tasks between the
-// LDS tile and the mid size (a wave runs one task at a time).
-size_t ws_bytes_host(uint32_t tcap, bool mat, uint32_t mwords) {
-    return (ws_bytes(tcap, mat, mwords) + 255) & ~(size_t)255;
-}
-
-constexpr int Q_SHARDS = 8;                 // rings per bucket in the dynamic order: one per XCD
-constexpr int NCTR = 2 * 4 * Q_SHARDS + 4;  // heads, tails (4 buckets x Q_SHARDS rings at most), pool top,
-                                            // hungry|pending, overflow, one spare
+constexpr int Q_SHARDS = 8;             // rings in the dynamic order: one per XCD
+constexpr int NCTR = 2 * Q_SHARDS + 4;  // heads, tails, pool top, hungry|pending, overflow, one spare
 
 struct RunState {
     unsigned long long ctr[NCTR];
@@ -120,10 +108,6 @@ int ensure(DBuf& b, size_t bytes) {
     return b.alloc(bytes);
 }
 
-// largest task that may use task-local matrices in the slab
-constexpr int MID_MAX = 4096;
-// largest pair of set masks kept in LDS (more would cost resident waves)
-constexpr size_t MASK_LDS_MAX = 4096;
 // LDS allocation granule of a workgroup on gfx950 (bytes), measured: single-
 // wave workgroups of 32000 B run 5 per 160 KB CU, of 32256 B 4; of 20480 B
 // 8, of 20736 B 7
@@ -152,9 +136,7 @@ int enumerate_persistent(const Instance* const* insts, const qc_params* params, 
         set_error("static scheduling deals ring positions to the waves in turn; cost order needs dynamic scheduling");
         return QC_EINVAL;
     }
-    const void* kern = TL == 64    ? (const void*)qcdev::expand_persistent<64>
-                       : TL == 128 ? (const void*)qcdev::expand_persistent<128>
-                                   : (const void*)qcdev::expand_persistent<256>;
+    const void* kern = (const void*)qcdev::expand_persistent;
 
     // roots and per-instance tables
     std::vector<TaskRef> roots;
@@ -199,23 +181,15 @@ int enumerate_persistent(const Instance* const* insts, const qc_params* params, 
     int dev = 0, n_cu = 0, per_cu = 0;
     QC_HIP(hipGetDevice(&dev));
     QC_HIP(hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, dev));
-    // wide tasks: per-vertex arrays in LDS up to this size (dynamic LDS)
-    const int wide_req = p.lds_wide < 0 ? 0 : (p.lds_wide > 0 ? (int)p.lds_wide : 512);
-    const uint32_t wide = wide_req > TL ? (uint32_t)std::min(std::min(wide_req, 1024), std::max(maxR, TL)) : 0u;
-    // the two set masks of tasks above the tile go to LDS after the wide
-    // arrays when they are small (rowpop reads the mask beside every row word)
-    const int mid_tile = std::min(p.mid_tile > 0 ? (int)p.mid_tile : 0, MID_MAX);
-    const uint32_t mid = (uint32_t)std::min(maxR, mid_tile);
-    const uint32_t midw = (mid + 63) / 64;
-    const size_t arr_b = wide ? ws_bytes(wide, false, 0) : (size_t)0;
-    const size_t mask_b = (size_t)2 * std::max<size_t>((size_t)maxrw, midw) * 8;
-    const bool mask_lds = mask_b <= MASK_LDS_MAX;
-    size_t lds_b = std::max(ws_bytes(TL, true, (TL + 63) / 64), arr_b + (mask_lds ? mask_b : 0));
     // (traces number every task by its ring position: no subtree runs unseen)
     const bool tiny = p.trace == 0;
-    // room for the children of any task of 64 vertices; the registers allow
-    // 8 waves per CU, and 8 x 16 KB fit its LDS
-    if (tiny) lds_b = std::max<size_t>(lds_b, (size_t)64 * 256);
+    // Dynamic LDS of a wave: the arrays of tasks of up to `wide` vertices (larger
+    // ones use the wave's HBM slab), and room for the children of any task
+    // of 64 vertices: the registers allow 8 waves per CU, and 8 x 16 KB fit its
+    // LDS.
+    const int wide_req = p.lds_wide < 0 ? 0 : (p.lds_wide > 0 ? (int)p.lds_wide : 512);
+    const uint32_t wide = (uint32_t)std::min(std::min(wide_req, 1024), maxR);
+    size_t lds_b = std::max<size_t>((size_t)64 * 256, wide_lds_bytes(wide, (uint32_t)maxrw));
     QC_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, 64, lds_b));
     {
         // A workgroup's LDS (static + dynamic) is allocated in granules of
@@ -233,11 +207,10 @@ int enumerate_persistent(const Instance* const* insts, const qc_params* params, 
         const size_t st = fa.sharedSizeBytes;
         auto alloc = [&](size_t dyn) { return (dyn + st + LDS_GRANULE - 1) / LDS_GRANULE * LDS_GRANULE; };
         per_cu = std::min(per_cu, (int)((size_t)lds_cu / alloc(lds_b)));
-        if (mask_lds && per_cu > 0) {
+        if (per_cu > 0) {
             // the resident waves leave part of the CU's LDS unused: the
             // dynamic region grows to the most that keeps per_cu waves
-            // resident, and tasks above the wide tier place arrays there
-            // (the masks sit at its end)
+            // resident, so larger tasks fit it
             size_t cand = (size_t)lds_cu / (size_t)per_cu / LDS_GRANULE * LDS_GRANULE;
             cand = std::min(cand, (size_t)lds_blk);
             cand = cand > st ? (cand - st) & ~(size_t)255 : 0;
@@ -250,9 +223,7 @@ int enumerate_persistent(const Instance* const* insts, const qc_params* params, 
     uint32_t grid = (uint32_t)std::max(1, n_cu) * (uint32_t)std::max(1, std::min(per_cu, 16));
     if (p.workgroups > 0) grid = std::min<uint32_t>(grid, (uint32_t)p.workgroups);
 
-    const bool use_mid = (int)mid > TL;
-    const size_t slab_b = std::max(ws_bytes_host((uint32_t)maxR, false, (uint32_t)maxrw),
-                                   use_mid ? ws_bytes_host(mid, true, midw) : (size_t)0);
+    const size_t slab_b = wide_slab_bytes((uint32_t)maxR);
     size_t freeb = 0, totalb = 0;
     QC_HIP(hipMemGetInfo(&freeb, &totalb));
     freeb += pool_cached_bytes(dev);
@@ -273,18 +244,17 @@ int enumerate_persistent(const Instance* const* insts, const qc_params* params, 
     // launch when a run overflows, unless the caller fixed them
     const bool fixed_tasks = p.task_capacity != 0, fixed_clq = p.clique_capacity != 0;
     const uint64_t max_pool = std::min<uint64_t>(budget / 2, (size_t)32 << 30) / sizeof(Vrec);
-    // the dynamic order spreads each bucket over Q_SHARDS rings (a wave pushes
-    // to its XCD's ring and takes from it first); static order deals the
-    // positions of one ring, and a trace numbers the tasks by position in one
+    // the dynamic order has Q_SHARDS rings (a wave pushes to its XCD's ring
+    // and takes from it first); static order deals the positions of one ring,
+    // and a trace numbers the tasks by position in one
     const bool trace = p.trace != 0;
-    const int ns = stat || trace ? 1 : Q_SHARDS;
-    const int nr = nb * ns;
+    const int nr = stat || trace ? 1 : Q_SHARDS;
     const uint64_t max_q = (1ull << 28) / nr;
     const uint64_t max_clq = std::min<uint64_t>(budget / 16 / 4, (uint64_t)1 << 31);
     uint64_t pool_cap = fixed_tasks ? p.task_capacity
                                     : std::max<uint64_t>(ws.pool_cap, std::min<uint64_t>(max_pool, 1ull << 26));
     pool_cap = std::max<uint64_t>(pool_cap, root_verts.size() + 1024);
-    uint64_t q_cap = std::max<uint64_t>(ws.q_cap / nr, std::min<uint64_t>(max_q, (1ull << 22) / ns));
+    uint64_t q_cap = std::max<uint64_t>(ws.q_cap / nr, std::min<uint64_t>(max_q, (1ull << 22) / nr));
     q_cap = std::max<uint64_t>(q_cap, roots.size() + 1024);
     uint64_t clq_slots = fixed_clq ? p.clique_capacity
                                    : std::max<uint64_t>(ws.clq_slots, std::min<uint64_t>(max_clq, 1ull << 24));
@@ -387,10 +357,6 @@ int enumerate_persistent(const Instance* const* insts, const qc_params* params, 
         A.slab = ws.slab.as<char>();
         A.slab_bytes = slab_b;
         A.slab_tcap = (uint32_t)maxR;
-        A.slab_mwords = (uint32_t)maxrw;
-        A.mid_tcap = use_mid ? mid : 0;
-        A.lds_wide = wide;
-        A.lds_masks = mask_lds ? (int32_t)(lds_b - mask_b) : -1;
         A.stats = ws.stats.as<DevStats>();
         A.error = ws.err.as<int>();
         A.queue_mode = 1;
@@ -421,9 +387,10 @@ int enumerate_persistent(const Instance* const* insts, const qc_params* params, 
         A.pool_top = ctr + 2 * nr * QSTRIDE;
         A.pending = ctr + (2 * nr + 1) * QSTRIDE;
         A.overflow = ctr + (2 * nr + 2) * QSTRIDE;
+        A.lds_bytes = (uint32_t)lds_b;
         A.tiny_cap = tiny ? (uint32_t)std::min<size_t>(TINY_STACK_MAX, lds_b / 256) : 0u;
         A.n_buckets = nb;
-        A.q_shards = ns;
+        A.q_shards = nr;
         A.n_roots = (int32_t)roots.size();
         A.cm_w = cost ? d_cmw.as<uint16_t>() : nullptr;
         A.cm_norm = cost ? d_cmn.as<float>() : nullptr;
@@ -451,7 +418,7 @@ int enumerate_persistent(const Instance* const* insts, const qc_params* params, 
         QC_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
         hipLaunchKernelGGL(qcdev::persist_reset, dim3(1024), dim3(256), 0, s, d_roots.as<TaskRef>(), nroots,
                            d_root_verts.as<Vrec>(), (uint64_t)root_verts.size(), ws.q.as<TaskRef>(),
-                           ws.seq.as<unsigned long long>(), q_cap, nb, ns, ws.pool.as<Vrec>(), ctr,
+                           ws.seq.as<unsigned long long>(), q_cap, (uint32_t)nr, ws.pool.as<Vrec>(), ctr,
                            ws.fl.as<unsigned long long>(), grid,
                            ws.clq_ctr.as<StreamCtr>(), ws.stats.as<DevStats>(), d_istats.as<DevStats>(),
                            (uint32_t)count, ws.err.as<int>(), d_rfeat.as<float>(), A.trace_feat, A.trace_parent,

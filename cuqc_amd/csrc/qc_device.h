@@ -45,20 +45,15 @@ __host__ __device__ constexpr uint32_t pow2_at_least(uint32_t x) {
     return p;
 }
 
-// Bytes of a per-wave workspace for tasks of up to `tcap` vertices: 15
-// per-vertex int arrays of pow2(tcap) entries, then (`mat`) the task-local
-// 1-hop / 2-hop matrices (tcap rows of ceil(tcap/64) words), then two masks of
-// `mwords` words (ceil(tcap/64) with local matrices, rw in root space).
-__host__ __device__ __attribute__((always_inline)) constexpr size_t ws_bytes(uint32_t tcap, bool mat, uint32_t mwords) {
-    uint32_t T2 = pow2_at_least(tcap < 64 ? 64 : tcap);
-    uint32_t W = (tcap + 63) / 64;
-    size_t b = 0;
-    b += (size_t)11 * T2 * 4;        // parent + child arrays
-    b += (size_t)4 * T2 * 4;         // lists / keys
-    b = (b + 15) & ~(size_t)15;
-    if (mat) b += (size_t)2 * tcap * W * 8;
-    b += (size_t)2 * mwords * 8;
-    return b;
+// LDS bytes of a task of t vertices: its arrays (20 bytes a vertex), two bit
+// masks over its positions, and three rows of rw words when they are staged
+__host__ __device__ __attribute__((always_inline)) constexpr uint32_t wide_T(uint32_t t) { return (t + 63u) & ~63u; }
+__host__ __device__ __attribute__((always_inline)) constexpr uint32_t wide_lds_bytes(uint32_t t, uint32_t rw) {
+    return 20u * wide_T(t) + wide_T(t) / 4u + (rw <= 256u ? 24u * rw : 0u);
+}
+// HBM slab bytes of a task of t vertices (52 a vertex, and the masks)
+__host__ __device__ __attribute__((always_inline)) constexpr size_t wide_slab_bytes(uint32_t t) {
+    return ((size_t)52 * wide_T(t) + wide_T(t) / 4u + 255) & ~(size_t)255;
 }
 
 struct TaskRef {
@@ -164,31 +159,25 @@ struct ExpandArgs {
     unsigned long long clq_ref_cap;
     unsigned long long clq_vert_cap;
 
-    // per-wave HBM workspace for tasks above the LDS tile
+    // per-wave HBM workspace for tasks whose arrays do not fit the LDS
     char* slab;
     unsigned long long slab_bytes;   // per wave
     uint32_t slab_tcap;              // vertices per slab
-    uint32_t slab_mwords;            // mask words per slab (root-space row words)
-    uint32_t mid_tcap;               // persistent mode: tasks above the LDS tile and up to
-                                     // this size use task-local matrices in the slab (0: none)
-    uint32_t lds_wide;               // persistent mode: tasks above the LDS tile and up to
-                                     // this size keep their per-vertex arrays in LDS (0: none)
-    int32_t lds_masks;               // persistent mode: byte offset in the dynamic LDS of the
-                                     // two set masks of tasks above the LDS tile (-1: slab)
+    uint32_t lds_bytes;              // size of the dynamic LDS
 
-    // persistent mode: n_buckets x q_shards shared ring queues of task refs
-    // plus one private LIFO stack per wave, over a vertex pool with free
-    // lists.  Ring r = b q_shards + s (bucket b, shard s) owns cells
-    // [r q_cap, (r+1) q_cap) of q_refs / q_seq and the position counters
-    // q_head[r QSTRIDE], q_tail[r QSTRIDE] (every shared counter sits on a
-    // 256-byte line of its own).  A wave pushes to its own shard and takes
-    // from it first, then from the other shards of the same bucket.
-    // Position p of a ring uses cell p mod q_cap, whose sequence word reads
-    // p while the cell is free for p, p + 1 once the ref of p is published
-    // and p + q_cap once it has been taken.  `pending` counts the tasks
-    // waiting in the rings plus the waves holding work (0 = search
-    // complete).  With a cost model, a child's bucket is its predicted log
-    // subtree size; waves take the highest non-empty bucket first.
+    // persistent mode: q_shards shared ring queues of task refs plus one
+    // private LIFO stack per wave, over a vertex pool with free lists.  Ring r
+    // owns cells [r q_cap, (r+1) q_cap) of q_refs / q_seq and the position
+    // counters q_head[r QSTRIDE], q_tail[r QSTRIDE] (every shared counter sits
+    // on a 256-byte line of its own).  Position p of a ring uses cell p mod
+    // q_cap, whose sequence word reads p while the cell is free for p, p + 1
+    // once the ref of p is published and p + q_cap once it has been taken.
+    // Consumers take positions ahead of their publication (one add on the
+    // head, which may pass the tail by the waves that wait) and wait for the
+    // position's own word.  `pending` counts the tasks waiting in the rings
+    // plus the waves holding work (0 = search complete).  With a cost model, a
+    // child's bucket is its predicted log subtree size; hand-overs give the
+    // highest buckets first.
     int32_t queue_mode;
     int32_t split_chunk;             // branches per split item (0: no splitting)
     uint32_t split_min_t;            // split tasks above this size
@@ -213,7 +202,7 @@ struct ExpandArgs {
     unsigned long long* pending;
     unsigned long long* overflow;    // pushes that found the ring and the private stack full
     // private stacks: wave w owns priv[w priv_cap, (w+1) priv_cap) (refs)
-    // and priv_bkt[...] (the bucket each ref would take in the rings);
+    // and priv_bkt[...] (each ref's predicted bucket);
     // children stay there (depth first) unless use_priv is 0, and the
     // oldest ones are handed to the rings while they run low
     TaskRef* priv;
@@ -229,10 +218,10 @@ struct ExpandArgs {
     unsigned int* trace_beyond;  // per slot: children past the depth window
 
     uint32_t tiny_cap;               // persistent mode: tasks of 64 vertices that the dynamic LDS holds
-                                     // (tiny_run; 0: tasks of that size take the general path)
+                                     // (tiny_run; 0: such tasks take the general path)
     int32_t n_buckets;               // 1 = FIFO
     int32_t n_roots;                 // root tasks of the launch (root split width)
-    int32_t q_shards;                // rings per bucket (ring b q_shards + s; wave w uses shard w mod q_shards)
+    int32_t q_shards;                // rings (wave w uses ring w mod q_shards)
     const uint16_t* cm_w;            // cost model: bf16 weights (5057)
     const float* cm_norm;            // mu[12] sd[12] ymu ysd thresholds[3]
 
