@@ -157,12 +157,20 @@ class SetList(Sequence):
         self.verts = verts
 
     @classmethod
-    def from_view(cls, count: int, off, verts) -> "SetList":
+    def from_view(cls, count: int, off, verts, owner) -> "SetList":
+        """Arrays over the library's own memory, which `owner` keeps: no copy.
+        Every array and view made from them keeps it too."""
         if count == 0:
             return cls(np.zeros(1, np.uint64), np.zeros(0, np.uint32))
-        o = np.ctypeslib.as_array(off, shape=(count + 1,)).copy()
-        v = np.ctypeslib.as_array(verts, shape=(int(o[-1]),)).copy() if o[-1] else np.zeros(0, np.uint32)
-        return cls(o, v)
+
+        def view(pointer, ctype, n, dtype):
+            buf = (ctype * n).from_address(C.addressof(pointer.contents))
+            buf._owner = owner
+            return np.frombuffer(buf, dtype=dtype)
+
+        o = view(off, C.c_uint64, count + 1, np.uint64)
+        nv = int(o[-1])
+        return cls(o, view(verts, C.c_uint32, nv, np.uint32) if nv else np.zeros(0, np.uint32))
 
     def __len__(self) -> int:
         return len(self.offsets) - 1
@@ -335,14 +343,28 @@ def write_sets(sets: Sequence[Sequence[int]], path) -> None:
             f.write(f"{len(s)} " + "".join(f"{int(x)} " for x in s) + "\n")
 
 
+class _ResultHandle:
+    """Frees a qc_result when the last array over its memory is gone."""
+
+    def __init__(self, h: C.c_void_p):
+        self._h = h
+
+    def __del__(self):
+        try:
+            load_library().qc_result_free(self._h)
+        except Exception:
+            pass
+
+
 def _result_from(h: C.c_void_p, rc: int) -> Result:
     L = load_library()
+    owner = _ResultHandle(C.c_void_p(h.value))
     try:
         cnt, off, v = C.c_uint64(), C.POINTER(C.c_uint64)(), C.POINTER(C.c_uint32)()
         _check(L.qc_result_view(h, C.byref(cnt), C.byref(off), C.byref(v)))
         maximal = _sets_from(cnt.value, off, v)
         _check(L.qc_result_raw(h, C.byref(cnt), C.byref(off), C.byref(v)))
-        raw = SetList.from_view(cnt.value, off, v)
+        raw = SetList.from_view(cnt.value, off, v, owner)
         st = _Stats()
         _check(L.qc_result_stats(h, C.byref(st)))
         stats = {n: int(getattr(st, n)) for n in _STAT_U64}
@@ -359,7 +381,7 @@ def _result_from(h: C.c_void_p, rc: int) -> Result:
             tsub = np.ctypeslib.as_array(sp, shape=(n,)).copy()
         return Result(maximal, raw, stats, rc, tf, tpar, tsub)
     finally:
-        L.qc_result_free(h)
+        del owner  # (the raw arrays may still hold it)
 
 
 def _params(gamma, min_size, scheduling, mode, order, lds_tile, workgroups, task_capacity, clique_capacity,

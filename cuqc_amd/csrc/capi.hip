@@ -4,6 +4,7 @@
 #include <chrono>
 #include <cmath>
 #include <cstdio>
+#include <cstdlib>
 #include <cstring>
 #include <map>
 #include <memory>
@@ -82,6 +83,103 @@ size_t pool_cached_bytes(int dev) {
     for (auto& kv : bc.free)
         if (kv.first.first == dev) b += kv.first.second * kv.second.size();
     return b;
+}
+
+// ---- host result blocks (see HostBuf) ----
+namespace {
+struct HostPool {
+    std::mutex mu;
+    std::vector<std::pair<size_t, void*>> free;  // pinned blocks, oldest first
+    size_t free_bytes = 0, pinned_bytes = 0;     // waiting, and pinned in all
+    // the oldest waiting blocks go back to HIP until at most `keep` bytes wait
+    void trim_locked(size_t keep) {
+        size_t n = 0;
+        for (; free_bytes > keep; n++) {
+            free_bytes -= free[n].first;
+            pinned_bytes -= free[n].first;
+            (void)hipHostFree(free[n].second);
+        }
+        free.erase(free.begin(), free.begin() + (std::ptrdiff_t)n);
+    }
+};
+HostPool& host_pool() {
+    static HostPool* h = new HostPool;  // lives until the process ends
+    return *h;
+}
+}  // namespace
+
+int HostBuf::alloc(size_t bytes) {
+    release();
+    if (bytes >= HOST_PINNED_MIN) {
+        // whole eighths of an octave: a result of nearly the same size reuses the block
+        size_t step = HOST_PINNED_MIN / 8;
+        while (step * 16 < bytes) step <<= 1;
+        const size_t want = (bytes + step - 1) / step * step;
+        HostPool& h = host_pool();
+        std::lock_guard<std::mutex> lock(h.mu);
+        size_t best = h.free.size();
+        for (size_t i = 0; i < h.free.size(); i++)
+            if (h.free[i].first >= want && h.free[i].first <= 4 * want &&
+                (best == h.free.size() || h.free[i].first < h.free[best].first))
+                best = i;
+        if (best < h.free.size()) {
+            cap = h.free[best].first;
+            p = h.free[best].second;
+            h.free_bytes -= cap;
+            h.free.erase(h.free.begin() + (std::ptrdiff_t)best);
+            pinned = true;
+            return QC_OK;
+        }
+        // a new block: waiting ones make room for it under the limit
+        if (h.pinned_bytes + want > HOST_PINNED_MAX) h.trim_locked(0);
+        if (h.pinned_bytes + want <= HOST_PINNED_MAX) {
+            void* q = nullptr;
+            if (hipHostMalloc(&q, want, hipHostMallocDefault) == hipSuccess && q) {
+                p = q;
+                cap = want;
+                pinned = true;
+                h.pinned_bytes += want;
+                return QC_OK;
+            }
+            (void)hipGetLastError();
+        }
+    }
+    p = malloc(bytes ? bytes : 1);
+    if (!p) {
+        // give the waiting blocks back and try once more
+        HostPool& h = host_pool();
+        {
+            std::lock_guard<std::mutex> lock(h.mu);
+            h.trim_locked(0);
+        }
+        p = malloc(bytes ? bytes : 1);
+    }
+    if (!p) {
+        set_error("host allocation of %zu bytes failed", bytes);
+        return QC_ENOMEM;
+    }
+    cap = bytes;
+    pinned = false;
+    return QC_OK;
+}
+
+void HostBuf::release() {
+    if (p && !pinned) ::free(p);
+    if (p && pinned) {
+        HostPool& h = host_pool();
+        std::lock_guard<std::mutex> lock(h.mu);
+        try {
+            h.free.push_back({cap, p});
+            h.free_bytes += cap;
+        } catch (...) {  // (no memory for the list: the block goes back to HIP)
+            h.pinned_bytes -= cap;
+            (void)hipHostFree(p);
+        }
+        h.trim_locked(HOST_POOL_MAX);
+    }
+    p = nullptr;
+    cap = 0;
+    pinned = false;
 }
 
 int load_serialized(const char* path, qc_graph* g);
@@ -201,8 +299,7 @@ int guarded(F&& f) {
 
 int finish_result(EnumOut& eo, const Instance& I, qc_result* r, double t0, double t_init, hipStream_t s) {
     int rc;
-    r->raw_off = std::move(eo.raw_off);
-    r->raw_v = std::move(eo.raw_v);
+    r->raw = std::move(eo.raw);
     r->trace_feat = std::move(eo.trace_feat);
     r->trace_parent = std::move(eo.trace_parent);
     r->trace_subtree = std::move(eo.trace_subtree);
@@ -230,7 +327,7 @@ int finish_result(EnumOut& eo, const Instance& I, qc_result* r, double t0, doubl
         r->st.t_nonmax_ms = eo.nonmax_ms;
     } else {
         const double tn = now_ms();
-        if ((rc = remove_nonmax_device(r->raw_off, r->raw_v, r->max_off, r->max_v, s, true))) return rc;
+        if ((rc = remove_nonmax_device(r->raw, r->max_off, r->max_v, s, true))) return rc;
         r->st.t_nonmax_ms = now_ms() - tn;
     }
     r->st.max_cliques = r->max_off.size() - 1;
@@ -451,9 +548,9 @@ int qc_result_view(const qc_result* r, uint64_t* count, const uint64_t** offsets
 
 int qc_result_raw(const qc_result* r, uint64_t* count, const uint64_t** offsets, const uint32_t** verts) {
     if (!r) return set_error("NULL result"), QC_EINVAL;
-    if (count) *count = r->raw_off.size() - 1;
-    if (offsets) *offsets = r->raw_off.data();
-    if (verts) *verts = r->raw_v.data();
+    if (count) *count = r->raw.count();
+    if (offsets) *offsets = r->raw.offp();
+    if (verts) *verts = r->raw.vp();
     return QC_OK;
 }
 
@@ -473,7 +570,7 @@ int qc_result_stats(const qc_result* r, qc_stats* s) {
     return QC_OK;
 }
 
-static int write_sets(const std::vector<uint64_t>& off, const std::vector<uint32_t>& v, const char* path) {
+static int write_sets(uint64_t count, const uint64_t* off, const uint32_t* v, const char* path) {
     FILE* f = fopen(path, "w");
     if (!f) {
         set_error("Error: cannot open file %s for write", path);
@@ -482,7 +579,7 @@ static int write_sets(const std::vector<uint64_t>& off, const std::vector<uint32
     std::vector<char> buf;
     buf.reserve(1 << 20);
     char tmp[16];
-    for (size_t i = 0; i + 1 < off.size(); i++) {
+    for (uint64_t i = 0; i < count; i++) {
         int l = snprintf(tmp, sizeof(tmp), "%d ", (int)(off[i + 1] - off[i]));
         buf.insert(buf.end(), tmp, tmp + l);
         for (uint64_t j = off[i]; j < off[i + 1]; j++) {
@@ -509,12 +606,12 @@ int qc_result_write(const qc_result* r, const char* path) {
         set_error("no quasi-cliques found; nothing written");
         return QC_EEMPTY;
     }
-    return write_sets(r->max_off, r->max_v, path);
+    return write_sets(r->max_off.size() - 1, r->max_off.data(), r->max_v.data(), path);
 }
 
 int qc_result_write_raw(const qc_result* r, const char* path) {
     if (!r || !path) return set_error("NULL argument"), QC_EINVAL;
-    return write_sets(r->raw_off, r->raw_v, path);
+    return write_sets(r->raw.count(), r->raw.offp(), r->raw.vp(), path);
 }
 
 void qc_result_free(qc_result* r) { delete r; }
@@ -537,10 +634,10 @@ int qc_remove_nonmax(uint64_t count, const uint64_t* offsets, const uint32_t* ve
         hipStream_t s;
         QC_HIP(hipStreamCreate(&s));
         std::unique_ptr<qc_result> r(new qc_result);
-        r->raw_off.assign(offsets, offsets + count + 1);
-        r->raw_v.assign(verts, verts + offsets[count]);
+        r->raw.off.assign(offsets, offsets + count + 1);
+        r->raw.v.assign(verts, verts + offsets[count]);
         double tn = now_ms();
-        int rc2 = remove_nonmax_device(r->raw_off, r->raw_v, r->max_off, r->max_v, s);
+        int rc2 = remove_nonmax_device(r->raw, r->max_off, r->max_v, s);
         r->st.t_nonmax_ms = now_ms() - tn;
         r->st.raw_cliques = count;
         r->st.max_cliques = r->max_off.size() - 1;

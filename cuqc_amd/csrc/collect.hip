@@ -68,9 +68,7 @@ namespace qc {
     } while (0)
 
 int collect_raw(const CliqueRef* d_refs, uint64_t taken, const uint32_t* d_verts, uint64_t k, uint64_t nv,
-                std::vector<uint64_t>& off, std::vector<uint32_t>& v, DBuf& sets, hipStream_t s) {
-    off.assign(1, 0);
-    v.clear();
+                RawSets& raw, DBuf& sets, hipStream_t s) {
     if (k == 0) return QC_OK;
     if (taken >= 0xFFFFFFFFull || nv >= (1ull << 40)) {
         set_error("raw set collection: %llu sets of %llu vertices exceed the key fields", (unsigned long long)k,
@@ -108,17 +106,17 @@ int collect_raw(const CliqueRef* d_refs, uint64_t taken, const uint32_t* d_verts
     hipLaunchKernelGGL(qcdev::rc_gather, dim3(nb), dim3(256), 0, s, sets.as<CliqueRef>(), oo.as<uint64_t>(), k, d_verts,
                        out.as<uint32_t>());
     QC_RC(hipGetLastError());
-    off.resize(k + 1);
-    QC_RC(hipMemcpyAsync(off.data(), oo.p, (k + 1) * 8, hipMemcpyDeviceToHost, s));
+    if ((rc = raw.off_buf.alloc((k + 1) * 8)) || (rc = raw.v_buf.alloc(std::max<uint64_t>(nv, 1) * 4))) return rc;
+    raw.k = k;
+    raw.nv = nv;
+    QC_RC(hipMemcpyAsync(raw.off_buf.p, oo.p, (k + 1) * 8, hipMemcpyDeviceToHost, s));
+    QC_RC(hipMemcpyAsync(raw.v_buf.p, out.p, nv * 4, hipMemcpyDeviceToHost, s));
     QC_RC(hipStreamSynchronize(s));
-    if (off[k] != nv) {
-        set_error("raw set collection: the sets hold %llu vertex slots, the stream %llu", (unsigned long long)off[k],
-                  (unsigned long long)nv);
+    if (raw.offp()[k] != nv) {
+        set_error("raw set collection: the sets hold %llu vertex slots, the stream %llu",
+                  (unsigned long long)raw.offp()[k], (unsigned long long)nv);
         return QC_EDEVICE;
     }
-    v.resize(nv);
-    QC_RC(hipMemcpyAsync(v.data(), out.p, nv * 4, hipMemcpyDeviceToHost, s));
-    QC_RC(hipStreamSynchronize(s));
     return QC_OK;
 }
 

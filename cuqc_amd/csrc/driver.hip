@@ -182,8 +182,8 @@ int enumerate_plain(const Instance& I, const qc_params& p, EnumOut& out, hipStre
         QC_HIP(hipMemcpyAsync(hverts.data(), d_clq_verts.p, cc.slots * 4, hipMemcpyDeviceToHost, s));
         QC_HIP(hipStreamSynchronize(s));
         for (auto& r : hrefs) {
-            out.raw_v.insert(out.raw_v.end(), hverts.begin() + r.off, hverts.begin() + r.off + r.len);
-            out.raw_off.push_back(out.raw_v.size());
+            out.raw.v.insert(out.raw.v.end(), hverts.begin() + r.off, hverts.begin() + r.off + r.len);
+            out.raw.off.push_back(out.raw.v.size());
         }
         QC_HIP(hipMemsetAsync(d_clq_ctr.p, 0, sizeof(StreamCtr), s));
         return QC_OK;

@@ -852,24 +852,26 @@ int remove_nonmax_sets(const NmInput& raw, int n_inst, std::vector<std::vector<u
     return QC_OK;
 }
 
-int remove_nonmax_device(const std::vector<uint64_t>& off, const std::vector<uint32_t>& v, std::vector<uint64_t>& mo,
-                         std::vector<uint32_t>& mv, hipStream_t s, bool distinct) {
+int remove_nonmax_device(const RawSets& raw, std::vector<uint64_t>& mo, std::vector<uint32_t>& mv, hipStream_t s,
+                         bool distinct) {
     int rc;
     mo.assign(1, 0);
     mv.clear();
-    const uint64_t k = off.size() - 1;
+    const uint64_t k = raw.count();
     if (k == 0) return QC_OK;
-    const uint64_t nv = v.size();
+    const uint64_t nv = raw.verts();
+    const uint64_t* off = raw.offp();
+    const uint32_t* v = raw.vp();
     uint32_t maxv = 0;
-    for (uint32_t x : v) maxv = std::max(maxv, x);
+    for (uint64_t i = 0; i < nv; i++) maxv = std::max(maxv, v[i]);
     if (maxv == 0xFFFFFFFFu) {
         set_error("vertex id 4294967295 is not supported");
         return QC_EINVAL;
     }
     DBuf d_off, d_v;
     if ((rc = d_off.alloc((k + 1) * 8, s)) || (rc = d_v.alloc(nv * 4, s))) return rc;
-    QC_HIP(hipMemcpyAsync(d_off.p, off.data(), (k + 1) * 8, hipMemcpyHostToDevice, s));
-    QC_HIP(hipMemcpyAsync(d_v.p, v.data(), nv * 4, hipMemcpyHostToDevice, s));
+    QC_HIP(hipMemcpyAsync(d_off.p, off, (k + 1) * 8, hipMemcpyHostToDevice, s));
+    QC_HIP(hipMemcpyAsync(d_v.p, v, nv * 4, hipMemcpyHostToDevice, s));
     NmInput in{};
     in.k = k;
     in.nv = nv;

@@ -576,25 +576,25 @@ int enumerate_persistent(const Instance* const* insts, const qc_params* params, 
     StreamCtr cc{raw_k, raw_nv};
     DBuf d_sets;  // the raw sets' refs, instances in order
     {
-        std::vector<uint64_t> go;
-        std::vector<uint32_t> gv;
+        RawSets g;
         const uint64_t taken = std::min<uint64_t>(last_items, clq_refs);
-        if ((rc = collect_raw(ws.clq_refs.as<CliqueRef>(), taken, ws.clq_verts.as<uint32_t>(), cc.items, cc.slots, go, gv,
+        if ((rc = collect_raw(ws.clq_refs.as<CliqueRef>(), taken, ws.clq_verts.as<uint32_t>(), cc.items, cc.slots, g,
                               d_sets, s)))
             return rc;
         if (count == 1) {
-            outs[0].raw_off = std::move(go);
-            outs[0].raw_v = std::move(gv);
+            outs[0].raw = std::move(g);
         } else {
             // instance i holds the next first_stats[i].raw_cliques sets
             uint64_t at = 0;
+            const uint64_t* go = g.offp();
+            const uint32_t* gv = g.vp();
             for (int i = 0; i < count; i++) {
                 const uint64_t n = first_stats[i].raw_cliques;
                 if (at + n > cc.items) break;
                 EnumOut& o = outs[i];
-                o.raw_off.resize(n + 1);
-                for (uint64_t j = 0; j <= n; j++) o.raw_off[j] = go[at + j] - go[at];
-                o.raw_v.assign(gv.begin() + go[at], gv.begin() + go[at + n]);
+                o.raw.off.resize(n + 1);
+                for (uint64_t j = 0; j <= n; j++) o.raw.off[j] = go[at + j] - go[at];
+                o.raw.v.assign(gv + go[at], gv + go[at + n]);
                 at += n;
             }
             if (at != cc.items) {

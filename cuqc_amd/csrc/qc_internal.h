@@ -11,13 +11,60 @@
 #include "qc_device.h"
 #include "qc_host.h"
 
+namespace qc {
+
+// Host memory that device results are copied into.  Blocks of a megabyte or
+// more are pinned (the copy runs at the link's rate, 57 GB/s against 18 into
+// pageable memory whose pages it also has to fault in) and go back to a pool
+// when their owner is freed: at most HOST_POOL_MAX bytes wait there, and at
+// most HOST_PINNED_MAX are pinned at a time, beyond which memory is pageable.
+constexpr size_t HOST_PINNED_MIN = (size_t)1 << 20;
+constexpr size_t HOST_PINNED_MAX = (size_t)4 << 30;
+constexpr size_t HOST_POOL_MAX = (size_t)1 << 30;
+struct HostBuf {
+    void* p = nullptr;
+    size_t cap = 0;
+    bool pinned = false;
+    HostBuf() = default;
+    HostBuf(const HostBuf&) = delete;
+    HostBuf& operator=(const HostBuf&) = delete;
+    HostBuf(HostBuf&& o) noexcept { swap(o); }
+    HostBuf& operator=(HostBuf&& o) noexcept {
+        swap(o);
+        return *this;
+    }
+    ~HostBuf() { release(); }
+    void swap(HostBuf& o) {
+        std::swap(p, o.p);
+        std::swap(cap, o.cap);
+        std::swap(pinned, o.pinned);
+    }
+    // contents undefined; QC_ENOMEM when there is no memory
+    int alloc(size_t bytes);
+    void release();
+};
+
+// Raw sets on the host: vectors, or (a persistent launch of one graph) the
+// blocks the device wrote them to.
+struct RawSets {
+    std::vector<uint64_t> off{0};
+    std::vector<uint32_t> v;
+    HostBuf off_buf, v_buf;  // in place of the vectors when off_buf.p is set
+    uint64_t k = 0, nv = 0;  // their sets and vertices
+    uint64_t count() const { return off_buf.p ? k : off.size() - 1; }
+    uint64_t verts() const { return off_buf.p ? nv : v.size(); }
+    const uint64_t* offp() const { return off_buf.p ? (const uint64_t*)off_buf.p : off.data(); }
+    const uint32_t* vp() const { return off_buf.p ? (const uint32_t*)v_buf.p : v.data(); }
+};
+
+}  // namespace qc
+
 struct qc_result {
     // maximal sets, lexicographic order, each ascending
     std::vector<uint64_t> max_off{0};
     std::vector<uint32_t> max_v;
     // raw sets as emitted
-    std::vector<uint64_t> raw_off{0};
-    std::vector<uint32_t> raw_v;
+    qc::RawSets raw;
     qc_stats st{};
     // task trace (qc_params.trace)
     std::vector<float> trace_feat;
@@ -179,8 +226,7 @@ inline void root_cut_counters(const RootCut& c, int32_t R, uint32_t small_max, D
 
 // plain / persistent enumeration (driver.hip, persist.hip)
 struct EnumOut {
-    std::vector<uint64_t> raw_off{0};
-    std::vector<uint32_t> raw_v;
+    RawSets raw;
     std::vector<float> trace_feat;
     std::vector<int64_t> trace_parent, trace_subtree;
     DevStats ds{};
@@ -234,13 +280,14 @@ int remove_nonmax_sets(const NmInput& in, int n_inst, std::vector<std::vector<ui
                        std::vector<std::vector<uint32_t>*> mv, hipStream_t s);
 // the raw sets of a persistent launch's clique stream (k sets of nv vertices
 // among `taken` refs) as one array, instances in order and each instance's sets
-// in vertex-slot order, on the host; their refs in that order stay in `sets`
-int collect_raw(const CliqueRef* d_refs, uint64_t taken, const uint32_t* d_verts, uint64_t k, uint64_t nv,
-                std::vector<uint64_t>& off, std::vector<uint32_t>& v, DBuf& sets, hipStream_t s);
+// in vertex-slot order, on the host (out's blocks); their refs in that order stay
+// in `sets`
+int collect_raw(const CliqueRef* d_refs, uint64_t taken, const uint32_t* d_verts, uint64_t k, uint64_t nv, RawSets& out,
+                DBuf& sets, hipStream_t s);
 // host raw sets (uploaded once); distinct: no set names a vertex twice (a
 // search's own raw sets), so the cover filter may be used: its masks test
 // subsets of vertices, while a caller's sets are compared as multisets
-int remove_nonmax_device(const std::vector<uint64_t>& off, const std::vector<uint32_t>& v, std::vector<uint64_t>& mo,
-                         std::vector<uint32_t>& mv, hipStream_t s, bool distinct = false);
+int remove_nonmax_device(const RawSets& raw, std::vector<uint64_t>& mo, std::vector<uint32_t>& mv, hipStream_t s,
+                         bool distinct = false);
 
 }  // namespace qc
