@@ -66,16 +66,19 @@ int enumerate_plain(const Instance& I, const qc_params& p, EnumOut& out, hipStre
         QC_HIP(hipGetDevice(&d));
         freeb += pool_cached_bytes(d);
     }
-    // Buffers start near what the root needs and grow on demand up to a
+    // Buffers start at 64 MB (what the block cache recycles), or near what the
+    // root needs, and grow on demand up to a
     // budget; task_capacity / clique_capacity pin them instead.
     const size_t budget = std::min<size_t>(freeb / 2, (size_t)96 << 30);
     const uint64_t max_slots = budget / 5 / sizeof(Vrec);
     uint64_t stg_slot_cap = p.task_capacity ? p.task_capacity
-                                            : std::min<uint64_t>(max_slots, std::max<uint64_t>(8ull << 20, 2 * root_bound));
+                                            : std::min<uint64_t>(max_slots, std::max<uint64_t>(4ull << 20, 2 * root_bound));
     uint64_t pool_cap = p.task_capacity ? p.task_capacity : stg_slot_cap;
     const bool grow = p.task_capacity == 0;
     uint64_t stage_refs = std::min<uint64_t>(stg_slot_cap / 2 + 4096, (uint64_t)128 << 20);
     uint64_t clq_slots = p.clique_capacity ? p.clique_capacity : (16ull << 20);
+    if (const char* ic = getenv("QCMINE_INITIAL_CAPACITY"))  // tests: launches made again
+        if (!p.clique_capacity && atoll(ic) > 0) clq_slots = std::min<uint64_t>(clq_slots, 8 * (uint64_t)atoll(ic));
     uint64_t clq_refs = std::min<uint64_t>(clq_slots / 4 + 4096, (uint64_t)64 << 20);
 
     Stack st[2];
@@ -88,20 +91,23 @@ int enumerate_plain(const Instance& I, const qc_params& p, EnumOut& out, hipStre
         if ((rc = stg_refs[k].alloc(stage_refs * sizeof(TaskRef)))) return rc;
         if ((rc = stg_verts[k].alloc(stg_slot_cap * sizeof(Vrec)))) return rc;
     }
-    DBuf d_ctr, d_clq_ctr, d_clq_refs, d_clq_verts, d_stats, d_err, d_task_ctr, d_args, d_in_refs;
-    if ((rc = d_ctr.alloc(2 * sizeof(StreamCtr)))) return rc;
-    if ((rc = d_clq_ctr.alloc(sizeof(StreamCtr)))) return rc;
+    DBuf d_clq_refs, d_clq_verts, d_stats, d_launch;
     if ((rc = d_clq_refs.alloc(clq_refs * sizeof(CliqueRef)))) return rc;
     if ((rc = d_clq_verts.alloc(clq_slots * 4))) return rc;
     if ((rc = d_stats.alloc(sizeof(DevStats)))) return rc;
-    if ((rc = d_err.alloc(sizeof(int)))) return rc;
-    if ((rc = d_task_ctr.alloc(sizeof(unsigned int)))) return rc;
-    if ((rc = d_args.alloc(sizeof(ExpandArgs)))) return rc;
     const uint32_t max_batch = 1u << 16;
-    if ((rc = d_in_refs.alloc((size_t)max_batch * sizeof(TaskRef)))) return rc;
-    QC_HIP(hipMemsetAsync(d_clq_ctr.p, 0, sizeof(StreamCtr), s));
+    // one launch's counters, arguments and task refs, sent with one copy
+    struct Launch {
+        LevelState st;
+        ExpandArgs a;
+    };
+    const size_t refs_at = (sizeof(Launch) + 63) & ~(size_t)63;
+    if ((rc = d_launch.alloc(refs_at + (size_t)max_batch * sizeof(TaskRef)))) return rc;
+    std::vector<char> launch(refs_at + (size_t)max_batch * sizeof(TaskRef));
+    Launch* const L = (Launch*)launch.data();
+    Launch* const dL = d_launch.as<Launch>();
+    LevelState done{};  // counters after the last launch
     QC_HIP(hipMemsetAsync(d_stats.p, 0, sizeof(DevStats), s));
-    QC_HIP(hipMemsetAsync(d_err.p, 0, sizeof(int), s));
 
     int dev = 0;
     QC_HIP(hipGetDevice(&dev));
@@ -139,25 +145,37 @@ int enumerate_plain(const Instance& I, const qc_params& p, EnumOut& out, hipStre
     memset(&A, 0, sizeof(A));
     A.g = I.dg;
     A.static_sched = p.scheduling != 0;
-    A.task_counter = d_task_ctr.as<unsigned int>();
+    A.task_counter = &dL->st.next_task;
     for (int k = 0; k < 2; k++) {
         A.out_refs[k] = stg_refs[k].as<TaskRef>();
         A.out_verts[k] = stg_verts[k].as<Vrec>();
         A.out_ref_cap[k] = stage_refs;
         A.out_vert_cap[k] = stg_slot_cap;
     }
-    A.out_ctr = d_ctr.as<StreamCtr>();
+    A.out_ctr = dL->st.out;
     A.small_max = TL;
     A.clq_refs = d_clq_refs.as<CliqueRef>();
     A.clq_verts = d_clq_verts.as<uint32_t>();
-    A.clq_ctr = d_clq_ctr.as<StreamCtr>();
+    A.clq_ctr = &dL->st.clq;
     A.clq_ref_cap = clq_refs;
     A.clq_vert_cap = clq_slots;
     A.slab = d_slab.as<char>();
     A.slab_bytes = slab_b;
     A.slab_tcap = (uint32_t)I.R;
     A.stats = d_stats.as<DevStats>();
-    A.error = d_err.as<int>();
+    A.error = &dL->st.error;
+    // Tasks above the small size are split into items of at most 64 branches,
+    // fewer when a launch has few of them (below): on one wave each, the six
+    // first-level tasks of a co-expression window kept 6 of 1,024 waves busy
+    // for most of its 87 ms (now 6).  Not under a caller's capacities, whose
+    // launches stay as they are without: a split record stays on the stack
+    // until its last item ran.
+    const bool fixed = !grow || p.clique_capacity != 0;
+    A.all_bounds = fixed;
+    const int split = fixed || p.split_chunk < 0 ? 0 : (p.split_chunk == 0 ? 64 : p.split_chunk);
+    A.split_min_t = (uint32_t)std::max<int>((int)TL, p.split_min);
+    A.n_roots = 1;
+    A.split_waves = n_slabs;
     A.g.root_b0 = cut.b0;
     A.g.root_b1 = cut.b1;
     A.g.root_cut = cut.cut;
@@ -170,10 +188,9 @@ int enumerate_plain(const Instance& I, const qc_params& p, EnumOut& out, hipStre
     std::vector<CliqueRef> hrefs;
     std::vector<uint32_t> hverts;
 
+    // brings the clique stream to the host (done.clq holds its counters)
     auto drain = [&](bool force) -> int {
-        StreamCtr cc;
-        QC_HIP(hipMemcpyAsync(&cc, d_clq_ctr.p, sizeof(cc), hipMemcpyDeviceToHost, s));
-        QC_HIP(hipStreamSynchronize(s));
+        const StreamCtr cc = done.clq;
         if (!force && cc.slots * 2 < clq_slots && cc.items * 2 < clq_refs) return QC_OK;
         if (cc.items == 0) return QC_OK;
         hrefs.resize(cc.items);
@@ -185,7 +202,7 @@ int enumerate_plain(const Instance& I, const qc_params& p, EnumOut& out, hipStre
             out.raw.v.insert(out.raw.v.end(), hverts.begin() + r.off, hverts.begin() + r.off + r.len);
             out.raw.off.push_back(out.raw.v.size());
         }
-        QC_HIP(hipMemsetAsync(d_clq_ctr.p, 0, sizeof(StreamCtr), s));
+        done.clq = StreamCtr{0, 0};
         return QC_OK;
     };
 
@@ -194,22 +211,30 @@ int enumerate_plain(const Instance& I, const qc_params& p, EnumOut& out, hipStre
     struct {
         uint64_t tasks = 0, buf = 0, buf_off = 0, clq = 0, clq_off = 0, child = 0, child_off = 0;
     } mx;
-    std::vector<TaskRef> batch, kids;
+    std::vector<TaskRef> batch, kids[2];
+    // a launch whose raw sets overflow the stream is made again with half the
+    // tasks (its counters and the stream put back), down to one task
+    uint32_t most = max_batch;
+    DBuf d_keep;
+    if ((rc = d_keep.alloc(sizeof(DevStats)))) return rc;
     while (!st[0].refs.empty() || !st[1].refs.empty()) {
         const int k = st[1].refs.empty() ? 0 : 1;
         Stack& S = st[k];
         // batch from the top: bounded count, children fit the staging buffers
-        const uint32_t bmax = k == 1 ? n_slabs : std::min<uint32_t>(max_batch, small_grid_max * 4);
-        uint64_t vol = 0;
+        const uint32_t bmax = std::min(most, k == 1 ? n_slabs : std::min<uint32_t>(max_batch, small_grid_max * 4));
+        uint64_t vol = 0, branches = 0;
         size_t take = 0;
         while (take < S.refs.size() && take < bmax) {
             const TaskRef& r = S.refs[S.refs.size() - 1 - take];
-            if (take > 0 && vol + r.bound > stg_slot_cap) break;
-            if (r.bound > stg_slot_cap) {
-                uint64_t want = std::max<uint64_t>(r.bound, 2 * stg_slot_cap);
-                if (!grow || r.bound > max_slots) {
+            // (a task to be split writes its record instead of children, and at
+            // most a ref per vertex: the staging holds half as many refs as slots)
+            const uint64_t need = split && k == 1 && r.b1 == 0 ? std::max<uint64_t>(r.bound, 2ull * r.t) : r.bound;
+            if (take > 0 && vol + need > stg_slot_cap) break;
+            if (need > stg_slot_cap) {
+                uint64_t want = std::max<uint64_t>(need, 2 * stg_slot_cap);
+                if (!grow || need > max_slots) {
                     set_error("task of %u vertices needs %llu child slots, staging holds %llu", r.t,
-                              (unsigned long long)r.bound, (unsigned long long)stg_slot_cap);
+                              (unsigned long long)need, (unsigned long long)stg_slot_cap);
                     return QC_EOVERFLOW;
                 }
                 stg_slot_cap = std::min(want, max_slots);
@@ -225,41 +250,54 @@ int enumerate_plain(const Instance& I, const qc_params& p, EnumOut& out, hipStre
                     A.out_vert_cap[j] = stg_slot_cap;
                 }
             }
-            vol += r.bound;
+            vol += need;
+            branches += r.b1 ? r.b1 - r.b0 : r.t;
             take++;
         }
         batch.assign(S.refs.end() - take, S.refs.end());
         S.refs.resize(S.refs.size() - take);
         const uint64_t base = batch.front().off;
-        QC_HIP(hipMemcpyAsync(d_in_refs.p, batch.data(), take * sizeof(TaskRef), hipMemcpyHostToDevice, s));
-        A.in_refs = d_in_refs.as<TaskRef>();
+        A.in_refs = (const TaskRef*)(d_launch.as<char>() + refs_at);
         A.in_verts = S.verts.as<Vrec>();
         A.n_in = (uint32_t)take;
         A.lds_bytes = (uint32_t)(k == 1 ? LARGE_LDS : SMALL_LDS);
         A.slab_bytes = k == 1 ? slab_b : small_slab_b;
-        QC_HIP(hipMemcpyAsync(d_args.p, &A, sizeof(A), hipMemcpyHostToDevice, s));
-        QC_HIP(hipMemsetAsync(d_ctr.p, 0, 2 * sizeof(StreamCtr), s));
-        QC_HIP(hipMemsetAsync(d_task_ctr.p, 0, sizeof(unsigned int), s));
+        // items: about one per wave over the launch's branches
+        A.split_chunk = split && k == 1 ? (int)std::max<uint64_t>(1, std::min<uint64_t>((uint64_t)split, branches / n_slabs)) : 0;
+        L->st = LevelState{{{0, 0}, {0, 0}}, done.clq, 0, 0};
+        L->a = A;
+        memcpy(launch.data() + refs_at, batch.data(), take * sizeof(TaskRef));
+        QC_HIP(hipMemcpyAsync(d_launch.p, launch.data(), refs_at + take * sizeof(TaskRef), hipMemcpyHostToDevice, s));
+        if (!fixed) QC_HIP(hipMemcpyAsync(d_keep.p, d_stats.p, sizeof(DevStats), hipMemcpyDeviceToDevice, s));
         QC_HIP(hipEventRecord(e0, s));
         const uint32_t grid = std::min<uint32_t>((uint32_t)take, k == 1 ? n_slabs : small_grid_max);
-        hipLaunchKernelGGL(qcdev::expand_level, dim3(grid), dim3(64), k == 1 ? LARGE_LDS : SMALL_LDS, s,
-                           d_args.as<ExpandArgs>());
+        hipLaunchKernelGGL(qcdev::expand_level, dim3(grid), dim3(64), k == 1 ? LARGE_LDS : SMALL_LDS, s, &dL->a);
         QC_HIP(hipGetLastError());
         QC_HIP(hipEventRecord(e1, s));
-        StreamCtr oc[2];
-        int err = 0;
-        QC_HIP(hipMemcpyAsync(oc, d_ctr.p, sizeof(oc), hipMemcpyDeviceToHost, s));
-        QC_HIP(hipMemcpyAsync(&err, d_err.p, sizeof(int), hipMemcpyDeviceToHost, s));
+        LevelState ls;
+        QC_HIP(hipMemcpyAsync(&ls, &dL->st, sizeof(ls), hipMemcpyDeviceToHost, s));
         QC_HIP(hipStreamSynchronize(s));
+        const StreamCtr* oc = ls.out;
         float ms = 0;
         QC_HIP(hipEventElapsedTime(&ms, e0, e1));
         kms += ms;
+        if (ls.error == 1 && !fixed && take > 1 &&
+            (ls.clq.slots > clq_slots || ls.clq.items > clq_refs)) {
+            QC_HIP(hipMemcpyAsync(d_stats.p, d_keep.p, sizeof(DevStats), hipMemcpyDeviceToDevice, s));
+            S.refs.insert(S.refs.end(), batch.begin(), batch.end());
+            most = (uint32_t)std::max<size_t>(1, take / 2);
+            if ((rc = drain(true))) return rc;
+            continue;
+        }
+        most = max_batch;
         out.levels++;
-        if (err) {
-            set_error("expansion buffers overflowed (error flags %d); raise task_capacity / clique_capacity", err);
+        if (ls.error) {
+            set_error("expansion buffers overflowed (error flags %d); raise task_capacity / clique_capacity", ls.error);
             return QC_EOVERFLOW;
         }
-        S.top = base;
+        done = ls;
+        // (a split record stays while items of it wait)
+        S.top = !S.refs.empty() && S.refs.back().b1 > 0 && S.refs.back().off == base ? base + batch.front().t : base;
         // push children: staging stream j -> stack j
         for (int j = 0; j < 2; j++) {
             if (oc[j].items == 0) continue;
@@ -278,13 +316,23 @@ int enumerate_plain(const Instance& I, const qc_params& p, EnumOut& out, hipStre
                           (unsigned long long)oc[j].slots, (unsigned long long)D.cap);
                 return QC_EOVERFLOW;
             }
-            kids.resize(oc[j].items);
-            QC_HIP(hipMemcpyAsync(kids.data(), stg_refs[j].p, oc[j].items * sizeof(TaskRef), hipMemcpyDeviceToHost, s));
+            kids[j].resize(oc[j].items);
+            QC_HIP(hipMemcpyAsync(kids[j].data(), stg_refs[j].p, oc[j].items * sizeof(TaskRef), hipMemcpyDeviceToHost, s));
             QC_HIP(hipMemcpyAsync(D.verts.as<Vrec>() + D.top, stg_verts[j].p, oc[j].slots * sizeof(Vrec),
                                   hipMemcpyDeviceToDevice, s));
-            QC_HIP(hipStreamSynchronize(s));
-            std::sort(kids.begin(), kids.end(), [](const TaskRef& x, const TaskRef& y) { return x.off < y.off; });
-            for (auto& r : kids) {
+        }
+        if (oc[0].items || oc[1].items) QC_HIP(hipStreamSynchronize(s));
+        uint64_t n_kids = 0, kid_slots = 0;  // children (items are parts of their task)
+        for (int j = 0; j < 2; j++) {
+            if (oc[j].items == 0) continue;
+            Stack& D = st[j];
+            // (items of one record stay together: their order among themselves is free)
+            std::sort(kids[j].begin(), kids[j].end(), [](const TaskRef& x, const TaskRef& y) { return x.off < y.off; });
+            for (auto& r : kids[j]) {
+                if (r.b1 == 0) {
+                    n_kids++;
+                    kid_slots += r.t;
+                }
                 r.off += D.top;
                 D.refs.push_back(r);
             }
@@ -294,24 +342,26 @@ int enumerate_plain(const Instance& I, const qc_params& p, EnumOut& out, hipStre
             // the reference's debug size report (main.cu:2635-2646): level,
             // tasks expanded (records, vertex slots), children written,
             // records waiting on the host stacks, raw cliques held
-            StreamCtr cc;
-            QC_HIP(hipMemcpyAsync(&cc, d_clq_ctr.p, sizeof(cc), hipMemcpyDeviceToHost, s));
-            QC_HIP(hipStreamSynchronize(s));
-            uint64_t bslots = 0;
-            for (const TaskRef& r : batch) bslots += r.t;
+            const StreamCtr cc = done.clq;
+            uint64_t bslots = 0, n_tasks = 0;
+            for (const TaskRef& r : batch)
+                if (r.b1 == 0) {
+                    n_tasks++;
+                    bslots += r.t;
+                }
             if (out.levels == 1) bslots += (uint64_t)cut.cut;  // the root as built
             const uint64_t wrefs = st[0].refs.size() + st[1].refs.size(), wslots = st[0].top + st[1].top;
             printf("L: %llu T1: %llu %llu T2: %llu %llu B: %llu %llu C: %llu %llu\n\n", (unsigned long long)out.levels,
-                   (unsigned long long)take, (unsigned long long)bslots,
-                   (unsigned long long)(oc[0].items + oc[1].items), (unsigned long long)(oc[0].slots + oc[1].slots),
+                   (unsigned long long)n_tasks, (unsigned long long)bslots, (unsigned long long)n_kids,
+                   (unsigned long long)kid_slots,
                    (unsigned long long)wrefs, (unsigned long long)wslots, cc.items, cc.slots);
             mx.tasks = std::max<uint64_t>(mx.tasks, bslots);
             mx.buf = std::max<uint64_t>(mx.buf, wslots);
             mx.buf_off = std::max<uint64_t>(mx.buf_off, wrefs);
             mx.clq = std::max<uint64_t>(mx.clq, cc.slots);
             mx.clq_off = std::max<uint64_t>(mx.clq_off, cc.items);
-            mx.child = std::max<uint64_t>(mx.child, oc[0].slots + oc[1].slots);
-            mx.child_off = std::max<uint64_t>(mx.child_off, oc[0].items + oc[1].items);
+            mx.child = std::max<uint64_t>(mx.child, kid_slots);
+            mx.child_off = std::max<uint64_t>(mx.child_off, n_kids);
         }
         if ((rc = drain(false))) return rc;
     }

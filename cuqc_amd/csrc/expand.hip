@@ -1227,7 +1227,8 @@ __device__ __attribute__((always_inline)) void tiny_level(Ctx& c, Tiny& y, uint3
         const int at = tiny_place(c, w, M, C);
         if (w & TW_PRESENT) a.out_verts[0][si + at] = Vrec{y.id, (w & TW_MEMBER) ? 1 : 0, tw_in(w), tw_ex(w)};
         // slot bound of this child's own children (see TaskRef)
-        const int bnd = wave_sum((C >> c.lane) & 1ull ? min(y.d2 + nm + 1, t) : 0);
+        const bool kids = a.all_bounds || !(c.g.max_depth >= 0 && (int)c.depth + 2 > c.g.max_depth);
+        const int bnd = wave_sum(kids && ((C >> c.lane) & 1ull) ? min(y.d2 + nm + 1, t) : 0);
         if (c.lane == 0) {
             TaskRef r;
             r.off = si;
@@ -1937,7 +1938,11 @@ __device__ __attribute__((always_inline)) void wide_child(Ctx& c, Wide<P>& z, in
     };
     for (int i = c.lane; i < m; i += WAVE) put(i, z.pid[z.cpos[i]], 1, z.cw[i]);
     unsigned long long bnd = 0;
-    auto bound_of = [&](uint32_t id) {  // slot bound of the child's own children (see TaskRef)
+    // slot bound of the child's own children (see TaskRef); past the depth
+    // window they are not written
+    const bool kids = c.a->all_bounds || !(c.g.max_depth >= 0 && (int)c.depth + 2 > c.g.max_depth);
+    auto bound_of = [&](uint32_t id) {
+        if (!kids) return 0ull;
         const unsigned long long x = (unsigned long long)z.d2r[id] + m + 1;
         return x < (unsigned long long)tc ? x : (unsigned long long)tc;
     };
@@ -2126,21 +2131,32 @@ __device__ __attribute__((always_inline)) void wide_split(Ctx& c, Wide<P>& z, co
     const int pre = bbeg;
     const int ts = t0 - pre;
     wide_bulk_remove(c, z, ts, pre);
-    // the record plus one Vrec after it whose id counts the items still
-    // to run (the last one frees the block)
-    unsigned long long slot = 0;
-    if (c.lane == 0) slot = pool_alloc(c, (uint32_t)ts + 1u);
+    // the record plus, in the pool, one Vrec after it whose id counts the items
+    // still to run (the last one frees the block); the level-synchronous form
+    // writes it to the stream of large tasks, every item a ref to it
+    const bool q = a.queue_mode != 0;
+    const int n_items = (hi - bbeg + ch - 1) / ch;
+    unsigned long long slot = 0, ri = 0;
+    if (c.lane == 0) {
+        if (q) {
+            slot = pool_alloc(c, (uint32_t)ts + 1u);
+        } else {
+            ri = atomicAdd(&a.out_ctr[1].items, (unsigned long long)n_items);
+            slot = atomicAdd(&a.out_ctr[1].slots, (unsigned long long)ts);
+        }
+    }
     slot = rdlane64(slot, 0);
-    if (slot == ~0ull) {
+    ri = rdlane64(ri, 0);
+    if (q ? slot == ~0ull : (ri + n_items > a.out_ref_cap[1] || slot + ts > a.out_vert_cap[1])) {
         if (c.lane == 0) atomicOr(a.error, 1);
         return;
     }
+    Vrec* dst = (q ? a.pool : a.out_verts[1]) + slot;
     for (int i = c.lane; i < ts; i += WAVE) {
         const typename P::word w = z.pw[i];
-        a.pool[slot + i] = Vrec{(int32_t)z.pid[i], (i < nm ? 1 : 0) | ((int32_t)z.pl2[i] << 4), P::in(w), P::ex(w)};
+        dst[i] = Vrec{(int32_t)z.pid[i], (i < nm ? 1 : 0) | ((int32_t)z.pl2[i] << 4), P::in(w), P::ex(w)};
     }
-    const int n_items = (hi - bbeg + ch - 1) / ch;
-    if (c.lane == 0) a.pool[slot + ts] = Vrec{n_items, 0, 0, 0};
+    if (q && c.lane == 0) dst[ts] = Vrec{n_items, 0, 0, 0};
     // item boundaries balance the work rather than the branch count:
     // branch b builds a child from about t0 - b vertices, so with
     // S(b) = sum of (t0 - x) over x in [bbeg, b), boundary j is the first
@@ -2173,6 +2189,17 @@ __device__ __attribute__((always_inline)) void wide_split(Ctx& c, Wide<P>& z, co
         r.b1 = (uint32_t)(boundary(j + 1) - pre);
         return r;
     };
+    if (!q) {
+        for (int j = c.lane; j < n_items; j += WAVE) {
+            TaskRef r = item_ref(j);
+            r.bound = 0;
+            if (c.keys)  // (the slots its children can take)
+                for (uint32_t b = r.b0; b < r.b1; b++)
+                    r.bound += (uint64_t)min((long long)z.d2r[z.pid[ts - 1 - (int)b]] + nm + 1, (long long)ts);
+            a.out_refs[1][ri + j] = r;
+        }
+        return;
+    }
     // the items go to the rings in chunks of up to 64 claimed at once
     // (lanes write the refs, one release fence per chunk), as many as wait at a
     // ring, the rest to this wave's own; what the rings cannot take stays on
@@ -2380,9 +2407,9 @@ __device__ __attribute__((always_inline)) bool process_wide(Ctx& c, const TaskRe
         // a root's branches are split finer, to about one item per resident
         // wave over all roots: until the roots' items produce children nothing
         // else can run
-        int ch = a.queue_mode ? a.split_chunk : 0;
+        int ch = a.split_chunk;
         if (root && ch > 0 && a.n_roots > 0) {
-            const long long want = ((long long)(bend - bbeg) * a.n_roots + gridDim.x - 1) / gridDim.x;
+            const long long want = ((long long)(bend - bbeg) * a.n_roots + a.split_waves - 1) / a.split_waves;
             ch = (int)max(1ll, min((long long)ch, want));
         }
         if (ch > 0 && (uint32_t)t0 > a.split_min_t && bend - bbeg > ch) {

@@ -392,6 +392,7 @@ int enumerate_persistent(const Instance* const* insts, const qc_params* params, 
         A.n_buckets = nb;
         A.q_shards = nr;
         A.n_roots = (int32_t)roots.size();
+        A.split_waves = grid;
         A.cm_w = cost ? d_cmw.as<uint16_t>() : nullptr;
         A.cm_norm = cost ? d_cmn.as<float>() : nullptr;
         A.q_cap = q_cap;

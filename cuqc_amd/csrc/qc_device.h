@@ -97,6 +97,15 @@ struct StreamCtr {
     unsigned long long slots;   // vertex slots
 };
 
+// Counters of one level-synchronous launch, set and read with one copy each
+// way: children per stream, the clique stream, the next task, error flags.
+struct LevelState {
+    StreamCtr out[2];
+    StreamCtr clq;
+    unsigned int next_task;
+    int error;
+};
+
 // Per-call statistics accumulated by the kernels.
 struct DevStats {
     unsigned long long tasks, branches, children, raw_cliques, sum_t, sum_t_written, sum_clique_len, large_tasks,
@@ -180,6 +189,8 @@ struct ExpandArgs {
     // highest buckets first.
     int32_t queue_mode;
     int32_t split_chunk;             // branches per split item (0: no splitting)
+    int32_t all_bounds;              // level form: slot bounds also for children that the depth window leaves unwritten
+    uint32_t split_waves;            // waves a root's items are meant for (with n_roots)
     uint32_t split_min_t;            // split tasks above this size
     uint32_t cost_min_t;             // cost order: children of at most this size skip the model (bucket 0)
     TaskRef* q_refs;

@@ -73,3 +73,37 @@ def test_forms(refs, name, form):
         assert res.stats[k] == ref["stats"][k], k
     assert oracle.canon(res.raw) == oracle.canon(ref["raw"])
     assert res.maximal_sorted_tuples() == oracle.nonmax(ref["raw"])
+
+
+# the level-synchronous form: tasks split into items across launches, against
+# the unsplit form and with a caller's capacities (where nothing is split)
+PLAIN = {
+    "items_of_1": dict(split_chunk=1, split_min=1, lds_tile=64),
+    "items_of_5": dict(split_chunk=5, lds_tile=64),
+    "unsplit": dict(split_chunk=-1),
+    "static": dict(scheduling=1),
+    "capacities": dict(task_capacity=1 << 23, clique_capacity=1 << 22),
+}
+
+
+@pytest.mark.parametrize("name", ["er190", "er200_g05", "er960", "l2_13bit"])
+@pytest.mark.parametrize("form", list(PLAIN))
+def test_plain_splits(refs, name, form):
+    g, gamma, ms, win, ref = refs[name]
+    print(f"[gpu] plain {name} {form}", flush=True)
+    res = qc.mine(g, gamma, ms, window=win, mode="plain", **PLAIN[form])
+    for k in COUNTERS:
+        assert res.stats[k] == ref["stats"][k], k
+    assert oracle.canon(res.raw) == oracle.canon(ref["raw"])
+
+
+def test_plain_clique_stream_overflows(refs, monkeypatch):
+    """A launch whose raw sets do not fit the stream is made again with half the
+    tasks: 65,536 vertices hold what two tasks of this graph emit, not a launch's."""
+    g, gamma, ms, win, ref = refs["er190"]
+    assert ref["stats"]["sum_clique_len"] > 3 * 65536
+    monkeypatch.setenv("QCMINE_INITIAL_CAPACITY", "8192")
+    res = qc.mine(g, gamma, ms, window=win, mode="plain")
+    for k in COUNTERS:
+        assert res.stats[k] == ref["stats"][k], k
+    assert oracle.canon(res.raw) == oracle.canon(ref["raw"])
