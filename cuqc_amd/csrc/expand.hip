@@ -581,6 +581,9 @@ __device__ __forceinline__ void ring_publish(Ctx& c, int b, unsigned long long p
 // is loaded at one check and read at the next, so its latency overlaps the
 // children built in between; a count one interval old only delays the answer.
 constexpr int SHARE_EVERY = 8;
+// fewest branches of an item when waves wait (an item loads its task's record,
+// which takes as long as one to three branches)
+constexpr int SPLIT_FINE = 4;
 constexpr uint32_t SHARE_MIN_T = 64;
 __device__ __forceinline__ bool share_child(Ctx& c) {
     const ExpandArgs& a = *c.a;
@@ -1326,7 +1329,7 @@ template <class P>
 struct Wide {
     uint64_t* row1;         // LDS: rows of the branch vertex (rl)
     uint64_t* row2;
-    uint64_t* lmask;        // LDS: a set of vertices in root space (rl)
+    uint64_t* lmask;        // LDS: a set of vertices in root space (ml)
     uint64_t* nbits;        // N of the branch vertex by parent position (LDS; in the slab when too large)
     uint64_t* flag;         // a bit per candidate (as nbits)
     typename P::u32p pid;   // parent: root-local id
@@ -1347,6 +1350,7 @@ struct Wide {
     int mdt;           // mindeg[lane]
     int mds;           // mindeg[min_size]
     bool rl;           // rows are staged in LDS
+    bool ml;           // lmask has room for a row
     int tb, ub1;       // cand_valid's lane-independent bounds, from the last wide_bounds
 };
 
@@ -1597,7 +1601,7 @@ __device__ __forceinline__ int wide_rowpop(gptr<const uint64_t> X, int rw, const
 // row, 64 rows at once, instead of the same words of one row).
 template <class P, class At>
 __device__ __attribute__((always_inline)) bool wide_set(Ctx& c, Wide<P>& z, int nl, At at) {
-    const bool mask = z.rl && nl > 2 * z.rw;
+    const bool mask = z.ml && nl > 2 * z.rw;
     if (mask) {
         for (int w = c.lane; w < z.rw; w += WAVE) z.lmask[w] = 0;
         lsync();
@@ -1874,6 +1878,88 @@ __device__ __forceinline__ void wide_sort(Ctx& c, int n, F swap_if) {
     }
 }
 
+// Descending radix sort of n 64-bit keys of `bits` bits in the slab: 8 bits a
+// pass, counters of a digit in LDS (256 words), the lanes of a chunk that share
+// a digit found by ballots.  Returns the array that holds the result.  For the
+// slab's children (thousands of candidates) the bitonic sort's 78 and more
+// passes over memory were most of the child: 2 ms for 3,000 candidates and 8
+// for 13,900, against 0.1 and 0.6.
+__device__ __attribute__((noinline)) gptr<uint64_t> wide_radix(gptr<uint64_t> src, gptr<uint64_t> dst, int n, int bits,
+                                                               uint32_t* cnt) {
+    constexpr int U = 4;
+    const int lane = lane_id();
+    for (int s = 0; s < bits; s += 8) {
+        for (int k = lane; k < 256; k += WAVE) cnt[k] = 0;
+        lsync();
+        for (int base = 0; base < n; base += U * WAVE) {
+            uint64_t key[U];
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const int i = base + u * WAVE + lane;
+                key[u] = i < n ? src[i] : 0;
+            }
+#pragma unroll
+            for (int u = 0; u < U; u++)
+                if (base + u * WAVE + lane < n) atomicAdd(&cnt[255 - (int)((key[u] >> s) & 255)], 1u);
+        }
+        lsync();
+        {
+            uint32_t v[4], t = 0;
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                v[k] = cnt[4 * lane + k];
+                t += v[k];
+            }
+            uint32_t before = t;
+            for (int d = 1; d < WAVE; d <<= 1) {
+                const uint32_t o = __shfl_up(before, d, WAVE);
+                if (lane >= d) before += o;
+            }
+            before -= t;
+            lsync();
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                cnt[4 * lane + k] = before;
+                before += v[k];
+            }
+        }
+        lsync();
+        for (int base = 0; base < n; base += U * WAVE) {
+            uint64_t key[U];
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const int i = base + u * WAVE + lane;
+                key[u] = i < n ? src[i] : 0;
+            }
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                if (base + u * WAVE >= n) break;
+                const bool in = base + u * WAVE + lane < n;
+                const int d = 255 - (int)((key[u] >> s) & 255);
+                uint64_t same = ballot(in);
+#pragma unroll
+                for (int b = 0; b < 8; b++) {
+                    const bool bit = (d >> b) & 1;
+                    const uint64_t bb = ballot(bit);
+                    same &= bit ? bb : ~bb;
+                }
+                const int rank = lanes_below(same);
+                uint32_t at = 0;
+                if (in) at = cnt[d] + (uint32_t)rank;
+                lsync();
+                if (in && rank == 0) cnt[d] = at + (uint32_t)__popcll(same);
+                lsync();
+                if (in) dst[at] = key[u];
+            }
+        }
+        lsync();
+        const gptr<uint64_t> t = src;
+        src = dst;
+        dst = t;
+    }
+    return src;
+}
+
 // The child's record: members, then the candidates in Q order
 // (main.cu:2059-2104: indeg, exdeg, lvl2adj, id, all descending).
 template <class P>
@@ -1986,7 +2072,45 @@ __device__ __attribute__((always_inline)) void wide_child(Ctx& c, Wide<P>& z, in
             put(m + i, (uint32_t)key & ((1u << z.idb) - 1u), 0, (uint32_t)(key >> 32));
         }
     } else {
-        // 128-bit keys (word, lvl2adj and id), in LDS when they fit there
+        // Many candidates: indeg and exdeg above their smallest values, lvl2adj
+        // and id in 64 bits.  Few, or values that need more bits: 128-bit keys
+        // (word, lvl2adj and id), in LDS when they fit there.  (Up to two chunks
+        // the bitonic sort has 28 passes in LDS, the radix sort 5 of several
+        // trips to the slab.)
+        const int rb = 32 - __builtin_clz((uint32_t)c.g.p->R);
+        int in0 = 0, ex0 = 0, eb = 0, bits = 64;
+        if (n > 2 * WAVE && z.spare_bytes >= 1024u) {
+            int il = INT32_MAX, ih = 0, el = INT32_MAX, eh = INT32_MIN;
+            for (int i = c.lane; i < n; i += WAVE) {
+                const typename P::word w = z.cw[m + i];
+                il = min(il, P::in(w));
+                ih = max(ih, P::in(w));
+                el = min(el, P::ex(w));
+                eh = max(eh, P::ex(w));
+            }
+            in0 = wave_min(il);
+            ex0 = wave_min(el);
+            const uint32_t ir = (uint32_t)(wave_max(ih) - in0), er = (uint32_t)(wave_max(eh) - ex0);
+            eb = er ? 32 - __builtin_clz(er) : 0;
+            bits = (ir ? 32 - __builtin_clz(ir) : 0) + eb + 2 * rb;
+        }
+        if (bits < 64) {
+            for (int i = c.lane; i < n; i += WAVE) {
+                const uint32_t p = z.cpos[m + i], id = z.pid[p];
+                const typename P::word w = z.cw[m + i];
+                z.keys[i] = ((uint64_t)(uint32_t)(P::in(w) - in0) << (eb + 2 * rb)) |
+                            ((uint64_t)(uint32_t)(P::ex(w) - ex0) << (2 * rb)) | ((uint64_t)z.pl2[p] << rb) | id;
+                if (!q) bnd += bound_of(id);
+            }
+            lsync();
+            const gptr<uint64_t> k = wide_radix(z.keys, z.keys + (size_t)z.T, n, bits, (uint32_t*)z.spare);
+            for (int i = c.lane; i < n; i += WAVE) {
+                const uint64_t key = k[i];
+                const int ex = (int)((key >> (2 * rb)) & ((1ull << eb) - 1ull));
+                put(m + i, (uint32_t)(key & ((1ull << rb) - 1ull)), 0,
+                    P::make((int)(key >> (eb + 2 * rb)) + in0, ex + ex0));
+            }
+        }
         auto run = [&](auto khi, auto klo) {
             for (int i = c.lane; i < n; i += WAVE) {
                 const uint32_t p = z.cpos[m + i], id = z.pid[p];
@@ -2006,7 +2130,9 @@ __device__ __attribute__((always_inline)) void wide_child(Ctx& c, Wide<P>& z, in
             });
             for (int i = c.lane; i < n; i += WAVE) put(m + i, (uint32_t)klo[i], 0, khi[i]);
         };
-        if (16u * (uint32_t)n <= z.spare_bytes)
+        if (bits < 64)
+            ;
+        else if (16u * (uint32_t)n <= z.spare_bytes)
             run((uint64_t*)z.spare, (uint64_t*)z.spare + n);
         else
             run(z.keys, z.keys + (size_t)z.T);
@@ -2285,6 +2411,10 @@ __device__ __attribute__((always_inline)) bool process_wide(Ctx& c, const TaskRe
         }
         z.spare = at;
         z.spare_bytes = lds_bytes - (uint32_t)(at - lds);
+        // rows too long to be staged can still have the mask (a batch's root of
+        // 17,193 vertices took 7.3 ms to apply its window's removals row by row)
+        z.ml = z.rl || 8u * (uint32_t)z.rw <= z.spare_bytes;
+        if (!z.rl) z.lmask = (uint64_t*)z.spare;
     }
     // ---- record ----
     bool bad = false;
@@ -2411,6 +2541,20 @@ __device__ __attribute__((always_inline)) bool process_wide(Ctx& c, const TaskRe
         if (root && ch > 0 && a.n_roots > 0) {
             const long long want = ((long long)(bend - bbeg) * a.n_roots + a.split_waves - 1) / a.split_waves;
             ch = (int)max(1ll, min((long long)ch, want));
+        } else if (ch > SPLIT_FINE && a.queue_mode && !a.static_sched) {
+            // other tasks too when more waves wait than the rings hold tasks
+            // for: a first-level task of 13,900 vertices whose 162-branch items
+            // made 162 large children each kept the other waves waiting (its
+            // window 365 -> 190 ms with the sort of the slab's children, a
+            // co-expression window 76 -> 57).  Not in the static order, which
+            // deals items to waves in turn, waiting or not (9 -> 19 ms).
+            unsigned long long ph = 0;
+            if (c.lane == 0) ph = __hip_atomic_load(a.pending, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            ph = rdlane64(ph, 0);
+            const long long hg = (long long)(ph >> 32), pd = (long long)(ph & 0xFFFFFFFFull);
+            const long long waiting = pd - ((long long)gridDim.x - hg);
+            const long long need = hg - (waiting > 0 ? waiting : 0);
+            if (need > 0) ch = (int)max((long long)SPLIT_FINE, min((long long)ch, (long long)(bend - bbeg) / need));
         }
         if (ch > 0 && (uint32_t)t0 > a.split_min_t && bend - bbeg > ch) {
             wide_split(c, z, ref, nm, bbeg, bend, ch);
