@@ -120,8 +120,6 @@ struct DevGraph {
     int32_t rw;           // words per root-space row
     const uint64_t* A1;   // R x rw
     const uint64_t* A2;   // R x rw
-    const int32_t* mindeg;
-    int32_t mindeg_n;
     const int32_t* ubq;
     int32_t ubq_n;
     int32_t min_size;

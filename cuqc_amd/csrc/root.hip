@@ -1,10 +1,11 @@
 // root.hip -- root task construction (initialize_tasks, main.cu:846-998) and
 // the device tables the expansion kernels read.
 //
-// Host part: the degree / |N2| filter (main.cu:872-885), the k-core peel
-// (main.cu:889-949), the cover vertex and covered set (main.cu:953-975) and
-// the Q-ordered root record (main.cu:978-995).
-// Device part: for every root vertex, its rows of the root-space 1-hop and
+// The degree / |N2| filter (main.cu:872-885) and the k-core peel (main.cu:889-949)
+// run on the device for large graphs, else on the host, as do the cover vertex
+// and covered set (main.cu:953-975) and the Q-ordered root record
+// (main.cu:978-995).
+// Device tables: for every root vertex, its rows of the root-space 1-hop and
 // 2-hop bit matrices and its full-graph |N2| (the third Q-order key), with
 // the 2-hop relation of adjToSer.cpp:115-156: N(v) u N(N(v)) minus v.
 //
@@ -92,15 +93,25 @@ __global__ __launch_bounds__(64) void root_rows(const uint64_t* __restrict__ off
     }
 }
 
-// The same rows and counts with the visited bitmap and both rows in LDS
-// (dynamic: ceil(n/64) + 2 rw words), for graphs whose bitmap fits.  Rows are
-// written whole, so A1 / A2 need no clearing.  NT threads share one vertex:
-// 256, or 1024 when the map leaves room for one workgroup per CU (then the
-// workgroup's waves are all the CU holds, and its loads of neighbour lists
-// are what hides the memory latency).
+// The same rows and counts with the visited map and the 1-hop row in LDS, for
+// graphs whose map fits, and with |N n root| and |N2 n root| (root_d2).
+//
+// A workgroup takes vertices from a counter (their work differs by orders of
+// magnitude).  The lists to walk are cut into segments of ROWS_SEG entries, as
+// many tables of them as they need, and every wave takes ROWS_AT_ONCE segments
+// at a time: their loads, 16 a lane, are in flight together.  (Lists walked one
+// after another waited for two dependent loads each, 2 us a list whatever its
+// length: 34.9 ms for the 70,088 root vertices of a power-law graph of a million,
+// whose 11.7 billion entries are now walked in 10.9, 4.3 TB/s; 3.0 -> 0.5 ms for a
+// co-expression graph's 1.1 billion, 1.8 -> 0.5 for 0.4 billion of a smaller
+// power-law graph.)  NT threads share a vertex: 256, or 1024 when the map leaves
+// room for one workgroup per CU.
 constexpr int ROWS_THREADS = 256;
 constexpr int ROWS_THREADS_WIDE = 1024;
-constexpr int ROWS_BIG_MAX = 512;  // long neighbour lists listed per vertex (LDS)
+constexpr int ROWS_SEG = 256;
+constexpr int ROWS_AT_ONCE = 4;
+constexpr int ROWS_TAB_MIN = 256;   // segments in the LDS table, at least
+constexpr int ROWS_TAB_MAX = 2048;
 
 __device__ __forceinline__ uint64_t rdl64(uint64_t x, int l) {
     const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)x, l);
@@ -111,131 +122,276 @@ __device__ __forceinline__ uint64_t rdl64(uint64_t x, int l) {
 template <bool BYTES, int NT>
 __global__ __launch_bounds__(NT) void root_rows_lds(const uint64_t* __restrict__ off, const uint32_t* __restrict__ adj,
                                                     const int32_t* __restrict__ loc, const uint32_t* __restrict__ orig,
-                                                    int32_t R, int32_t rw, int32_t n, uint64_t* A1, uint64_t* A2,
-                                                    int32_t* n2out) {
+                                                    int32_t R, int32_t rw, int32_t n, int32_t tab_n, uint64_t* A1,
+                                                    uint64_t* A2, int32_t* n2out, int32_t* d1r, int32_t* d2r,
+                                                    uint32_t* next) {
     // vis: {v} u N(v) u N(N(v)) over all n vertices, as a byte map (BYTES:
     // plain stores of 1, no read-modify-write) or a bitmap (atomics without
-    // return); r1: root-space row of N(v).  |N2(v)| and the A2 row are read
-    // off the map afterwards.
-    // NT / 64 waves share one vertex: each takes every nwv-th group
-    // of neighbour lists and every nwv-th block of row words.  Lists of NT
-    // entries or more (the hubs of a power-law graph) are walked by all the
-    // workgroup's threads together instead: in a group they kept one wave
-    // busy while the others had finished (on config 4 the busiest wave of a
-    // vertex held 5.5x the average share).
+    // return); r1: root-space row of N(v); seg: list start << 16 | entries.
+    // |N2(v)| and the A2 row are read off the map afterwards.
     extern __shared__ unsigned long long sh[];
-    __shared__ int s_cnt;
-    __shared__ int s_nbig;
-    __shared__ uint32_t s_big[ROWS_BIG_MAX];
+    __shared__ uint32_t s_a, s_tot, s_cnt, s_d1, s_d2;
     const int lane = threadIdx.x & 63;
-    const int tid = threadIdx.x, nt = blockDim.x;
-    const int wv = threadIdx.x >> 6, nwv = blockDim.x >> 6;
+    const int tid = threadIdx.x;
+    const int wv = threadIdx.x >> 6;
+    constexpr int NWV = NT / 64;
     const int nw = BYTES ? (n + 7) / 8 : (n + 63) / 64;  // 64-bit words of the map
-    unsigned long long* vis = sh;
-    unsigned char* vis8 = (unsigned char*)sh;
-    unsigned long long* r1 = sh + nw;
+    unsigned long long* const vis = sh;
+    uint32_t* const vis32 = (uint32_t*)sh;
+    unsigned char* const vis8 = (unsigned char*)sh;
+    unsigned long long* const r1 = sh + nw;
+    unsigned long long* const seg = r1 + rw;
     auto mark = [&](uint32_t x) {
         if (BYTES)
             vis8[x] = 1;
         else
-            atomicOr(&vis[x >> 6], 1ull << (x & 63));
+            atomicOr(&vis32[x >> 5], 1u << (x & 31));
     };
-    auto seen = [&](uint32_t x) -> bool { return BYTES ? vis8[x] != 0 : ((vis[x >> 6] >> (x & 63)) & 1ull); };
-    constexpr int G = 8;  // neighbours u whose lists are walked together
-    for (int a = blockIdx.x; a < R; a += gridDim.x) {
-        const uint32_t v = orig[a];
-        for (int w = tid; w < nw; w += nt) vis[w] = 0;
-        for (int w = tid; w < rw; w += nt) r1[w] = 0;
+    auto seen = [&](uint32_t x) -> bool { return BYTES ? vis8[x] != 0 : ((vis32[x >> 5] >> (x & 31)) & 1u) != 0; };
+    for (;;) {
+        __syncthreads();  // (the vertex before is done with everything shared)
         if (tid == 0) {
-            s_cnt = 0;
-            s_nbig = 0;
+            s_a = atomicAdd(next, 1u);
+            s_tot = s_cnt = s_d1 = s_d2 = 0;
         }
+        for (int w = tid; w < nw; w += NT) vis[w] = 0;
+        for (int w = tid; w < rw; w += NT) r1[w] = 0;
         __syncthreads();
+        const uint32_t a = s_a;
+        if (a >= (uint32_t)R) break;
+        const uint32_t v = orig[a];
         if (tid == 0) mark(v);
         const uint64_t b0 = off[v], b1 = off[v + 1];
-        for (uint64_t j = b0 + tid; j < b1; j += nt) {
-            const uint32_t u = adj[j];
-            mark(u);
-            const int la = loc[u];
-            if (la >= 0) atomicOr(&r1[la >> 6], 1ull << (la & 63));
-            if (off[u + 1] - off[u] >= (uint64_t)NT) {
-                const int q = atomicAdd(&s_nbig, 1);
-                if (q < ROWS_BIG_MAX) s_big[q] = u;
-            }
-        }
-        __syncthreads();
-        // the long lists, one after another, every thread on each; when more
-        // than ROWS_BIG_MAX were found the groups below walk all long lists
-        // again (marking twice changes nothing)
-        const int nbig = min(s_nbig, ROWS_BIG_MAX);
-        const bool big_done = s_nbig <= ROWS_BIG_MAX;
-        for (int q = 0; q < nbig; q++) {
-            const uint32_t u = s_big[q];
-            const uint64_t e1 = off[u + 1];
-            for (uint64_t k = off[u] + tid; k < e1; k += nt) mark(adj[k]);
-        }
-        // N(u) for G neighbours u at a time as one flat range of entries:
-        // lane i < G holds u_i's list start and the prefix of list lengths
-        for (uint64_t j0 = b0 + (uint64_t)wv * G; j0 < b1; j0 += (uint64_t)nwv * G) {
+        for (uint64_t j0 = b0; j0 < b1; j0 += NT) {
+            // a neighbour per thread: marked, and its list as segments
             uint64_t st = 0, len = 0;
-            if (lane < G && j0 + lane < b1) {
-                const uint32_t u = adj[j0 + lane];
+            if (j0 + tid < b1) {
+                const uint32_t u = adj[j0 + tid];
+                mark(u);
+                const int la = loc[u];
+                if (la >= 0) atomicOr(&r1[la >> 6], 1ull << (la & 63));
                 st = off[u];
                 len = off[u + 1] - st;
-                if (big_done && len >= (uint64_t)NT) len = 0;
             }
-            uint64_t pre = len;  // inclusive prefix over lanes 0..G-1
-            for (int o = 1; o < G; o <<= 1) {
-                const uint64_t y = __shfl_up(pre, o, 64);
-                if (lane >= o) pre += y;
+            const uint32_t ns = (uint32_t)((len + ROWS_SEG - 1) / ROWS_SEG);
+            uint32_t pos = ns;  // inclusive prefix over the wave
+            for (int o = 1; o < 64; o <<= 1) {
+                const uint32_t y = __shfl_up(pos, o, 64);
+                if (lane >= o) pos += y;
             }
-            // segment ends and starts as wave-uniform values (the G lists
-            // of one group hold far fewer than 2^32 entries)
-            uint32_t e[G];
-            uint64_t sv[G];
+            uint32_t at = 0;
+            if (lane == 63) at = atomicAdd(&s_tot, pos);
+            pos += (uint32_t)__builtin_amdgcn_readlane((int)at, 63) - ns;
+            __syncthreads();
+            const uint32_t tot = s_tot;
+            for (uint32_t lo = 0; lo < tot; lo += (uint32_t)tab_n) {
+                const uint32_t hi = min(tot, lo + (uint32_t)tab_n);
+                for (uint32_t q = max(pos, lo); q < min(pos + ns, hi); q++) {
+                    const uint64_t d = (uint64_t)(q - pos) * ROWS_SEG;
+                    seg[q - lo] = ((st + d) << 16) | min(len - d, (uint64_t)ROWS_SEG);
+                }
+                __syncthreads();
+                const int m = (int)(hi - lo);
+                for (int g = wv * ROWS_AT_ONCE; g < m; g += NWV * ROWS_AT_ONCE) {
+                    uint64_t sg = 0;
+                    if (lane < ROWS_AT_ONCE && g + lane < m) sg = seg[g + lane];
+                    uint32_t x[ROWS_AT_ONCE][ROWS_SEG / 64];
 #pragma unroll
-            for (int q = 0; q < G; q++) {
-                e[q] = (uint32_t)rdl64(pre, q);
-                sv[q] = rdl64(st, q);
-            }
-            const uint32_t total = e[G - 1];
-#pragma unroll 8
-            for (uint32_t p = lane; p < total; p += 64) {
-                uint64_t s0 = sv[0];
-                uint32_t base = 0;
+                    for (int q = 0; q < ROWS_AT_ONCE; q++) {
+                        const uint64_t e = rdl64(sg, q);
+                        const uint32_t* const p = adj + (e >> 16);
+                        const int l = (int)(e & 0xFFFFull);
 #pragma unroll
-                for (int q = 0; q < G - 1; q++)
-                    if (p >= e[q]) {
-                        s0 = sv[q + 1];
-                        base = e[q];
+                        for (int k = 0; k < ROWS_SEG / 64; k++) {
+                            x[q][k] = 0xFFFFFFFFu;
+                            if (k * 64 + lane < l) x[q][k] = p[k * 64 + lane];
+                        }
                     }
-                mark(adj[s0 + (p - base)]);
+#pragma unroll
+                    for (int q = 0; q < ROWS_AT_ONCE; q++)
+#pragma unroll
+                        for (int k = 0; k < ROWS_SEG / 64; k++)
+                            if (x[q][k] != 0xFFFFFFFFu) mark(x[q][k]);
+                }
+                __syncthreads();
             }
+            if (tid == 0) s_tot = 0;
+            __syncthreads();
         }
         __syncthreads();
-        int cnt = 0;
-        for (int w = tid; w < nw; w += nt) cnt += __popcll(vis[w]);  // bytes are 0 or 1
-        for (int o = 32; o > 0; o >>= 1) cnt += __shfl_xor(cnt, o, 64);
-        if (lane == 0) atomicAdd(&s_cnt, cnt);
-        for (int w = tid; w < rw; w += nt) A1[(size_t)a * rw + w] = r1[w];
+        int cnt = 0, c1 = 0, c2 = 0;
+        for (int w = tid; w < nw; w += NT) cnt += __popcll(vis[w]);  // bytes are 0 or 1
+        for (int w = tid; w < rw; w += NT) {
+            A1[(size_t)a * rw + w] = r1[w];
+            c1 += __popcll(r1[w]);
+        }
+        for (int o = 32; o > 0; o >>= 1) {
+            cnt += __shfl_xor(cnt, o, 64);
+            c1 += __shfl_xor(c1, o, 64);
+        }
         // A2 row: bit b iff orig[b] was reached (b != a), one ballot per
-        // word; eight words per step keep eight orig loads in flight
-        for (int w0 = wv * 8; w0 < rw; w0 += nwv * 8) {
+        // word; eight words per step keep eight orig loads in flight, and the
+        // words leave in one store
+        for (int w0 = wv * 8; w0 < rw; w0 += NWV * 8) {
             uint32_t xs[8];
 #pragma unroll
             for (int k = 0; k < 8; k++) {
                 const int b = (w0 + k) * 64 + lane;
                 xs[k] = (w0 + k < rw && b < R) ? orig[b] : 0xFFFFFFFFu;
             }
+            unsigned long long mine = 0;
 #pragma unroll
             for (int k = 0; k < 8; k++) {
-                const int b = (w0 + k) * 64 + lane;
+                const uint32_t b = (uint32_t)((w0 + k) * 64 + lane);
                 const unsigned long long word = __ballot(xs[k] != 0xFFFFFFFFu && b != a && seen(xs[k]));
-                if (lane == 0 && w0 + k < rw) A2[(size_t)a * rw + w0 + k] = word;
+                c2 += __popcll(word);
+                if (lane == k) mine = word;
             }
+            if (lane < 8 && w0 + lane < rw) A2[(size_t)a * rw + w0 + lane] = mine;
+        }
+        if (lane == 0) {
+            atomicAdd(&s_cnt, (uint32_t)cnt);
+            atomicAdd(&s_d1, (uint32_t)c1);
+            atomicAdd(&s_d2, (uint32_t)c2);
         }
         __syncthreads();
-        if (tid == 0) n2out[a] = s_cnt - 1;  // v itself is in the map
+        if (tid == 0) {
+            n2out[a] = (int32_t)s_cnt - 1;  // v itself is in the map
+            d1r[a] = (int32_t)s_d1;
+            d2r[a] = (int32_t)s_d2;
+        }
+    }
+}
+
+// ---- filter and peel on the device (large graphs) ----
+// State of a peel: queue lengths per round, the core's size, and how many of
+// its vertices have fewer than min_size - 1 neighbours.
+constexpr int PEEL_ROUNDS = 48;
+struct PeelState {
+    uint32_t cnt[PEEL_ROUNDS + 1];
+    uint32_t R;
+    uint32_t n_check;
+};
+constexpr int SCAN_PER = 4096;  // vertices per block of the compaction
+
+// The degree filter (thr, and lists of min_size - 1 second neighbours when the
+// graph has them), a bit per vertex: the count below reads one for every entry
+// of every list, from a table that the caches hold.
+__global__ __launch_bounds__(256) void peel_pass(const uint64_t* __restrict__ off, const uint64_t* __restrict__ off2,
+                                                 int32_t n, int32_t thr, int64_t need2, uint64_t* __restrict__ pass) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const bool ok = i < n && (int64_t)(off[i + 1] - off[i]) >= thr &&
+                    (!off2 || (int64_t)(off2[i + 1] - off2[i]) >= need2);
+    const unsigned long long m = __ballot(ok);
+    if ((threadIdx.x & 63) == 0 && i < n) pass[i >> 6] = m;
+}
+
+// Degrees inside the vertices that pass, and the first round of the peel's
+// queue.  exd < 0 marks what did not pass.  A wave takes 64 vertices and walks the
+// lists of those that pass, one after the other.
+__global__ __launch_bounds__(256) void peel_count(const uint64_t* __restrict__ off, const uint32_t* __restrict__ adj,
+                                                  const uint64_t* __restrict__ pass, int32_t n, int32_t thr,
+                                                  int32_t* __restrict__ exd, uint32_t* __restrict__ queue,
+                                                  PeelState* ps) {
+    const int lane = threadIdx.x & 63;
+    const int64_t wave = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6), nwave = (int64_t)gridDim.x * 4;
+    for (int64_t b = wave * 64; b < n; b += nwave * 64) {
+        const unsigned long long word = pass[b >> 6];
+        if (b + lane < n && !((word >> lane) & 1ull)) exd[b + lane] = -1;
+        for (unsigned long long m = word; m; m &= m - 1) {
+            const int64_t v = b + __builtin_ctzll(m);
+            const uint64_t e = off[v + 1];
+            int d = 0;
+#pragma unroll 4
+            for (uint64_t j = off[v] + lane; j < e; j += 64) {
+                const uint32_t u = adj[j];
+                d += (int)((pass[u >> 6] >> (u & 63)) & 1ull);
+            }
+            for (int o = 32; o > 0; o >>= 1) d += __shfl_xor(d, o, 64);
+            if (lane == 0) {
+                exd[v] = d;
+                if (d < thr) queue[atomicAdd(&ps->cnt[0], 1u)] = (uint32_t)v;
+            }
+        }
+    }
+}
+
+// One round: the lists of the vertices queued by the round before; a neighbour
+// whose degree comes down to thr - 1 joins the next round (once, since degrees
+// go down by one at a time; those queued first are below already).
+__global__ __launch_bounds__(256) void peel_round(const uint64_t* __restrict__ off, const uint32_t* __restrict__ adj,
+                                                  int32_t thr, int32_t* exd, uint32_t* queue, PeelState* ps, int r) {
+    const int lane = threadIdx.x & 63;
+    const uint32_t wave = blockIdx.x * 4 + (threadIdx.x >> 6), nwave = gridDim.x * 4;
+    uint32_t lo = 0;
+    for (int k = 0; k < r; k++) lo += ps->cnt[k];
+    const uint32_t hi = lo + ps->cnt[r];
+    for (uint32_t q = lo + wave; q < hi; q += nwave) {
+        const uint32_t v = queue[q];
+        const uint64_t e = off[v + 1];
+        for (uint64_t j = off[v] + lane; j < e; j += 64) {
+            const uint32_t u = adj[j];
+            // (what did not pass stays negative)
+            if (exd[u] >= 0 && atomicSub(&exd[u], 1) == thr) queue[hi + atomicAdd(&ps->cnt[r + 1], 1u)] = u;
+        }
+    }
+}
+
+// The core's vertices in input order: per block, their number (first), then
+// their places.
+__global__ __launch_bounds__(256) void core_count(const int32_t* __restrict__ exd, int32_t n, int32_t thr,
+                                                  uint32_t* __restrict__ sums) {
+    __shared__ uint32_t s;
+    if (threadIdx.x == 0) s = 0;
+    __syncthreads();
+    const int64_t b = (int64_t)blockIdx.x * SCAN_PER;
+    uint32_t k = 0;
+    for (int i = threadIdx.x; i < SCAN_PER; i += 256)
+        if (b + i < n && exd[b + i] >= thr) k++;
+    for (int o = 32; o > 0; o >>= 1) k += __shfl_xor(k, o, 64);
+    if ((threadIdx.x & 63) == 0) atomicAdd(&s, k);
+    __syncthreads();
+    if (threadIdx.x == 0) sums[blockIdx.x] = s;
+}
+__global__ __launch_bounds__(64) void core_scan(uint32_t* sums, int32_t nb, PeelState* ps) {
+    const int lane = threadIdx.x;
+    uint32_t run = 0;
+    for (int b = 0; b < nb; b += 64) {
+        const uint32_t x = b + lane < nb ? sums[b + lane] : 0u;
+        uint32_t y = x;
+        for (int o = 1; o < 64; o <<= 1) {
+            const uint32_t t = __shfl_up(y, o, 64);
+            if (lane >= o) y += t;
+        }
+        if (b + lane < nb) sums[b + lane] = run + y - x;
+        run += (uint32_t)__builtin_amdgcn_readlane((int)y, 63);
+    }
+    if (lane == 0) {
+        ps->R = run;
+        ps->n_check = 0;
+    }
+}
+__global__ __launch_bounds__(64) void core_write(const int32_t* __restrict__ exd, const uint64_t* __restrict__ off,
+                                                 int32_t n, int32_t thr, int64_t need, const uint32_t* __restrict__ sums,
+                                                 int32_t* __restrict__ loc, uint32_t* __restrict__ orig,
+                                                 int32_t* __restrict__ core_deg, uint32_t* __restrict__ check,
+                                                 PeelState* ps) {
+    const int lane = threadIdx.x;
+    const int64_t b = (int64_t)blockIdx.x * SCAN_PER;
+    uint32_t at = sums[blockIdx.x];
+    for (int i = 0; i < SCAN_PER && b + i < n; i += 64) {
+        const int64_t v = b + i + lane;
+        const int d = v < n ? exd[v] : -1;
+        const bool in = v < n && d >= thr;
+        const uint64_t m = __ballot(in);
+        const uint32_t p = at + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
+        if (v < n) loc[v] = in ? (int32_t)p : -1;
+        if (in) {
+            orig[p] = (uint32_t)v;
+            core_deg[p] = d;
+            if ((int64_t)(off[v + 1] - off[v]) < need) check[atomicAdd(&ps->n_check, 1u)] = (uint32_t)v;
+        }
+        at += (uint32_t)__popcll(m);
     }
 }
 
@@ -281,6 +437,14 @@ namespace qc {
 
 namespace {
 
+// The filter and the peel run on the device from this many vertices or list
+// entries on: 0.3 ms or more of launches and round trips there, while the host
+// took 1.9 ms for a power-law graph of 100,000 vertices and 2 million entries,
+// 0.5 to 0.8 for a co-expression graph of 8,000 and 2 million, and 0.1 to 0.3 for
+// the smaller ones.
+constexpr int PEEL_DEVICE_MIN = 32768;
+constexpr size_t PEEL_DEVICE_ENTRIES = (size_t)1 << 20;
+
 // min(|N2(v)|, cap) over the full graph: the walk stops at the cap-th
 // distinct vertex (a neighbour that is a hub would otherwise cost its whole
 // list for a vertex that passed long before)
@@ -306,6 +470,52 @@ long n2_capped(const qc_graph* g, int v, std::vector<int>& mark, long cap) {
 }
 
 inline int label_rank(int l) { return l == 1 ? 0 : l == 2 ? 1 : l == 0 ? 2 : l == 3 ? 3 : 4; }
+
+inline int bits_of(uint32_t x) { return x ? 32 - __builtin_clz(x) : 0; }
+
+// root-local ids in the root's Q order.  The four keys in one word where they
+// fit, sorted by 11 bits a pass (70,000 vertices: 1 ms against 6 by comparing).
+void q_order(int R, int max_ex, int max_l2, const std::vector<int32_t>& label, const std::vector<int32_t>& exd,
+             const std::vector<int32_t>& l2, std::vector<int32_t>& order) {
+    const int be = bits_of((uint32_t)max_ex), bl = bits_of((uint32_t)max_l2), bi = bits_of((uint32_t)(R - 1));
+    if (3 + be + bl + bi > 64) {
+        for (int a = 0; a < R; a++) order[a] = a;
+        std::sort(order.begin(), order.end(), [&](int x, int y) {
+            const int rx = label_rank(label[x]), ry = label_rank(label[y]);
+            if (rx != ry) return rx < ry;
+            if (exd[x] != exd[y]) return exd[x] > exd[y];
+            if (l2[x] != l2[y]) return l2[x] > l2[y];
+            return x > y;
+        });
+        return;
+    }
+    // (ascending: the descending keys as their distance from the largest)
+    std::vector<uint64_t> key(R);
+    for (int a = 0; a < R; a++)
+        key[a] = ((((uint64_t)label_rank(label[a]) << be | (uint64_t)(max_ex - exd[a])) << bl |
+                   (uint64_t)(max_l2 - l2[a]))
+                  << bi) |
+                 (uint64_t)(R - 1 - a);
+    if (R < 4096) {
+        std::sort(key.begin(), key.end());
+    } else {
+        std::vector<uint64_t> tmp(R);
+        std::vector<uint32_t> cnt(2048);
+        for (int sh = 0; sh < 3 + be + bl + bi; sh += 11) {
+            std::fill(cnt.begin(), cnt.end(), 0u);
+            for (uint64_t k : key) cnt[(k >> sh) & 2047]++;
+            uint32_t at = 0;
+            for (uint32_t& c : cnt) {
+                const uint32_t x = c;
+                c = at;
+                at += x;
+            }
+            for (uint64_t k : key) tmp[cnt[(k >> sh) & 2047]++] = k;
+            key.swap(tmp);
+        }
+    }
+    for (int a = 0; a < R; a++) order[a] = R - 1 - (int)(key[a] & ((1ull << bi) - 1ull));
+}
 
 }  // namespace
 
@@ -362,31 +572,16 @@ int device_csr(const qc_graph* g, DevCSR** out, hipStream_t s) {
 }
 }  // namespace
 
-int upload_graph(const qc_graph* g, hipStream_t s) {
-    DevCSR* d = nullptr;
-    return device_csr(g, &d, s);
-}
-
-int graph_device_arrays(const qc_graph* g, const uint64_t** off, const uint32_t** adj, hipStream_t s) {
-    DevCSR* d = nullptr;
-    const int rc = device_csr(g, &d, s);
-    if (rc) return rc;
-    *off = d->off.as<uint64_t>();
-    *adj = d->adj.as<uint32_t>();
-    return QC_OK;
-}
-
 namespace {
-int build_instance_impl(const qc_graph* g, double gamma, int ms, Instance& I, hipStream_t s) {
-    const auto t_start = std::chrono::steady_clock::now();
-    const int n = g->n;
-    I.n = n;
-    I.gamma = gamma;
-    I.min_size = ms;
-    build_tables(gamma, n, ms, I.mindeg, I.ubq);
-    const int thr = I.mindeg[ms];
 
-    // ---- filter (main.cu:872-885) ----
+// Filter (main.cu:872-885) and peel (main.cu:889-949).  The reference's rounds and
+// queue compute the core in which every vertex has at least thr neighbours
+// inside it (unique, whatever the removal order), with exd = the degree inside
+// it.  Here: degrees inside the filtered set (host threads over the vertices),
+// then one queue that only walks the lists of removed filtered vertices.
+void peel_host(const qc_graph* g, int thr, int ms, std::vector<uint32_t>& orig, std::vector<int32_t>& core_deg,
+               std::vector<int32_t>& loc) {
+    const int n = g->n;
     std::vector<int32_t> lab(n), exd(n);
     std::vector<int32_t> rem;
     std::vector<int> mark(n, -1);
@@ -399,13 +594,6 @@ int build_instance_impl(const qc_graph* g, double gamma, int ms, Instance& I, hi
         lab[i] = pass ? 0 : -1;
         if (pass) rem.push_back(i);
     }
-    const auto t_filter = std::chrono::steady_clock::now();
-    // ---- peel (main.cu:889-949) ----
-    // The reference's rounds and queue compute the core in which every
-    // vertex has at least thr neighbours inside it (unique, whatever the
-    // removal order), with exd = the degree inside it.  Here: degrees inside
-    // the filtered set (host threads over the vertices), then one queue that
-    // only walks the lists of removed filtered vertices.
     {
         const unsigned hw = std::max(1u, std::min(16u, std::thread::hardware_concurrency()));
         const size_t nrem = rem.size();
@@ -427,7 +615,6 @@ int build_instance_impl(const qc_graph* g, double gamma, int ms, Instance& I, hi
             for (auto& x : th) x.join();
         }
     }
-    const auto t_count = std::chrono::steady_clock::now();
     std::vector<int32_t> queue;
     for (int v : rem)
         if (exd[v] < thr) {
@@ -444,60 +631,187 @@ int build_instance_impl(const qc_graph* g, double gamma, int ms, Instance& I, hi
             }
         }
     }
-    const auto t_host = std::chrono::steady_clock::now();
-    // ---- root-local ids ----
-    I.orig.clear();
-    std::vector<int32_t> loc(n, -1);
+    // root-local ids
+    loc.assign(n, -1);
+    orig.clear();
+    core_deg.clear();
     for (int i = 0; i < n; i++)
         if (lab[i] == 0) {
-            loc[i] = (int32_t)I.orig.size();
-            I.orig.push_back((uint32_t)i);
+            loc[i] = (int32_t)orig.size();
+            orig.push_back((uint32_t)i);
+            core_deg.push_back(exd[i]);
         }
+}
+
+// The same on the device.  Without second-neighbour lists the filter's |N2|
+// >= min_size - 1 is left out there and looked up for the core's vertices of
+// degree below min_size - 1: a core whose vertices all have it is the filtered
+// core too (it contains that one, and is one).  done = false, to be done on the
+// host: a vertex of the core does not have it, or the peel takes more rounds
+// than PEEL_ROUNDS (a long chain would cost a launch for each of its vertices).
+// A power-law graph of a million vertices and 30 million entries: 45 ms on 16
+// host threads, 1.2 here, bound by the latency of the rounds' launches and the
+// random reads of the count.
+int peel_device(const qc_graph* g, const DevCSR& G, int thr, int ms, Instance& I, std::vector<int32_t>& core_deg,
+                DBuf& d_loc, bool& done, hipStream_t s) {
+    using namespace qcdev;
+    const int n = g->n;
+    done = false;
+    if (thr < 0) return QC_OK;
+    DBuf d_exd, d_queue, d_state, d_sums, d_deg, d_pass, d_check;
+    int rc;
+    const int nb = (int)(((int64_t)n + SCAN_PER - 1) / SCAN_PER);
+    if ((rc = d_exd.alloc((size_t)n * 4, s)) || (rc = d_queue.alloc((size_t)n * 4, s)) ||
+        (rc = d_state.alloc(sizeof(PeelState), s)) || (rc = d_sums.alloc((size_t)nb * 4, s)) ||
+        (rc = d_deg.alloc((size_t)n * 4, s)) || (rc = d_loc.alloc((size_t)n * 4, s)) ||
+        (rc = d_pass.alloc(((size_t)n + 63) / 64 * 8, s)) || (rc = d_check.alloc((size_t)n * 4, s)) ||
+        (rc = I.d_orig.alloc((size_t)n * 4)))
+        return rc;
+    QC_HIP(hipMemsetAsync(d_state.p, 0, sizeof(PeelState), s));
+    PeelState* ps = d_state.as<PeelState>();
+    const uint64_t* off = G.off.as<uint64_t>();
+    const uint32_t* adj = G.adj.as<uint32_t>();
+    hipLaunchKernelGGL(peel_pass, dim3((n + 255) / 256), dim3(256), 0, s, off,
+                       g->has_n2 ? G.off2.as<uint64_t>() : (const uint64_t*)nullptr, n, thr, (int64_t)ms - 1,
+                       d_pass.as<uint64_t>());
+    hipLaunchKernelGGL(peel_count, dim3(std::min((n + 255) / 256, 2048)), dim3(256), 0, s, off, adj,
+                       d_pass.as<uint64_t>(), n, thr, d_exd.as<int32_t>(), d_queue.as<uint32_t>(), ps);
+    QC_HIP(hipGetLastError());
+    // (12 rounds between looks at the queue: a round of nothing takes 3 us, a look 20)
+    PeelState h;
+    int r = 0;
+    for (;;) {
+        for (int k = 0; k < 12; k++, r++)
+            hipLaunchKernelGGL(peel_round, dim3(512), dim3(256), 0, s, off, adj, thr, d_exd.as<int32_t>(),
+                               d_queue.as<uint32_t>(), ps, r);
+        hipLaunchKernelGGL(core_count, dim3(nb), dim3(256), 0, s, d_exd.as<int32_t>(), n, thr, d_sums.as<uint32_t>());
+        hipLaunchKernelGGL(core_scan, dim3(1), dim3(64), 0, s, d_sums.as<uint32_t>(), nb, ps);
+        hipLaunchKernelGGL(core_write, dim3(nb), dim3(64), 0, s, d_exd.as<int32_t>(), off, n, thr,
+                           g->has_n2 ? (int64_t)0 : (int64_t)ms - 1, d_sums.as<uint32_t>(), d_loc.as<int32_t>(),
+                           I.d_orig.as<uint32_t>(), d_deg.as<int32_t>(), d_check.as<uint32_t>(), ps);
+        QC_HIP(hipGetLastError());
+        QC_HIP(hipMemcpyAsync(&h, ps, sizeof(h), hipMemcpyDeviceToHost, s));
+        QC_HIP(hipStreamSynchronize(s));
+        if (h.cnt[r] == 0) break;
+        if (r + 12 > PEEL_ROUNDS) return QC_OK;
+    }
+    I.orig.resize(h.R);
+    core_deg.resize(h.R);
+    std::vector<uint32_t> check(h.n_check);
+    if (h.R) {
+        QC_HIP(hipMemcpyAsync(I.orig.data(), I.d_orig.p, (size_t)h.R * 4, hipMemcpyDeviceToHost, s));
+        QC_HIP(hipMemcpyAsync(core_deg.data(), d_deg.p, (size_t)h.R * 4, hipMemcpyDeviceToHost, s));
+    }
+    if (h.n_check) QC_HIP(hipMemcpyAsync(check.data(), d_check.p, (size_t)h.n_check * 4, hipMemcpyDeviceToHost, s));
+    QC_HIP(hipStreamSynchronize(s));
+    if (!check.empty()) {
+        std::vector<int> mark(n, -1);
+        for (uint32_t v : check)
+            if (n2_capped(g, (int)v, mark, ms - 1) < ms - 1) return QC_OK;
+    }
+    done = true;
+    return QC_OK;
+}
+
+}  // namespace
+
+int upload_graph(const qc_graph* g, hipStream_t s) {
+    DevCSR* d = nullptr;
+    return device_csr(g, &d, s);
+}
+
+int graph_device_arrays(const qc_graph* g, const uint64_t** off, const uint32_t** adj, hipStream_t s) {
+    DevCSR* d = nullptr;
+    const int rc = device_csr(g, &d, s);
+    if (rc) return rc;
+    *off = d->off.as<uint64_t>();
+    *adj = d->adj.as<uint32_t>();
+    return QC_OK;
+}
+
+namespace {
+int build_instance_impl(const qc_graph* g, double gamma, int ms, Instance& I, hipStream_t s) {
+    const auto t_start = std::chrono::steady_clock::now();
+    const int n = g->n;
+    I.n = n;
+    I.gamma = gamma;
+    I.min_size = ms;
+    const int thr = (int32_t)std::ceil(gamma * (double)(ms - 1));  // mindeg[min_size]
+    int rc;
+    I.orig.clear();
+    I.root.clear();
+    // of the root's vertices, by root-local id: degree in the core
+    std::vector<int32_t> exd;
+    DevCSR* G = nullptr;
+    DBuf d_loc;
+    bool on_device = false;
+    std::vector<int32_t> loc;  // (host path: in use until its copy has run)
+    if (n >= PEEL_DEVICE_MIN || g->adj.size() >= PEEL_DEVICE_ENTRIES) {
+        if ((rc = device_csr(g, &G, s))) return rc;
+        if ((rc = peel_device(g, *G, thr, ms, I, exd, d_loc, on_device, s))) return rc;
+    }
+    if (!on_device) {
+        peel_host(g, thr, ms, I.orig, exd, loc);
+        if (!I.orig.empty()) {
+            if ((rc = device_csr(g, &G, s))) return rc;
+            if ((rc = d_loc.alloc((size_t)n * 4, s)) || (rc = I.d_orig.alloc(I.orig.size() * 4))) return rc;
+            QC_HIP(hipMemcpyAsync(d_loc.p, loc.data(), (size_t)n * 4, hipMemcpyHostToDevice, s));
+            QC_HIP(hipMemcpyAsync(I.d_orig.p, I.orig.data(), I.orig.size() * 4, hipMemcpyHostToDevice, s));
+        }
+    }
+    const auto t_host = std::chrono::steady_clock::now();
     const int R = (int)I.orig.size();
     I.R = R;
     I.rw = (R + 63) / 64;
-    I.root.clear();
     if (R == 0) return QC_OK;
+    // (the total degree of a member, which indexes the table, is below R)
+    I.ubq.resize((size_t)R + 2);
+    for (int d = 0; d < R + 2; d++) I.ubq[d] = (int32_t)std::floor((double)d / gamma);
 
     // ---- device tables ----
-    int rc;
     const size_t mat_bytes = (size_t)R * I.rw * 8;
     if ((rc = I.A1.alloc(mat_bytes))) return rc;
     if ((rc = I.A2.alloc(mat_bytes))) return rc;
-    // LDS form: visited map + the 1-hop row of one root vertex per wave; a
+    // LDS form: visited map, the 1-hop row and a table of list segments; a
     // byte map (plain stores) up to 32K vertices, a bitmap (atomics) above
     const bool byte_map = n <= 32768;
     const size_t map_words = byte_map ? ((size_t)n + 7) / 8 : ((size_t)n + 63) / 64;
-    const size_t lds_bytes = (map_words + (size_t)I.rw) * 8;
-    int lds_max = 0, cur_dev = 0;
+    const size_t map_bytes = (map_words + (size_t)I.rw) * 8;
+    int lds_max = 0, cur_dev = 0, n_cu = 0;
     QC_HIP(hipGetDevice(&cur_dev));
     if (hipDeviceGetAttribute(&lds_max, hipDeviceAttributeMaxSharedMemoryPerBlock, cur_dev) != hipSuccess)
         lds_max = 64 * 1024;
+    QC_HIP(hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, cur_dev));
     // one workgroup per CU when two maps do not fit: then 16 waves per vertex
-    const bool rows_wide = !byte_map && lds_bytes * 2 > (size_t)lds_max;
+    const bool rows_wide = !byte_map && map_bytes * 2 > (size_t)lds_max;
     const int rows_threads = rows_wide ? qcdev::ROWS_THREADS_WIDE : qcdev::ROWS_THREADS;
     const void* rows_kernel = byte_map    ? (const void*)qcdev::root_rows_lds<true, qcdev::ROWS_THREADS>
                               : rows_wide ? (const void*)qcdev::root_rows_lds<false, qcdev::ROWS_THREADS_WIDE>
                                           : (const void*)qcdev::root_rows_lds<false, qcdev::ROWS_THREADS>;
-    // (the kernel's static LDS, the long-list table, comes on top)
-    bool lds_rows = !g->has_n2 && lds_bytes + sizeof(uint32_t) * (qcdev::ROWS_BIG_MAX + 4) <= (size_t)lds_max;
+    // the segment table takes what is left (64: the kernel's static LDS), at
+    // most four segments a thread or ROWS_TAB_MAX
+    const size_t left = map_bytes + 64 < (size_t)lds_max ? ((size_t)lds_max - map_bytes - 64) / 8 : 0;
+    const int tab_n = (int)std::min<size_t>(left, std::min(qcdev::ROWS_TAB_MAX, 4 * rows_threads));
+    const size_t lds_bytes = map_bytes + (size_t)tab_n * 8;
+    bool lds_rows = !g->has_n2 && tab_n >= qcdev::ROWS_TAB_MIN;
     if (lds_rows && lds_bytes > 48 * 1024 &&
         hipFuncSetAttribute(rows_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes) != hipSuccess)
+        lds_rows = false;
+    int occ = 0;
+    if (lds_rows && (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, rows_kernel, rows_threads, lds_bytes) !=
+                         hipSuccess ||
+                     occ < 1))
         lds_rows = false;
     if (!lds_rows) {
         QC_HIP(hipMemsetAsync(I.A1.p, 0, mat_bytes, s));
         QC_HIP(hipMemsetAsync(I.A2.p, 0, mat_bytes, s));
     }
-    DevCSR* G = nullptr;
-    if ((rc = device_csr(g, &G, s))) return rc;
     // temporaries carry the stream: released on an error return while the
     // kernels below still run, they are not handed out again before those end
-    DBuf d_loc, d_n2, d_vis;
-    if ((rc = d_loc.alloc((size_t)n * 4, s))) return rc;
-    if ((rc = d_n2.alloc((size_t)R * 4, s))) return rc;
-    if ((rc = I.d_orig.alloc((size_t)R * 4))) return rc;
-    QC_HIP(hipMemcpyAsync(d_loc.p, loc.data(), (size_t)n * 4, hipMemcpyHostToDevice, s));
-    QC_HIP(hipMemcpyAsync(I.d_orig.p, I.orig.data(), (size_t)R * 4, hipMemcpyHostToDevice, s));
+    DBuf d_n2, d_vis, d_next;
+    if ((rc = d_n2.alloc((size_t)R * 4, s)) || (rc = I.d_d2r.alloc((size_t)R * 4)) ||
+        (rc = I.d_d1r.alloc((size_t)R * 4)))
+        return rc;
     int blocks = std::min(R, 2048);
     uint64_t vis_words = ((uint64_t)n + 63) / 64;
     const bool phases = getenv("QCMINE_PHASES") != nullptr;
@@ -507,20 +821,22 @@ int build_instance_impl(const qc_graph* g, double gamma, int ms, Instance& I, hi
     };
     const auto t_up = stamp();
     if (lds_rows) {
-        // one block per root vertex: the dispatcher hands the next vertex to
-        // whichever slot frees first (their costs differ by orders of magnitude)
-        const int lblocks = std::min(R, 1 << 20);
+        if ((rc = d_next.alloc(4, s))) return rc;
+        QC_HIP(hipMemsetAsync(d_next.p, 0, 4, s));
         const uint64_t* offp = G->off.as<uint64_t>();
         const uint32_t* adjp = G->adj.as<uint32_t>();
         const int32_t* locp = d_loc.as<int32_t>();
         const uint32_t* origp = I.d_orig.as<uint32_t>();
-        int32_t Rv = R, rwv = I.rw, nv = n;
+        int32_t Rv = R, rwv = I.rw, nv = n, tabv = tab_n;
         uint64_t* A1p = I.A1.as<uint64_t>();
         uint64_t* A2p = I.A2.as<uint64_t>();
         int32_t* n2p = d_n2.as<int32_t>();
-        void* rargs[] = {(void*)&offp, (void*)&adjp, (void*)&locp, (void*)&origp, (void*)&Rv,
-                         (void*)&rwv,  (void*)&nv,   (void*)&A1p,  (void*)&A2p,   (void*)&n2p};
-        QC_HIP(hipLaunchKernel(rows_kernel, dim3(lblocks), dim3(rows_threads), rargs, lds_bytes, s));
+        int32_t* d1p = I.d_d1r.as<int32_t>();
+        int32_t* d2p = I.d_d2r.as<int32_t>();
+        uint32_t* nextp = d_next.as<uint32_t>();
+        void* rargs[] = {(void*)&offp, (void*)&adjp, (void*)&locp, (void*)&origp, (void*)&Rv,  (void*)&rwv, (void*)&nv,
+                         (void*)&tabv, (void*)&A1p,  (void*)&A2p,  (void*)&n2p,   (void*)&d1p, (void*)&d2p, (void*)&nextp};
+        QC_HIP(hipLaunchKernel(rows_kernel, dim3(std::min(R, occ * n_cu)), dim3(rows_threads), rargs, lds_bytes, s));
     } else {
         if (!g->has_n2) {
             if ((rc = d_vis.alloc((size_t)blocks * vis_words * 8, s))) return rc;
@@ -530,72 +846,60 @@ int build_instance_impl(const qc_graph* g, double gamma, int ms, Instance& I, hi
                            G->adj.as<uint32_t>(), G->off2.as<uint64_t>(), G->adj2.as<uint32_t>(), d_loc.as<int32_t>(),
                            I.d_orig.as<uint32_t>(), R, I.rw, I.A1.as<uint64_t>(), I.A2.as<uint64_t>(),
                            d_n2.as<int32_t>(), d_vis.as<unsigned long long>(), vis_words, g->has_n2 ? 1 : 0);
+        hipLaunchKernelGGL(qcdev::root_d2, dim3(blocks), dim3(64), 0, s, I.A2.as<uint64_t>(), I.A1.as<uint64_t>(), R,
+                           I.rw, I.d_d2r.as<int32_t>(), I.d_d1r.as<int32_t>());
     }
     QC_HIP(hipGetLastError());
     const auto t_rows = stamp();
-    if ((rc = I.d_d2r.alloc((size_t)R * 4))) return rc;
-    if ((rc = I.d_d1r.alloc((size_t)R * 4))) return rc;
-    hipLaunchKernelGGL(qcdev::root_d2, dim3(blocks), dim3(64), 0, s, I.A2.as<uint64_t>(), I.A1.as<uint64_t>(), R,
-                       I.rw, I.d_d2r.as<int32_t>(), I.d_d1r.as<int32_t>());
-    QC_HIP(hipGetLastError());
     I.d2r.resize(R);
     QC_HIP(hipMemcpyAsync(I.d2r.data(), I.d_d2r.p, (size_t)R * 4, hipMemcpyDeviceToHost, s));
     std::vector<int32_t> n2(R);
     QC_HIP(hipMemcpyAsync(n2.data(), d_n2.p, (size_t)R * 4, hipMemcpyDeviceToHost, s));
-    if ((rc = I.d_mindeg.alloc(I.mindeg.size() * 4))) return rc;
     if ((rc = I.d_ubq.alloc(I.ubq.size() * 4))) return rc;
-    QC_HIP(hipMemcpyAsync(I.d_mindeg.p, I.mindeg.data(), I.mindeg.size() * 4, hipMemcpyHostToDevice, s));
     QC_HIP(hipMemcpyAsync(I.d_ubq.p, I.ubq.data(), I.ubq.size() * 4, hipMemcpyHostToDevice, s));
     QC_HIP(hipStreamSynchronize(s));
     if (phases) {
         const auto t_dev = std::chrono::steady_clock::now();
         auto ms = [](auto a, auto b) { return std::chrono::duration<double, std::milli>(b - a).count(); };
         fprintf(stderr,
-                "[qcmine] root: R=%d host filter/peel %.2f ms (from call; filter %.2f, degrees %.2f, peel %.2f), "
-                "device rows %.2f ms (%s; uploads %.2f, rows %.2f, degrees and tables %.2f)\n",
-                R, ms(t_start, t_host), ms(t_start, t_filter), ms(t_filter, t_count), ms(t_count, t_host),
-                ms(t_host, t_dev), lds_rows ? "lds" : "global", ms(t_host, t_up), ms(t_up, t_rows), ms(t_rows, t_dev));
+                "[qcmine] root: R=%d filter/peel %.2f ms (%s), device rows %.2f ms (%s; uploads %.2f, rows %.2f, "
+                "tables %.2f)\n",
+                R, ms(t_start, t_host), on_device ? "device" : "host", ms(t_host, t_dev), lds_rows ? "lds" : "global",
+                ms(t_host, t_up), ms(t_up, t_rows), ms(t_rows, t_dev));
     }
 
     // ---- cover vertex and covered set (main.cu:953-975) ----
-    int maxd = 0, maxi = -1;
+    int maxd = 0, maxi = -1, maxl2 = 0;
     for (int a = 0; a < R; a++) {
-        int v = (int)I.orig[a];
-        if (exd[v] > maxd) {
-            maxd = exd[v];
+        if (exd[a] > maxd) {
+            maxd = exd[a];
             maxi = a;
         }
+        maxl2 = std::max(maxl2, n2[a]);
     }
-    struct RV {
-        int32_t id, label, exdeg, l2;
-    };
-    std::vector<RV> rv(R);
-    for (int a = 0; a < R; a++) rv[a] = {a, 0, exd[I.orig[a]], n2[a]};
+    std::vector<int32_t> label(R, 0);
     if (maxi >= 0) {
-        rv[maxi].label = 3;
-        int v = (int)I.orig[maxi];
+        label[maxi] = 3;
+        const uint32_t v = I.orig[maxi];
         for (uint64_t j = g->off[v]; j < g->off[v + 1]; j++) {
-            int la = loc[g->adj[j]];
-            if (la >= 0 && rv[la].label == 0) rv[la].label = 2;
+            // (input ids ascend with root-local ones)
+            const auto it = std::lower_bound(I.orig.begin(), I.orig.end(), g->adj[j]);
+            if (it == I.orig.end() || *it != g->adj[j]) continue;
+            const size_t la = (size_t)(it - I.orig.begin());
+            if (label[la] == 0) label[la] = 2;
         }
     }
     // ---- Q order (main.cu:2059-2104); indeg is 0 for every root vertex ----
-    std::sort(rv.begin(), rv.end(), [](const RV& x, const RV& y) {
-        int rx = label_rank(x.label), ry = label_rank(y.label);
-        if (rx != ry) return rx < ry;
-        if (x.exdeg != y.exdeg) return x.exdeg > y.exdeg;
-        if (x.l2 != y.l2) return x.l2 > y.l2;
-        return x.id > y.id;
-    });
+    // label rank ascending, then exdeg, |N2| and id descending
+    std::vector<int32_t> order(R);
+    q_order(R, maxd, maxl2, label, exd, n2, order);
     I.root.resize(R);
-    for (int a = 0; a < R; a++) I.root[a] = Vrec{rv[a].id, rv[a].label, 0, rv[a].exdeg};
+    for (int a = 0; a < R; a++) I.root[a] = Vrec{order[a], label[order[a]], 0, exd[order[a]]};
 
     I.dg.R = R;
     I.dg.rw = I.rw;
     I.dg.A1 = I.A1.as<uint64_t>();
     I.dg.A2 = I.A2.as<uint64_t>();
-    I.dg.mindeg = I.d_mindeg.as<int32_t>();
-    I.dg.mindeg_n = (int32_t)I.mindeg.size();
     I.dg.ubq = I.d_ubq.as<int32_t>();
     I.dg.ubq_n = (int32_t)I.ubq.size();
     I.dg.min_size = ms;
