@@ -6,9 +6,10 @@
 // remove-one-vertex, add-one-vertex with diameter and degree pruning,
 // critical-vertex pruning, the clique test and the Q-ordered child write.
 //
-// Three forms of the same steps, by the task's size: up to 64 vertices in
+// Four forms of the same steps, by the task's size: up to 64 vertices in
 // registers, with the whole subtree below (tiny_*); up to what the wave's LDS
-// holds (WideLds); larger ones from the wave's HBM slab (WideSlab).
+// holds (WideLds); larger ones from the wave's HBM slab, in 16- and 32-bit
+// arrays up to 4,095 vertices (WideMid), else in 32- and 64-bit ones (WideSlab).
 //
 // Adjacency.  Every task is a subset of the root task, so vertex ids are
 // root-local (0..R-1) and the 1-hop / 2-hop relations are kept as R x R bit
@@ -27,6 +28,8 @@
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+
+#include <type_traits>
 
 #include "qc_device.h"
 
@@ -128,7 +131,7 @@ struct LStats {
 struct GConst {
     const DevGraph* p;
     double gamma;
-    int32_t ubq_n, min_size, max_depth;
+    int32_t min_size, max_depth;
 };
 
 __device__ __forceinline__ int32_t uni32(int32_t x) { return __builtin_amdgcn_readfirstlane(x); }
@@ -142,7 +145,6 @@ __device__ __forceinline__ GConst load_graph(const DevGraph* p) {
     GConst g;
     g.p = p;
     g.gamma = __longlong_as_double(uni64(__double_as_longlong(p->gamma)));
-    g.ubq_n = uni32(p->ubq_n);
     g.min_size = uni32(p->min_size);
     g.max_depth = uni32(p->max_depth);
     return g;
@@ -204,6 +206,9 @@ __device__ __forceinline__ void ph_flush(Ctx& c) {
 __device__ __forceinline__ int md(const Ctx& c, int i) {
     return i < 1 ? 0 : (int)ceil(c.g.gamma * (double)(i - 1));
 }
+// floor(d / gamma), the same IEEE division as on the host, in place of a table:
+// a dependent load on the way to every bound
+__device__ __forceinline__ int ub_quot(const Ctx& c, int d) { return (int)floor((double)d / c.g.gamma); }
 __device__ __forceinline__ int get_mindeg(const Ctx& c, int s) {
     int ms = c.g.min_size;
     return s < ms ? md(c, ms) : md(c, s);
@@ -730,6 +735,7 @@ struct Tiny {
     uint32_t orig;        // input id
     int d1, d2;           // |N n root|, |N2 n root|
     int mdt;              // mindeg[lane]
+    int ubt;              // floor(lane / gamma)
     uint32_t s;           // word of the task to run next
     uint32_t hot;         // the child pushed last, not yet in the LDS
     int fr, ff;           // lane k: removed vertex and smallest failing member of the k-th failed removal
@@ -794,6 +800,7 @@ __device__ __attribute__((always_inline)) bool tiny_load(Ctx& c, const TaskRef& 
         }
     }
     y.mdt = md(c, lane);
+    y.ubt = ub_quot(c, lane);
     y.depth = ref.depth;
     y.hot_on = false;
     y.hot = 0;
@@ -878,7 +885,8 @@ __device__ __forceinline__ bool tiny_bounds(Ctx& c, const Tiny& y, uint64_t M, i
         const int min_tot = wave_min(mem ? in + ex : INT32_MAX);
         // (a stale exdeg can make the sum negative: floor(d / gamma) is then
         // below 0 and the bound too)
-        const int tq = min_tot < 0 ? -1 : c.g.p->ubq[min(min_tot, c.g.ubq_n - 1)];
+        // (from 63 on floor(d / gamma) + 1 - m is nc or more)
+        const int tq = min_tot < 0 ? -1 : rdlane(y.ubt, min(min_tot, WAVE - 1));
         ub = tq + 1 - m;
         if (ub > nc) ub = nc;
         if (lb < ub) {
@@ -918,9 +926,11 @@ __device__ __forceinline__ bool tiny_bounds(Ctx& c, const Tiny& y, uint64_t M, i
 
 // degree_pruning over lane masks: `alive` are the candidates that may stay,
 // `dead` the others; on return `alive` holds those that stay.  True: fails.
+// again: whether the same call on what it leaves could end otherwise (the last
+// bounds counted fewer candidates than stay).
 __device__ __attribute__((always_inline)) bool tiny_prune(Ctx& c, const Tiny& y, uint64_t M, int m, uint64_t& alive,
                                                           uint64_t dead, int in, int& ex, bool map_empty, int mds, int& ub,
-                                                          int& lb, int& med) {
+                                                          int& lb, int& med, bool& again) {
     const int ms = c.g.min_size;
     const uint64_t me = 1ull << c.lane;
     int T = 0, U = 0;
@@ -957,6 +967,7 @@ __device__ __attribute__((always_inline)) bool tiny_prune(Ctx& c, const Tiny& y,
         cnt_set = ballot((rem & me) && valid());
     }
     alive = rem;
+    again = cnt_set != rem;
     return false;
 }
 
@@ -1025,9 +1036,9 @@ __device__ __attribute__((always_inline)) void tiny_task(Ctx& c, Tiny& y, uint32
         const int a1 = (int)((y.r1 >> v) & 1ull);
         int ci = in + a1, ce = ex - a1;
         int ub = 0, lb = 0, med = 0;
-        bool map_empty = false, first = true, fails;
+        bool map_empty = false, first = true, fails, again = true;
         for (;;) {
-            fails = tiny_prune(c, y, Mc, m, alive, dead, ci, ce, map_empty, mds, ub, lb, med);
+            fails = tiny_prune(c, y, Mc, m, alive, dead, ci, ce, map_empty, mds, ub, lb, med, again);
             if (!first || fails) break;
             first = false;
             // critical_prep
@@ -1037,6 +1048,9 @@ __device__ __attribute__((always_inline)) void tiny_task(Ctx& c, Tiny& y, uint32
             const uint64_t F = cm ? ballot((alive & me) && (y.r1 & cm)) : 0ull;
             dead = 0;
             if (F == 0) {
+                // nothing changed: the closing degree pruning ends as the first
+                // one did, unless that one's last bounds counted fewer
+                if (!again) break;
                 map_empty = true;
                 continue;
             }
@@ -1270,7 +1284,7 @@ __device__ __attribute__((always_inline)) void tiny_level(Ctx& c, Tiny& y, uint3
 //     address for 64 lanes, neighbouring words) while the set is small.
 // The order of members and of candidates inside a child is free: the record
 // written is sorted by a key that is unique.
-constexpr uint32_t WIDE_LDS_MAX = 4095;   // WideLds: positions, indegrees and the sort key's fields
+constexpr uint32_t WIDE_LDS_MAX = WIDE_TASK_MAX;   // WideLds: positions, indegrees and the sort key's fields
 constexpr int WIDE_LDS_R_MAX = 1 << 20;   // WideLds: ids in a sort key
 constexpr int WIDE_ROW_WORDS = 256;       // rows up to this size (R <= 16,384) are staged in LDS
 
@@ -1321,6 +1335,20 @@ struct WideSlab : WideWord<uint64_t, 32, 1 << 30, 1 << 29> {
     using keyp = gptr<uint64_t>;
 };
 
+// the slab with 16-bit ids and positions and WideLds' words: half the bytes
+// that a branch reads and writes per vertex, which bound the first branches of a
+// power-law graph (tasks of 3,000 vertices, 2,048 slabs: 160 -> 146 ms)
+struct WideMid : WideWord<uint32_t, 20, 1 << 17, 1 << 16> {
+    static constexpr bool slab = true;
+    static constexpr int U = 4;
+    using u32p = gptr<uint16_t>;
+    using wordp = gptr<uint32_t>;
+    using posp = gptr<uint16_t>;
+    using pos_t = uint16_t;
+    using keyp = gptr<uint64_t>;
+};
+constexpr int WIDE_MID_R_MAX = 1 << 16;
+
 __device__ __forceinline__ bool wide_rows_staged(uint32_t rw, uint32_t lds_bytes) {
     return rw <= (uint32_t)WIDE_ROW_WORDS && 24u * rw <= lds_bytes;
 }
@@ -1349,6 +1377,7 @@ struct Wide {
     int idb;           // WideLds: bits of the id in a sort key
     int mdt;           // mindeg[lane]
     int mds;           // mindeg[min_size]
+    int ubt;           // floor(lane / gamma)
     bool rl;           // rows are staged in LDS
     bool ml;           // lmask has room for a row
     int tb, ub1;       // cand_valid's lane-independent bounds, from the last wide_bounds
@@ -1376,7 +1405,7 @@ __device__ __attribute__((always_inline)) bool wide_bounds(Ctx& c, Wide<P>& z, i
     auto gm = [&](int s) { return s < ms ? z.mds : wide_md(c, z, s); };
     // smallest (indeg, exdeg) pair, exdeg compared as an unsigned value
     int min_in, min_in_ex, min_tot = INT32_MAX, sum_in = 0;
-    if constexpr (!P::slab) {
+    if constexpr (sizeof(typename P::word) == 4) {
         // (in one word, compared as signed with the top bit flipped)
         int pair = INT32_MAX;
         for (int i = c.lane; i < m; i += WAVE) {
@@ -1423,12 +1452,18 @@ __device__ __attribute__((always_inline)) bool wide_bounds(Ctx& c, Wide<P>& z, i
         min_tot = wave_min(min_tot);
         // (a stale exdeg can make the sum negative: floor(d / gamma) is then
         // below 0 and the bound too)
-        const int tq = min_tot < 0 ? -1 : glob(c.g.p->ubq)[min(min_tot, c.g.ubq_n - 1)];
+        const int tq = min_tot < 0 ? -1 : min_tot < WAVE ? rdlane(z.ubt, min_tot) : uni(ub_quot(c, min_tot));
         ub = tq + 1 - m;
         if (ub > nc) ub = nc;
         ub = uni(ub);
         if (lb < ub) {
-            const long long sum_all = wave_sum64((long long)sum_in);
+            // (32-bit words: t <= 4,095, so degree sums and products fit 32 bits)
+            using num = typename std::conditional<sizeof(typename P::word) == 8, long long, int>::type;
+            num sum_all;
+            if constexpr (sizeof(typename P::word) == 8)
+                sum_all = wave_sum64((long long)sum_in);
+            else
+                sum_all = wave_sum(sum_in);
             // C[v] = #{indeg >= v}: lane v holds it while every value is
             // below 64, else a table
             int V = 0, creg = 0;
@@ -1438,7 +1473,33 @@ __device__ __attribute__((always_inline)) bool wide_bounds(Ctx& c, Wide<P>& z, i
                 const typename P::word w = z.cw[i];
                 return !sub || wide_valid<P>(c, tb0, ub0, m, w) ? P::in(w) : 0;
             };
-            if (m < 16 && n > 2 * WAVE) {
+            if (m <= 4 && n > 2 * WAVE) {
+                // values 1 to 4, the first levels of a search: as below with
+                // one word a lane and two sums
+                int cnt[5] = {0, 0, 0, 0, 0};
+                for (int b0 = m; b0 < m + n; b0 += 255 * WAVE) {
+                    uint32_t acc = 0;
+                    const int b1 = min(m + n, b0 + 255 * WAVE);
+#pragma unroll 4
+                    for (int base = b0; base < b1; base += WAVE) {
+                        const int x = indeg(base + c.lane);
+                        acc += x ? 1u << (x * 8 - 8) : 0u;
+                    }
+                    const uint32_t f0 = (uint32_t)wave_sum((int)(acc & 0x00FF00FFu));
+                    const uint32_t f1 = (uint32_t)wave_sum((int)((acc >> 8) & 0x00FF00FFu));
+                    cnt[1] += (int)(f0 & 0xFFFFu);
+                    cnt[2] += (int)(f1 & 0xFFFFu);
+                    cnt[3] += (int)(f0 >> 16);
+                    cnt[4] += (int)(f1 >> 16);
+                }
+                int run = 0;
+#pragma unroll
+                for (int v = 4; v >= 1; v--) {
+                    run += cnt[v];
+                    if (run && V == 0) V = v;
+                    if (c.lane == v) creg = run;
+                }
+            } else if (m < 16 && n > 2 * WAVE) {
                 // values below 16: every lane counts its own in 8-bit fields
                 // (of at most 255 chunks at a time), then sums of 16- and
                 // 32-bit fields over the lanes
@@ -1505,7 +1566,7 @@ __device__ __attribute__((always_inline)) bool wide_bounds(Ctx& c, Wide<P>& z, i
             // first 64 on either side)
             auto holds = [&](int base) -> uint64_t {
                 const int idx = base + c.lane;
-                long long p = 0;
+                num p = 0;
                 if (reg) {
                     int q = 0;
                     for (int v = 1; v <= V; v++) q += min(rdlane(creg, v), idx);
@@ -1513,7 +1574,7 @@ __device__ __attribute__((always_inline)) bool wide_bounds(Ctx& c, Wide<P>& z, i
                 } else {
                     for (int v = 1; v <= V; v++) p += min((int)z.tab[v], idx);
                 }
-                return ballot(idx <= ub && idx >= lb && sum_all + p >= (long long)m * md(c, m + idx));
+                return ballot(idx <= ub && idx >= lb && sum_all + p >= (num)m * md(c, m + idx));
             };
             int first = -1, last = -1, base = lb & ~(WAVE - 1);
             uint64_t ok = 0;
@@ -1567,7 +1628,7 @@ __device__ __attribute__((always_inline)) bool wide_bounds(Ctx& c, Wide<P>& z, i
 }
 
 // |row(id) n L| for this lane's id against the vertices of L: lane k of
-// `ids` holds L's k-th vertex of the group, nl <= 64 of them (X: A1 or A2)
+// `ids` holds L's k-th vertex of the group, nl <= 64 of them (X: A1 or A2).
 __device__ __forceinline__ int wide_count(gptr<const uint64_t> X, int rw, int ids, int nl, int id) {
     const int wd = id >> 6, sh = id & 63;
     int n = 0, k = 0;
@@ -1580,6 +1641,46 @@ __device__ __forceinline__ int wide_count(gptr<const uint64_t> X, int rw, int id
     }
     for (; k < nl; k++) n += (int)((X[(size_t)rdlane(ids, k) * rw + wd] >> sh) & 1ull);
     return n;
+}
+// the same for four chunks of ids: 16 words in flight, where rows are long and
+// far apart (a recount of 700 candidates against each other on rows of 1,096
+// words took 4 ms a chunk at a time)
+struct Count4 {
+    int n0, n1, n2, n3;
+};
+__device__ __forceinline__ Count4 wide_count4(gptr<const uint64_t> X, int rw, int ids, int nl, int i0, int i1, int i2,
+                                              int i3) {
+    Count4 c{0, 0, 0, 0};
+    const int w0 = i0 >> 6, w1 = i1 >> 6, w2 = i2 >> 6, w3 = i3 >> 6;
+    auto bit = [](uint64_t x, int i) { return (int)((x >> (i & 63)) & 1ull); };
+    int k = 0;
+    for (; k + 4 <= nl; k += 4) {
+        uint64_t x[4][4];
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            gptr<const uint64_t> r = X + (size_t)rdlane(ids, k + q) * rw;
+            x[q][0] = r[w0];
+            x[q][1] = r[w1];
+            x[q][2] = r[w2];
+            x[q][3] = r[w3];
+        }
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            c.n0 += bit(x[q][0], i0);
+            c.n1 += bit(x[q][1], i1);
+            c.n2 += bit(x[q][2], i2);
+            c.n3 += bit(x[q][3], i3);
+        }
+    }
+    for (; k < nl; k++) {
+        gptr<const uint64_t> r = X + (size_t)rdlane(ids, k) * rw;
+        const uint64_t x0 = r[w0], x1 = r[w1], x2 = r[w2], x3 = r[w3];
+        c.n0 += bit(x0, i0);
+        c.n1 += bit(x1, i1);
+        c.n2 += bit(x2, i2);
+        c.n3 += bit(x3, i3);
+    }
+    return c;
 }
 // the same against a mask in LDS
 __device__ __forceinline__ int wide_rowpop(gptr<const uint64_t> X, int rw, const uint64_t* mask, int id) {
@@ -1620,6 +1721,48 @@ __device__ __attribute__((always_inline)) int wide_in_set(Ctx& c, Wide<P>& z, gp
         n += wide_count(X, z.rw, ids, min(nl - g, WAVE), id);
     }
     return n;
+}
+
+// |N n set| of places [0, n), place i's id = id_of(i), given to put(i, count).
+// (A task in LDS keeps its registers for the branch loop: one chunk at a time.)
+template <class P, class At, class Id, class Put>
+__device__ __attribute__((always_inline)) void wide_counts(Ctx& c, Wide<P>& z, bool mask, int nl, At at, int n, Id id_of,
+                                                           Put put) {
+    if (mask || !P::slab) {
+        for (int base = 0; base < n; base += WAVE) {
+            const int i = base + c.lane;
+            const int k = wide_in_set(c, z, z.A1, mask, nl, at, i < n ? id_of(i) : 0);
+            if (i < n) put(i, k);
+        }
+        return;
+    }
+    for (int base = 0; base < n; base += 4 * WAVE) {
+        int id[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const int i = base + u * WAVE + c.lane;
+            id[u] = i < n ? id_of(i) : 0;
+        }
+        int k[4] = {0, 0, 0, 0};
+        for (int g = 0; g < nl; g += WAVE) {
+            const int ids = g + c.lane < nl ? (int)at(g + c.lane) : 0;
+            const int gn = min(nl - g, WAVE);
+            if (n - base <= WAVE) {
+                k[0] += wide_count(z.A1, z.rw, ids, gn, id[0]);
+            } else {
+                const Count4 q = wide_count4(z.A1, z.rw, ids, gn, id[0], id[1], id[2], id[3]);
+                k[0] += q.n0;
+                k[1] += q.n1;
+                k[2] += q.n2;
+                k[3] += q.n3;
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const int i = base + u * WAVE + c.lane;
+            if (i < n) put(i, k[u]);
+        }
+    }
 }
 
 // Keeps the candidates [m, m + n) valid under (z.tb, z.ub1), in place; the
@@ -1674,10 +1817,12 @@ __device__ __attribute__((always_inline)) int wide_keep(Ctx& c, Wide<P>& z, int 
 // degree_pruning (main.cu:1735-1855): members [0, m), candidates [m, m + n),
 // nl removed ones on the list.  True: the record fails (n is then meaningless).
 // map_empty: the reference's id->position map holds no entry during this call
-// (critical-vertex pruning without critical-adjacent candidates).
+// (critical-vertex pruning without critical-adjacent candidates).  again: whether
+// the same call on what it leaves could end otherwise (the last bounds counted
+// fewer candidates than stay).
 template <class P>
 __device__ __attribute__((always_inline)) bool wide_prune(Ctx& c, Wide<P>& z, int m, int& n, int nl, bool map_empty, int& ub,
-                                                          int& lb, int& med) {
+                                                          int& lb, int& med, bool& again) {
     int nc = n;
     bool sub = false;
     int tb0 = 0, ub0 = 0;
@@ -1686,6 +1831,7 @@ __device__ __attribute__((always_inline)) bool wide_prune(Ctx& c, Wide<P>& z, in
         const bool fail = wide_bounds(c, z, m, n, nc, sub, tb0, ub0, ub, lb, med);
         ph_mark(c, PH_LU);
         if (fail) return true;
+        again = nc != n;
         if (sub) nl = 0;
         n = wide_keep(c, z, m, n, nl);
         lsync();
@@ -1703,29 +1849,22 @@ __device__ __attribute__((always_inline)) bool wide_prune(Ctx& c, Wide<P>& z, in
         tb0 = z.tb;
         ub0 = z.ub1;
         sub = true;
+        auto put = [&](int i, int k) {
+            const typename P::word w = z.cw[i];
+            z.cw[i] = P::set_ex(w, rc ? k : P::ex(w) - k);
+        };
+        if (!map_empty) {
+            wide_counts(c, z, mask, k, at, m + n, [&](int i) { return (int)z.pid[z.cpos[i]]; }, put);
+        } else if (rc) {
+            for (int i = c.lane; i < m + n; i += WAVE) z.cw[i] = P::set_ex(z.cw[i], 0);
+        }
+        lsync();
+        // indegrees of the candidates valid under the old bounds with the new
+        // exdeg (main.cu:1811-1815)
         nc = 0;
-        for (int base = 0; base < m + n; base += WAVE) {
+        for (int base = 0; base < n; base += WAVE) {
             const int i = base + c.lane;
-            bool ok = false;
-            typename P::word w = 0;
-            int id = 0;
-            if (i < m + n) {
-                w = z.cw[i];
-                id = (int)z.pid[z.cpos[i]];
-            }
-            if (!map_empty) {
-                const int cnt = wide_in_set(c, z, z.A1, mask, k, at, id);
-                w = P::set_ex(w, rc ? cnt : P::ex(w) - cnt);
-            } else if (rc) {
-                w = P::set_ex(w, 0);
-            }
-            if (i < m + n) {
-                z.cw[i] = w;
-                // indegrees of the candidates valid under the old bounds
-                // with the new exdeg (main.cu:1811-1815)
-                ok = i >= m && wide_valid<P>(c, tb0, ub0, m, w);
-            }
-            nc += __popcll(ballot(ok));
+            nc += __popcll(ballot(i < n && wide_valid<P>(c, tb0, ub0, m, z.cw[m + (i < n ? i : 0)])));
         }
         lsync();
         ph_mark(c, PH_DEGUPD);
@@ -1733,8 +1872,9 @@ __device__ __attribute__((always_inline)) bool wide_prune(Ctx& c, Wide<P>& z, in
 }
 
 // critical vertex pruning (main.cu:1526-1707) up to its closing degree pruning:
-// 2 when the record fails, else 0 with the candidates, the list and map_empty
-// as that pruning takes them.
+// 2 when the record fails, 1 when nothing changed (no critical-adjacent
+// candidates), else 0 with the candidates, the list and map_empty as that pruning
+// takes them.
 template <class P>
 __device__ __attribute__((always_inline)) int wide_critical(Ctx& c, Wide<P>& z, int& m, int& n, int& nl, int lb,
                                                             bool& map_empty) {
@@ -1757,7 +1897,7 @@ __device__ __attribute__((always_inline)) int wide_critical(Ctx& c, Wide<P>& z, 
     }
     nl = 0;
     map_empty = true;
-    if (ncm == 0) return 0;
+    if (ncm == 0) return 1;
     wadj_lanes(c, sw);
     lsync();
     // critical-adjacent candidates, moved to the front of the candidates: the
@@ -1773,7 +1913,7 @@ __device__ __attribute__((always_inline)) int wide_critical(Ctx& c, Wide<P>& z, 
         if (c.lane == 0) z.flag[base / WAVE] = bf;
         ncrit += __popcll(bf);
     }
-    if (ncrit == 0) return 0;
+    if (ncrit == 0) return 1;
     map_empty = false;
     lsync();
     int na = 0, nb = 0;
@@ -2175,12 +2315,8 @@ __device__ __attribute__((always_inline)) void wide_bulk_remove(Ctx& c, Wide<P>&
     if (nr <= 0) return;
     auto gone = [&](int q) { return z.pid[keep + q]; };
     const bool mask = wide_set(c, z, nr, gone);
-    for (int base = 0; base < keep; base += WAVE) {
-        const int i = base + c.lane;
-        const int id = i < keep ? (int)z.pid[i] : 0;
-        const int k = wide_in_set(c, z, z.A1, mask, nr, gone, id);
-        if (i < keep) z.pw[i] -= (typename P::word)k;
-    }
+    wide_counts(c, z, mask, nr, gone, keep, [&](int i) { return (int)z.pid[i]; },
+                [&](int i, int k) { z.pw[i] -= (typename P::word)k; });
     lsync();
 }
 
@@ -2390,12 +2526,12 @@ __device__ __attribute__((always_inline)) bool process_wide(Ctx& c, const TaskRe
             z.nbits = (uint64_t*)at;
             z.flag = z.nbits + T / 64;
         } else {
-            // WIDE_SLAB bytes a vertex
+            // (52 bytes a vertex, WideMid: 34)
             gptr<char> g = globw(slab);
             z.keys = (gptr<uint64_t>)g;
-            z.pw = z.keys + (size_t)2 * T;
-            z.cw = z.keys + (size_t)3 * T;
-            gptr<uint32_t> u = (gptr<uint32_t>)(z.keys + (size_t)4 * T);
+            z.pw = (typename P::wordp)(z.keys + (size_t)2 * T);
+            z.cw = z.pw + (size_t)T;
+            typename P::posp u = (typename P::posp)(z.cw + (size_t)T);
             z.pid = u;
             z.pl2 = u + (size_t)T;
             z.cpos = u + (size_t)2 * T;
@@ -2421,7 +2557,7 @@ __device__ __attribute__((always_inline)) bool process_wide(Ctx& c, const TaskRe
     int nm = 0, cov = 0;
     gptr<const Vrec> src = glob(a.in_verts + ref.off);
     // lvl2adj has to fit its field (an item of the root takes it from the whole root)
-    const uint32_t l2_max = P::slab ? 0xFFFFFFFFu : z.idb == 16 ? 0xFFFFu : 0xFFFu;
+    const uint32_t l2_max = sizeof(typename P::pos_t) == 4 ? 0xFFFFFFFFu : P::slab || z.idb == 16 ? 0xFFFFu : 0xFFFu;
     for (int base = 0; base < t0; base += P::U * WAVE) {
         typedef int v4 __attribute__((ext_vector_type(4)));
         v4 v[P::U];
@@ -2468,6 +2604,7 @@ __device__ __attribute__((always_inline)) bool process_wide(Ctx& c, const TaskRe
     z.d2r = glob(c.g.p->d2r);
     z.mdt = md(c, c.lane);
     z.mds = uni(md(c, c.g.min_size));
+    z.ubt = ub_quot(c, c.lane);
     lsync();
     ph_mark(c, PH_LOAD);
 
@@ -2717,16 +2854,21 @@ __device__ __attribute__((always_inline)) bool process_wide(Ctx& c, const TaskRe
         int ub = 0, lb = 0, med = 0;
         // degree pruning, then critical-vertex pruning, which ends in a
         // second degree pruning
-        bool first = true, map_empty = false, fails;
+        bool first = true, map_empty = false, fails, again = true;
         for (;;) {
-            fails = wide_prune(c, z, m, n, nl, map_empty, ub, lb, med);
+            fails = wide_prune(c, z, m, n, nl, map_empty, ub, lb, med, again);
             if (!first || fails) break;
             first = false;
-            if (wide_critical(c, z, m, n, nl, lb, map_empty) == 2) {
+            const int cr = wide_critical(c, z, m, n, nl, lb, map_empty);
+            if (cr == 2) {
                 m = -1;  // neither a clique test nor a child
                 break;
             }
             ph_mark(c, PH_CRIT);
+            // (most children: the closing degree pruning would end as the first
+            // one did, on the same degrees; with it the bounds were 37% of a
+            // co-expression window's time)
+            if (cr == 1 && !again) break;
         }
         if (m < 0) {
             ph_mark(c, PH_CRIT);
@@ -2753,11 +2895,127 @@ __device__ __forceinline__ bool wide_fits(const Ctx& c, uint32_t t, uint32_t lds
            wide_lds_bytes(t, (uint32_t)c.g.p->rw) <= lds_bytes;
 }
 
-// a task of any size and kind
+// What a task in the slab takes from the wave's state and changes in it.
+template <class T>
+using lptr = __attribute__((address_space(3))) T*;
+struct Far {
+    const ExpandArgs* a;
+    const DevGraph* g;
+    char* slab;
+    TaskRef ref;
+    long long slot, wadj_l, ph_t;
+    unsigned long long share_v;
+    lptr<char> lds;
+    lptr<LStats> st;
+    lptr<unsigned long long> ph, clq;
+    lptr<TaskRef> ptopref;
+    lptr<uint32_t> fl, fln;
+    uint32_t lds_bytes, inst, ptopi, pbot, ptop;
+    int shard, share_n, share_left;
+    bool share_ok, phase_on;
+};
+template <class T>
+__device__ __forceinline__ T* unip(T* p) {
+    return (T*)uni64((long long)p);
+}
+template <class T>
+__device__ __forceinline__ T* unil(lptr<T> p) {
+    return (T*)(lptr<T>)(uintptr_t)(uint32_t)uni32((int)(uint32_t)(uintptr_t)p);
+}
+// A function of its own: with its code inside the kernel the registers of both
+// forms of the branch loop did not fit (116 of them in memory, 25 without), and
+// the tasks in LDS paid for it, which are most.
+template <class P>
+__device__ __attribute__((noinline)) bool process_far(Far* f) {
+    Ctx c;
+    c.a = unip(f->a);
+    c.g = load_graph(unip(f->g));
+    c.lane = lane_id();
+    c.st = unil(f->st);
+    c.depth = 0;
+    c.inst = (uint32_t)uni32((int)f->inst);
+    c.slot = uni64(f->slot);
+    c.ph = unil(f->ph);
+    c.ph_t = uni64(f->ph_t);
+    c.wadj_l = f->wadj_l;
+    c.phase_on = uni32(f->phase_on) != 0;
+    c.keys = false;
+    c.shard = uni32(f->shard);
+    c.ptopref = unil(f->ptopref);
+    c.ptopi = (uint32_t)uni32((int)f->ptopi);
+    c.clq = unil(f->clq);
+    c.fl = unil(f->fl);
+    c.fln = unil(f->fln);
+    c.pstack = c.a->priv + (size_t)blockIdx.x * c.a->priv_cap;
+    c.pbkt = c.a->priv_bkt + (size_t)blockIdx.x * c.a->priv_cap;
+    c.pbot = (uint32_t)uni32((int)f->pbot);
+    c.ptop = (uint32_t)uni32((int)f->ptop);
+    c.share_v = f->share_v;
+    c.share_n = uni32(f->share_n);
+    c.share_left = uni32(f->share_left);
+    c.share_ok = uni32(f->share_ok) != 0;
+    const TaskRef r = bcast_ref(f->ref, 0);
+    const bool ok = process_wide<P>(c, r, unil(f->lds), (uint32_t)uni32((int)f->lds_bytes), unip(f->slab));
+    f->ph_t = c.ph_t;
+    f->wadj_l = c.wadj_l;
+    f->ptopi = c.ptopi;
+    f->pbot = c.pbot;
+    f->ptop = c.ptop;
+    f->share_v = c.share_v;
+    f->share_n = c.share_n;
+    f->share_left = c.share_left;
+    return ok;
+}
+
+// a task of any size and kind; FAR: the slab's forms are there (without them
+// every task fits the wave's LDS, see enumerate_persistent)
+template <bool FAR>
 __device__ __attribute__((always_inline)) void process_task(Ctx& c, const TaskRef& ref, char* lds, uint32_t lds_bytes,
                                                             char* slab) {
     if (wide_fits(c, ref.t, lds_bytes) && process_wide<WideLds>(c, ref, lds, lds_bytes, slab)) return;
-    process_wide<WideSlab>(c, ref, lds, lds_bytes, slab);
+    if constexpr (!FAR) {
+        if (c.lane == 0) atomicOr(c.a->error, 2);
+        return;
+    }
+    Far f;
+    f.a = c.a;
+    f.g = c.g.p;
+    f.slab = slab;
+    f.ref = ref;
+    f.slot = c.slot;
+    f.wadj_l = c.wadj_l;
+    f.ph_t = c.ph_t;
+    f.share_v = c.share_v;
+    f.lds = (lptr<char>)lds;
+    f.st = (lptr<LStats>)c.st;
+    f.ph = (lptr<unsigned long long>)c.ph;
+    f.clq = (lptr<unsigned long long>)c.clq;
+    f.ptopref = (lptr<TaskRef>)c.ptopref;
+    f.fl = (lptr<uint32_t>)c.fl;
+    f.fln = (lptr<uint32_t>)c.fln;
+    f.lds_bytes = lds_bytes;
+    f.inst = c.inst;
+    f.ptopi = c.ptopi;
+    f.pbot = c.pbot;
+    f.ptop = c.ptop;
+    f.shard = c.shard;
+    f.share_n = c.share_n;
+    f.share_left = c.share_left;
+    f.share_ok = c.share_ok;
+    f.phase_on = c.phase_on;
+    // (positions and indegrees of at most 12 bits, ids of 16; degrees that do
+    // not fit are found at load)
+    bool done = false;
+    if (ref.t <= WIDE_LDS_MAX && c.g.p->R <= WIDE_MID_R_MAX) done = process_far<WideMid>(&f);
+    if (!done) process_far<WideSlab>(&f);
+    c.wadj_l = f.wadj_l;
+    c.ph_t = uni64(f.ph_t);
+    c.ptopi = (uint32_t)uni32((int)f.ptopi);
+    c.pbot = (uint32_t)uni32((int)f.pbot);
+    c.ptop = (uint32_t)uni32((int)f.ptop);
+    c.share_v = f.share_v;
+    c.share_n = uni32(f.share_n);
+    c.share_left = uni32(f.share_left);
 }
 
 // ---------------------------------------------------------------------------
@@ -2823,7 +3081,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void ex
             y.cap = TINY_MAX;
             tiny_level(c, y, (uint32_t*)lds, s_dep);
         } else {
-            process_task(c, ref, lds, a.lds_bytes, slab);
+            process_task<true>(c, ref, lds, a.lds_bytes, slab);
         }
         wsync();
         if (a.static_sched) {
@@ -2866,6 +3124,7 @@ __device__ __attribute__((always_inline)) void release_record(Ctx& c, const Task
 // rings until the pending counter reaches zero
 // ---------------------------------------------------------------------------
 // (two resident waves per SIMD: the register allocation is held to 256)
+template <bool FAR>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void expand_persistent(
     const ExpandArgs* __restrict__ ap) {
     const ExpandArgs& a = *ap;
@@ -3162,7 +3421,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void ex
         if (ref.t > a.slab_tcap) {
             if (c.lane == 0) atomicOr(a.error, 2);
         } else {
-            process_task(c, ref, lds, a.lds_bytes, slab);
+            process_task<FAR>(c, ref, lds, a.lds_bytes, slab);
         }
         wsync();
         if (a.timeline && gslot >= 0) timeline_row(c, ref, gslot, tl_start);
@@ -3178,5 +3437,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void ex
     else
         flush_stats(c);
 }
+
+template __global__ void expand_persistent<false>(const ExpandArgs* __restrict__);
+template __global__ void expand_persistent<true>(const ExpandArgs* __restrict__);
 
 }  // namespace qcdev

@@ -21,7 +21,10 @@
 #include "qc_internal.h"
 
 namespace qcdev {
+template <bool FAR>
 __global__ void expand_persistent(const ExpandArgs*);
+extern template __global__ void expand_persistent<false>(const ExpandArgs*);
+extern template __global__ void expand_persistent<true>(const ExpandArgs*);
 
 // Queue state for a fresh run: the roots dealt over the nr rings (root i
 // at position i / nr of ring i mod nr, published), every other cell free for
@@ -136,7 +139,6 @@ int enumerate_persistent(const Instance* const* insts, const qc_params* params, 
         set_error("static scheduling deals ring positions to the waves in turn; cost order needs dynamic scheduling");
         return QC_EINVAL;
     }
-    const void* kern = (const void*)qcdev::expand_persistent;
 
     // roots and per-instance tables
     std::vector<TaskRef> roots;
@@ -178,6 +180,14 @@ int enumerate_persistent(const Instance* const* insts, const qc_params* params, 
     }
     if (roots.empty()) return QC_OK;
 
+    // Where the largest root fits the LDS that every wave has, the kernel without
+    // the slab's forms: the calls to those, though never made, cost the others
+    // registers (a full search of 1.86 million tasks 13.3 against 11.4 ms, 3,051
+    // tasks 1.05 against 0.85; where they are needed, the first branches of a
+    // power-law graph take 146 ms with the calls and 160 with the code in place).
+    const bool far = maxR > WIDE_TASK_MAX || wide_lds_bytes((uint32_t)maxR, (uint32_t)maxrw) > MIN_WAVE_LDS;
+    const void* kern = far ? (const void*)qcdev::expand_persistent<true> : (const void*)qcdev::expand_persistent<false>;
+
     int dev = 0, n_cu = 0, per_cu = 0;
     QC_HIP(hipGetDevice(&dev));
     QC_HIP(hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, dev));
@@ -189,7 +199,7 @@ int enumerate_persistent(const Instance* const* insts, const qc_params* params, 
     // LDS.
     const int wide_req = p.lds_wide < 0 ? 0 : (p.lds_wide > 0 ? (int)p.lds_wide : 512);
     const uint32_t wide = (uint32_t)std::min(std::min(wide_req, 1024), maxR);
-    size_t lds_b = std::max<size_t>((size_t)64 * 256, wide_lds_bytes(wide, (uint32_t)maxrw));
+    size_t lds_b = std::max<size_t>(MIN_WAVE_LDS, wide_lds_bytes(wide, (uint32_t)maxrw));
     QC_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, 64, lds_b));
     {
         // A workgroup's LDS (static + dynamic) is allocated in granules of

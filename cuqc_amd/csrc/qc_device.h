@@ -51,6 +51,10 @@ __host__ __device__ __attribute__((always_inline)) constexpr uint32_t wide_T(uin
 __host__ __device__ __attribute__((always_inline)) constexpr uint32_t wide_lds_bytes(uint32_t t, uint32_t rw) {
     return 20u * wide_T(t) + wide_T(t) / 4u + (rw <= 256u ? 24u * rw : 0u);
 }
+// dynamic LDS of a persistent wave, at least (64 words for each of the 64 children
+// of a task in registers)
+constexpr size_t MIN_WAVE_LDS = 64 * 256;
+constexpr int WIDE_TASK_MAX = 4095;  // tasks in LDS: positions and indegrees of 12 bits
 // HBM slab bytes of a task of t vertices (52 a vertex, and the masks)
 __host__ __device__ __attribute__((always_inline)) constexpr size_t wide_slab_bytes(uint32_t t) {
     return ((size_t)52 * wide_T(t) + wide_T(t) / 4u + 255) & ~(size_t)255;
@@ -114,14 +118,12 @@ struct DevStats {
 
 // Graph tables on the device: root-space 1-hop / 2-hop bit matrices
 // (row a, bit b set iff b in N(a) / N2(a); rows of `rw` 64-bit words),
-// the integer tables and the id translation.
+// and the id translation.
 struct DevGraph {
     int32_t R;            // root vertices
     int32_t rw;           // words per root-space row
     const uint64_t* A1;   // R x rw
     const uint64_t* A2;   // R x rw
-    const int32_t* ubq;
-    int32_t ubq_n;
     int32_t min_size;
     int32_t pad;
     const uint32_t* orig; // root-local id -> input vertex id

@@ -182,11 +182,10 @@ struct Instance {
     int32_t min_size = 0;
     std::vector<Vrec> root;           // root task record (root-local ids)
     std::vector<uint32_t> orig;       // root-local -> input id
-    std::vector<int32_t> ubq;         // floor(d / gamma) for total degrees d
     std::vector<int32_t> d2r;         // |N2(a) n root|
     uint64_t root_bound = 0;          // children slot bound of the root task
     uint64_t root_branches = 0;       // branches of the root task
-    DBuf A1, A2, d_ubq, d_orig, d_d2r, d_d1r;
+    DBuf A1, A2, d_orig, d_d2r, d_d1r;
     DevGraph dg{};
 };
 

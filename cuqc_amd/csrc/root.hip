@@ -764,9 +764,6 @@ int build_instance_impl(const qc_graph* g, double gamma, int ms, Instance& I, hi
     I.R = R;
     I.rw = (R + 63) / 64;
     if (R == 0) return QC_OK;
-    // (the total degree of a member, which indexes the table, is below R)
-    I.ubq.resize((size_t)R + 2);
-    for (int d = 0; d < R + 2; d++) I.ubq[d] = (int32_t)std::floor((double)d / gamma);
 
     // ---- device tables ----
     const size_t mat_bytes = (size_t)R * I.rw * 8;
@@ -855,8 +852,6 @@ int build_instance_impl(const qc_graph* g, double gamma, int ms, Instance& I, hi
     QC_HIP(hipMemcpyAsync(I.d2r.data(), I.d_d2r.p, (size_t)R * 4, hipMemcpyDeviceToHost, s));
     std::vector<int32_t> n2(R);
     QC_HIP(hipMemcpyAsync(n2.data(), d_n2.p, (size_t)R * 4, hipMemcpyDeviceToHost, s));
-    if ((rc = I.d_ubq.alloc(I.ubq.size() * 4))) return rc;
-    QC_HIP(hipMemcpyAsync(I.d_ubq.p, I.ubq.data(), I.ubq.size() * 4, hipMemcpyHostToDevice, s));
     QC_HIP(hipStreamSynchronize(s));
     if (phases) {
         const auto t_dev = std::chrono::steady_clock::now();
@@ -900,8 +895,6 @@ int build_instance_impl(const qc_graph* g, double gamma, int ms, Instance& I, hi
     I.dg.rw = I.rw;
     I.dg.A1 = I.A1.as<uint64_t>();
     I.dg.A2 = I.A2.as<uint64_t>();
-    I.dg.ubq = I.d_ubq.as<int32_t>();
-    I.dg.ubq_n = (int32_t)I.ubq.size();
     I.dg.min_size = ms;
     I.dg.gamma = gamma;
     I.dg.orig = I.d_orig.as<uint32_t>();
