@@ -12,7 +12,8 @@
 // Refs that a wave took and did not use (inst CLQ_NONE) sort last.
 //   1. key = inst << 40 | off per ref, radix sort of (key, ref index);
 //   2. set lengths in that order, exclusive scan -> output offsets;
-//   3. one thread per set copies its vertices to its output offset.
+//   3. the vertices are gathered in that order, straight into the host's block
+//      when it is pinned.
 
 #include <cstring>
 
@@ -45,14 +46,39 @@ __global__ void rc_lens(const CliqueRef* __restrict__ refs, const uint32_t* __re
     if (j == k) lens[k] = 0;
 }
 
-__global__ __launch_bounds__(256) void rc_gather(const CliqueRef* __restrict__ sets, const uint64_t* __restrict__ oo,
-                                                 uint64_t k, const uint32_t* __restrict__ v,
-                                                 uint32_t* __restrict__ out) {
-    const uint64_t j = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x;
-    if (j >= k) return;
-    const CliqueRef r = sets[j];
-    const uint64_t o = oo[j];
-    for (uint32_t t = 0; t < r.len; t++) out[o + t] = v[r.off + t];
+// 256 consecutive sets a workgroup; its threads take the places of their output
+// one after another (reads and writes of neighbouring words), each finding its
+// set among the offsets in LDS.  `out` may be host memory: the link's rate
+// bounds the kernel then (57 GB/s; 194 MB of a full search 3.4 ms, against
+// 1.2 for a thread per set into a device buffer, 3.4 for the copy and 0.4 for
+// the buffer).
+constexpr int RC_SETS = 256;
+__global__ __launch_bounds__(RC_SETS) void rc_gather(const CliqueRef* __restrict__ sets, const uint64_t* __restrict__ oo,
+                                                     uint64_t k, const uint32_t* __restrict__ v, uint32_t* out) {
+    __shared__ uint32_t at[RC_SETS + 1];
+    __shared__ uint64_t from[RC_SETS];
+    const uint64_t j0 = (uint64_t)blockIdx.x * RC_SETS;
+    const int n = (int)min((uint64_t)RC_SETS, k - j0);
+    const uint64_t o0 = oo[j0];
+    const int t = threadIdx.x;
+    if (t < n) {
+        from[t] = sets[j0 + t].off;
+        at[t] = (uint32_t)(oo[j0 + t] - o0);
+    }
+    if (t == 0) at[n] = (uint32_t)(oo[j0 + n] - o0);
+    __syncthreads();
+    const uint32_t total = at[n];
+    for (uint32_t p = t; p < total; p += RC_SETS) {
+        int lo = 0, hi = n;  // at[lo] <= p < at[hi]
+        while (hi - lo > 1) {
+            const int mid = (lo + hi) >> 1;
+            if (at[mid] <= p)
+                lo = mid;
+            else
+                hi = mid;
+        }
+        out[o0 + p] = v[from[lo] + (p - at[lo])];
+    }
 }
 
 }  // namespace qcdev
@@ -88,7 +114,7 @@ int collect_raw(const CliqueRef* d_refs, uint64_t taken, const uint32_t* d_verts
     int rc;
     if ((rc = keys.alloc(taken * 8, s)) || (rc = skeys.alloc(taken * 8, s)) || (rc = idx.alloc(taken * 4, s)) ||
         (rc = sidx.alloc(taken * 4, s)) || (rc = lens.alloc((k + 1) * 8, s)) || (rc = oo.alloc((k + 1) * 8, s)) ||
-        (rc = sets.alloc(k * sizeof(CliqueRef), s)) || (rc = out.alloc(std::max<uint64_t>(nv, 1) * 4, s)) ||
+        (rc = sets.alloc(k * sizeof(CliqueRef), s)) ||
         (rc = temp.alloc(std::max(sort_b, scan_b), s)))
         return rc;
     const unsigned nt = (unsigned)((taken + 255) / 256);
@@ -103,20 +129,32 @@ int collect_raw(const CliqueRef* d_refs, uint64_t taken, const uint32_t* d_verts
     QC_RC(hipGetLastError());
     QC_RC(rocprim::exclusive_scan(temp.p, scan_b, lens.as<uint64_t>(), oo.as<uint64_t>(), (uint64_t)0, (size_t)k + 1,
                                   rocprim::plus<uint64_t>(), s));
-    hipLaunchKernelGGL(qcdev::rc_gather, dim3(nb), dim3(256), 0, s, sets.as<CliqueRef>(), oo.as<uint64_t>(), k, d_verts,
-                       out.as<uint32_t>());
-    QC_RC(hipGetLastError());
     if ((rc = raw.off_buf.alloc((k + 1) * 8)) || (rc = raw.v_buf.alloc(std::max<uint64_t>(nv, 1) * 4))) return rc;
+    void* to = nullptr;
+    if (raw.v_buf.pinned && hipHostGetDevicePointer(&to, raw.v_buf.p, 0) != hipSuccess) {
+        (void)hipGetLastError();
+        to = nullptr;
+    }
+    if (!to && (rc = out.alloc(std::max<uint64_t>(nv, 1) * 4, s))) return rc;
     raw.k = k;
     raw.nv = nv;
     QC_RC(hipMemcpyAsync(raw.off_buf.p, oo.p, (k + 1) * 8, hipMemcpyDeviceToHost, s));
-    QC_RC(hipMemcpyAsync(raw.v_buf.p, out.p, nv * 4, hipMemcpyDeviceToHost, s));
-    QC_RC(hipStreamSynchronize(s));
-    if (raw.offp()[k] != nv) {
+    auto check = [&]() -> int {
+        if (raw.offp()[k] == nv) return QC_OK;
         set_error("raw set collection: the sets hold %llu vertex slots, the stream %llu",
                   (unsigned long long)raw.offp()[k], (unsigned long long)nv);
         return QC_EDEVICE;
+    };
+    if (to) {  // (looked at before anything is written to the host's block)
+        QC_RC(hipStreamSynchronize(s));
+        if ((rc = check())) return rc;
     }
+    hipLaunchKernelGGL(qcdev::rc_gather, dim3((unsigned)((k + qcdev::RC_SETS - 1) / qcdev::RC_SETS)), dim3(qcdev::RC_SETS),
+                       0, s, sets.as<CliqueRef>(), oo.as<uint64_t>(), k, d_verts, to ? (uint32_t*)to : out.as<uint32_t>());
+    QC_RC(hipGetLastError());
+    if (!to) QC_RC(hipMemcpyAsync(raw.v_buf.p, out.p, nv * 4, hipMemcpyDeviceToHost, s));
+    QC_RC(hipStreamSynchronize(s));
+    if ((rc = check())) return rc;
     return QC_OK;
 }
 

@@ -162,25 +162,23 @@ __global__ void nm_total(const uint32_t* __restrict__ pos, const uint32_t* __res
 
 __global__ void nm_count(const uint64_t* __restrict__ off, const uint32_t* __restrict__ v,
                          const uint32_t* __restrict__ uniq, const uint32_t* __restrict__ nu_p,
-                         uint32_t* __restrict__ cnt) {
+                         uint32_t* __restrict__ cnt, uint32_t* __restrict__ rank) {
     const uint32_t nu = *nu_p;
     for (uint32_t u = blockIdx.x; u < nu; u += gridDim.x) {
         uint32_t s = uniq[u];
-        for (uint64_t j = off[s] + threadIdx.x; j < off[s + 1]; j += blockDim.x) atomicAdd(&cnt[v[j]], 1u);
+        for (uint64_t j = off[s] + threadIdx.x; j < off[s + 1]; j += blockDim.x) rank[j] = atomicAdd(&cnt[v[j]], 1u);
     }
 }
 
 __global__ void nm_scatter(const uint64_t* __restrict__ off, const uint32_t* __restrict__ v,
                            const uint32_t* __restrict__ uniq, const uint32_t* __restrict__ nu_p,
-                           const uint32_t* __restrict__ start, uint32_t* __restrict__ cursor,
+                           const uint32_t* __restrict__ start, const uint32_t* __restrict__ rank,
                            uint32_t* __restrict__ post) {
     const uint32_t nu = *nu_p;
     for (uint32_t u = blockIdx.x; u < nu; u += gridDim.x) {
         uint32_t s = uniq[u];
         for (uint64_t j = off[s] + threadIdx.x; j < off[s + 1]; j += blockDim.x) {
-            uint32_t x = v[j];
-            uint32_t at = atomicAdd(&cursor[x], 1u);
-            post[start[x] + at] = s;
+            post[start[v[j]] + rank[j]] = s;
         }
     }
 }
@@ -692,17 +690,16 @@ int nonmax_run(const NmInput& in, char* scr, size_t scr_bytes, const NmOutput& o
 
     // 3. inverted index
     hipLaunchKernelGGL(qcdev::nm_fill<uint32_t>, dim3(gn), dim3(256), 0, s, U32(P.cnt), (uint64_t)nkeys, 0u);
-    hipLaunchKernelGGL(qcdev::nm_fill<uint32_t>, dim3(gn), dim3(256), 0, s, U32(P.cur), (uint64_t)nkeys, 0u);
-    hipLaunchKernelGGL(qcdev::nm_count, dim3(gw), dim3(64), 0, s, off, keys, U32(P.uniq), nu_p, U32(P.cnt));
+    hipLaunchKernelGGL(qcdev::nm_count, dim3(gw), dim3(64), 0, s, off, keys, U32(P.uniq), nu_p, U32(P.cnt),
+                       U32(P.pkey));
     QC_HIP(hipGetLastError());
     tb = P.temp_bytes;
     QC_RP(rocprim::exclusive_scan(temp, tb, U32(P.cnt), U32(P.start), 0u, (size_t)nkeys, rocprim::plus<uint32_t>(),
                                   s));
     hipLaunchKernelGGL(qcdev::nm_scatter, dim3(gw), dim3(64), 0, s, off, keys, U32(P.uniq), nu_p, U32(P.start),
-                       U32(P.cur), U32(P.post));
+                       U32(P.pkey), U32(P.post));
     QC_HIP(hipGetLastError());
-    // every postings list: largest sets first (the cursor array is free
-    // again and takes the segment ends)
+    // every postings list: largest sets first (P.cur takes the segment ends)
     const unsigned gv = (unsigned)std::min<uint64_t>((std::max<uint64_t>(nv, nkeys) + 255) / 256, 16384);
     hipLaunchKernelGGL(qcdev::nm_post_keys, dim3(gv), dim3(256), 0, s, off, U32(P.post), U32(P.start), U32(P.cnt),
                        nkeys, nv, U32(P.pkey), U32(P.cur));
