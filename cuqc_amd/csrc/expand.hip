@@ -1319,8 +1319,10 @@ struct WideWord {
 struct WideLds : WideWord<uint32_t, 20, 1 << 17, 1 << 16> {
     static constexpr bool slab = false;
     static constexpr int U = 2;  // chunks of 64 in flight
+    static constexpr bool cw_lds = true;
     using u32p = uint32_t*;
     using wordp = uint32_t*;
+    using cwordp = uint32_t*;
     using posp = uint16_t*;
     using pos_t = uint16_t;
     using keyp = uint64_t*;
@@ -1329,7 +1331,9 @@ struct WideSlab : WideWord<uint64_t, 32, 1 << 30, 1 << 29> {
     static constexpr bool slab = true;
     static constexpr int U = 4;
     using u32p = gptr<uint32_t>;
+    static constexpr bool cw_lds = false;
     using wordp = gptr<uint64_t>;
+    using cwordp = gptr<uint64_t>;
     using posp = gptr<uint32_t>;
     using pos_t = uint32_t;
     using keyp = gptr<uint64_t>;
@@ -1341,11 +1345,19 @@ struct WideSlab : WideWord<uint64_t, 32, 1 << 30, 1 << 29> {
 struct WideMid : WideWord<uint32_t, 20, 1 << 17, 1 << 16> {
     static constexpr bool slab = true;
     static constexpr int U = 4;
+    static constexpr bool cw_lds = false;
     using u32p = gptr<uint16_t>;
     using wordp = gptr<uint32_t>;
+    using cwordp = gptr<uint32_t>;
     using posp = gptr<uint16_t>;
     using pos_t = uint16_t;
     using keyp = gptr<uint64_t>;
+};
+// the same with the child's words in LDS, which every pass over the child's
+// candidates reads: up to 3,200 vertices with 20 KB a wave
+struct WideMidLds : WideMid {
+    static constexpr bool cw_lds = true;
+    using cwordp = uint32_t*;
 };
 constexpr int WIDE_MID_R_MAX = 1 << 16;
 
@@ -1364,7 +1376,7 @@ struct Wide {
     typename P::wordp pw;   //         indeg / exdeg word
     typename P::posp pl2;   //         lvl2adj
     typename P::posp cpos;  // child: position in the parent
-    typename P::wordp cw;   //        word
+    typename P::cwordp cw;  //        word
     typename P::posp list;  // positions (parent) of removed candidates, and other short lists (T entries)
     typename P::posp tab;   // counts per indegree (T entries)
     typename P::keyp keys;  // sort keys (WideLds: in the place of cw, list and tab; WideSlab: 2 T entries)
@@ -1697,6 +1709,54 @@ __device__ __forceinline__ int wide_rowpop(gptr<const uint64_t> X, int rw, const
     return s;
 }
 
+// the same for 64 rows, 8 at a time: the lanes share a row's words (a lane on its
+// own row touches 64 lines with every load, which the L1 does not keep until
+// the row's next words are read).  Sums of two rows share a word (R <= 16,384).
+// For the slab's tasks: one in LDS has no registers to spare for it, and gained
+// nothing.
+__device__ __forceinline__ int wide_rowpop_shared(const Ctx& c, gptr<const uint64_t> X, int rw, const uint64_t* mask, int id) {
+    int out = 0;
+#pragma unroll 1
+    for (int g = 0; g < 8; g++) {
+        uint32_t s[4] = {0, 0, 0, 0};
+        gptr<const uint64_t> r[8];
+#pragma unroll
+        for (int k = 0; k < 8; k++) r[k] = X + (size_t)rdlane(id, g * 8 + k) * rw;
+#pragma unroll 2
+        for (int w0 = 0; w0 < rw; w0 += WAVE) {
+            const int wd = w0 + c.lane;
+            uint64_t x[8];
+            uint64_t mk = 0;
+            if (wd < rw) mk = mask[wd];
+#pragma unroll
+            for (int k = 0; k < 8; k++) {
+                x[k] = 0;
+                if (wd < rw) x[k] = r[k][wd];
+            }
+#pragma unroll
+            for (int k = 0; k < 8; k++) s[k >> 1] += (uint32_t)__popcll(x[k] & mk) << (16 * (k & 1));
+        }
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            int v = (int)s[k];
+            v += dpp32<0xb1, 0xf>(0, v);
+            v += dpp32<0x4e, 0xf>(0, v);
+            v += dpp32<0x141, 0xf>(0, v);
+            v += dpp32<0x140, 0xf>(0, v);
+            s[k] = (uint32_t)v;
+        }
+        // lane l takes row l & 7 of the group
+        const int q = (c.lane >> 1) & 3;
+        uint32_t t = q == 0 ? s[0] : q == 1 ? s[1] : q == 2 ? s[2] : s[3];
+        t += (uint32_t)__shfl_xor((int)t, 16, WAVE);
+        t += (uint32_t)__shfl_xor((int)t, 32, WAVE);
+        const int v = (int)((c.lane & 1) ? t >> 16 : t & 0xFFFFu);
+        if ((c.lane >> 3) == g) out = v;
+    }
+    return out;
+}
+constexpr int WIDE_SHARED_MIN = 48;  // row words from which rows are shared (below, most lanes have no word)
+
 // A set of nl vertices, vertex k = at(k): counts by its rows, or by a mask of
 // it when it has more than two vertices per row word (a lane then reads its own
 // row, 64 rows at once, instead of the same words of one row).
@@ -1714,6 +1774,7 @@ __device__ __attribute__((always_inline)) bool wide_set(Ctx& c, Wide<P>& z, int 
 template <class P, class At>
 __device__ __attribute__((always_inline)) int wide_in_set(Ctx& c, Wide<P>& z, gptr<const uint64_t> X, bool mask, int nl,
                                                           At at, int id) {
+    if (mask && P::slab && z.rl && z.rw >= WIDE_SHARED_MIN) return wide_rowpop_shared(c, X, z.rw, z.lmask, id);
     if (mask) return wide_rowpop(X, z.rw, z.lmask, id);
     int n = 0;
     for (int g = 0; g < nl; g += WAVE) {
@@ -2422,9 +2483,14 @@ __device__ __attribute__((always_inline)) void wide_split(Ctx& c, Wide<P>& z, co
     // item boundaries balance the work rather than the branch count:
     // branch b builds a child from about t0 - b vertices, so with
     // S(b) = sum of (t0 - x) over x in [bbeg, b), boundary j is the first
-    // b with S(b) >= j S(hi) / n_items (kept strictly increasing)
+    // b with S(b) >= j S(hi) / n_items (kept strictly increasing).  At the
+    // window's last level the children are not written, and a branch costs about
+    // the same wherever it starts: items of equal counts (first branches of
+    // a power-law graph 133 -> 125 ms; with equal counts on every level a
+    // cost-ordered co-expression window took 19.5 ms instead of 17.0).
     const long long t0l = t0;
-    auto S = [&](long long b) { return (b - bbeg) * t0l - (b * (b - 1) - (long long)bbeg * (bbeg - 1)) / 2; };
+    const long long fall = c.keys ? 1 : 0;
+    auto S = [&](long long b) { return (b - bbeg) * t0l - fall * ((b * (b - 1) - (long long)bbeg * (bbeg - 1)) / 2); };
     const long long s_tot = S(hi);
     auto boundary = [&](int j) -> int {
         if (j <= 0) return bbeg;
@@ -2530,8 +2596,13 @@ __device__ __attribute__((always_inline)) bool process_wide(Ctx& c, const TaskRe
             gptr<char> g = globw(slab);
             z.keys = (gptr<uint64_t>)g;
             z.pw = (typename P::wordp)(z.keys + (size_t)2 * T);
-            z.cw = z.pw + (size_t)T;
-            typename P::posp u = (typename P::posp)(z.cw + (size_t)T);
+            if constexpr (P::cw_lds) {
+                z.cw = (uint32_t*)at;
+                at += 4 * T;
+            } else {
+                z.cw = z.pw + (size_t)T;
+            }
+            typename P::posp u = (typename P::posp)(z.pw + (size_t)2 * T);
             z.pid = u;
             z.pl2 = u + (size_t)T;
             z.cpos = u + (size_t)2 * T;
@@ -3006,7 +3077,14 @@ __device__ __attribute__((always_inline)) void process_task(Ctx& c, const TaskRe
     // (positions and indegrees of at most 12 bits, ids of 16; degrees that do
     // not fit are found at load)
     bool done = false;
-    if (ref.t <= WIDE_LDS_MAX && c.g.p->R <= WIDE_MID_R_MAX) done = process_far<WideMid>(&f);
+    if (ref.t <= WIDE_LDS_MAX && c.g.p->R <= WIDE_MID_R_MAX) {
+        const uint32_t rw = (uint32_t)c.g.p->rw, T = wide_T(ref.t);
+        // (rows, the child's words, the masks, and the radix sort's counters)
+        if ((wide_rows_staged(rw, lds_bytes) ? 24u * rw : 0u) + 4u * T + T / 4u + 1024u <= lds_bytes)
+            done = process_far<WideMidLds>(&f);
+        else
+            done = process_far<WideMid>(&f);
+    }
     if (!done) process_far<WideSlab>(&f);
     c.wadj_l = f.wadj_l;
     c.ph_t = uni64(f.ph_t);
