@@ -6,16 +6,15 @@ the schedule is a runtime choice and this module picks it per workload by
 timing candidate schedules on the workload itself (or on a sample window of
 it):
 
-* ``lds_tile``    tasks up to this many vertices run from LDS (64/128/256);
+* ``lds_tile``    tasks above this many vertices count as large (64/128/256);
 * ``split_chunk`` branch-range work items of this many branches (-1: never
                   split);
 * ``split_min``   split only tasks above this many vertices (0: the library
                   default, the LDS tile for a single graph and 512 for a
                   batch; values below the LDS tile mean the tile);
-* ``mid_tile``    tasks above the LDS tile and up to this size build task-local
-                  bit matrices in HBM (0: none, read the root matrices);
-* ``lds_wide``    tasks above the LDS tile and up to this size keep their
-                  per-vertex arrays in LDS (-1: none, 0: 512);
+* ``mid_tile``    accepted by the library, without effect;
+* ``lds_wide``    the LDS of a wave holds tasks of up to this size at least
+                  (-1: what 16 KB hold, 0: 512);
 * ``workgroups``  resident waves of the persistent launch (0: as many as fit).
 
 The search is coordinate descent from the library defaults, one parameter at

@@ -108,8 +108,10 @@ int enumerate_plain(const Instance& I, const qc_params& p, EnumOut& out, hipStre
     };
     const size_t refs_at = (sizeof(Launch) + 63) & ~(size_t)63;
     if ((rc = d_launch.alloc(refs_at + (size_t)max_batch * sizeof(TaskRef)))) return rc;
-    std::vector<char> launch(refs_at + (size_t)max_batch * sizeof(TaskRef));
-    Launch* const L = (Launch*)launch.data();
+    std::vector<char> launch_mem(refs_at + (size_t)max_batch * sizeof(TaskRef) + alignof(Launch));
+    char* const launch =
+        (char*)(((uintptr_t)launch_mem.data() + alignof(Launch) - 1) & ~(uintptr_t)(alignof(Launch) - 1));
+    Launch* const L = (Launch*)launch;
     Launch* const dL = d_launch.as<Launch>();
     LevelState done{};  // counters after the last launch
     QC_HIP(hipMemsetAsync(d_stats.p, 0, sizeof(DevStats), s));
@@ -271,8 +273,8 @@ int enumerate_plain(const Instance& I, const qc_params& p, EnumOut& out, hipStre
         A.split_chunk = split && k == 1 ? (int)std::max<uint64_t>(1, std::min<uint64_t>((uint64_t)split, branches / n_slabs)) : 0;
         L->st = LevelState{{{0, 0}, {0, 0}}, done.clq, 0, 0};
         L->a = A;
-        memcpy(launch.data() + refs_at, batch.data(), take * sizeof(TaskRef));
-        QC_HIP(hipMemcpyAsync(d_launch.p, launch.data(), refs_at + take * sizeof(TaskRef), hipMemcpyHostToDevice, s));
+        memcpy(launch + refs_at, batch.data(), take * sizeof(TaskRef));
+        QC_HIP(hipMemcpyAsync(d_launch.p, launch, refs_at + take * sizeof(TaskRef), hipMemcpyHostToDevice, s));
         if (!fixed) QC_HIP(hipMemcpyAsync(d_keep.p, d_stats.p, sizeof(DevStats), hipMemcpyDeviceToDevice, s));
         QC_HIP(hipEventRecord(e0, s));
         const uint32_t grid = std::min<uint32_t>((uint32_t)take, k == 1 ? n_slabs : small_grid_max);

@@ -3474,8 +3474,6 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void ex
         }
         c.slot = ref.b1 > 0 ? (long long)ref.bound : gslot;
         c.share_ok = ref.t >= SHARE_MIN_T;
-        // workspace: LDS with local matrices, LDS arrays with root
-        // matrices, slab with local matrices, or slab in root space
         // A task that fits one vertex a lane runs with its whole subtree in
         // registers.  64 is the width of a wave and of a mask in scalar
         // registers; split items (prepared records) and the root (labels

@@ -95,10 +95,13 @@ constexpr uint32_t CLQ_NONE = 0xFFFFFFFFu;
 // most tasks of at most 64 vertices a wave keeps in its dynamic LDS
 constexpr uint32_t TINY_STACK_MAX = 256;
 
-// Counters of one output stream (children or cliques).
-struct StreamCtr {
-    unsigned long long items;   // records
-    unsigned long long slots;   // vertex slots
+// Counters of one output stream (children or cliques).  Every counter that the
+// waves add to has a cache line of its own: the L2 takes the atomics of one line
+// one after another (a level-synchronous launch's seven counters on one line
+// made its deep levels of small tasks twice as long).
+struct alignas(256) StreamCtr {
+    unsigned long long items;               // records
+    alignas(128) unsigned long long slots;  // vertex slots
 };
 
 // Counters of one level-synchronous launch, set and read with one copy each
@@ -106,8 +109,8 @@ struct StreamCtr {
 struct LevelState {
     StreamCtr out[2];
     StreamCtr clq;
-    unsigned int next_task;
-    int error;
+    alignas(128) unsigned int next_task;
+    alignas(128) int error;
 };
 
 // Per-call statistics accumulated by the kernels.
@@ -248,7 +251,7 @@ struct ExpandArgs {
 };
 
 enum PhaseId {
-    PH_LOAD = 0,      // record load and local matrices
+    PH_LOAD = 0,      // record load (of a subtree in registers: its matrices too)
     PH_LOOKAHEAD,     // lookahead
     PH_REMOVE,        // remove_one_vertex steps and item catch-up
     PH_ADD,           // add_one_vertex and diameter pruning

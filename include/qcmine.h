@@ -57,9 +57,11 @@ typedef struct qc_params {
     int32_t mode;            /* qc_mode */
     int32_t order;           /* qc_order */
     int32_t workgroups;      /* 0 = auto (persistent: CUs x occupancy) */
-    int32_t lds_tile;        /* largest task (vertices) staged in LDS; 0 = auto */
-    int32_t split_chunk;     /* persistent mode: branches per work item when a task above
-                                split_min is split across waves; 0 = 64, < 0 = never split */
+    int32_t lds_tile;        /* 64, 128 or 256: tasks above it count as large; the default of
+                                split_min for a single graph; 0 = auto */
+    int32_t split_chunk;     /* branches per work item, at most, when a task above split_min is
+                                split across waves (plain mode: unless a capacity is fixed);
+                                0 = 64, < 0 = never split */
     int32_t max_depth;       /* search window: expand tasks of depth <= max_depth; <= 0: all */
     uint64_t task_capacity;  /* vertex slots per task pool; 0 = auto */
     uint64_t clique_capacity;/* raw-clique vertex slots; 0 = auto */
@@ -71,14 +73,11 @@ typedef struct qc_params {
                                 require identical counters from every replay; <= 1: once */
     int32_t trace;           /* persistent mode: record the cost-model features of every expanded
                                 task and its subtree size (qc_result_trace) */
-    int32_t split_min;       /* persistent mode: split only tasks above this many vertices (and
-                                above the LDS tile); 0 = the LDS tile for a single graph, 512 for
-                                a batch */
-    int32_t mid_tile;        /* persistent mode: tasks above the LDS tile and up to this size
-                                (<= 4096) build task-local bit matrices in HBM; <= 0 = none (read
-                                the root matrices) */
-    int32_t lds_wide;        /* persistent mode: tasks above the LDS tile and up to this size
-                                (<= 1024) keep their per-vertex arrays in LDS; 0 = 512, < 0 = none */
+    int32_t split_min;       /* split only tasks above this many vertices (and above lds_tile);
+                                0 = lds_tile for a single graph, 512 for a batch */
+    int32_t mid_tile;        /* accepted; has no effect */
+    int32_t lds_wide;        /* persistent mode: the LDS of a wave holds tasks of up to this size
+                                (<= 1024) at least; 0 = 512, < 0 = what 16 KB hold */
 } qc_params;
 
 typedef struct qc_stats {
