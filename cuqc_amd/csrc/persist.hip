@@ -29,7 +29,7 @@ extern template __global__ void expand_persistent<true>(const ExpandArgs*);
 // Queue state for a fresh run: the roots dealt over the nr rings (root i
 // at position i / nr of ring i mod nr, published), every other cell free for
 // its first lap, the free lists empty, counters reset.  ctr = heads[nr],
-// tails[nr], pool top, hungry|pending, overflow, QSTRIDE words apart.  Root records sit at the start of the
+// tails[nr], pool top, hungry|pending, overflow, done, QSTRIDE words apart.  Root records sit at the start of the
 // pool; allocated blocks start at the next unit boundary.
 __global__ void persist_reset(const TaskRef* __restrict__ roots, uint32_t nroots, const Vrec* __restrict__ root_verts,
                               uint64_t root_slots, TaskRef* q_refs, unsigned long long* q_seq, uint64_t q_cap,
@@ -63,6 +63,7 @@ __global__ void persist_reset(const TaskRef* __restrict__ roots, uint32_t nroots
         ctr[2ull * nr * QSTRIDE] = (root_slots + POOL_UNIT - 1) / POOL_UNIT * POOL_UNIT;  // pool top
         ctr[(2ull * nr + 1) * QSTRIDE] = (uint64_t)n_waves << 32 | nroots;  // hungry: every wave, pending: the roots
         ctr[(2ull * nr + 2) * QSTRIDE] = 0;                      // overflow
+        ctr[(2ull * nr + 3) * QSTRIDE] = 0;                      // done
         clq_ctr->items = 0;
         clq_ctr->slots = 0;
         *stats = DevStats{0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
@@ -76,7 +77,7 @@ namespace qc {
 namespace {
 
 constexpr int Q_SHARDS = 8;             // rings in the dynamic order: one per XCD
-constexpr int NCTR = 2 * Q_SHARDS + 4;  // heads, tails, pool top, hungry|pending, overflow, one spare
+constexpr int NCTR = 2 * Q_SHARDS + 4;  // heads, tails, pool top, hungry|pending, overflow, done
 
 struct RunState {
     unsigned long long ctr[NCTR];
@@ -396,6 +397,7 @@ int enumerate_persistent(const Instance* const* insts, const qc_params* params, 
         A.q_tail = ctr + nr * QSTRIDE;
         A.pool_top = ctr + 2 * nr * QSTRIDE;
         A.pending = ctr + (2 * nr + 1) * QSTRIDE;
+        A.done = ctr + (2 * nr + 3) * QSTRIDE;
         A.overflow = ctr + (2 * nr + 2) * QSTRIDE;
         A.lds_bytes = (uint32_t)lds_b;
         A.tiny_cap = tiny ? (uint32_t)std::min<size_t>(TINY_STACK_MAX, lds_b / 256) : 0u;

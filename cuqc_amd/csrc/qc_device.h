@@ -214,6 +214,7 @@ struct ExpandArgs {
     // none (they ask the busy ones to hand some over).  Both stay below 2^31
     // and never go negative: every decrement follows its increment.
     unsigned long long* pending;
+    unsigned long long* done;        // set once when the launch is finished (polled by idle waves)
     unsigned long long* overflow;    // pushes that found the ring and the private stack full
     // private stacks: wave w owns priv[w priv_cap, (w+1) priv_cap) (refs)
     // and priv_bkt[...] (each ref's predicted bucket);
