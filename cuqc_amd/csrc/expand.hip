@@ -2632,8 +2632,11 @@ __device__ __attribute__((always_inline)) bool process_wide(Ctx& c, const TaskRe
     bool bad = false;
     int nm = 0, cov = 0;
     gptr<const Vrec> src = glob(a.in_verts + ref.off);
-    // lvl2adj has to fit its field (an item of the root takes it from the whole root)
+    // lvl2adj has to fit its field: an item brings it with its record, a root
+    // that a window shortened takes the whole root's (below), more than its own
+    // vertices
     const uint32_t l2_max = sizeof(typename P::pos_t) == 4 ? 0xFFFFFFFFu : P::slab || z.idb == 16 ? 0xFFFFu : 0xFFFu;
+    if (root && !item && (uint32_t)c.g.p->max_d2r > l2_max) return false;
     for (int base = 0; base < t0; base += P::U * WAVE) {
         typedef int v4 __attribute__((ext_vector_type(4)));
         v4 v[P::U];

@@ -128,7 +128,7 @@ struct DevGraph {
     const uint64_t* A1;   // R x rw
     const uint64_t* A2;   // R x rw
     int32_t min_size;
-    int32_t pad;
+    int32_t max_d2r;      // largest |N2(a) n root|
     const uint32_t* orig; // root-local id -> input vertex id
     const int32_t* d2r;   // |N2(a) n root| per root vertex
     const int32_t* d1r;   // |N(a) n root| per root vertex

@@ -896,6 +896,7 @@ int build_instance_impl(const qc_graph* g, double gamma, int ms, Instance& I, hi
     I.dg.A1 = I.A1.as<uint64_t>();
     I.dg.A2 = I.A2.as<uint64_t>();
     I.dg.min_size = ms;
+    I.dg.max_d2r = *std::max_element(I.d2r.begin(), I.d2r.end());
     I.dg.gamma = gamma;
     I.dg.orig = I.d_orig.as<uint32_t>();
     I.dg.d2r = I.d_d2r.as<int32_t>();
