@@ -220,7 +220,8 @@ int enumerate_plain(const Instance& I, const qc_params& p, EnumOut& out, hipStre
     } mx;
     std::vector<TaskRef> batch, kids[2];
     // a launch whose raw sets overflow the stream is made again with half the
-    // tasks (its counters and the stream put back), down to one task
+    // tasks (its counters and the stream put back), down to one task on an empty
+    // stream
     uint32_t most = max_batch;
     DBuf d_keep;
     if ((rc = d_keep.alloc(sizeof(DevStats)))) return rc;
@@ -288,7 +289,7 @@ int enumerate_plain(const Instance& I, const qc_params& p, EnumOut& out, hipStre
         float ms = 0;
         QC_HIP(hipEventElapsedTime(&ms, e0, e1));
         kms += ms;
-        if (ls.error == 1 && !fixed && take > 1 &&
+        if (ls.error == 1 && !fixed && (take > 1 || done.clq.items > 0) &&
             (ls.clq.slots > clq_slots || ls.clq.items > clq_refs)) {
             QC_HIP(hipMemcpyAsync(d_stats.p, d_keep.p, sizeof(DevStats), hipMemcpyDeviceToDevice, s));
             S.refs.insert(S.refs.end(), batch.begin(), batch.end());
