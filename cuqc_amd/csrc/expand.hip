@@ -2561,7 +2561,10 @@ __device__ __attribute__((always_inline)) void wide_split(Ctx& c, Wide<P>& z, co
 // One task or split item.  False, with nothing done, when a degree or lvl2adj
 // does not fit WideLds' fields (WideSlab then runs it; its own are never
 // exceeded).  The caller has checked wide_fits (WideLds) or the slab's size.
-template <class P>
+// CUT: a root may be one that a window shortened (not where the whole root fits
+// the LDS, whose counts fit the fields: 43 registers in memory there, 51 with
+// the check).
+template <class P, bool CUT = true>
 __device__ __attribute__((always_inline)) bool process_wide(Ctx& c, const TaskRef ref, char* lds, uint32_t lds_bytes,
                                                             char* slab) {
     const ExpandArgs& a = *c.a;
@@ -2636,7 +2639,7 @@ __device__ __attribute__((always_inline)) bool process_wide(Ctx& c, const TaskRe
     // that a window shortened takes the whole root's (below), more than its own
     // vertices
     const uint32_t l2_max = sizeof(typename P::pos_t) == 4 ? 0xFFFFFFFFu : P::slab || z.idb == 16 ? 0xFFFFu : 0xFFFu;
-    if (root && !item && (uint32_t)c.g.p->max_d2r > l2_max) return false;
+    if (CUT && root && !item && (uint32_t)c.g.p->max_d2r > l2_max) return false;
     for (int base = 0; base < t0; base += P::U * WAVE) {
         typedef int v4 __attribute__((ext_vector_type(4)));
         v4 v[P::U];
@@ -3051,7 +3054,7 @@ __device__ __attribute__((noinline)) bool process_far(Far* f) {
 template <bool FAR>
 __device__ __attribute__((always_inline)) void process_task(Ctx& c, const TaskRef& ref, char* lds, uint32_t lds_bytes,
                                                             char* slab) {
-    if (wide_fits(c, ref.t, lds_bytes) && process_wide<WideLds>(c, ref, lds, lds_bytes, slab)) return;
+    if (wide_fits(c, ref.t, lds_bytes) && process_wide<WideLds, FAR>(c, ref, lds, lds_bytes, slab)) return;
     if constexpr (!FAR) {
         if (c.lane == 0) atomicOr(c.a->error, 2);
         return;
