@@ -3246,12 +3246,9 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void ex
     c.ph = s_ph;
     if (c.lane == 0) s_st = LStats{0, 0, 0, 0, 0, 0, 0, 0, 0};
     ph_start(c);
-    // consecutive idle polls before the launch is declared stuck (about a
-    // minute of back-off): every wave then leaves with error bit 4
-    constexpr int IDLE_LIMIT = 1 << 24;
     const unsigned long long G = gridDim.x;
-    int idle = 0;       // consecutive empty polls (back-off)
-    int idle_total = 0;
+    int idle = 0;             // consecutive empty polls (back-off)
+    uint32_t idle_total = 0;  // the same, not capped, since the last look that found a working wave
     int sinst = -1;     // instance the wave's counters belong to
     // static order: this wave takes positions blockIdx.x, +G, +2G, ... of
     // the single ring
@@ -3427,29 +3424,35 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void ex
                 // Finished once nothing is pending (no ring task and no busy
                 // wave: a wave counts itself out only when its stack is
                 // empty, after pushing what it made): looked up on every
-                // fourth poll, as is a lost task or another wave's fault
-                // (error bit 4), by one wave in 16, which tells the others
+                // fourth poll by one wave in 16, which tells the others
                 // through a word that is written once: with every idle wave
                 // reading it, the busy ones' adds to the pending word waited.
+                // A task is lost (error bit 4, and every wave leaves) when
+                // tasks are pending and no wave works, for longer than one
+                // that waits for its position takes to see it.  How long this
+                // wave has waited says nothing: tasks may go to other rings,
+                // or one wave run a root that is not split.
                 // Polls are relaxed: an acquire invalidates the CU's vector L1
                 // under the waves still working.
-                if ((idle_total & 3) == 0) {
-                    int leave = 0;
+                if ((idle_total++ & 3u) == 0) {
+                    int look = 0;  // 1: leave, 2: a wave works
                     if (c.lane == 0) {
                         if ((blockIdx.x & 15u) == 0) {
                             const unsigned long long pd = __hip_atomic_load(a.pending, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                            const int er = __hip_atomic_load(a.error, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                            leave = (pd & 0xFFFFFFFFull) == 0 || (er & 4) != 0;
-                            if (leave) __hip_atomic_store(a.done, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                            int er = __hip_atomic_load(a.error, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                            if ((pd >> 32) < G)
+                                look = 2;
+                            else if ((uint32_t)pd != 0 && idle_total / 4 >= a.idle_limit)
+                                er |= atomicOr(a.error, 4) | 4;
+                            if ((uint32_t)pd == 0 || (er & 4) != 0) look = 1;
+                            if (look == 1) __hip_atomic_store(a.done, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                         } else {
-                            leave = __hip_atomic_load(a.done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
+                            look = __hip_atomic_load(a.done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
                         }
                     }
-                    if (rdlane(leave, 0)) break;
-                }
-                if (++idle_total >= IDLE_LIMIT) {
-                    if (c.lane == 0) atomicOr(a.error, 4);
-                    break;
+                    look = rdlane(look, 0);
+                    if (look == 1) break;
+                    if (look == 2) idle_total = 1;
                 }
                 idle = idle < 8 ? idle + 1 : 8;
                 for (int k = 0; k < idle; k++) __builtin_amdgcn_s_sleep(16);

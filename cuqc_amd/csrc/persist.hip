@@ -410,6 +410,8 @@ int enumerate_persistent(const Instance* const* insts, const qc_params* params, 
         A.q_shards = nr;
         A.n_roots = (int32_t)roots.size();
         A.split_waves = grid;
+        A.idle_limit = 1u << 22;  // (about a minute of back-off)
+        if (const char* il = getenv("QCMINE_IDLE_LIMIT")) A.idle_limit = (uint32_t)std::max(1, atoi(il));  // tests
         A.cm_w = cost ? d_cmw.as<uint16_t>() : nullptr;
         A.cm_norm = cost ? d_cmn.as<float>() : nullptr;
         A.q_cap = q_cap;

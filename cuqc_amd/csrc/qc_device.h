@@ -194,6 +194,8 @@ struct ExpandArgs {
     int32_t split_chunk;             // branches per split item (0: no splitting)
     int32_t all_bounds;              // level form: slot bounds also for children that the depth window leaves unwritten
     uint32_t split_waves;            // waves a root's items are meant for (with n_roots)
+    uint32_t idle_limit;             // persistent mode: looks in a row at a launch with tasks and no working wave
+                                     // (every fourth poll) after which it is given up
     uint32_t split_min_t;            // split tasks above this size
     uint32_t cost_min_t;             // cost order: children of at most this size skip the model (bucket 0)
     TaskRef* q_refs;
