@@ -494,8 +494,7 @@ __device__ __attribute__((always_inline)) void pool_free(Ctx& c, unsigned long l
 // Claims up to n (<= 64) consecutive free cells of ring b for producers
 // (whole wave; lane j checks the cell of position pos + j).  Returns how
 // many were claimed (0: the ring is full, or max_tries attempts lost to
-// other producers), their first position in *pos.  With a trace the ring
-// must not wrap (positions index the trace rows).
+// other producers), their first position in *pos.
 __device__ __attribute__((always_inline)) int ring_claim(Ctx& c, int b, int n, unsigned long long* pos_out,
                                                         int max_tries = 1 << 16) {
     const ExpandArgs& a = *c.a;
@@ -512,11 +511,10 @@ __device__ __attribute__((always_inline)) int ring_claim(Ctx& c, int b, int n, u
         const uint64_t fullm = ballot(c.lane < n && sq < p);
         int k = freem == ~0ull ? WAVE : __builtin_ctzll(~freem);
         k = min(k, n);
-        if (a.trace_feat && pos + (unsigned long long)k > a.q_cap) k = (int)(pos < a.q_cap ? a.q_cap - pos : 0);
         if (k == 0) {
             // lane 0's cell still holds the entry of the previous lap: full;
             // otherwise the tail moved under us
-            if ((fullm & 1ull) || (a.trace_feat && pos >= a.q_cap)) return 0;
+            if (fullm & 1ull) return 0;
             continue;
         }
         int ok = 0;
@@ -533,6 +531,21 @@ __device__ __attribute__((always_inline)) int ring_claim(Ctx& c, int b, int n, u
         }
     }
     return 0;
+}
+
+// The same with a trace, whose one ring must not wrap (positions index the
+// trace rows): its cells are free for their only lap, and one add takes the
+// positions.  Every task goes through the ring then: 1,024 waves that tried to
+// move its tail by compare and swap for each child spent 77% of a co-expression
+// window's time on it.
+__device__ __forceinline__ int ring_claim_trace(Ctx& c, int n, unsigned long long* pos_out) {
+    const ExpandArgs& a = *c.a;
+    unsigned long long pos = 0;
+    if (c.lane == 0)
+        pos = __hip_atomic_fetch_add(&a.q_tail[0], (unsigned long long)n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    pos = rdlane64(pos, 0);
+    *pos_out = pos;
+    return pos + (unsigned long long)n <= a.q_cap ? n : 0;
 }
 
 // The ring a producer's next task goes to: this wave's own shard when waves wait
@@ -620,7 +633,7 @@ __device__ __attribute__((always_inline)) bool push_ref(Ctx& c, const TaskRef& r
         if (ring) {
             const int rg = ring_for(c);
             unsigned long long pos = 0;
-            if (ring_claim(c, rg, 1, &pos) == 1) {
+            if ((a.trace_feat ? ring_claim_trace(c, 1, &pos) : ring_claim(c, rg, 1, &pos)) == 1) {
                 const unsigned long long gi = (unsigned long long)rg * a.q_cap + pos % a.q_cap;
                 if (c.lane == 0) {
                     __hip_atomic_fetch_add(a.pending, 1ull, __ATOMIC_RELAXED,
@@ -2542,7 +2555,8 @@ __device__ __attribute__((always_inline)) void wide_split(Ctx& c, Wide<P>& z, co
         unsigned long long pos = 0;
         int waiting = 0;
         const int rg = ring_for(c, &waiting);
-        const int k = ring_claim(c, rg, min(n_items - done, waiting > 0 ? min(waiting, WAVE) : WAVE), &pos);
+        const int want = min(n_items - done, waiting > 0 ? min(waiting, WAVE) : WAVE);
+        const int k = a.trace_feat ? ring_claim_trace(c, want, &pos) : ring_claim(c, rg, want, &pos);
         if (k == 0) break;
         if (c.lane == 0)
             __hip_atomic_fetch_add(a.pending, (unsigned long long)k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
