@@ -231,11 +231,13 @@ int enumerate_persistent(const Instance* const* insts, const qc_params* params, 
         }
     }
     // every wave must be resident: the queue hand-off waits on producers
-    // (static order and traces send every task through one ring: with 8 waves per
-    // CU instead of 4 a power-law window of 252,000 small tasks took 89 ms instead
-    // of 61, its trace 3.5 s instead of 2.4; a co-expression window of large
-    // tasks, static, 5.9 instead of 6.8)
-    const int max_per_cu = stat || p.trace ? 4 : 16;
+    // (static order sends every task through one ring: with 8 waves per CU instead
+    // of 4 a power-law window of 252,000 small tasks took 89 ms instead of 61; a
+    // co-expression window of large tasks 5.9 instead of 6.8.  Traces use one ring
+    // too, but take their places with one add: with 4 waves per CU instead of 8
+    // that power-law window took 21.6 ms instead of 23.3, the first branches of a
+    // power-law graph 212 instead of 127.)
+    const int max_per_cu = stat ? 4 : 16;
     uint32_t grid = (uint32_t)std::max(1, n_cu) * (uint32_t)std::max(1, std::min(per_cu, max_per_cu));
     if (p.workgroups > 0) grid = std::min<uint32_t>(grid, (uint32_t)p.workgroups);
 
