@@ -201,6 +201,13 @@ int enumerate_persistent(const Instance* const* insts, const qc_params* params, 
     const int wide_req = p.lds_wide < 0 ? 0 : (p.lds_wide > 0 ? (int)p.lds_wide : 512);
     const uint32_t wide = (uint32_t)std::min(std::min(wide_req, 1024), maxR);
     size_t lds_b = std::max<size_t>(MIN_WAVE_LDS, wide_lds_bytes(wide, (uint32_t)maxrw));
+    // (static order sends every task through one ring: with 8 waves per CU instead
+    // of 4 a power-law window of 252,000 small tasks took 89 ms instead of 61; a
+    // co-expression window of large tasks 5.9 instead of 6.8.  Traces use one ring
+    // too, but take their places with one add: with 4 waves per CU instead of 8
+    // that power-law window took 21.6 ms instead of 23.3, the first branches of a
+    // power-law graph 212 instead of 127.)
+    const int max_per_cu = stat ? 4 : 16;
     QC_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, 64, lds_b));
     {
         // A workgroup's LDS (static + dynamic) is allocated in granules of
@@ -217,7 +224,7 @@ int enumerate_persistent(const Instance* const* insts, const qc_params* params, 
         QC_HIP(hipFuncGetAttributes(&fa, kern));
         const size_t st = fa.sharedSizeBytes;
         auto alloc = [&](size_t dyn) { return (dyn + st + LDS_GRANULE - 1) / LDS_GRANULE * LDS_GRANULE; };
-        per_cu = std::min(per_cu, (int)((size_t)lds_cu / alloc(lds_b)));
+        per_cu = std::min({per_cu, (int)((size_t)lds_cu / alloc(lds_b)), max_per_cu});
         if (per_cu > 0) {
             // the resident waves leave part of the CU's LDS unused: the
             // dynamic region grows to the most that keeps per_cu waves
@@ -231,14 +238,7 @@ int enumerate_persistent(const Instance* const* insts, const qc_params* params, 
         }
     }
     // every wave must be resident: the queue hand-off waits on producers
-    // (static order sends every task through one ring: with 8 waves per CU instead
-    // of 4 a power-law window of 252,000 small tasks took 89 ms instead of 61; a
-    // co-expression window of large tasks 5.9 instead of 6.8.  Traces use one ring
-    // too, but take their places with one add: with 4 waves per CU instead of 8
-    // that power-law window took 21.6 ms instead of 23.3, the first branches of a
-    // power-law graph 212 instead of 127.)
-    const int max_per_cu = stat ? 4 : 16;
-    uint32_t grid = (uint32_t)std::max(1, n_cu) * (uint32_t)std::max(1, std::min(per_cu, max_per_cu));
+    uint32_t grid = (uint32_t)std::max(1, n_cu) * (uint32_t)std::max(1, per_cu);
     if (p.workgroups > 0) grid = std::min<uint32_t>(grid, (uint32_t)p.workgroups);
 
     const size_t slab_b = wide_slab_bytes((uint32_t)maxR);
@@ -584,7 +584,7 @@ int enumerate_persistent(const Instance* const* insts, const qc_params* params, 
                                       "lu", "degupd", "classify", "critical", "compact", "hist", "pool", "pop", "give", "sync", "tiny"};
         double tot = 0;
         for (int k = 0; k < PH_CYCLES; k++) tot += (double)ph[k];
-        fprintf(stderr, "[qcmine] phases (grid %u waves, %.3g wave-cycles):", grid, tot);
+        fprintf(stderr, "[qcmine] phases (grid %u waves, %zu B of LDS each, %.3g wave-cycles):", grid, lds_b, tot);
         for (int k = 0; k < PH_CYCLES; k++)
             fprintf(stderr, " %s %.1f%%", names[k], 100.0 * ph[k] / (tot > 0 ? tot : 1));
         fprintf(stderr, "; tasks from own stacks %llu, from rings %llu, handed over %llu\n", ph[PH_N_OWN],
