@@ -12,10 +12,13 @@ it):
 * ``split_min``   split only tasks above this many vertices (0: the library
                   default, the LDS tile for a single graph and 512 for a
                   batch; values below the LDS tile mean the tile);
-* ``mid_tile``    accepted by the library, without effect;
 * ``lds_wide``    the LDS of a wave holds tasks of up to this size at least
-                  (-1: what 16 KB hold, 0: 512);
-* ``workgroups``  resident waves of the persistent launch (0: as many as fit).
+                  (0: 512, which it nearly always does in any case);
+* ``workgroups``  resident waves of the persistent launch (0: as many as fit, 2,048 on
+                  256 CUs).
+
+``mid_tile`` is accepted by the library, without effect: a schedule keeps it
+(cached ones name it), the search does not vary it.
 
 The search is coordinate descent from the library defaults, one parameter at
 a time, repeated while a full sweep improves the time by more than
@@ -38,13 +41,12 @@ from dataclasses import asdict, dataclass, field
 SPACE: dict[str, list[int]] = {
     "split_chunk": [16, 32, 64, 128, -1],
     "split_min": [0, 1, 512, 1024],
-    "mid_tile": [0, 512, 1024],
-    "lds_wide": [-1, 256, 512, 1024],
+    "lds_wide": [0, 1024],
     "lds_tile": [64, 128, 256],
-    "workgroups": [1024, 2048, 3072, 0],
+    "workgroups": [1024, 0],
 }
 DEFAULT = {"lds_tile": 128, "split_chunk": 64, "split_min": 0, "mid_tile": 0, "lds_wide": 0, "workgroups": 0}
-ORDER = ("split_chunk", "lds_wide", "split_min", "mid_tile", "lds_tile", "workgroups")
+ORDER = ("split_chunk", "lds_wide", "split_min", "lds_tile", "workgroups")
 
 _INVARIANT = ("tasks", "branches", "children", "raw_cliques", "w_adj", "beyond")
 

@@ -77,7 +77,9 @@ typedef struct qc_params {
                                 0 = lds_tile for a single graph, 512 for a batch */
     int32_t mid_tile;        /* accepted; has no effect */
     int32_t lds_wide;        /* persistent mode: the LDS of a wave holds tasks of up to this size
-                                (<= 1024) at least; 0 = 512, < 0 = what 16 KB hold */
+                                (<= 1024) at least, for fewer resident waves if need be; 0 = 512,
+                                < 0 = no such size. The waves that are resident share the CU's
+                                LDS in any case (about 900 vertices each with 8 of them) */
 } qc_params;
 
 typedef struct qc_stats {

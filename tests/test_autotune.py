@@ -79,3 +79,24 @@ def test_lucky_single_timing_does_not_leave_the_defaults(monkeypatch):
     s = at.tune([G()], [0.9], [10], reps=1)
     assert s.split_chunk == at.DEFAULT["split_chunk"]
     assert s.kernel_ms == 100.0
+
+
+def test_every_candidate_is_another_launch(monkeypatch):
+    # options without effect are not timed against themselves
+    tried = []
+
+    def fake_mine(g, ga, ms, sched, mode, window, **kw):
+        tried.append((kw["mid_tile"], 512 if kw["lds_wide"] <= 512 else kw["lds_wide"], kw["split_chunk"], kw["split_min"],
+                      kw["lds_tile"], kw["workgroups"]))
+        return _Res(100.0)
+
+    import cuqc_amd
+    monkeypatch.setattr(cuqc_amd, "mine", fake_mine)
+
+    class G:
+        def checksum(self):
+            return 1
+
+    at.tune([G()], [0.9], [10], reps=1)
+    assert len(set(tried)) == len(tried)
+    assert {t[0] for t in tried} == {0}
