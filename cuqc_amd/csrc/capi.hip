@@ -92,14 +92,33 @@ struct HostPool {
     std::vector<std::pair<size_t, void*>> free;  // pinned blocks, oldest first
     size_t free_bytes = 0, pinned_bytes = 0;     // waiting, and pinned in all
     // the oldest waiting blocks go back to HIP until at most `keep` bytes wait
-    void trim_locked(size_t keep) {
-        size_t n = 0;
-        for (; free_bytes > keep; n++) {
-            free_bytes -= free[n].first;
-            pinned_bytes -= free[n].first;
-            (void)hipHostFree(free[n].second);
+    // (outside the lock: results are freed from any thread, and unpinning 100 MB
+    // takes milliseconds that no other call has to wait for)
+    void trim(size_t keep) {
+        for (;;) {
+            std::pair<size_t, void*> b;
+            {
+                std::lock_guard<std::mutex> lock(mu);
+                if (free_bytes <= keep) return;
+                b = free.front();
+                free.erase(free.begin());
+                free_bytes -= b.first;
+            }
+            (void)hipHostFree(b.second);
+            std::lock_guard<std::mutex> lock(mu);
+            pinned_bytes -= b.first;
         }
-        free.erase(free.begin(), free.begin() + (std::ptrdiff_t)n);
+    }
+    // room for a new block under the limit, counted as pinned
+    bool reserve(size_t want) {
+        std::lock_guard<std::mutex> lock(mu);
+        if (pinned_bytes + want > HOST_PINNED_MAX) return false;
+        pinned_bytes += want;
+        return true;
+    }
+    void unreserve(size_t want) {
+        std::lock_guard<std::mutex> lock(mu);
+        pinned_bytes -= want;
     }
 };
 HostPool& host_pool() {
@@ -116,42 +135,44 @@ int HostBuf::alloc(size_t bytes) {
         while (step * 16 < bytes) step <<= 1;
         const size_t want = (bytes + step - 1) / step * step;
         HostPool& h = host_pool();
-        std::lock_guard<std::mutex> lock(h.mu);
-        size_t best = h.free.size();
-        for (size_t i = 0; i < h.free.size(); i++)
-            if (h.free[i].first >= want && h.free[i].first <= 4 * want &&
-                (best == h.free.size() || h.free[i].first < h.free[best].first))
-                best = i;
-        if (best < h.free.size()) {
-            cap = h.free[best].first;
-            p = h.free[best].second;
-            h.free_bytes -= cap;
-            h.free.erase(h.free.begin() + (std::ptrdiff_t)best);
-            pinned = true;
-            return QC_OK;
+        {
+            std::lock_guard<std::mutex> lock(h.mu);
+            size_t best = h.free.size();
+            for (size_t i = 0; i < h.free.size(); i++)
+                if (h.free[i].first >= want && h.free[i].first <= 4 * want &&
+                    (best == h.free.size() || h.free[i].first < h.free[best].first))
+                    best = i;
+            if (best < h.free.size()) {
+                cap = h.free[best].first;
+                p = h.free[best].second;
+                h.free_bytes -= cap;
+                h.free.erase(h.free.begin() + (std::ptrdiff_t)best);
+                pinned = true;
+                return QC_OK;
+            }
         }
         // a new block: waiting ones make room for it under the limit
-        if (h.pinned_bytes + want > HOST_PINNED_MAX) h.trim_locked(0);
-        if (h.pinned_bytes + want <= HOST_PINNED_MAX) {
+        bool room = h.reserve(want);
+        if (!room) {
+            h.trim(0);
+            room = h.reserve(want);
+        }
+        if (room) {
             void* q = nullptr;
             if (hipHostMalloc(&q, want, hipHostMallocDefault) == hipSuccess && q) {
                 p = q;
                 cap = want;
                 pinned = true;
-                h.pinned_bytes += want;
                 return QC_OK;
             }
             (void)hipGetLastError();
+            h.unreserve(want);
         }
     }
     p = malloc(bytes ? bytes : 1);
     if (!p) {
         // give the waiting blocks back and try once more
-        HostPool& h = host_pool();
-        {
-            std::lock_guard<std::mutex> lock(h.mu);
-            h.trim_locked(0);
-        }
+        host_pool().trim(0);
         p = malloc(bytes ? bytes : 1);
     }
     if (!p) {
@@ -167,15 +188,22 @@ void HostBuf::release() {
     if (p && !pinned) ::free(p);
     if (p && pinned) {
         HostPool& h = host_pool();
-        std::lock_guard<std::mutex> lock(h.mu);
-        try {
-            h.free.push_back({cap, p});
-            h.free_bytes += cap;
-        } catch (...) {  // (no memory for the list: the block goes back to HIP)
-            h.pinned_bytes -= cap;
-            (void)hipHostFree(p);
+        bool kept = true;
+        {
+            std::lock_guard<std::mutex> lock(h.mu);
+            try {
+                h.free.push_back({cap, p});
+                h.free_bytes += cap;
+            } catch (...) {  // (no memory for the list: the block goes back to HIP)
+                kept = false;
+            }
         }
-        h.trim_locked(HOST_POOL_MAX);
+        if (kept) {
+            h.trim(HOST_POOL_MAX);
+        } else {
+            (void)hipHostFree(p);
+            h.unreserve(cap);
+        }
     }
     p = nullptr;
     cap = 0;
