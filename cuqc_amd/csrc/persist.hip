@@ -268,7 +268,12 @@ int enumerate_persistent(const Instance* const* insts, const qc_params* params, 
     const bool trace = p.trace != 0;
     const int nr = stat || trace ? 1 : Q_SHARDS;
     const uint64_t max_q = (1ull << 28) / nr;
-    const uint64_t max_clq = std::min<uint64_t>(budget / 16 / 4, (uint64_t)1 << 31);
+    // (the waves take slots of the clique stream several at a time and leave less
+    // than a quarter of them unused, see clq_reserve: the stream may grow to what
+    // a search of `raw_max` raw vertices takes at most)
+    auto clq_stream = [&](uint64_t verts) { return verts + verts / 3 + (uint64_t)grid * CLQ_SLOTS; };
+    const uint64_t raw_max = std::min<uint64_t>(budget / 16 / 4, (uint64_t)1 << 31);
+    const uint64_t max_clq = clq_stream(raw_max);
     uint64_t pool_cap = fixed_tasks ? p.task_capacity
                                     : std::max<uint64_t>(ws.pool_cap, std::min<uint64_t>(max_pool, 1ull << 26));
     pool_cap = std::max<uint64_t>(pool_cap, root_verts.size() + 1024);
@@ -278,11 +283,10 @@ int enumerate_persistent(const Instance* const* insts, const qc_params* params, 
                                    : std::max<uint64_t>(ws.clq_slots, std::min<uint64_t>(max_clq, 1ull << 24));
     uint64_t clq_refs = std::max<uint64_t>(ws.clq_refs_cap, clq_slots / 8 + 1024);
     // a caller's clique capacity bounds the raw sets' vertices (and their
-    // number); the waves take refs and slots several at a time, so the stream
-    // itself is larger by what they can leave unused
+    // number); the stream itself is larger by what the waves can leave unused
     const uint64_t fixed_slots = clq_slots, fixed_refs = clq_slots / 8 + 1024;
     if (fixed_clq) {
-        clq_slots = clq_slots + clq_slots / 3 + (uint64_t)grid * CLQ_SLOTS;
+        clq_slots = clq_stream(clq_slots);
         clq_refs = std::max<uint64_t>(clq_refs, fixed_refs + (uint64_t)grid * CLQ_REFS);
     }
     // private stacks: a power of two of refs per wave (the stack is a ring
@@ -345,10 +349,20 @@ int enumerate_persistent(const Instance* const* insts, const qc_params* params, 
     float first_ms = 0;
     uint64_t last_items = 0;
     uint64_t raw_k = 0, raw_nv = 0;  // raw sets and their vertices, over all instances
+    // (a caller's capacity that only fits the memory without the waves' part is
+    // taken as it is: enough unless the raw sets come close to it)
+    auto clq_verts_alloc = [&]() -> int {
+        int e = ensure(ws.clq_verts, clq_slots * 4);
+        if (e == QC_ENOMEM && fixed_clq && clq_slots > fixed_slots) {
+            clq_slots = fixed_slots;
+            e = ensure(ws.clq_verts, clq_slots * 4);
+        }
+        return e;
+    };
     for (int attempt = 0;; attempt++) {
         if ((rc = ensure(ws.pool, pool_cap * sizeof(Vrec))) || (rc = ensure(ws.q, nr * q_cap * sizeof(TaskRef))) ||
             (rc = ensure(ws.seq, nr * q_cap * 8)) || (rc = ensure(ws.clq_refs, clq_refs * sizeof(CliqueRef))) ||
-            (rc = ensure(ws.clq_verts, clq_slots * 4)) || (rc = ensure(ws.priv, (size_t)grid * priv_cap * sizeof(TaskRef))) ||
+            (rc = clq_verts_alloc()) || (rc = ensure(ws.priv, (size_t)grid * priv_cap * sizeof(TaskRef))) ||
             (rc = ensure(ws.pbkt, (size_t)grid * priv_cap)))
             return rc;
         if (trace && ((rc = d_tfeat.alloc(q_cap * 12 * sizeof(float))) || (rc = d_tpar.alloc(q_cap * 8)) ||
