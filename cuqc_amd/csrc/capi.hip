@@ -1,5 +1,6 @@
 // capi.hip -- the C ABI of include/qcmine.h.
 
+#include <algorithm>
 #include <atomic>
 #include <chrono>
 #include <cmath>
@@ -292,6 +293,12 @@ int check_params(const qc_params* p) {
     if (p->order == QC_ORDER_COST && !p->cost_model) {
         set_error("cost-ordered scheduling needs a cost model");
         return QC_EINVAL;
+    }
+    // (far above any device's memory, far below where their bytes overflow)
+    if (p->task_capacity > 1ull << 48 || p->clique_capacity > 1ull << 48) {
+        set_error("a capacity of %llu does not fit device memory",
+                  (unsigned long long)std::max(p->task_capacity, p->clique_capacity));
+        return QC_ENOMEM;
     }
     return QC_OK;
 }
