@@ -572,7 +572,7 @@ __device__ __attribute__((always_inline)) int ring_for(Ctx& c, int* waiting = nu
     return r;
 }
 
-// Publishes positions [pos, pos + k) of bucket b (their refs are written):
+// Publishes positions [pos, pos + k) of ring b (their refs are written):
 // one release fence for the wave's record and ref stores, then the
 // sequence words (lanes < k).
 __device__ __forceinline__ void ring_publish(Ctx& c, int b, unsigned long long pos, int k) {
@@ -723,7 +723,6 @@ constexpr uint32_t TINY_MAX = WAVE;
 constexpr int TINY_EX_MAX = 8000;  // largest exdeg the word holds (stale exdegs can pass the task's size)
 constexpr int TINY_EX_MIN = -64;   // smallest at load: a subtree lowers an exdeg by at most 63 more
 constexpr int TINY_BIAS = 128;
-constexpr uint32_t TINY_ENTRY = WAVE * 4;  // bytes of a stack entry
 
 // State word of a vertex: [12:0] exdeg + 128, [18:13] indeg, [24:19] order
 // (lvl2adj, or 63 - position for a task loaded from a record), [25] member,
@@ -3306,7 +3305,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void ex
             if (!a.static_sched && c.ptop - c.pbot > own) {
                 // more waves wait for work than the rings hold: hand over
                 // the oldest (shallowest, so largest) records, up to 16 at
-                // once, into the bucket of the oldest one.  The rings hold
+                // once, to one ring (ring_for).  The rings hold
                 // pending - (G - hungry) tasks; handing over more than the
                 // waiting waves take turns the search breadth first and
                 // multiplies the live records.

@@ -1,10 +1,11 @@
 // persist.hip -- persistent-kernel enumeration: one launch for one or many
 // mining instances.
 //
-// The roots of all instances seed one device FIFO queue; every wave of
-// expand_persistent pops task refs (tagged with their instance), expands
-// them against that instance's tables and pushes the children it writes,
-// until the pending-task counter drops to zero.  There is no host round trip
+// The roots of all instances are dealt over device rings; every wave of
+// expand_persistent takes task refs (tagged with their instance) from them,
+// expands them against that instance's tables, keeps the children it writes on
+// a stack of its own and hands some to the rings while other waves wait, until
+// nothing is pending.  There is no host round trip
 // between levels (the reference returns to the host after every level,
 // main.cu:606-678).  The reset of the queue state and the launch are captured
 // in a hipGraph; the reset is a kernel (no memset nodes), so the graph can be
@@ -29,8 +30,9 @@ extern template __global__ void expand_persistent<true>(const ExpandArgs*);
 // Queue state for a fresh run: the roots dealt over the nr rings (root i
 // at position i / nr of ring i mod nr, published), every other cell free for
 // its first lap, the free lists empty, counters reset.  ctr = heads[nr],
-// tails[nr], pool top, hungry|pending, overflow, done, QSTRIDE words apart.  Root records sit at the start of the
-// pool; allocated blocks start at the next unit boundary.
+// tails[nr], pool top, hungry|pending, overflow, done, QSTRIDE words apart.
+// Root records sit at the start of the pool; allocated blocks start at the next
+// unit boundary.
 __global__ void persist_reset(const TaskRef* __restrict__ roots, uint32_t nroots, const Vrec* __restrict__ root_verts,
                               uint64_t root_slots, TaskRef* q_refs, unsigned long long* q_seq, uint64_t q_cap,
                               uint32_t nr, Vrec* pool, unsigned long long* ctr, unsigned long long* fl_head,
@@ -595,7 +597,7 @@ int enumerate_persistent(const Instance* const* insts, const qc_params* params, 
         unsigned long long ph[PH_COUNT];
         QC_HIP(hipMemcpy(ph, d_phase.p, sizeof(ph), hipMemcpyDeviceToHost));
         static const char* names[] = {"load", "lookahead", "remove", "add", "prune", "child", "prepare", "idle",
-                                      "lu", "degupd", "classify", "critical", "compact", "hist", "pool", "pop", "give", "sync", "tiny"};
+                                      "lu", "degupd", "compact", "critical", "pool", "pop", "give", "sync", "tiny"};
         double tot = 0;
         for (int k = 0; k < PH_CYCLES; k++) tot += (double)ph[k];
         fprintf(stderr, "[qcmine] phases (grid %u waves, %zu B of LDS each, %.3g wave-cycles):", grid, lds_b, tot);

@@ -39,12 +39,6 @@ __host__ __device__ inline int pool_class(uint32_t nvrec, uint32_t& units) {
     return 8 + (e - 3) * 4 + (int)(k - 1);
 }
 
-__host__ __device__ constexpr uint32_t pow2_at_least(uint32_t x) {
-    uint32_t p = 1;
-    while (p < x) p <<= 1;
-    return p;
-}
-
 // LDS bytes of a task of t vertices: its arrays (20 bytes a vertex), two bit
 // masks over its positions, and three rows of rw words when they are staged
 __host__ __device__ __attribute__((always_inline)) constexpr uint32_t wide_T(uint32_t t) { return (t + 63u) & ~63u; }
@@ -264,10 +258,8 @@ enum PhaseId {
     PH_IDLE,          // persistent form: waiting for work (empty polls and back-off)
     PH_LU,            // LU bounds and member checks
     PH_DEGUPD,        // degree-pruning exdeg updates
-    PH_COMPACT,       // degree-pruning classification
+    PH_COMPACT,       // degree-pruning classification and compaction
     PH_CRIT,          // critical-vertex step
-    PH_MOVE,          // degree-pruning compaction of the kept candidates
-    PH_HIST,          // candidate indegree tables for the LU bounds
     PH_POOL,          // persistent form: record blocks taken and given back, task refs pushed
     PH_POP,           // persistent form: taking the next task (own stack, rings)
     PH_GIVE,          // persistent form: deciding on and making hand-overs from the own stack
