@@ -3,7 +3,6 @@ however many the order of the search allows."""
 import re
 
 import pytest
-import torch
 
 import cuqc_amd as qc
 from tests.graphs import planted
@@ -11,13 +10,16 @@ from tests.graphs import planted
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("form", [dict(), dict(scheduling=1), dict(trace=True)], ids=["dynamic", "static", "trace"])
-def test_lds_of_a_cu_is_used(form, monkeypatch, capfd):
+def test_lds_of_a_cu_is_used(monkeypatch, capfd):
     monkeypatch.setenv("QCMINE_PHASES", "1")
     g = qc.Graph.from_csr(*planted(700, 0.15, [40], 0.95, 43))
-    qc.mine(g, 0.6, 20, window=(0, 1, 1), mode="persistent", **form)
-    m = re.search(r"grid (\d+) waves, (\d+) B of LDS each", capfd.readouterr().err)
-    per_cu = int(m[1]) // torch.cuda.get_device_properties(0).multi_processor_count
-    # (160 KB a CU in granules of 1,280 B, less 1.1 KB of static LDS a wave)
-    assert per_cu * (int(m[2]) + 1120 + 1280 + 256) >= 160 * 1024
-    assert per_cu * (int(m[2]) + 1120) <= 160 * 1024
+    lds = {}
+    for order, form in (("dynamic", dict()), ("static", dict(scheduling=1)), ("trace", dict(trace=True))):
+        qc.mine(g, 0.6, 20, window=(0, 1, 1), mode="persistent", **form)
+        m = re.search(r"grid (\d+) waves, (\d+) B of LDS each", capfd.readouterr().err)
+        lds[order] = (int(m[1]), int(m[2]))
+    # (with 1.1 KB of static LDS a wave, in granules of 1,280 B a workgroup)
+    whole = lds["dynamic"][0] * (lds["dynamic"][1] + 1120)
+    for waves, each in lds.values():
+        assert 0.95 * whole <= waves * (each + 1120) <= 1.05 * whole
+    assert lds["static"][0] < lds["dynamic"][0]
